@@ -1,5 +1,5 @@
-// Autotuner: picks the block size of the density, force and reorder passes,
-// the keys per thread of the sort's digit passes, whether density and force
+// Autotuner: picks the block size of the density and force passes (and, of
+// the radix sort, the gather's block and the keys per thread of the digit passes), whether density and force
 // run as persistent blocks over tile queues and whether the force and
 // density passes stage their rows in LDS, by timing each candidate
 // with HIP events on the handle's own state.  The state is saved first and
@@ -100,8 +100,9 @@ extern "C" int sph_autotune(sph_handle* h) {
                    {&best.reorder_block, blocks, 4, SPH_PASS_REORDER},
                    {&best.sort_items, items, 4, SPH_PASS_SORT}};
     for (const Axis& ax : axes) {
-        // Keys per thread only shape the radix sort's digit passes.
-        if (ax.field == &best.sort_items && best.sort_mode != kSortRadix) continue;
+        // The gather's block and the keys per thread only shape the radix sort.
+        if ((ax.field == &best.sort_items || ax.field == &best.reorder_block) && best.sort_mode != kSortRadix)
+            continue;
         double best_ms = 1e30;
         int best_v = *ax.field;
         for (int c = 0; c < ax.ncand; ++c) {

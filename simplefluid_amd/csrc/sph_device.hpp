@@ -5,12 +5,13 @@
 //                                sorted order pos.w = p/rho^2 and vel.w = 1/rho
 //                                (written by the density pass for the force pass)
 //   id[2]           uint32 x N   original particle id, state / sorted order
-//   key0, rank0     uint32 x N   cell key of the state positions and the slot taken
-//                                in its cell count (written by integrate)
-//   sort ping-pong  2 x (uint32 key + uint32 value) x N (radix mode)
-//   count           uint32 x C+2T particles per cell, then per scan tile of 4096 cells
-//                                (atomic, built by the integrate pass), then the
+//   key0            uint32 x N   cell key of the state positions (written by integrate)
+//   head            uint32 x C+2T per cell, the newest run of particles that entered it
+//                                (0: none; built by the integrate pass, cleared by the
+//                                sort), then particles per tile of 1024 cells, then the
 //                                exclusive scan of the tile sums
+//   next            uint32 x N   per run (at its first particle), the cell's run before it
+//   radix ping-pong 2 x (uint32 key + uint32 value) x N (radix mode)
 //   cstart          uint32 x C+1 lower-bound cell-start table: cstart[c] = #particles with key < c
 //   rho             float  x N   density (sorted order)
 //   mask            uint32 x 9N  neighbour bits, row-major [row][particle] (layout at
@@ -332,41 +333,63 @@ __device__ __forceinline__ uint32_t cell_key(const SceneConst& sc, float x, floa
     return sc.cell_offset + ((uint32_t)cz * (uint32_t)sc.G[1] + (uint32_t)cy) * (uint32_t)sc.G[0] + (uint32_t)cx;
 }
 
-// Atomic add of each active lane's 1 to arr[idx], one atomic per run of
-// equal idx in consecutive lanes.  Returns the slot this lane took (the old
-// value plus its place in the run).  All lanes of the wave must call it;
-// `active` marks the lanes that hold a particle.
-__device__ __forceinline__ uint32_t run_add(uint32_t* __restrict__ arr, uint32_t idx, bool active) {
+// Cells per tile of the sort (1024): the integrate pass also sums particles
+// per tile, so every sort block finds its prefix without waiting.
+constexpr uint32_t kTileShift = 10;
+constexpr uint32_t kTileCells = 1u << kTileShift;
+
+// Runs.  A cell's members are kept as a chain of runs: consecutive particles
+// of one wave with the same key, at most 15 of them so that a run packs into
+// one word (first particle in 28 bits, length in 4; 0 is the chain's end).
+// Lanes follow the last sorted order, so a cell mostly has one or two runs.
+constexpr uint32_t kRunMax = 15;
+constexpr uint32_t kRunMask = (1u << 28) - 1u;
+__device__ __forceinline__ uint32_t run_first(uint32_t r) { return r & kRunMask; }
+__device__ __forceinline__ uint32_t run_len(uint32_t r) { return r >> 28; }
+
+// Lane masks of the wave's runs of equal v (active lanes only).  first: this
+// lane starts one; end: the lane after the last of this lane's run.
+struct LaneRun {
+    bool first;
+    int leader, end;
+};
+__device__ __forceinline__ LaneRun lane_run(uint32_t v, bool active) {
     const int lane = (int)(threadIdx.x & 63u);
-    const uint32_t kk = active ? idx : 0xffffffffu;
+    const uint32_t kk = active ? v : 0xffffffffu;
     const uint32_t prev = __shfl_up(kk, 1, 64);
-    const bool start = active && (lane == 0 || prev != kk);
-    const uint64_t starts = __ballot(start);
+    LaneRun r;
+    r.first = active && (lane == 0 || prev != kk);
+    const uint64_t starts = __ballot(r.first);
     const uint64_t act = __ballot(active);
-    // Leader of this lane's run: the highest run start at or below the lane.
-    const uint64_t le = starts & (lane == 63 ? ~0ull : ((2ull << lane) - 1ull));
-    const int leader = le ? 63 - __clzll(le) : lane;
-    // Run length: up to the next start or the first inactive lane above.
-    const uint64_t above = (starts | ~act) & ~((2ull << lane) - 1ull) & (lane == 63 ? 0ull : ~0ull);
-    const int next = above ? __ffsll((long long)above) - 1 : 64;
-    uint32_t base = 0;
-    if (start) base = atomicAdd(&arr[kk], (uint32_t)(next - lane));
-    base = __shfl(base, leader, 64);
-    return base + (uint32_t)(lane - leader);
+    const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+    const uint64_t le = starts & upto;
+    r.leader = le ? 63 - __clzll(le) : lane;
+    const uint64_t above = (starts | ~act) & ~upto;
+    r.end = above ? __ffsll((long long)above) - 1 : 64;
+    return r;
 }
 
-// Cells per tile of the cell-start scan (4096): the integrate pass also sums
-// particles per tile, so every scan block finds its prefix without waiting.
-constexpr uint32_t kScanTileShift = 12;
+// Links particle k (lanes hold consecutive particles) into its cell's chain,
+// one exchange per run.  All lanes of the wave must call it; `active` marks
+// the lanes that hold a particle.
+__device__ __forceinline__ void push_run(uint32_t* __restrict__ head, uint32_t* __restrict__ next, uint32_t key,
+                                         uint32_t k, bool active) {
+    const int lane = (int)(threadIdx.x & 63u);
+    const LaneRun r = lane_run(key, active);
+    // A run's lanes 0, 15, 30, 45 and 60 each start a link.
+    const uint64_t links = 0x1000200040008001ull;
+    if (active && ((links >> (lane - r.leader)) & 1ull)) {
+        const int len = min(r.end - lane, (int)kRunMax);
+        next[k] = atomicExch(head + key, k | ((uint32_t)len << 28));
+    }
+}
 
-// Per-cell count (lanes follow sorted order, so most neighbours share a
-// cell) and the per-tile sums that follow the C cell counts.  Returns the
-// slot this lane took in its cell.
-__device__ __forceinline__ uint32_t count_slot(uint32_t* __restrict__ count, uint32_t* __restrict__ tsum,
-                                               uint32_t key, bool active) {
-    const uint32_t slot = run_add(count, key, active);
-    (void)run_add(tsum, key >> kScanTileShift, active);
-    return slot;
+// Adds the wave's particles to their tiles' sums: one atomic per run of
+// lanes in one tile.
+__device__ __forceinline__ void add_tile_sums(uint32_t* __restrict__ tsum, uint32_t key, bool active) {
+    const LaneRun r = lane_run(key >> kTileShift, active);
+    const int lane = (int)(threadIdx.x & 63u);
+    if (r.first) atomicAdd(tsum + (key >> kTileShift), (uint32_t)(r.end - lane));
 }
 
 // Adds the wave's largest |v|^2 to arr[idx] (float bits; atomic max on the

@@ -201,8 +201,8 @@ StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     a.id_s = w.id_s.p;
     a.id_o = h->id.p;
     a.key0 = h->key0.p;
-    a.rank0 = h->rank0.p;
-    a.count = h->count.p;
+    a.next = h->next.p;
+    a.head = h->head.p;
     a.cstart = w.cstart.p;
     a.rho = w.rho.p;
     a.mask = w.mask.p;
@@ -229,11 +229,8 @@ int alloc_step_bufs(sph_handle* h, StepBufs& w) {
     // is rewritten at the next scan.
     chk(w.tile_pre.ensure(scan_tiles(h->ncells)));
     if (e == hipSuccess) chk(launch_fill_u32(h->stream, w.tile_pre.p, 0xffffffffu, scan_tiles(h->ncells)));
-    if (h->tune.sort_mode == kSortCellCount) {
-        chk(w.tmp.ensure(n));
-    } else {
+    if (h->tune.sort_mode == kSortRadix)
         for (int i = 0; i < 2; ++i) { chk(w.kbuf[i].ensure(n)); chk(w.vbuf[i].ensure(n)); }
-    }
     chk(w.rho.ensure(n));
     chk(w.mask.ensure((size_t)kRows * n));
     if (h->keep_acc) chk(w.acc.ensure(n));
@@ -248,10 +245,11 @@ static int ensure_buffers(sph_handle* h) {
     chk(h->vel.ensure(n));
     chk(h->id.ensure(n));
     chk(h->key0.ensure(n));
-    chk(h->rank0.ensure(n));
-    const size_t count_words = (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells);
-    const bool fresh_count = h->count.count < count_words || !h->count.p;
-    chk(h->count.ensure(count_words));
+    chk(h->next.ensure(n));
+    chk(h->tmp.ensure(n));
+    const size_t head_words = (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells);
+    const bool fresh_head = h->head.count < head_words || !h->head.p;
+    chk(h->head.ensure(head_words));
     chk(h->hist.ensure(kMaxPasses * 256));
     chk(h->status.ensure((size_t)kMaxPasses * sort_tiles((uint32_t)n, 4) * 256 + 256));
     chk(h->tickets.ensure(kMaxPasses));
@@ -267,7 +265,7 @@ static int ensure_buffers(sph_handle* h) {
     chk(launch_fill_u32(h->stream, h->err.p, 0u, 1));
     chk(launch_fill_u32(h->stream, h->queue.p, 0u, kQueueWords));
     chk(launch_fill_u32(h->stream, h->vmax2.p, 0u, h->sc_h.size()));
-    if (fresh_count) chk(launch_fill_u32(h->stream, h->count.p, 0u, count_words));
+    if (fresh_head) chk(launch_fill_u32(h->stream, h->head.p, 0u, head_words));
     chk(hipMemcpyAsync(h->sc_d.p, h->sc_h.data(), h->sc_h.size() * sizeof(SceneConst), hipMemcpyHostToDevice, h->stream));
     if (e != hipSuccess) return hip_fail(h, e, "buffer init");
     return alloc_step_bufs(h, h->work);
@@ -294,13 +292,13 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     const uint8_t hashed = h->keys_valid ? 0 : 1;
     if (record_prof) prof_record(h, 0);
     if (!h->keys_valid) {
-        // New state: counts start from zero, then every particle is hashed.
-        hipError_t e = launch_fill_u32(st, h->count.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells));
+        // New state: the chains start empty, then every particle is hashed.
+        hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells));
         if (e == hipSuccess && h->cfl) e = launch_fill_u32(st, h->vmax2.p, 0u, h->sc_h.size());
         uint32_t nt = 0;
         const uint2* tl = tiles_for(h, 256, nt);
         if (e == hipSuccess)
-            e = launch_hash(st, 256, nt, h->pos.p, h->vel.p, h->key0.p, h->rank0.p, h->count.p, h->ncells,
+            e = launch_hash(st, 256, nt, h->pos.p, h->vel.p, h->key0.p, h->next.p, h->head.p, h->ncells,
                             h->cfl ? h->vmax2.p : nullptr, h->sc_d.p, tl, nt);
         if (e != hipSuccess) return hip_fail(h, e, "hash launch");
         h->keys_valid = true;
@@ -314,11 +312,11 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     sp.items = h->tune.sort_items;
     sp.reorder_block = h->tune.reorder_block;
     sp.key0 = h->key0.p;
-    sp.rank0 = h->rank0.p;
-    sp.count = h->count.p;
+    sp.head = h->head.p;
+    sp.next = h->next.p;
     sp.cstart = w.cstart.p;
     sp.tile_pre = w.tile_pre.p;
-    sp.tmp = w.tmp.p;
+    sp.tmp = h->tmp.p;
     for (int i = 0; i < 2; ++i) { sp.kbuf[i] = w.kbuf[i].p; sp.vbuf[i] = w.vbuf[i].p; }
     sp.skey = w.skey.p;
     sp.perm = w.perm.p;

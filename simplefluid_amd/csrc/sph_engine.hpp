@@ -78,8 +78,7 @@ struct StepBufs {
     DevBuf<uint32_t> id_s;
     DevBuf<uint32_t> skey, perm;   // sorted keys, sorted index -> state index
     DevBuf<uint32_t> cstart;       // C + 1 lower-bound cell-start table
-    DevBuf<uint32_t> tile_pre;     // per scan tile of cstart: prefix held by an empty tile, or ~0u
-    DevBuf<uint32_t> tmp;          // cell-count sort slots
+    DevBuf<uint32_t> tile_pre;     // per tile of cstart: prefix held by an empty tile, or ~0u
     DevBuf<uint32_t> kbuf[2], vbuf[2];  // radix ping-pong (radix mode only)
     DevBuf<float> rho;
     DevBuf<uint32_t> mask;
@@ -148,7 +147,8 @@ struct sph_handle {
     hipStream_t stream = nullptr;
     // State (state order) and per-step buffers.
     sph::DevBuf<float4> pos, vel;
-    sph::DevBuf<uint32_t> id, key0, rank0, count;
+    sph::DevBuf<uint32_t> id, key0, next, head;
+    sph::DevBuf<uint32_t> tmp;             // cell-count sort: members of the tiles too full for LDS
     sph::StepBufs work;
     sph::DevBuf<uint32_t> hist, status, tickets, err, queue;
     bool cfl = false;                      // adaptive step (single scene)

@@ -21,12 +21,12 @@ struct SortPlan {
     int items = 8;                    // radix: keys per thread of a digit-pass tile
     int reorder_block = 256;
     const uint32_t* key0 = nullptr;   // unsorted keys (state order)
-    const uint32_t* rank0 = nullptr;  // slot each particle took in its cell's count
-    uint32_t* count = nullptr;        // C cell counts (zeroed by the scan) + per-tile sums
-    uint32_t* cstart = nullptr;       // C + 1, written by the scan
-    uint32_t* tile_pre = nullptr;     // per scan tile: the prefix this cstart holds in all its cells
+    uint32_t* head = nullptr;         // C chain heads (cleared by the sort), T tile sums, T words for their scan
+    const uint32_t* next = nullptr;   // per run, the cell's run before it
+    uint32_t* cstart = nullptr;       // C + 1, written by the sort
+    uint32_t* tile_pre = nullptr;     // per tile: the prefix this cstart holds in all its cells
                                       // when the tile was empty at its last write, else 0xffffffff
-    uint32_t* tmp = nullptr;          // cell-count: slot -> particle
+    uint32_t* tmp = nullptr;          // cell-count: members of the tiles too full for LDS (n)
     uint32_t* kbuf[2] = {nullptr, nullptr};  // radix ping-pong
     uint32_t* vbuf[2] = {nullptr, nullptr};
     uint32_t* skey = nullptr;         // sorted keys
@@ -35,7 +35,7 @@ struct SortPlan {
     uint32_t* status = nullptr;       // radix: passes x tiles x 256
     uint32_t* tickets = nullptr;      // radix: kMaxPasses
     uint32_t* err = nullptr;
-    uint32_t* queue = nullptr;        // kQueueWords tile counters, zeroed by the scan
+    uint32_t* queue = nullptr;        // kQueueWords tile counters, zeroed by the sort
     const uint32_t* halt = nullptr;   // device frame loop: non-zero word skips the step (cell-count mode)
     const float4* pos_in = nullptr;
     const float4* vel_in = nullptr;
@@ -48,13 +48,13 @@ struct SortPlan {
 };
 
 uint32_t sort_tiles(uint32_t n, int items);
-// Tiles of 4096 cells.  count holds C cell counts, then T = scan_tiles(C)
+// Tiles of 1024 cells.  head holds C chain heads, then T = scan_tiles(C)
 // per-tile sums, then their exclusive scan (T words).
 uint32_t scan_tiles(uint32_t ncells);
 int sort_key_passes(uint32_t ncells);
-// Cell-start table plus the sort proper (keys and permutation) ...
+// Cell-start table and the sort; cell-count mode gathers the state too ...
 hipError_t launch_sort_keys(hipStream_t st, const SortPlan& sp);
-// ... then the gather of the state into sorted order.
+// ... radix mode: the gather of the state into sorted order.
 hipError_t launch_sort_gather(hipStream_t st, const SortPlan& sp);
 
 // Arguments of the per-particle passes.  Work is split in tiles of blockDim
@@ -68,8 +68,8 @@ struct StepArgs {
     const uint32_t* id_s;
     uint32_t* id_o;
     uint32_t* key0;          // next step's unsorted keys
-    uint32_t* rank0;         // next step's slot in its cell count
-    uint32_t* count;         // next step's per-cell counts, then per-scan-tile sums (atomic)
+    uint32_t* head;          // next step's chain heads, then per-tile sums (atomic)
+    uint32_t* next;          // next step's runs
     const uint32_t* cstart;  // cell-start table of this step
     float* rho;
     uint32_t* mask;
@@ -79,17 +79,17 @@ struct StepArgs {
     uint32_t ntiles;
     uint32_t n;
     uint32_t ncells;
-    uint32_t* queue;         // persistent launch: 8 tile counters (zeroed by the scan), else null
+    uint32_t* queue;         // persistent launch: 8 tile counters (zeroed by the sort), else null
     uint32_t* vmax2;         // CFL: per-scene max |v|^2 (float bits) of the new state, else null
     const uint32_t* halt;    // device frame loop: non-zero word skips the step, else null
 };
 
 // Tile counters of the persistent density and force launches (8 each),
-// zeroed by the cell-start scan of every step.
+// zeroed by the sort of every step.
 constexpr int kQueueWords = 16;
 
 hipError_t launch_hash(hipStream_t st, int block, uint32_t grid, const float4* pos, const float4* vel,
-                       uint32_t* key0, uint32_t* rank0, uint32_t* count, uint32_t ncells, uint32_t* vmax2,
+                       uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t ncells, uint32_t* vmax2,
                        const SceneConst* scenes, const uint2* tiles, uint32_t ntiles);
 // CFL step of every scene from its max |v|^2 (scenes with cfl = 0 keep dt);
 // clears vmax2 and stores scene 0's step in *dt_out.  With a frame state

@@ -14,7 +14,7 @@
 // largest x subdivision of 4, 2, 1 whose grid fits is used, as a handle of
 // that size would pick).  Every call on one GPU shares that GPU's scratch:
 // calls that overlap on one GPU race, and each call rewrites the scratch
-// from the start (counts, tile prefixes, error word and tile queues are
+// from the start (chain heads, tile prefixes, error word and tile queues are
 // cleared by kernels, not by memset, so the call may be graph-captured).
 #include <cstring>
 #include <mutex>
@@ -29,7 +29,7 @@ constexpr uint32_t kMaxParticles = 65536;
 constexpr uint32_t kMaxCells = 1u << 20;
 constexpr int kBlock = 256;
 constexpr uint32_t kMaxTiles = kMaxParticles / kBlock;
-constexpr uint32_t kScanTilesMax = (kMaxCells + 4095u) / 4096u;
+constexpr uint32_t kScanTilesMax = (kMaxCells + kTileCells - 1u) / kTileCells;
 
 // Byte offsets of the arrays inside the scratch, each 256-byte aligned.
 constexpr size_t align256(size_t x) { return (x + 255u) & ~(size_t)255u; }
@@ -43,14 +43,14 @@ struct Layout {
     static constexpr size_t id = align256(soa + 12 * N);
     static constexpr size_t id_s = align256(id + 4 * N);
     static constexpr size_t key0 = align256(id_s + 4 * N);
-    static constexpr size_t rank0 = align256(key0 + 4 * N);
-    static constexpr size_t skey = align256(rank0 + 4 * N);
+    static constexpr size_t next = align256(key0 + 4 * N);
+    static constexpr size_t skey = align256(next + 4 * N);
     static constexpr size_t perm = align256(skey + 4 * N);
     static constexpr size_t tmp = align256(perm + 4 * N);
     static constexpr size_t rho = align256(tmp + 4 * N);
     static constexpr size_t mask = align256(rho + 4 * N);
-    static constexpr size_t count = align256(mask + 4 * (size_t)kRows * N);
-    static constexpr size_t cstart = align256(count + 4 * ((size_t)kMaxCells + 2 * kScanTilesMax));
+    static constexpr size_t head = align256(mask + 4 * (size_t)kRows * N);
+    static constexpr size_t cstart = align256(head + 4 * ((size_t)kMaxCells + 2 * kScanTilesMax));
     static constexpr size_t tile_pre = align256(cstart + 4 * ((size_t)kMaxCells + 1));
     static constexpr size_t tiles = align256(tile_pre + 4 * (size_t)kScanTilesMax);
     static constexpr size_t scene = align256(tiles + 8 * (size_t)kMaxTiles);
@@ -139,29 +139,29 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     float4* pos = reinterpret_cast<float4*>(at(Layout::pos));
     float4* vel = reinterpret_cast<float4*>(at(Layout::vel));
     uint32_t* id = reinterpret_cast<uint32_t*>(at(Layout::id));
-    uint32_t* count = reinterpret_cast<uint32_t*>(at(Layout::count));
+    uint32_t* head = reinterpret_cast<uint32_t*>(at(Layout::head));
     const uint32_t T = scan_tiles(C);
     const uint32_t ntiles = (n + kBlock - 1) / kBlock;
 
     hipLaunchKernelGGL(noalloc_setup_kernel, dim3((n + 255) / 256), dim3(256), 0, st, sc, n, base);
     e = hipGetLastError();
-    if (e == hipSuccess) e = launch_fill_u32(st, count, 0u, (size_t)C + 2 * (size_t)T);
+    if (e == hipSuccess) e = launch_fill_u32(st, head, 0u, (size_t)C + 2 * (size_t)T);
     if (e == hipSuccess) e = launch_fill_u32(st, reinterpret_cast<uint32_t*>(at(Layout::tile_pre)), 0xffffffffu, T);
     if (e == hipSuccess) e = launch_pack3(st, n, xyz_in, pos);
     if (e == hipSuccess) e = launch_pack3(st, n, vel_in, vel);
     const SceneConst* scd = reinterpret_cast<const SceneConst*>(at(Layout::scene));
     const uint2* tiles = reinterpret_cast<const uint2*>(at(Layout::tiles));
     uint32_t* key0 = reinterpret_cast<uint32_t*>(at(Layout::key0));
-    uint32_t* rank0 = reinterpret_cast<uint32_t*>(at(Layout::rank0));
-    if (e == hipSuccess) e = launch_hash(st, kBlock, ntiles, pos, vel, key0, rank0, count, C, nullptr, scd, tiles, ntiles);
+    uint32_t* next = reinterpret_cast<uint32_t*>(at(Layout::next));
+    if (e == hipSuccess) e = launch_hash(st, kBlock, ntiles, pos, vel, key0, next, head, C, nullptr, scd, tiles, ntiles);
     SortPlan sp;
     sp.n = n;
     sp.ncells = C;
     sp.mode = kSortCellCount;
     sp.reorder_block = kBlock;
     sp.key0 = key0;
-    sp.rank0 = rank0;
-    sp.count = count;
+    sp.head = head;
+    sp.next = next;
     sp.cstart = reinterpret_cast<uint32_t*>(at(Layout::cstart));
     sp.tile_pre = reinterpret_cast<uint32_t*>(at(Layout::tile_pre));
     sp.tmp = reinterpret_cast<uint32_t*>(at(Layout::tmp));
@@ -188,8 +188,8 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     a.id_s = sp.id_out;
     a.id_o = id;
     a.key0 = key0;
-    a.rank0 = rank0;
-    a.count = count;
+    a.next = next;
+    a.head = head;
     a.cstart = sp.cstart;
     a.rho = reinterpret_cast<float*>(at(Layout::rho));
     a.mask = reinterpret_cast<uint32_t*>(at(Layout::mask));

@@ -3,17 +3,14 @@
 // Both sort modes produce the same stable permutation (ties keep the input
 // order) and the same lower-bound table cstart[c] = #particles with key < c.
 //
-// Cell-count sort (default): a one-digit radix sort whose digit is the whole
-// cell key.  The integrate pass already counted particles per cell with
-// atomics (count[key]++, keeping the returned slot in rank0).  Then
-//   cell_scan        exclusive scan of count -> cstart; each block of 4096
-//                    cells takes its prefix from the per-tile sums the
-//                    integrate pass also counted (zeroes count for the next step)
-//   cell_scatter     tmp[cstart[key] + rank0] = k   (slot order within a
-//                    cell is whatever order the atomics ran in)
-//   cell_rank        the deterministic rank of k in its cell is the number of
-//                    members with a smaller input index; k is gathered
-//                    straight into its sorted place (pos, vel, id, key, perm)
+// Cell-count sort (default): one kernel.  The integrate pass already linked
+// each particle into its cell's chain of runs and counted particles per tile
+// of 1024 cells, so a block of cell_sort_kernel owns a tile: it takes its
+// prefix from the tile sums, counts its cells by following their chains,
+// scans the counts (cstart), lists the members cell by cell in LDS, ranks
+// each in its cell (the number of members with a smaller input index) and
+// gathers its state straight into its sorted place (pos, vel, id, key,
+// perm).  No block waits for another.
 // Radix sort: one histogram kernel for all 8-bit digits, then one kernel per
 // digit that ranks a tile of keys in LDS (wave64 ballot-matching of the
 // digit bits, so equal digits rank in lane order without LDS atomics) and
@@ -95,240 +92,361 @@ __device__ __forceinline__ uint32_t look_back(const uint32_t* status, uint32_t s
 
 // ---------------------------------------------------------------- cell count
 
-// Exclusive scan of the T per-tile sums (count[C .. C+T)) into
-// count[C+T .. C+2T), one block of 1024 threads, each over a contiguous run.
-constexpr int kTileScanBlock = 1024;
-constexpr uint32_t kInlineTiles = 1024;
-
-__global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __restrict__ count, uint32_t C,
-                                                                   uint32_t T, const uint32_t* __restrict__ halt) {
-    if (halt && *halt) return;
-    // Rounds of 4096 tile sums: thread t takes 4 consecutive ones (16-byte
-    // access when aligned), a block scan adds the round's carry.
-    __shared__ uint32_t s_w[kTileScanBlock / 64];
-    __shared__ uint32_t s_carry;
-    const uint32_t* tsum = count + C;
-    uint32_t* tpre = count + C + T;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) s_carry = 0u;
-    __syncthreads();
-    for (uint32_t r0 = 0; r0 < T; r0 += 4u * kTileScanBlock) {
-        const uint32_t i0 = r0 + 4u * (uint32_t)tid;
-        uint32_t v[4];
+// Exclusive scan of one value per thread over a block of BLOCK threads;
+// total receives the block sum.
+template <int BLOCK>
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s_w, uint32_t& total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t x = v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = i0 + e < T ? tsum[i0 + e] : 0u;
-        const uint32_t own = v[0] + v[1] + v[2] + v[3];
-        uint32_t x = own;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (lane == 63) s_w[wave] = x;
-        __syncthreads();
-        uint32_t run = s_carry + x - own;
-        uint32_t tot = 0;
-        for (int w = 0; w < kTileScanBlock / 64; ++w) {
-            if (w < wave) run += s_w[w];
-            tot += s_w[w];
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (i0 + e < T) tpre[i0 + e] = run;
-            run += v[e];
-        }
-        __syncthreads();
-        if (tid == 0) s_carry += tot;
-        __syncthreads();
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
     }
+    if (lane == 63) s_w[wave] = x;
+    __syncthreads();
+    uint32_t pre = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; ++w) {
+        const uint32_t sw = s_w[w];
+        if (w < wave) pre += sw;
+        tot += sw;
+    }
+    total = tot;
+    return pre + x - v;
 }
 
-// Block b scans the counts of cells [4096 b, 4096 (b + 1)).  Its prefix is
-// the exclusive scan of the tile sums (counted by the integrate pass next to
-// the cell counts): summed here when there are at most kInlineTiles tiles,
-// else read from tile_scan_kernel's output.  No block waits for another; a
-// tile with no particles only writes its prefix.  Wave w takes 1024 cells in 4 rounds of 64 lanes x
-// 4 consecutive cells (16-byte loads and stores); the counts are zeroed for
-// the next step as they are read.
-__global__ __launch_bounds__(kSortBlock) void cell_scan_kernel(uint32_t* __restrict__ count,
-                                                               uint32_t* __restrict__ cstart, uint32_t C,
-                                                               uint32_t* __restrict__ queue,
-                                                               const uint32_t* __restrict__ halt,
-                                                               uint32_t* __restrict__ tile_pre) {
+// Exclusive scan of the T per-tile sums (head[C .. C+T)) into
+// head[C+T .. C+2T).  Block i scans sums [1024 i, 1024 (i + 1)) and adds up
+// all the ones before itself: the reads are coalesced, independent and in
+// cache, where one block over all of them waited on itself round by round
+// (22k tiles: 14 us).
+constexpr int kTileScanBlock = 1024;
+// Up to this many tiles each sort block sums the tiles before its own itself
+// (8 words per thread at most); above it tile_scan_kernel runs first.
+constexpr uint32_t kInlineTiles = 2048;
+
+__global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __restrict__ head, uint32_t C,
+                                                                   uint32_t T, const uint32_t* __restrict__ halt) {
     if (halt && *halt) return;
-    __shared__ uint32_t s_tot[kSortWaves];
-    const uint32_t b = blockIdx.x;
+    __shared__ uint32_t s_w[kTileScanBlock / 64];
+    __shared__ uint32_t s_pre[kTileScanBlock / 64];
+    const uint32_t* tsum = head + C;
+    const uint32_t i0 = blockIdx.x * (uint32_t)kTileScanBlock, i = i0 + threadIdx.x;
+    uint32_t before = 0;
+#pragma unroll 8
+    for (uint32_t e = threadIdx.x; e < i0; e += (uint32_t)kTileScanBlock) before += tsum[e];
+    const uint32_t own = i < T ? tsum[i] : 0u;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    if ((threadIdx.x & 63u) == 0u) s_pre[threadIdx.x >> 6] = before;
+    uint32_t total;
+    uint32_t run = block_scan<kTileScanBlock>(own, s_w, total);
+#pragma unroll
+    for (int w = 0; w < kTileScanBlock / 64; ++w) run += s_pre[w];
+    if (i < T) head[C + T + i] = run;
+}
+
+// Members a cell may hold for the stable in-cell rank (a member's rank scans
+// its cell).  Rest-density fluid holds a few per cell.
+constexpr uint32_t kMaxRankCell = 1024;
+// Members of a tile listed in LDS; a fuller tile lists them in global memory.
+constexpr uint32_t kTileMembers = 4096;
+// Links of one cell followed in its chain; a longer chain (a pile of
+// particles in one cell, or an upload in random order of a very full one)
+// makes the block find the tile's members by scanning all keys instead.
+constexpr int kMaxLinks = 256;
+
+struct CellSortArgs {
+    uint32_t n, C;
+    uint32_t* head;
+    const uint32_t* next;
+    const uint32_t* key0;
+    uint32_t* cstart;
+    uint32_t* tile_pre;
+    uint32_t* tmp;       // members of the tiles too full for LDS, at their sorted place
+    const float4* pos_in;
+    const float4* vel_in;
+    const uint32_t* id_in;
+    float4* pos_out;
+    float4* vel_out;
+    uint32_t* id_out;
+    uint32_t* skey;
+    uint32_t* perm;
+    float* soa;
+    uint32_t* queue;
+    uint32_t* err;
+    const uint32_t* halt;
+    int gather;          // 0: the cell-start table only (radix mode)
+};
+
+// Block b sorts the particles of cells [1024 b, 1024 (b + 1)).  Thread t owns
+// V consecutive cells; their chains are followed together, so a wave waits
+// once per link for the longest chain among its cells, and the first
+// kHeldLinks links stay in registers for the listing.  The kernel is bound
+// by the latency of its dependent steps at small sizes (tile sums and heads,
+// the links, the members' state) and by memory at large ones; one particle's
+// state is moved once.
+constexpr int kHeldLinks = 4;
+
+// One thread per cell up to this many tiles, where the chip waits on each
+// block's dependent steps; above it four cells per thread, where 1024-lane
+// blocks only hold up each other's phases.  Measured, 1024 against 256
+// threads: DoubleDambreak at resolution 24 (54 tiles) 7.0 against 11.5 us,
+// 65k dam break (489 tiles) 7.8 against 11.3 us, 1M (2013 tiles) 29.2 against
+// 23.1 us.
+constexpr uint32_t kWideTiles = 1024;
+
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
+    if (a.halt && *a.halt) return;
+    constexpr int V = (int)kTileCells / BLOCK;
+    constexpr int kWaves = BLOCK / 64;
+    static_assert(V == 1 || V == 4, "one head, or four in one 16-byte load, per thread");
+    __shared__ uint32_t s_w[kWaves];
+    __shared__ uint32_t s_pre[kWaves];
+    __shared__ uint32_t s_big;
+    __shared__ uint32_t s_off[kTileCells + 1];
+    __shared__ uint32_t s_mem[kTileMembers];
+    __shared__ uint16_t s_cell[kTileMembers];
+    const uint32_t b = blockIdx.x, C = a.C;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // Tile counters of this step's persistent density and force launches.
-    if (b == 0 && tid < kQueueWords && queue) queue[tid] = 0u;
-    const uint32_t T = (C + (1u << kScanTileShift) - 1u) >> kScanTileShift;
-    uint32_t pre;
-    if (T <= kInlineTiles) {
-        __shared__ uint32_t s_pre[kSortWaves];
-        uint32_t x = 0;
-        for (uint32_t i = (uint32_t)tid; i < b; i += kSortBlock) x += count[C + i];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-        if (lane == 0) s_pre[wave] = x;
-        __syncthreads();
-        pre = s_pre[0] + s_pre[1] + s_pre[2] + s_pre[3];
+    if (b == 0 && tid < kQueueWords && a.queue) a.queue[tid] = 0u;
+    const uint32_t T = (C + kTileCells - 1u) >> kTileShift;
+    const uint32_t base = b << kTileShift;
+    const uint32_t i0 = base + (uint32_t)(V * tid);
+    uint32_t r[kHeldLinks + 1][V];
+    const bool whole = i0 + (uint32_t)V <= C;
+    if (V == 4 && whole) {
+        const uint4 hv = *reinterpret_cast<const uint4*>(a.head + i0);
+        r[0][0] = hv.x;
+        r[0][V > 1 ? 1 : 0] = V > 1 ? hv.y : hv.x;
+        r[0][V > 2 ? 2 : 0] = V > 2 ? hv.z : hv.x;
+        r[0][V > 3 ? 3 : 0] = V > 3 ? hv.w : hv.x;
     } else {
-        pre = count[C + T + b];
+#pragma unroll
+        for (int v = 0; v < V; ++v) r[0][v] = i0 + (uint32_t)v < C ? a.head[i0 + v] : 0u;
     }
     // What the table holds for this tile, read by every thread before any
     // thread of the block rewrites it.
-    const uint32_t held = tile_pre[b];
-    __syncthreads();
-    if (count[C + b] == 0u) {
+    const uint32_t held = a.tile_pre[b];
+    const uint32_t members = a.head[C + b];
+    uint32_t pre;
+    if (T <= kInlineTiles) {
+        uint32_t x = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < kInlineTiles / BLOCK; ++e) {
+            const uint32_t i = e * BLOCK + (uint32_t)tid;
+            if (i < b) x += a.head[C + i];
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+        if (lane == 0) s_pre[wave] = x;
+        if (tid == 0) s_big = 0u;
+        __syncthreads();
+        pre = 0u;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) pre += s_pre[w];
+    } else {
+        pre = a.head[C + T + b];
+        if (tid == 0) s_big = 0u;
+        __syncthreads();
+    }
+    if (members == 0u) {
         // An empty tile's cells all hold its prefix; skip the rewrite when
         // this table already holds that prefix there (most empty tiles of
         // a sparse grid keep theirs from step to step).
         if (held == pre) return;
-        if (tid == 0) tile_pre[b] = pre;
-        const uint32_t t0 = b << kScanTileShift;
-        const uint32_t t1 = t0 + (1u << kScanTileShift) < C ? t0 + (1u << kScanTileShift) : C;
-        const uint4 v4 = make_uint4(pre, pre, pre, pre);
-        for (uint32_t i = t0 + 4u * (uint32_t)tid; i < t1; i += 4u * kSortBlock) {
-            if (i + 4u <= t1) {
-                *reinterpret_cast<uint4*>(cstart + i) = v4;
-            } else {
-                for (uint32_t e = i; e < t1; ++e) cstart[e] = pre;
+        if (tid == 0) a.tile_pre[b] = pre;
+        if (V == 4 && whole) {
+            *reinterpret_cast<uint4*>(a.cstart + i0) = make_uint4(pre, pre, pre, pre);
+        } else {
+            for (uint32_t e = i0; e < C && e < i0 + (uint32_t)V; ++e) a.cstart[e] = pre;
+        }
+        if (b == T - 1u && tid == 0) a.cstart[C] = pre;
+        return;
+    }
+    if (tid == 0) a.tile_pre[b] = 0xffffffffu;
+    const __amdgpu_buffer_rsrc_t rnext = buffer_of(a.next, a.n);
+    // The run before r in its cell; for the empty run, past the array's end, 0.
+    auto link = [&](uint32_t run) -> uint32_t {
+        return __builtin_amdgcn_raw_buffer_load_b32(rnext, (int)(run ? run_first(run) << 2 : 0xfffffffcu), 0, 0);
+    };
+    auto any = [&](const uint32_t* q) -> bool {
+        uint32_t o = 0;
+#pragma unroll
+        for (int v = 0; v < V; ++v) o |= q[v];
+        return o != 0u;
+    };
+    uint32_t cnt[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) cnt[v] = run_len(r[0][v]);
+#pragma unroll
+    for (int l = 0; l < kHeldLinks; ++l) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) r[l + 1][v] = 0u;
+        if (__ballot(any(r[l]))) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) r[l + 1][v] = link(r[l][v]);
+#pragma unroll
+            for (int v = 0; v < V; ++v) cnt[v] += run_len(r[l + 1][v]);
+        }
+    }
+    // The heads are empty again for the integrate pass.
+    if (any(r[0])) {
+        if (V == 4 && whole) {
+            *reinterpret_cast<uint4*>(a.head + i0) = make_uint4(0u, 0u, 0u, 0u);
+        } else {
+            for (uint32_t e = i0; e < C && e < i0 + (uint32_t)V; ++e) a.head[e] = 0u;
+        }
+    }
+    {
+        uint32_t q[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) q[v] = r[kHeldLinks][v];
+        int links = kHeldLinks;
+        while (any(q)) {
+            if (++links > kMaxLinks) {
+                s_big = 1u;
+                break;
+            }
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                q[v] = link(q[v]);
+                cnt[v] += run_len(q[v]);
             }
         }
-        if (t1 == C && tid == 0) cstart[C] = pre;
-        return;
     }
-    if (tid == 0) tile_pre[b] = 0xffffffffu;
-    const uint32_t base = (b << kScanTileShift) + (uint32_t)wave * 1024u;
-    uint4 v[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t i0 = base + 256u * (uint32_t)r + 4u * (uint32_t)lane;
-        if (i0 + 4u <= C) {
-            v[r] = *reinterpret_cast<const uint4*>(count + i0);
-            *reinterpret_cast<uint4*>(count + i0) = make_uint4(0u, 0u, 0u, 0u);
-        } else {
-            v[r].x = i0 < C ? count[i0] : 0u;
-            v[r].y = i0 + 1u < C ? count[i0 + 1u] : 0u;
-            v[r].z = i0 + 2u < C ? count[i0 + 2u] : 0u;
-            v[r].w = i0 + 3u < C ? count[i0 + 3u] : 0u;
-            for (uint32_t e = 0; e < 4u; ++e)
-                if (i0 + e < C) count[i0 + e] = 0u;
-        }
-    }
-    // Wave-local exclusive prefix of each lane's four cells, round by round.
-    uint32_t ex[4];
-    uint32_t carry = 0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t own = v[r].x + v[r].y + v[r].z + v[r].w;
-        uint32_t x = own;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        ex[r] = carry + x - own;
-        carry += __shfl(x, 63, 64);
-    }
-    if (lane == 0) s_tot[wave] = carry;
     __syncthreads();
-    uint32_t off = pre;
-#pragma unroll
-    for (int w = 0; w < kSortWaves; ++w)
-        if (w < wave) off += s_tot[w];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t i0 = base + 256u * (uint32_t)r + 4u * (uint32_t)lane;
-        uint4 o;
-        o.x = off + ex[r];
-        o.y = o.x + v[r].x;
-        o.z = o.y + v[r].y;
-        o.w = o.z + v[r].z;
-        const uint32_t end = o.w + v[r].w;
-        if (i0 + 4u <= C) {
-            *reinterpret_cast<uint4*>(cstart + i0) = o;
-        } else {
-            const uint32_t val[4] = {o.x, o.y, o.z, o.w};
-            for (uint32_t e = 0; e < 4u; ++e)
-                if (i0 + e < C) cstart[i0 + e] = val[e];
+    const bool big = s_big != 0u;
+    if (big) {
+        // Count by scanning all keys (s_off as the counters).
+        for (uint32_t i = (uint32_t)tid; i < kTileCells; i += BLOCK) s_off[i] = 0u;
+        __syncthreads();
+        for (uint32_t k = (uint32_t)tid; k < a.n; k += BLOCK) {
+            const uint32_t c = a.key0[k] - base;
+            if (c < kTileCells) atomicAdd(&s_off[c], 1u);
         }
-        if (i0 < C && C <= i0 + 4u) {
-            const uint32_t val[5] = {o.x, o.y, o.z, o.w, end};
-            cstart[C] = val[C - i0];
-        }
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < V; ++v) cnt[v] = s_off[V * tid + v];
+        __syncthreads();
     }
-}
-
-__global__ void cell_scatter_kernel(uint32_t n, uint32_t C, const uint32_t* __restrict__ key0,
-                                    const uint32_t* __restrict__ rank0, const uint32_t* __restrict__ cstart,
-                                    uint32_t* __restrict__ tmp, uint32_t* __restrict__ err,
-                                    const uint32_t* __restrict__ halt) {
-    if (halt && *halt) return;
-    const uint32_t k = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const uint32_t key = key0[k];
-    const uint32_t slot = key < C ? cstart[key] + rank0[k] : 0xffffffffu;
-    if (slot < n)
-        tmp[slot] = k;
-    else
-        atomicOr(err, 2u);
-}
-
-// Members a cell may hold for the stable in-cell rank (cell_rank_kernel
-// scans its cell once per member).  Rest-density fluid holds a few per cell.
-constexpr uint32_t kMaxRankCell = 1024;
-
-__global__ void cell_rank_kernel(uint32_t n, uint32_t C, const uint32_t* __restrict__ key0,
-                                 const uint32_t* __restrict__ rank0,
-                                 const uint32_t* __restrict__ cstart, const uint32_t* __restrict__ tmp,
-                                 const float4* __restrict__ pos_in, const float4* __restrict__ vel_in,
-                                 const uint32_t* __restrict__ id_in, float4* __restrict__ pos_out,
-                                 float4* __restrict__ vel_out, uint32_t* __restrict__ id_out,
-                                 uint32_t* __restrict__ skey, uint32_t* __restrict__ perm,
-                                 uint32_t* __restrict__ tsum, uint32_t tsum_words,
-                                 uint32_t* __restrict__ err, float* __restrict__ soa,
-                                 const uint32_t* __restrict__ halt) {
-    if (halt && *halt) return;
-    // The scan has read the tile sums; clear them for the integrate pass.
-    if (blockIdx.x == 0)
-        for (uint32_t i = threadIdx.x; i < tsum_words; i += blockDim.x) tsum[i] = 0u;
-    const uint32_t k = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const uint32_t key = key0[k];
-    if (key >= C) {
-        atomicOr(err, 4u);
-        return;
-    }
-    const uint32_t lo = cstart[key], hi = cstart[key + 1];
-    uint32_t r;
-    if (hi - lo <= kMaxRankCell) {
-        r = 0;
-        for (uint32_t t = lo; t < hi; ++t) r += tmp[t] < k ? 1u : 0u;
+    uint32_t own = 0, total;
+#pragma unroll
+    for (int v = 0; v < V; ++v) own += cnt[v];
+    uint32_t off[V];
+    off[0] = block_scan<BLOCK>(own, s_w, total);
+#pragma unroll
+    for (int v = 1; v < V; ++v) off[v] = off[v - 1] + cnt[v - 1];
+    if (V == 4 && whole) {
+        *reinterpret_cast<uint4*>(a.cstart + i0) = make_uint4(pre + off[0], pre + off[V > 1 ? 1 : 0],
+                                                              pre + off[V > 2 ? 2 : 0], pre + off[V > 3 ? 3 : 0]);
     } else {
-        // A cell this full only arises from collapsed or non-finite
-        // positions (clamped into one cell).  Ranking it costs its size per
-        // member, so it keeps the arrival order (a valid permutation, not
-        // the stable one) and raises the error flag instead.
-        r = rank0[k];
-        atomicOr(err, 8u);
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (i0 + (uint32_t)v < C) a.cstart[i0 + v] = pre + off[v];
     }
-    const uint32_t dst = lo + r;
-    if (dst >= hi || hi > n) {
-        atomicOr(err, 4u);
+    if (b == T - 1u && tid == 0) a.cstart[C] = pre + total;
+    if (!a.gather) return;
+    if (pre > a.n || total > a.n - pre) {  // inconsistent sums: never write out of bounds
+        if (tid == 0) atomicOr(a.err, 2u);
         return;
     }
-    perm[dst] = k;
-    skey[dst] = key;
-    const float4 pk = pos_in[k];
-    pos_out[dst] = pk;
-    if (soa) {  // the planes, for the gathered density pass
-        soa[dst] = pk.x;
-        soa[n + dst] = pk.y;
-        soa[2 * (size_t)n + dst] = pk.z;
+#pragma unroll
+    for (int v = 0; v < V; ++v) s_off[V * tid + v] = off[v];
+    if (tid == 0) s_off[kTileCells] = total;
+    // The members, cell by cell, in the order their runs come.
+    const bool in_lds = total <= kTileMembers && !big;
+    uint32_t* const tmp = a.tmp + pre;
+    if (!big) {
+        auto list = [&](const uint32_t* q) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const uint32_t k = run_first(q[v]), len = run_len(q[v]);
+                for (uint32_t t = 0; t < len; ++t) {
+                    if (in_lds) {
+                        s_mem[off[v] + t] = k + t;
+                        s_cell[off[v] + t] = (uint16_t)(V * tid + v);
+                    } else {
+                        tmp[off[v] + t] = k + t;
+                    }
+                }
+                off[v] += len;
+            }
+        };
+#pragma unroll
+        for (int l = 0; l <= kHeldLinks; ++l)
+            if (any(r[l])) list(r[l]);
+        uint32_t q[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) q[v] = r[kHeldLinks][v];
+        while (any(q)) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) q[v] = link(q[v]);
+            list(q);
+        }
+    } else {
+        __syncthreads();
+        for (uint32_t k = (uint32_t)tid; k < a.n; k += BLOCK) {
+            const uint32_t c = a.key0[k] - base;
+            if (c < kTileCells) tmp[atomicAdd(&s_off[c], 1u)] = k;
+        }
+        __syncthreads();
+        // The counters ended at the next cell's start.
+#pragma unroll
+        for (int v = 0; v < V; ++v) s_off[V * tid + v] = off[v];
     }
-    vel_out[dst] = vel_in[k];
-    id_out[dst] = id_in[k];
+    __threadfence_block();
+    __syncthreads();
+    for (uint32_t j = (uint32_t)tid; j < total; j += BLOCK) {
+        const uint32_t k = in_lds ? s_mem[j] : tmp[j];
+        if (k >= a.n) {
+            atomicOr(a.err, 4u);
+            continue;
+        }
+        const float4 pk = a.pos_in[k];
+        const float4 vk = a.vel_in[k];
+        const uint32_t ik = a.id_in[k];
+        const uint32_t c = in_lds ? (uint32_t)s_cell[j] : a.key0[k] - base;
+        if (c >= kTileCells) {
+            atomicOr(a.err, 4u);
+            continue;
+        }
+        const uint32_t lo = s_off[c], hi = s_off[c + 1u];
+        uint32_t d = j;
+        if (hi - lo <= kMaxRankCell) {
+            d = lo;
+            if (in_lds) {
+                for (uint32_t t = lo; t < hi; ++t) d += s_mem[t] < k ? 1u : 0u;
+            } else {
+                for (uint32_t t = lo; t < hi; ++t) d += tmp[t] < k ? 1u : 0u;
+            }
+        } else {
+            // A cell this full only arises from collapsed or non-finite
+            // positions (clamped into one cell).  Ranking it costs its size
+            // per member, so it keeps the order its members were listed in
+            // (a valid permutation, not the stable one) and raises the error
+            // flag instead.
+            atomicOr(a.err, 8u);
+        }
+        const uint32_t dst = pre + d;
+        if (dst >= a.n) {
+            atomicOr(a.err, 4u);
+            continue;
+        }
+        if (a.perm) a.perm[dst] = k;
+        if (a.skey) a.skey[dst] = base + c;
+        a.pos_out[dst] = pk;
+        if (a.soa) {  // the planes, for the gathered density pass
+            a.soa[dst] = pk.x;
+            a.soa[a.n + dst] = pk.y;
+            a.soa[2 * (size_t)a.n + dst] = pk.z;
+        }
+        a.vel_out[dst] = vk;
+        a.id_out[dst] = ik;
+    }
 }
 
 // --------------------------------------------------------------------- radix
@@ -485,12 +603,10 @@ __global__ void radix_reorder_kernel(uint32_t n, const uint32_t* __restrict__ pe
                                      const float4* __restrict__ pos_in, const float4* __restrict__ vel_in,
                                      const uint32_t* __restrict__ id_in, float4* __restrict__ pos_out,
                                      float4* __restrict__ vel_out, uint32_t* __restrict__ id_out,
-                                     uint32_t* __restrict__ hist_zero, uint32_t* __restrict__ tsum,
-                                     uint32_t tsum_words, uint32_t* __restrict__ err, float* __restrict__ soa) {
-    if (blockIdx.x == 0) {
+                                     uint32_t* __restrict__ hist_zero, uint32_t* __restrict__ err,
+                                     float* __restrict__ soa) {
+    if (blockIdx.x == 0)
         for (uint32_t i = threadIdx.x; i < (uint32_t)(kMaxPasses * kBins); i += blockDim.x) hist_zero[i] = 0u;
-        for (uint32_t i = threadIdx.x; i < tsum_words; i += blockDim.x) tsum[i] = 0u;
-    }
     const uint32_t k = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const uint32_t s = perm[k];
@@ -518,7 +634,7 @@ uint32_t sort_tiles(uint32_t n, int items) {
     return (n + tile - 1) / tile;
 }
 
-uint32_t scan_tiles(uint32_t C) { return (C + (1u << kScanTileShift) - 1u) >> kScanTileShift; }
+uint32_t scan_tiles(uint32_t C) { return (C + kTileCells - 1u) >> kTileShift; }
 
 int sort_key_passes(uint32_t ncells) {
     int bits = 1;
@@ -526,20 +642,46 @@ int sort_key_passes(uint32_t ncells) {
     return (bits + 7) / 8;
 }
 
+static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
+    const uint32_t tiles = scan_tiles(sp.ncells);
+    if (tiles > kInlineTiles)
+        hipLaunchKernelGGL(tile_scan_kernel, dim3((tiles + kTileScanBlock - 1) / kTileScanBlock), dim3(kTileScanBlock),
+                           0, st, sp.head, sp.ncells, tiles, sp.halt);
+    CellSortArgs a;
+    a.n = sp.n;
+    a.C = sp.ncells;
+    a.head = sp.head;
+    a.next = sp.next;
+    a.key0 = sp.key0;
+    a.cstart = sp.cstart;
+    a.tile_pre = sp.tile_pre;
+    a.tmp = sp.tmp;
+    a.pos_in = sp.pos_in;
+    a.vel_in = sp.vel_in;
+    a.id_in = sp.id_in;
+    a.pos_out = sp.pos_out;
+    a.vel_out = sp.vel_out;
+    a.id_out = sp.id_out;
+    a.skey = sp.skey;
+    a.perm = sp.perm;
+    a.soa = sp.soa_out;
+    a.queue = sp.queue;
+    a.err = sp.err;
+    a.halt = sp.halt;
+    a.gather = gather;
+    if (tiles <= kWideTiles)
+        hipLaunchKernelGGL(cell_sort_kernel<1024>, dim3(tiles), dim3(1024), 0, st, a);
+    else
+        hipLaunchKernelGGL(cell_sort_kernel<256>, dim3(tiles), dim3(256), 0, st, a);
+}
+
 hipError_t launch_sort_keys(hipStream_t st, const SortPlan& sp) {
     if (sp.n == 0) return hipSuccess;
-    // The cell-start table (both modes).
-    const uint32_t stiles = scan_tiles(sp.ncells);
-    if (stiles > kInlineTiles)
-        hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(kTileScanBlock), 0, st, sp.count, sp.ncells, stiles,
-                           sp.halt);
-    hipLaunchKernelGGL(cell_scan_kernel, dim3(stiles), dim3(kSortBlock), 0, st, sp.count, sp.cstart, sp.ncells,
-                       sp.queue, sp.halt, sp.tile_pre);
     if (sp.mode == kSortCellCount) {
-        hipLaunchKernelGGL(cell_scatter_kernel, dim3(blocks_for(sp.n, 256)), dim3(256), 0, st, sp.n, sp.ncells,
-                           sp.key0, sp.rank0, sp.cstart, sp.tmp, sp.err, sp.halt);
+        launch_cell_sort(st, sp, 1);
         return hipGetLastError();
     }
+    launch_cell_sort(st, sp, 0);
     if (sp.halt) return hipErrorInvalidValue;  // the frame loop runs the cell-count sort only
     const uint32_t tiles = sort_tiles(sp.n, sp.items);
     const uint32_t hist_blocks = (sp.n + kSortBlock * kHistItems - 1) / (kSortBlock * kHistItems);
@@ -578,17 +720,10 @@ hipError_t launch_sort_keys(hipStream_t st, const SortPlan& sp) {
 
 hipError_t launch_sort_gather(hipStream_t st, const SortPlan& sp) {
     if (sp.n == 0) return hipSuccess;
-    uint32_t* tsum = sp.count + sp.ncells;  // per-tile sums, cleared once the scan has read them
-    const uint32_t tsum_words = scan_tiles(sp.ncells);
-    if (sp.mode == kSortCellCount)
-        hipLaunchKernelGGL(cell_rank_kernel, dim3(blocks_for(sp.n, sp.reorder_block)), dim3(sp.reorder_block), 0,
-                           st, sp.n, sp.ncells, sp.key0, sp.rank0, sp.cstart, sp.tmp, sp.pos_in, sp.vel_in, sp.id_in,
-                           sp.pos_out, sp.vel_out, sp.id_out, sp.skey, sp.perm, tsum,
-                           tsum_words, sp.err, sp.soa_out, sp.halt);
-    else
+    if (sp.mode == kSortRadix)
         hipLaunchKernelGGL(radix_reorder_kernel, dim3(blocks_for(sp.n, sp.reorder_block)), dim3(sp.reorder_block),
                            0, st, sp.n, sp.perm, sp.pos_in, sp.vel_in, sp.id_in, sp.pos_out, sp.vel_out,
-                           sp.id_out, sp.hist, tsum, tsum_words, sp.err, sp.soa_out);
+                           sp.id_out, sp.hist, sp.err, sp.soa_out);
     return hipGetLastError();
 }
 

@@ -514,9 +514,18 @@ __device__ __forceinline__ uint32_t force_one_staged(const StepArgs& a, const Sc
     return active ? force_finish(a, sc, k, pi, vi, f) : 0u;
 }
 
+// The sort has read the tile sums; the density pass clears them for the
+// integrate pass.
+__device__ __forceinline__ void clear_tile_sums(const StepArgs& a) {
+    const uint32_t words = (a.ncells + kTileCells - 1u) >> kTileShift;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
+        a.head[a.ncells + i] = 0u;
+}
+
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void density_kernel(StepArgs a) {
     if (a.halt && *a.halt) return;
+    clear_tile_sums(a);
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
     const __amdgpu_buffer_rsrc_t rx = buffer_of(a.soa, a.n);
     const __amdgpu_buffer_rsrc_t ry = buffer_of(a.soa + a.n, a.n);
@@ -535,6 +544,7 @@ __global__ __launch_bounds__(BLOCK) void density_kernel(StepArgs a) {
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void density_staged_kernel(StepArgs a) {
     if (a.halt && *a.halt) return;
+    clear_tile_sums(a);
     __shared__ DensitySlot s_slot[BLOCK / 64];
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
     const __amdgpu_buffer_rsrc_t rcs = buffer_of(a.cstart, a.ncells + 1u);
@@ -562,17 +572,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
         const bool active = k < sc.p_end;
         uint32_t key = 0;
         if (active) key = force_one(a, sc, k, rpos, rvel, rcs);
-        // Next step's key and its slot in the per-cell count (whole wave).
-        const uint32_t slot = count_slot(a.count, a.count + a.ncells, key, active);
+        // Next step's key, its run in the cell's chain and the tile sums (whole wave).
+        push_run(a.head, a.next, key, k, active);
+        add_tile_sums(a.head + a.ncells, key, active);
         if (a.vmax2) {
             float4 vn = make_float4(0.f, 0.f, 0.f, 0.f);
             if (active) vn = a.vel_o[k];
             wave_max_v2(a.vmax2, ti.x, vn.x, vn.y, vn.z, active);
         }
-        if (active) {
-            a.key0[k] = key;
-            a.rank0[k] = slot;
-        }
+        if (active) a.key0[k] = key;
     });
 }
 
@@ -596,23 +604,35 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
         const uint32_t k = ti.y + threadIdx.x;
         const bool active = k < sc.p_end;
         const uint32_t key = force_one_staged(a, sc, k, active, rpos, rvel, rcs, slot_a, slot_b);
-        const uint32_t cslot = count_slot(a.count, a.count + a.ncells, key, active);
+        // Next step's key, its run in the cell's chain and the tile sums (whole wave).
+        push_run(a.head, a.next, key, k, active);
+        add_tile_sums(a.head + a.ncells, key, active);
         if (a.vmax2) {
             float4 vn = make_float4(0.f, 0.f, 0.f, 0.f);
             if (active) vn = a.vel_o[k];
             wave_max_v2(a.vmax2, ti.x, vn.x, vn.y, vn.z, active);
         }
-        if (active) {
-            a.key0[k] = key;
-            a.rank0[k] = cslot;
-        }
+        if (active) a.key0[k] = key;
     });
 }
 
+// Uploads come in any order, a lattice's fastest axis often across the
+// cells' rows, so a wave's particles can lie in as many tiles as it has lanes
+// and one atomic per run would queue on the few tile sums of a small grid: a
+// block counts them in LDS first (grids of up to kHashTiles tiles).
+constexpr uint32_t kHashTiles = 2048;
+
 __global__ void hash_kernel(const float4* __restrict__ pos, const float4* __restrict__ vel,
-                            uint32_t* __restrict__ key0, uint32_t* __restrict__ rank0, uint32_t* __restrict__ count,
+                            uint32_t* __restrict__ key0, uint32_t* __restrict__ next, uint32_t* __restrict__ head,
                             uint32_t ncells, uint32_t* __restrict__ vmax2, const SceneConst* __restrict__ scenes,
                             const uint2* __restrict__ tiles, uint32_t ntiles) {
+    __shared__ uint32_t s_sum[kHashTiles];
+    const uint32_t gt = (ncells + kTileCells - 1u) >> kTileShift;
+    const bool local = gt <= kHashTiles;
+    if (local) {
+        for (uint32_t i = threadIdx.x; i < gt; i += blockDim.x) s_sum[i] = 0u;
+        __syncthreads();
+    }
     uint32_t t0, t1;
     tile_span(ntiles, t0, t1);
     for (uint32_t t = t0; t < t1; ++t) {
@@ -625,16 +645,22 @@ __global__ void hash_kernel(const float4* __restrict__ pos, const float4* __rest
             const float4 p = pos[k];
             key = cell_key(sc, p.x, p.y, p.z);
         }
-        const uint32_t slot = count_slot(count, count + ncells, key, active);
-        if (active) {
-            key0[k] = key;
-            rank0[k] = slot;
-        }
+        push_run(head, next, key, k, active);
+        if (!local)
+            add_tile_sums(head + ncells, key, active);
+        else if (active)
+            atomicAdd(&s_sum[key >> kTileShift], 1u);
+        if (active) key0[k] = key;
         if (vmax2) {
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
             if (active) v = vel[k];
             wave_max_v2(vmax2, ti.x, v.x, v.y, v.z, active);
         }
+    }
+    if (local) {
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < gt; i += blockDim.x)
+            if (s_sum[i]) atomicAdd(head + ncells + i, s_sum[i]);
     }
 }
 
@@ -793,10 +819,10 @@ int force_blocks_per_cu(int block, int staged) {
 }
 
 hipError_t launch_hash(hipStream_t st, int block, uint32_t grid, const float4* pos, const float4* vel,
-                       uint32_t* key0, uint32_t* rank0, uint32_t* count, uint32_t ncells, uint32_t* vmax2,
+                       uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t ncells, uint32_t* vmax2,
                        const SceneConst* scenes, const uint2* tiles, uint32_t ntiles) {
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL(hash_kernel, dim3(grid), dim3(block), 0, st, pos, vel, key0, rank0, count, ncells, vmax2,
+    hipLaunchKernelGGL(hash_kernel, dim3(grid), dim3(block), 0, st, pos, vel, key0, next, head, ncells, vmax2,
                        scenes, tiles, ntiles);
     return hipGetLastError();
 }
