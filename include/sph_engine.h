@@ -161,7 +161,7 @@ int  sph_scene_sample_ball(uint64_t seed, const float* centre, float radius, flo
  * hipMalloc): one step of n particles whose state the caller holds in device
  * memory, enqueued on `stream` (a hipStream_t; NULL = the default stream),
  * with every intermediate in a fixed scratch array of the library (about
- * 17 MB per GPU, held until the process ends).  xyz_in, vel_in (may be NULL:
+ * 24 MB per GPU, held until the process ends).  xyz_in, vel_in (may be NULL:
  * zero velocity), xyz_out, vel_out: device arrays of 3n floats in the
  * caller's particle order.  The step and its results equal the first
  * sph_advance_steps step of a handle given the same particles and params
@@ -234,8 +234,10 @@ int  sph_autotune(sph_handle* h);
  * force run as persistent blocks taking tiles from per-XCD queues (clear:
  * one block per tile), bit 1 set when the force pass stages each row's
  * candidates in LDS (clear: it gathers them from global memory), bit 2 the
- * same for the density pass.  Every choice gives the same results bit for
- * bit.                                                                      */
+ * same for the density pass.  A handle of at most 40,960 particles (640 tiles
+ * of 64, scene by scene) runs density and force in a form of its own that
+ * none of these shape, until sph_set_tuning asks for the forms above.  Every
+ * choice gives the same results bit for bit.                                */
 int  sph_get_tuning(const sph_handle* h, int* cfg5);
 int  sph_set_tuning(sph_handle* h, const int* cfg5);
 /* Sort used to order particles by cell (no reference counterpart; both give

@@ -5,7 +5,8 @@
 // with HIP events on the handle's own state.  The state is saved first and
 // restored before every trial, so all candidates run the same steps.
 // Results are cached per process, keyed by device arch, particle-count
-// bucket (power of two) and scene count.
+// bucket (power of two) and scene count.  A handle small enough for the split
+// form runs that, which has no shape to choose.
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -39,6 +40,11 @@ extern "C" int sph_autotune(sph_handle* h) {
     BudgetScope budget_scope(h ? &h->mem : nullptr);
     if (!h) return SPH_E_INVALID;
     if (!h->ready) return fail(h, SPH_E_NOT_READY, "call sph_make_ready first");
+    h->tune.split = 1;
+    if (split_form(h)) {  // has no shape to choose
+        invalidate_graph(h);
+        return SPH_OK;
+    }
     const std::string key = cache_key(h);
     {
         std::lock_guard<std::mutex> lk(g_mu);
@@ -100,6 +106,7 @@ extern "C" int sph_autotune(sph_handle* h) {
                    {&best.reorder_block, blocks, 4, SPH_PASS_REORDER},
                    {&best.sort_items, items, 4, SPH_PASS_SORT}};
     for (const Axis& ax : axes) {
+        if (rc != SPH_OK) break;
         // The gather's block and the keys per thread only shape the radix sort.
         if ((ax.field == &best.sort_items || ax.field == &best.reorder_block) && best.sort_mode != kSortRadix)
             continue;

@@ -181,20 +181,26 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const T* p, uint32_t
     return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, (int)(n * (uint32_t)sizeof(T)), 0x00020000);
 }
 
-// Window [lo, hi) of row (dy, dz); rcs is a buffer over cstart.
-__device__ __forceinline__ void row_window(__amdgpu_buffer_rsrc_t rcs, const SceneConst& sc, const RowGeom& g,
-                                           int dy, int dz, uint32_t& lo, uint32_t& hi) {
+// Window [lo, hi) of the row whose cell (x = 0) is c, for a particle whose
+// chord there has the squared half length w2; rcs is a buffer over cstart.
+__device__ __forceinline__ void chord_window(__amdgpu_buffer_rsrc_t rcs, const SceneConst& sc, float fx, float w2,
+                                             uint32_t c, uint32_t& lo, uint32_t& hi) {
     lo = 0u;
     hi = 0u;
-    const float w2 = sc.hc2 - (g.qy[dy + 1] + g.qz[dz + 1]);
     if (!(w2 > 0.0f)) return;
     const float wx = __builtin_amdgcn_sqrtf(w2) * sc.xsubf + sc.wmargin;
     const float gmax = (float)(sc.G[0] - 1);
-    const uint32_t x0 = (uint32_t)(int)fminf(fmaxf(g.fx - wx, 0.0f), gmax);
-    const uint32_t x1 = (uint32_t)(int)fminf(fmaxf(g.fx + wx, 0.0f), gmax);
-    const uint32_t c = g.row0 + (uint32_t)(dz * sc.G[1] + dy) * (uint32_t)sc.G[0];
+    const uint32_t x0 = (uint32_t)(int)fminf(fmaxf(fx - wx, 0.0f), gmax);
+    const uint32_t x1 = (uint32_t)(int)fminf(fmaxf(fx + wx, 0.0f), gmax);
     lo = __builtin_amdgcn_raw_buffer_load_b32(rcs, (int)((c + x0) << 2), 0, 0);
     hi = __builtin_amdgcn_raw_buffer_load_b32(rcs, (int)((c + x1 + 1u) << 2), 0, 0);
+}
+
+// Window of row (dy, dz).
+__device__ __forceinline__ void row_window(__amdgpu_buffer_rsrc_t rcs, const SceneConst& sc, const RowGeom& g,
+                                           int dy, int dz, uint32_t& lo, uint32_t& hi) {
+    const float w2 = sc.hc2 - (g.qy[dy + 1] + g.qz[dz + 1]);
+    chord_window(rcs, sc, g.fx, w2, g.row0 + (uint32_t)(dz * sc.G[1] + dy) * (uint32_t)sc.G[0], lo, hi);
 }
 
 // Row masks.  The density pass tests a row's candidates [lo, hi) four at a
@@ -228,6 +234,23 @@ __device__ __forceinline__ void row_neighbors(uint32_t lo, uint32_t hi, uint32_t
 __device__ __forceinline__ uint32_t row_first(uint32_t lo, uint32_t hi) {
     const uint32_t span = mask_span(lo, hi);
     return span > 32u ? lo + span - 32u : lo;
+}
+
+// The same for `words` words together (the one before the mask holds the 32
+// slots before the mask's).
+__device__ __forceinline__ uint32_t row_first(uint32_t lo, uint32_t hi, uint32_t words) {
+    const uint32_t span = mask_span(lo, hi), w = words * 32u;
+    return span > w ? lo + span - w : lo;
+}
+
+// A word's slots as bits in ascending order of candidates: of the word whose
+// last slot is `after` slots before the row's end, bit i is candidate
+// row_first(lo, hi, 1 + after / 32) + i.
+__device__ __forceinline__ uint32_t mask_ascending(uint32_t word, uint32_t span, uint32_t after) {
+    uint32_t r = __builtin_bitreverse32(word);
+    const uint32_t slots = span - after;
+    if (slots - 1u < 31u) r >>= 32u - slots;
+    return r;
 }
 
 // row_neighbors with the mask's visits given as offsets: g(i) for candidate
@@ -356,7 +379,8 @@ struct LaneRun {
 __device__ __forceinline__ LaneRun lane_run(uint32_t v, bool active) {
     const int lane = (int)(threadIdx.x & 63u);
     const uint32_t kk = active ? v : 0xffffffffu;
-    const uint32_t prev = __shfl_up(kk, 1, 64);
+    // The lane below's value (DPP wave_shr:1).
+    const uint32_t prev = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)kk, 0x138, 0xF, 0xF, false);
     LaneRun r;
     r.first = active && (lane == 0 || prev != kk);
     const uint64_t starts = __ballot(r.first);
@@ -385,11 +409,19 @@ __device__ __forceinline__ void push_run(uint32_t* __restrict__ head, uint32_t* 
 }
 
 // Adds the wave's particles to their tiles' sums: one atomic per run of
-// lanes in one tile.
+// lanes in one tile, or one in all where the wave has a single tile.
 __device__ __forceinline__ void add_tile_sums(uint32_t* __restrict__ tsum, uint32_t key, bool active) {
-    const LaneRun r = lane_run(key >> kTileShift, active);
-    const int lane = (int)(threadIdx.x & 63u);
-    if (r.first) atomicAdd(tsum + (key >> kTileShift), (uint32_t)(r.end - lane));
+    const uint32_t lane = threadIdx.x & 63u, tile = key >> kTileShift;
+    const uint64_t act = __ballot(active);
+    if (act == 0u) return;
+    const uint32_t first = (uint32_t)__builtin_ctzll(act);
+    const uint32_t one = (uint32_t)__builtin_amdgcn_readlane((int)tile, (int)first);
+    if (__ballot(active && tile != one) == 0u) {
+        if (lane == first) atomicAdd(tsum + one, (uint32_t)__popcll(act));
+        return;
+    }
+    const LaneRun r = lane_run(tile, active);
+    if (r.first) atomicAdd(tsum + tile, (uint32_t)(r.end - (int)lane));
 }
 
 // Adds the wave's largest |v|^2 to arr[idx] (float bits; atomic max on the

@@ -190,6 +190,10 @@ uint32_t grid_for(sph_handle* h, int block, uint32_t ntiles, uint32_t** queue, i
     return resident;
 }
 
+bool split_form(const sph_handle* h) {
+    return h->tune.split && h->split_tiles <= kSplitTiles && h->nlist.p && h->ncount.p;
+}
+
 StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     StepArgs a;
     std::memset(&a, 0, sizeof(a));
@@ -206,6 +210,8 @@ StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     a.cstart = w.cstart.p;
     a.rho = w.rho.p;
     a.mask = w.mask.p;
+    a.nlist = h->nlist.p;
+    a.ncount = h->ncount.p;
     a.acc = (h->keep_acc || w.acc.p) ? w.acc.p : nullptr;
     a.scenes = h->sc_d.p;
     a.tiles = tiles_for(h, block, a.ntiles);
@@ -268,7 +274,15 @@ static int ensure_buffers(sph_handle* h) {
     if (fresh_head) chk(launch_fill_u32(h->stream, h->head.p, 0u, head_words));
     chk(hipMemcpyAsync(h->sc_d.p, h->sc_h.data(), h->sc_h.size() * sizeof(SceneConst), hipMemcpyHostToDevice, h->stream));
     if (e != hipSuccess) return hip_fail(h, e, "buffer init");
-    return alloc_step_bufs(h, h->work);
+    const int rc = alloc_step_bufs(h, h->work);
+    if (rc != SPH_OK) return rc;
+    // Only speeds small steps up: a handle with no room for it does without.
+    if (h->split_tiles <= kSplitTiles && (h->nlist.ensure((size_t)kListMax * n) != hipSuccess || h->ncount.ensure(n) != hipSuccess)) {
+        h->nlist.release();
+        h->mem.refused = 0;
+        (void)hipGetLastError();
+    }
+    return SPH_OK;
 }
 
 static void prof_record(sph_handle* h, int slot) {
@@ -329,7 +343,8 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     sp.vel_in = h->vel.p;
     sp.id_in = h->id.p;
     sp.pos_out = w.pos_s.p;
-    sp.soa_out = h->tune.density_staged ? nullptr : w.soa.p;
+    const bool split = split_form(h);
+    sp.soa_out = h->tune.density_staged || split ? nullptr : w.soa.p;
     sp.halt = frame;
     sp.vel_out = w.vel_s.p;
     sp.id_out = w.id_s.p;
@@ -339,7 +354,12 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     e = launch_sort_gather(st, sp);
     if (e != hipSuccess) return hip_fail(h, e, "reorder launch");
     if (record_prof) prof_record(h, 3);
-    {
+    if (split) {
+        StepArgs a = step_args(h, w, kSplitTile);
+        a.halt = frame;
+        e = launch_density_split(st, a);
+        if (e != hipSuccess) return hip_fail(h, e, "density launch");
+    } else {
         StepArgs a = step_args(h, w, h->tune.density_block);
         a.halt = frame;
         const uint32_t grid = grid_for(h, h->tune.density_block, a.ntiles, &a.queue);
@@ -352,7 +372,13 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
         e = launch_cfl(st, (uint32_t)h->sc_h.size(), h->sc_d.p, h->vmax2.p, h->dt_dev.p, frame);
         if (e != hipSuccess) return hip_fail(h, e, "cfl launch");
     }
-    {
+    if (split) {
+        StepArgs a = step_args(h, w, kSplitTile);
+        a.vmax2 = h->cfl ? h->vmax2.p : nullptr;
+        a.halt = frame;
+        e = launch_force_split(st, a);
+        if (e != hipSuccess) return hip_fail(h, e, "force launch");
+    } else {
         StepArgs a = step_args(h, w, h->tune.force_block);
         a.vmax2 = h->cfl ? h->vmax2.p : nullptr;
         a.halt = frame;
@@ -449,6 +475,8 @@ static int configure(sph_handle* h, const std::vector<sph_params>& ps, const std
     h->n = (uint32_t)p_off;
     h->ncells = (uint32_t)cell_off;
     h->passes = sort_key_passes(h->ncells);
+    h->split_tiles = 0;
+    for (uint32_t v : ns) h->split_tiles += (v + kSplitTile - 1) / kSplitTile;
     h->xsub = xsub;
     h->cfl = ps.size() == 1 && ps[0].cfl_number > 0.f;
     h->tiles.clear();
@@ -638,7 +666,7 @@ static int capture_graph(sph_handle* h, GraphKind kind = kGraphOne) {
     // Tile tables are built on first use with a synchronous copy, which a
     // capturing stream does not allow: build the ones the step uses first
     // (a block size set after steps have run has none yet).
-    const int blocks[] = {h->tune.density_block, h->tune.force_block};
+    const int blocks[] = {h->tune.density_block, h->tune.force_block, kSplitTile};
     for (int b : blocks) {
         uint32_t nt = 0;
         if (!tiles_for(h, b, nt)) return fail(h, SPH_E_OOM, "tile table");
@@ -1086,6 +1114,7 @@ int sph_set_tuning(sph_handle* h, const int* cfg) {
     h->tune.persistent = cfg[4] & 1;
     h->tune.force_staged = (cfg[4] >> 1) & 1;
     h->tune.density_staged = (cfg[4] >> 2) & 1;
+    h->tune.split = 0;
     invalidate_graph(h);
     return SPH_OK;
 }

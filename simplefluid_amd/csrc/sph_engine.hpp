@@ -93,6 +93,8 @@ struct Tuning {
     int persistent = 0;   // density and force: 0 one block per tile, 1 persistent blocks over tile queues
     int force_staged = 0; // force: 1 each row's candidates staged in LDS, 0 gathered from global memory
     int density_staged = 0;  // density: the same choice
+    int split = 1;        // density and force: 1 the split form where it applies (split_form), 0 the forms above
+                          // (sph_set_tuning)
     int sort_mode = kSortCellCount;
 };
 
@@ -133,6 +135,7 @@ struct sph_handle {
     uint32_t n = 0;
     uint32_t ncells = 0;
     int passes = 1;
+    uint32_t split_tiles = 0;              // tiles of the split form, scene by scene
     int xsub = 1;                          // x cells per y/z cell size
     int xsub_override = 0;                 // 0 = automatic
     bool ready = false;
@@ -148,6 +151,8 @@ struct sph_handle {
     // State (state order) and per-step buffers.
     sph::DevBuf<float4> pos, vel;
     sph::DevBuf<uint32_t> id, key0, next, head;
+    sph::DevBuf<uint16_t> nlist;           // split form's neighbour lists (left out under a memory limit
+    sph::DevBuf<uint32_t> ncount;          // they do not fit)
     sph::DevBuf<uint32_t> tmp;             // cell-count sort: members of the tiles too full for LDS
     sph::StepBufs work;
     sph::DevBuf<uint32_t> hist, status, tickets, err, queue;
@@ -217,6 +222,9 @@ uint2* tiles_for(sph_handle* h, int block, uint32_t& ntiles);
 // the launch is persistent, else null.
 // blocks_per_cu: the kernel's resident blocks per CU (0: 2048 lanes' worth).
 uint32_t grid_for(sph_handle* h, int block, uint32_t ntiles, uint32_t** queue, int blocks_per_cu = 0);
+// Density and force run in the split form: few enough tiles, its lists
+// allocated, and no other form asked for (sph_set_tuning).
+bool split_form(const sph_handle* h);
 StepArgs step_args(sph_handle* h, StepBufs& w, int block);
 // Enqueue one step reading/writing the state buffers with intermediates in w.
 // frame: device frame state (every kernel of the step skips once it is

@@ -63,16 +63,20 @@ struct StepArgs {
     float4* pos_s;           // sorted positions; w <- p/rho^2 (density pass)
     const float* soa;        // the same positions as x, y, z planes (3 N floats)
     float4* vel_s;           // sorted velocities; w <- 1/rho (density pass)
-    float4* pos_o;           // state out (integrate)
+    float4* pos_o;           // state out (integrate), or null with xyz_out
     float4* vel_o;
     const uint32_t* id_s;
     uint32_t* id_o;
     uint32_t* key0;          // next step's unsorted keys
-    uint32_t* head;          // next step's chain heads, then per-tile sums (atomic)
+    uint32_t* head;          // next step's chain heads, then per-tile sums (atomic); null: no next step
     uint32_t* next;          // next step's runs
     const uint32_t* cstart;  // cell-start table of this step
     float* rho;
     uint32_t* mask;
+    uint16_t* nlist;         // split form: neighbour lists, else null
+    uint32_t* ncount;        // split form: their lengths
+    float* xyz_out;          // state out in original order too (3 n floats each), or null
+    float* vel_out;
     float4* acc;             // optional: acceleration (sorted order)
     const SceneConst* scenes;
     const uint2* tiles;
@@ -91,6 +95,10 @@ constexpr int kQueueWords = 16;
 hipError_t launch_hash(hipStream_t st, int block, uint32_t grid, const float4* pos, const float4* vel,
                        uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t ncells, uint32_t* vmax2,
                        const SceneConst* scenes, const uint2* tiles, uint32_t ntiles);
+// Upload and hash of one scene in one pass (vel_in null: zero velocity).
+hipError_t launch_upload_hash(hipStream_t st, const float* xyz, const float* vel_in, float4* pos, float4* vel,
+                              uint32_t* id, uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t n,
+                              uint32_t ncells, const SceneConst& sc);
 // CFL step of every scene from its max |v|^2 (scenes with cfl = 0 keep dt);
 // clears vmax2 and stores scene 0's step in *dt_out.  With a frame state
 // (below) the kernel does nothing once the frame is halted, and otherwise
@@ -108,6 +116,24 @@ hipError_t launch_frame_gate(hipStream_t st, uint32_t* frame);
 hipError_t launch_density(hipStream_t st, int block, uint32_t grid, const StepArgs& a, int staged = 0);
 // staged: the force pass reads each row's candidates from LDS (same results).
 hipError_t launch_force(hipStream_t st, int block, uint32_t grid, const StepArgs& a, int staged = 0);
+// The split form of both passes, for at most kSplitMax particles: tiles of 64
+// particles, a block of nine waves (density) or four (force) each; the
+// density pass leaves every particle's neighbours as a list of kListMax
+// indices for the force pass (a particle with more is walked by its masks).
+// Same results as the other forms, bit for bit.
+constexpr uint32_t kSplitMax = 65536;   // the lists hold 16-bit indices
+constexpr uint32_t kListMax = 64;
+constexpr int kSplitTile = 64;
+// Tiles up to which handles take it.  Two force blocks fit a CU, so 512 tiles
+// run at once; from there on the chip is full and its extra work shows.
+// Measured per step, the split form against the best of the others: 512
+// particles 17.9 against 30.2 us, 4,096 18.0 against 27.8, 23,520 21.7 against
+// 31.9, 32,768 (512 tiles) 22.6 against 30.6, 40,960 (640) 31.0 against 31.8,
+// 49,152 (768) 32.5 against 32.5, 57,800 39.0 against 34.3.
+constexpr uint32_t kSplitTiles = 640;
+static_assert(kSplitTiles * kSplitTile <= kSplitMax, "every handle of so many tiles has 16-bit indices");
+hipError_t launch_density_split(hipStream_t st, const StepArgs& a);
+hipError_t launch_force_split(hipStream_t st, const StepArgs& a);
 // Resident blocks per CU of the force kernel at this block size and form
 // (the runtime's occupancy figure; 0 if it cannot say).
 int force_blocks_per_cu(int block, int staged);

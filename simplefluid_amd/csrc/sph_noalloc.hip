@@ -7,15 +7,15 @@
 //
 // The step is the one sph_advance_steps runs as the first step after
 // sph_set_particles (hash, cell-count sort, gather, density, force), with the
-// same kernels, the same grid rule and the default launch shape, so its
-// results equal that entry point's bit for bit.
+// same kernels in their split form and the same grid rule, so its results
+// equal that entry point's bit for bit.
 //
 // Limits: at most kMaxParticles particles and kMaxCells grid cells (the
 // largest x subdivision of 4, 2, 1 whose grid fits is used, as a handle of
 // that size would pick).  Every call on one GPU shares that GPU's scratch:
 // calls that overlap on one GPU race, and each call rewrites the scratch
-// from the start (chain heads, tile prefixes, error word and tile queues are
-// cleared by kernels, not by memset, so the call may be graph-captured).
+// from the start (chain heads, tile prefixes and the error word are cleared by
+// a kernel, not by memset, so the call may be graph-captured).
 #include <cstring>
 #include <mutex>
 
@@ -27,8 +27,8 @@ namespace {
 
 constexpr uint32_t kMaxParticles = 65536;
 constexpr uint32_t kMaxCells = 1u << 20;
-constexpr int kBlock = 256;
-constexpr uint32_t kMaxTiles = kMaxParticles / kBlock;
+constexpr uint32_t kMaxTiles = kMaxParticles / kSplitTile;
+static_assert(kMaxParticles <= kSplitMax, "the step runs in the split form");
 constexpr uint32_t kScanTilesMax = (kMaxCells + kTileCells - 1u) / kTileCells;
 
 // Byte offsets of the arrays inside the scratch, each 256-byte aligned.
@@ -39,27 +39,25 @@ struct Layout {
     static constexpr size_t vel = align256(pos + 16 * N);
     static constexpr size_t pos_s = align256(vel + 16 * N);
     static constexpr size_t vel_s = align256(pos_s + 16 * N);
-    static constexpr size_t soa = align256(vel_s + 16 * N);
-    static constexpr size_t id = align256(soa + 12 * N);
+    static constexpr size_t id = align256(vel_s + 16 * N);
     static constexpr size_t id_s = align256(id + 4 * N);
     static constexpr size_t key0 = align256(id_s + 4 * N);
     static constexpr size_t next = align256(key0 + 4 * N);
-    static constexpr size_t skey = align256(next + 4 * N);
-    static constexpr size_t perm = align256(skey + 4 * N);
-    static constexpr size_t tmp = align256(perm + 4 * N);
-    static constexpr size_t rho = align256(tmp + 4 * N);
+    static constexpr size_t tmp = align256(next + 4 * N);
+    static constexpr size_t nlist = align256(tmp + 4 * N);
+    static constexpr size_t ncount = align256(nlist + 2 * (size_t)kListMax * N);
+    static constexpr size_t rho = align256(ncount + 4 * N);
     static constexpr size_t mask = align256(rho + 4 * N);
     static constexpr size_t head = align256(mask + 4 * (size_t)kRows * N);
-    static constexpr size_t cstart = align256(head + 4 * ((size_t)kMaxCells + 2 * kScanTilesMax));
+    static constexpr size_t cstart = align256(head + 4 * ((size_t)kMaxCells + 2 * kScanTilesMax) + 16);
     static constexpr size_t tile_pre = align256(cstart + 4 * ((size_t)kMaxCells + 1));
     static constexpr size_t tiles = align256(tile_pre + 4 * (size_t)kScanTilesMax);
     static constexpr size_t scene = align256(tiles + 8 * (size_t)kMaxTiles);
     static constexpr size_t err = align256(scene + sizeof(SceneConst));
-    static constexpr size_t queue = align256(err + 4);
-    static constexpr size_t total = align256(queue + 4 * (size_t)kQueueWords);
+    static constexpr size_t total = align256(err + 4);
 };
 
-// The step's scratch on each GPU the library runs on (about 17 MB), held
+// The step's scratch on each GPU the library runs on (about 24 MB), held
 // until the process ends.  Host code reaches it only through the address
 // hipGetSymbolAddress returns on that device.
 static __device__ __align__(256) uint8_t scratch[Layout::total];
@@ -68,17 +66,23 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 void* g_scratch[kMaxDevices] = {};
 
-// Scene constants, the tile table (scene 0, first particle t * kBlock), the
-// identity ids, and the error word and tile queues cleared.
-__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t n, uint8_t* __restrict__ base) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k == 0) *reinterpret_cast<SceneConst*>(base + Layout::scene) = sc;
-    if (k < (uint32_t)kQueueWords) reinterpret_cast<uint32_t*>(base + Layout::queue)[k] = 0u;
-    if (k == 0) *reinterpret_cast<uint32_t*>(base + Layout::err) = 0u;
-    if (k < n) {
-        reinterpret_cast<uint32_t*>(base + Layout::id)[k] = k;
-        if (k % kBlock == 0) reinterpret_cast<uint2*>(base + Layout::tiles)[k / kBlock] = make_uint2(0u, k);
+// Scene constants, the tile table (scene 0, first particle t * kSplitTile),
+// empty chains, tile sums and tile prefixes, and the error word cleared.
+__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint8_t* __restrict__ base) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    if (i == 0) {
+        *reinterpret_cast<SceneConst*>(base + Layout::scene) = sc;
+        *reinterpret_cast<uint32_t*>(base + Layout::err) = 0u;
     }
+    const uint32_t T = (ncells + kTileCells - 1u) >> kTileShift;
+    uint32_t* head = reinterpret_cast<uint32_t*>(base + Layout::head);
+    // Whole 16-byte words; the scratch behind the last tile sum is unused.
+    for (uint32_t w = i; w < (ncells + 2u * T + 3u) / 4u; w += stride)
+        reinterpret_cast<uint4*>(head)[w] = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t* tile_pre = reinterpret_cast<uint32_t*>(base + Layout::tile_pre);
+    for (uint32_t t = i; t < T; t += stride) tile_pre[t] = 0xffffffffu;
+    uint2* tiles = reinterpret_cast<uint2*>(base + Layout::tiles);
+    for (uint32_t t = i; t * kSplitTile < sc.p_end; t += stride) tiles[t] = make_uint2(0u, t * kSplitTile);
 }
 
 // The scratch address on the current device, looked up once per device.
@@ -140,68 +144,52 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     float4* vel = reinterpret_cast<float4*>(at(Layout::vel));
     uint32_t* id = reinterpret_cast<uint32_t*>(at(Layout::id));
     uint32_t* head = reinterpret_cast<uint32_t*>(at(Layout::head));
-    const uint32_t T = scan_tiles(C);
-    const uint32_t ntiles = (n + kBlock - 1) / kBlock;
-
-    hipLaunchKernelGGL(noalloc_setup_kernel, dim3((n + 255) / 256), dim3(256), 0, st, sc, n, base);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = launch_fill_u32(st, head, 0u, (size_t)C + 2 * (size_t)T);
-    if (e == hipSuccess) e = launch_fill_u32(st, reinterpret_cast<uint32_t*>(at(Layout::tile_pre)), 0xffffffffu, T);
-    if (e == hipSuccess) e = launch_pack3(st, n, xyz_in, pos);
-    if (e == hipSuccess) e = launch_pack3(st, n, vel_in, vel);
-    const SceneConst* scd = reinterpret_cast<const SceneConst*>(at(Layout::scene));
-    const uint2* tiles = reinterpret_cast<const uint2*>(at(Layout::tiles));
     uint32_t* key0 = reinterpret_cast<uint32_t*>(at(Layout::key0));
     uint32_t* next = reinterpret_cast<uint32_t*>(at(Layout::next));
-    if (e == hipSuccess) e = launch_hash(st, kBlock, ntiles, pos, vel, key0, next, head, C, nullptr, scd, tiles, ntiles);
+    const SceneConst* scd = reinterpret_cast<const SceneConst*>(at(Layout::scene));
+
+    // Five launches: setup, upload and hash, sort, density, force (which
+    // writes the caller's arrays itself).
+    hipLaunchKernelGGL(noalloc_setup_kernel, dim3(256), dim3(256), 0, st, sc, C, base);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = launch_upload_hash(st, xyz_in, vel_in, pos, vel, id, key0, next, head, n, C, sc);
     SortPlan sp;
     sp.n = n;
     sp.ncells = C;
     sp.mode = kSortCellCount;
-    sp.reorder_block = kBlock;
     sp.key0 = key0;
     sp.head = head;
     sp.next = next;
     sp.cstart = reinterpret_cast<uint32_t*>(at(Layout::cstart));
     sp.tile_pre = reinterpret_cast<uint32_t*>(at(Layout::tile_pre));
     sp.tmp = reinterpret_cast<uint32_t*>(at(Layout::tmp));
-    sp.skey = reinterpret_cast<uint32_t*>(at(Layout::skey));
-    sp.perm = reinterpret_cast<uint32_t*>(at(Layout::perm));
     sp.err = reinterpret_cast<uint32_t*>(at(Layout::err));
-    sp.queue = reinterpret_cast<uint32_t*>(at(Layout::queue));
     sp.pos_in = pos;
     sp.vel_in = vel;
     sp.id_in = id;
     sp.pos_out = reinterpret_cast<float4*>(at(Layout::pos_s));
     sp.vel_out = reinterpret_cast<float4*>(at(Layout::vel_s));
     sp.id_out = reinterpret_cast<uint32_t*>(at(Layout::id_s));
-    sp.soa_out = reinterpret_cast<float*>(at(Layout::soa));
     if (e == hipSuccess) e = launch_sort_keys(st, sp);
-    if (e == hipSuccess) e = launch_sort_gather(st, sp);
     StepArgs a;
     std::memset(&a, 0, sizeof(a));
     a.pos_s = sp.pos_out;
-    a.soa = sp.soa_out;
     a.vel_s = sp.vel_out;
-    a.pos_o = pos;   // the new state, in sorted order, back into the input slots
-    a.vel_o = vel;
     a.id_s = sp.id_out;
-    a.id_o = id;
-    a.key0 = key0;
-    a.next = next;
-    a.head = head;
+    a.xyz_out = xyz_out;
+    a.vel_out = vel_out;
     a.cstart = sp.cstart;
     a.rho = reinterpret_cast<float*>(at(Layout::rho));
     a.mask = reinterpret_cast<uint32_t*>(at(Layout::mask));
+    a.nlist = reinterpret_cast<uint16_t*>(at(Layout::nlist));
+    a.ncount = reinterpret_cast<uint32_t*>(at(Layout::ncount));
     a.scenes = scd;
-    a.tiles = tiles;
-    a.ntiles = ntiles;
+    a.tiles = reinterpret_cast<const uint2*>(at(Layout::tiles));
+    a.ntiles = (n + kSplitTile - 1) / kSplitTile;
     a.n = n;
     a.ncells = C;
-    if (e == hipSuccess) e = launch_density(st, kBlock, ntiles, a);
-    if (e == hipSuccess) e = launch_force(st, kBlock, ntiles, a);
-    if (e == hipSuccess) e = launch_unpermute3(st, n, pos, id, xyz_out);
-    if (e == hipSuccess) e = launch_unpermute3(st, n, vel, id, vel_out);
+    if (e == hipSuccess) e = launch_density_split(st, a);
+    if (e == hipSuccess) e = launch_force_split(st, a);
     if (e != hipSuccess) return fail_noalloc(SPH_E_HIP, "sph_step_noalloc: kernel launch failed");
     return SPH_OK;
 }

@@ -59,6 +59,20 @@ __device__ __forceinline__ void density_trip(const float4& pi, float h2, const f
     }
 }
 
+// Density, EOS and their stores from the neighbours' sum and the walls'.
+__device__ __forceinline__ void density_finish(const StepArgs& a, const SceneConst& sc, uint32_t k, float sum,
+                                               float wr) {
+    const float rho = sc.cD * sum + sc.rho0 * wr;
+    const float p = eos(sc, rho);
+    const float ir = 1.0f / rho;
+    a.rho[k] = rho;
+    // p/rho^2 and 1/rho ride in the unused w of the sorted position and
+    // velocity, so the force pass gets them with the same loads.  Neighbour
+    // reads of pos_s in this pass take x, y, z only.
+    reinterpret_cast<float*>(a.pos_s + k)[3] = (p * ir) * ir;
+    reinterpret_cast<float*>(a.vel_s + k)[3] = ir;
+}
+
 __device__ __forceinline__ void density_one(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                             __amdgpu_buffer_rsrc_t rpos, __amdgpu_buffer_rsrc_t rx,
                                             __amdgpu_buffer_rsrc_t ry, __amdgpu_buffer_rsrc_t rz,
@@ -102,15 +116,7 @@ __device__ __forceinline__ void density_one(const StepArgs& a, const SceneConst&
         wr += wall_rho((pk[d] - sc.bmin[d]) * sc.inv_h);
         wr += wall_rho((sc.wmax[d] - pk[d]) * sc.inv_h);
     }
-    const float rho = sc.cD * sum + sc.rho0 * wr;
-    const float p = eos(sc, rho);
-    const float ir = 1.0f / rho;
-    a.rho[k] = rho;
-    // p/rho^2 and 1/rho ride in the unused w of the sorted position and
-    // velocity, so the force pass gets them with the same loads.  Neighbour
-    // reads of pos_s in this pass take x, y, z only.
-    reinterpret_cast<float*>(a.pos_s + k)[3] = (p * ir) * ir;
-    reinterpret_cast<float*>(a.vel_s + k)[3] = ir;
+    density_finish(a, sc, k, sum, wr);
 }
 
 // Candidates a wave stages per row in the density pass, plus the slots a
@@ -297,12 +303,7 @@ __device__ __forceinline__ void density_one_staged(const StepArgs& a, const Scen
         wr += wall_rho((pk[d] - sc.bmin[d]) * sc.inv_h);
         wr += wall_rho((sc.wmax[d] - pk[d]) * sc.inv_h);
     }
-    const float rho = sc.cD * sum + sc.rho0 * wr;
-    const float p = eos(sc, rho);
-    const float ir = 1.0f / rho;
-    a.rho[k] = rho;
-    reinterpret_cast<float*>(a.pos_s + k)[3] = (p * ir) * ir;
-    reinterpret_cast<float*>(a.vel_s + k)[3] = ir;
+    density_finish(a, sc, k, sum, wr);
 }
 
 struct ForceAcc {
@@ -334,6 +335,13 @@ __device__ __forceinline__ void force_pair(const SceneConst& sc, const float4& p
 __device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                                  const float4& pi, const float4& vi, const ForceAcc& f);
 
+// The centre row's mask word (its last slot `after` slots before the row's
+// end) without particle k's own bit.
+__device__ __forceinline__ uint32_t without_self(uint32_t word, uint32_t lo, uint32_t hi, uint32_t k, uint32_t after) {
+    const uint32_t b = mask_bit(lo, hi, k) - after;
+    return b < (uint32_t)kMaskBits ? word & ~(1u << b) : word;
+}
+
 __device__ __forceinline__ uint32_t force_one(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                               __amdgpu_buffer_rsrc_t rpos, __amdgpu_buffer_rsrc_t rvel,
                                               __amdgpu_buffer_rsrc_t rcs) {
@@ -346,10 +354,7 @@ __device__ __forceinline__ uint32_t force_one(const StepArgs& a, const SceneCons
         row_window(rcs, sc, g, row % 3 - 1, row / 3 - 1, lo[row], hi[row]);
         mk[row] = a.mask[(size_t)row * a.n + k];
     }
-    {
-        const uint32_t b = mask_bit(lo[4], hi[4], k);  // own bit, in the centre row
-        if (b < (uint32_t)kMaskBits) mk[4] &= ~(1u << b);
-    }
+    mk[4] = without_self(mk[4], lo[4], hi[4], k, 0u);
     ForceAcc f = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int row = 0; row < kRows; ++row) {
@@ -383,17 +388,17 @@ __device__ __forceinline__ uint32_t force_one(const StepArgs& a, const SceneCons
     return force_finish(a, sc, k, pi, vi, f);
 }
 
-// Walls, integrate, clamp and stores of particle k; returns its next key.
+// Integrate, clamp and stores of particle k, given its neighbours' sums, the
+// walls' differences wj and its id; returns its next key.
 __device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
-                                                 const float4& pi, const float4& vi, const ForceAcc& f) {
+                                                 const float4& pi, const float4& vi, const ForceAcc& f,
+                                                 const float wj[3], uint32_t id) {
     const float cvi = sc.cV * vi.w;
     // The walls' pressure term at this particle's own p/rho^2.
     const float cwi = sc.cW * pi.w;
-    const float pk[3] = {pi.x, pi.y, pi.z};
     float aw[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-        aw[d] = cwi * (wall_j((pk[d] - sc.bmin[d]) * sc.inv_h) - wall_j((sc.wmax[d] - pk[d]) * sc.inv_h));
+    for (int d = 0; d < 3; ++d) aw[d] = cwi * wj[d];
     const float a0 = ((sc.cP * f.px + cvi * f.vx) + sc.g[0]) + aw[0];
     const float a1 = ((sc.cP * f.py + cvi * f.vy) + sc.g[1]) + aw[1];
     const float a2 = ((sc.cP * f.pz + cvi * f.vz) + sc.g[2]) + aw[2];
@@ -410,10 +415,29 @@ __device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneC
             if (v[d] > 0.0f) v[d] = -sc.e * v[d];
         }
     }
-    a.pos_o[k] = make_float4(p[0], p[1], p[2], 0.0f);
-    a.vel_o[k] = make_float4(v[0], v[1], v[2], 0.0f);
-    a.id_o[k] = a.id_s[k];
+    if (a.pos_o) {
+        a.pos_o[k] = make_float4(p[0], p[1], p[2], 0.0f);
+        a.vel_o[k] = make_float4(v[0], v[1], v[2], 0.0f);
+        a.id_o[k] = id;
+    }
+    if (a.xyz_out) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            a.xyz_out[3 * (size_t)id + d] = p[d];
+            a.vel_out[3 * (size_t)id + d] = v[d];
+        }
+    }
     return cell_key(sc, p[0], p[1], p[2]);
+}
+
+__device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
+                                                 const float4& pi, const float4& vi, const ForceAcc& f) {
+    const float pk[3] = {pi.x, pi.y, pi.z};
+    float wj[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        wj[d] = wall_j((pk[d] - sc.bmin[d]) * sc.inv_h) - wall_j((sc.wmax[d] - pk[d]) * sc.inv_h);
+    return force_finish(a, sc, k, pi, vi, f, wj, a.id_s[k]);
 }
 
 // Candidates a wave stages per row: its lanes' windows of one row lie in
@@ -450,10 +474,7 @@ __device__ __forceinline__ uint32_t force_one_staged(const StepArgs& a, const Sc
         mk[row] = active ? a.mask[(size_t)row * a.n + k] : 0u;
         if (!active) lo[row] = hi[row] = 0u;
     }
-    {
-        const uint32_t b = mask_bit(lo[4], hi[4], k);
-        if (active && b < (uint32_t)kMaskBits) mk[4] &= ~(1u << b);
-    }
+    if (active) mk[4] = without_self(mk[4], lo[4], hi[4], k, 0u);
     const uint32_t lane = threadIdx.x & 63u;
     ForceAcc f = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     // Each row's union of windows is copied into one of two slots by direct
@@ -517,9 +538,25 @@ __device__ __forceinline__ uint32_t force_one_staged(const StepArgs& a, const Sc
 // The sort has read the tile sums; the density pass clears them for the
 // integrate pass.
 __device__ __forceinline__ void clear_tile_sums(const StepArgs& a) {
+    if (!a.head) return;
     const uint32_t words = (a.ncells + kTileCells - 1u) >> kTileShift;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
         a.head[a.ncells + i] = 0u;
+}
+
+// Next step's key, its run in the cell's chain, the tile sums and the largest
+// speed (whole wave).
+__device__ __forceinline__ void finish_particle(const StepArgs& a, uint32_t scene, uint32_t k, uint32_t key,
+                                                bool active) {
+    if (!a.head) return;  // a single step: there is no next one
+    add_tile_sums(a.head + a.ncells, key, active);
+    if (a.vmax2) {
+        float4 vn = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (active) vn = a.vel_o[k];
+        wave_max_v2(a.vmax2, scene, vn.x, vn.y, vn.z, active);
+    }
+    if (active) a.key0[k] = key;
+    push_run(a.head, a.next, key, k, active);  // last: it waits for its exchange's answer
 }
 
 template <int BLOCK>
@@ -572,15 +609,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
         const bool active = k < sc.p_end;
         uint32_t key = 0;
         if (active) key = force_one(a, sc, k, rpos, rvel, rcs);
-        // Next step's key, its run in the cell's chain and the tile sums (whole wave).
-        push_run(a.head, a.next, key, k, active);
-        add_tile_sums(a.head + a.ncells, key, active);
-        if (a.vmax2) {
-            float4 vn = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (active) vn = a.vel_o[k];
-            wave_max_v2(a.vmax2, ti.x, vn.x, vn.y, vn.z, active);
-        }
-        if (active) a.key0[k] = key;
+        finish_particle(a, ti.x, k, key, active);
     });
 }
 
@@ -604,16 +633,447 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
         const uint32_t k = ti.y + threadIdx.x;
         const bool active = k < sc.p_end;
         const uint32_t key = force_one_staged(a, sc, k, active, rpos, rvel, rcs, slot_a, slot_b);
-        // Next step's key, its run in the cell's chain and the tile sums (whole wave).
-        push_run(a.head, a.next, key, k, active);
-        add_tile_sums(a.head + a.ncells, key, active);
-        if (a.vmax2) {
-            float4 vn = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (active) vn = a.vel_o[k];
-            wave_max_v2(a.vmax2, ti.x, vn.x, vn.y, vn.z, active);
-        }
-        if (active) a.key0[k] = key;
+        finish_particle(a, ti.x, k, key, active);
     });
+}
+
+// ------------------------------------------------------------- split form
+//
+// With few particles the chip is idle and a pass lasts as long as one wave's
+// serial chain: nine rows one after the other, each waiting for its copy or
+// its gathers (500 particles, 8 waves: density 12.5 us, force 11.3 us; 24k:
+// 13.4 and 13.9 us).  The split form shortens that chain.  Density: nine
+// waves per 64 particles, one per row, so all copies are in flight together
+// and every row's trips run at the same time; the rows' neighbours then go
+// into one list per particle, with their terms, and the first wave adds the
+// terms in list order, so the sum is the other forms' bit for bit.  The force
+// pass walks that list, without windows, masks or rows.
+
+constexpr uint32_t kKept = 5;        // a gathered row's terms kept in its copy's place
+constexpr uint32_t kListOver = 0xffffu;
+
+static_assert(kKept * kSplitTile * 4 <= sizeof(DensitySlot), "the kept terms fit a row's copy");
+
+struct SplitShared {
+    DensitySlot rec[kRows];                        // the rows' copies, as planes: lanes read them in step,
+                                                   // which records of 16 bytes would serve four at a time
+    float term[kListMax + 8][kSplitTile];          // the neighbours' terms, itself included
+    uint16_t id[kListMax + 4][kSplitTile];         // the neighbours; the particle itself goes to the last place
+    uint32_t count[3][kSplitTile];                 // neighbours per row, one byte a row (itself included)
+    uint32_t over;                                 // some row or list does not fit
+    float wall[kSplitTile];
+};
+
+// The window of one row (dy, dz) of a particle: row_geom and row_window for
+// that row alone.
+__device__ __forceinline__ void split_window(__amdgpu_buffer_rsrc_t rcs, const SceneConst& sc, const float4& p, int dy,
+                                             int dz, uint32_t& lo, uint32_t& hi) {
+    const float fx = (p.x - sc.bmin[0]) * sc.inv_csx;
+    const float f[2] = {(p.y - sc.bmin[1]) * sc.inv_cs, (p.z - sc.bmin[2]) * sc.inv_cs};
+    const int d[2] = {dy, dz};
+    int c[2];
+    float q[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        c[i] = (int)fminf(fmaxf(f[i], 0.0f), (float)(sc.G[i + 1] - 1));
+        const float m = 0.0009765625f;
+        const float r = fminf(fmaxf(f[i] - (float)c[i], 0.0f), 1.0f);
+        const float near = fmaxf((d[i] < 0 ? r : 1.0f - r) - m, 0.0f);
+        const bool in = d[i] < 0 ? c[i] > 0 : c[i] < sc.G[i + 1] - 1;
+        q[i] = d[i] == 0 ? 0.0f : in ? near * near : 4.0f;
+    }
+    lo = hi = 0u;
+    if (!(__builtin_isfinite(p.x) && __builtin_isfinite(p.y) && __builtin_isfinite(p.z))) return;
+    const uint32_t row = ((uint32_t)(c[1] + dz) * (uint32_t)sc.G[1] + (uint32_t)(c[0] + dy)) * (uint32_t)sc.G[0];
+    chord_window(rcs, sc, fx, sc.hc2 - (q[0] + q[1]), sc.cell_offset + row, lo, hi);
+}
+
+// One candidate's term c = min(d^2 - h^2, 0), formed as density_trip forms it.
+__device__ __forceinline__ float split_term(const float4& pi, float h2, float x, float y, float z) {
+    return dist2(pi.x - x, pi.y - y, pi.z - z) - h2;
+}
+
+// Runs a row's trips: candidate j's term goes to f(c), m and mh receive the
+// mask words.  quad(j, X, Y, Z): the coordinates of candidates j .. j + 3; it
+// may be asked for up to seven past the row, whose values are not used.
+struct Quad {
+    float4 X, Y, Z;
+};
+template <class G, class F>
+__device__ __forceinline__ void split_trips(G&& quad, const float4& pi, float h2, uint32_t lo, uint32_t hi,
+                                            uint32_t& m, uint32_t& mh, F&& f) {
+    m = 0u;
+    mh = 0u;
+    const bool two = __ballot(mask_span(lo, hi) > 32u) != 0u;
+    if (lo >= hi) return;
+    Quad cur, nxt;
+    auto test = [&](const Quad& q, uint32_t left) {
+        const float xs[4] = {q.X.x, q.X.y, q.X.z, q.X.w}, ys[4] = {q.Y.x, q.Y.y, q.Y.z, q.Y.w},
+                    zs[4] = {q.Z.x, q.Z.y, q.Z.z, q.Z.w};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            float t = split_term(pi, h2, xs[u], ys[u], zs[u]);
+            if (u != 0) t = (uint32_t)u < left ? t : 1.0f;
+            const float c = fminf(t, 0.0f);
+            m = push_sign(m, c);
+            f(c);
+        }
+    };
+    uint32_t j = lo;
+    const uint32_t full_end = lo + ((hi - lo) & ~3u);
+    quad(j, cur);
+    if (two) {
+        const uint32_t jm = row_first(lo, hi);
+        for (; j != full_end; j += 4u) {
+            if (j == jm) mh = m;
+            quad(j + 4u, nxt);
+            test(cur, 4u);
+            cur = nxt;
+        }
+        if (j == jm) mh = m;
+        if (j != hi) test(cur, hi - j);
+        return;
+    }
+    // The next trip's records load while this one's are tested, the two
+    // register sets in turn.
+    for (;;) {
+        if (j == full_end) {
+            if (j != hi) test(cur, hi - j);
+            break;
+        }
+        quad(j + 4u, nxt);
+        test(cur, 4u);
+        j += 4u;
+        if (j == full_end) {
+            if (j != hi) test(nxt, hi - j);
+            break;
+        }
+        quad(j + 4u, cur);
+        test(nxt, 4u);
+        j += 4u;
+    }
+}
+
+// Visits the candidates of a word's ascending bits (bit i: j0 + i), the next
+// one's record loading while this one's is used.
+template <class G, class F>
+__device__ __forceinline__ void split_bits(uint32_t r, uint32_t j0, G&& get, F&& f) {
+    if (!r) return;
+    uint32_t j = j0 + (uint32_t)__builtin_ctz(r);
+    float4 p = get(j);
+#pragma unroll 2
+    for (;;) {
+        r &= r - 1u;
+        const uint32_t jn = r ? j0 + (uint32_t)__builtin_ctz(r) : j;
+        const float4 pn = get(jn);
+        f(j, p);
+        if (!r) break;
+        j = jn;
+        p = pn;
+    }
+}
+
+__global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
+    if (a.halt && *a.halt) return;
+    clear_tile_sums(a);
+    __shared__ SplitShared sh;
+    const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
+    const __amdgpu_buffer_rsrc_t rcs = buffer_of(a.cstart, a.ncells + 1u);
+    const uint2 ti = tile_at(a.tiles, xcd_block(blockIdx.x, gridDim.x));
+    const SceneConst sc = scene_at(a.scenes, ti.x);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t k = ti.y + lane;
+    const bool active = k < sc.p_end;
+    const float4 pi = load4(rpos, k << 4);  // zeros past the buffer end
+    uint32_t lo, hi;
+    split_window(rcs, sc, pi, w % 3 - 1, w / 3 - 1, lo, hi);
+    if (!active) lo = hi = 0u;
+    if (threadIdx.x == 0) sh.over = 0u;
+    // The row's union of windows.
+    const bool has = hi > lo;
+    const uint32_t ulo = wave_umin(has ? lo : 0xffffffffu);
+    const uint32_t uhi = wave_umax(has ? hi : 0u);
+    const bool fit = ulo < uhi && uhi - ulo <= kStageD;
+    if (fit) {
+        float* v = sh.rec[w].v;
+        const bool c0 = lane < uhi - ulo, c1 = lane + 64u < uhi - ulo;
+        float4 n0, n1;
+        if (c0) n0 = load4(rpos, (ulo + lane) << 4);
+        if (c1) n1 = load4(rpos, (ulo + lane + 64u) << 4);
+        if (c0) {
+            v[lane] = n0.x;
+            v[kPlaneD + lane] = n0.y;
+            v[2 * kPlaneD + lane] = n0.z;
+        }
+        if (c1) {
+            v[lane + 64u] = n1.x;
+            v[kPlaneD + lane + 64u] = n1.y;
+            v[2 * kPlaneD + lane + 64u] = n1.z;
+        }
+        wave_lds_sync();
+    }
+    auto staged = [&](uint32_t j, Quad& q) {
+        const float* p = sh.rec[w].v + (j - ulo);
+        q.X = slot_quad(p, 0);
+        q.Y = slot_quad(p, 1);
+        q.Z = slot_quad(p, 2);
+    };
+    auto gathered = [&](uint32_t j, Quad& q) { load_quad(rpos, j, q.X, q.Y, q.Z); };
+    auto staged_one = [&](uint32_t j) {
+        const float* p = sh.rec[w].v + (j - ulo);
+        return make_float4(p[0], p[kPlaneD], p[2 * kPlaneD], 0.0f);
+    };
+    auto gathered_one = [&](uint32_t j) { return load4(rpos, j << 4); };
+    uint32_t m, mh, nkept = 0u;
+    float* const kept = sh.rec[w].v + lane;
+    if (fit)
+        split_trips(staged, pi, sc.h2, lo, hi, m, mh, [](float) {});
+    else
+        split_trips(gathered, pi, sc.h2, lo, hi, m, mh, [&](float c) {
+            if (c < 0.0f) {
+                if (nkept < kKept) kept[nkept * kSplitTile] = c;
+                ++nkept;
+            }
+        });
+    if (active) a.mask[(size_t)w * a.n + k] = m;
+    const uint32_t span = mask_span(lo, hi);
+    if (span <= 32u) mh = 0u;
+    const uint32_t cnt = (uint32_t)__popc(m) + (uint32_t)__popc(mh);
+    reinterpret_cast<uint8_t*>(sh.count)[(((uint32_t)w >> 2) * kSplitTile + lane) * 4u + ((uint32_t)w & 3u)] = (uint8_t)cnt;
+    if (__ballot(span > 64u) != 0u && lane == 0u) sh.over = 1u;
+    __syncthreads();
+    // Where this row's neighbours go in the list, and how many there are.
+    uint32_t base = 0u, total = 0u;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+        const uint32_t c = sh.count[g][lane];
+        const uint32_t before = w >= 4 * g + 4 ? 0xffffffffu : w > 4 * g ? (1u << (8 * (w - 4 * g))) - 1u : 0u;
+        base = __builtin_amdgcn_sad_u8(c & before, 0u, base);
+        total = __builtin_amdgcn_sad_u8(g == 2 ? c & 0xffu : c, 0u, total);
+    }
+    // The list leaves the particle itself out (its term is in the sum).
+    if (__ballot(total > kListMax + 1u) != 0u && lane == 0u && w == 0) sh.over = 1u;
+    const bool fits = __ballot(total > kListMax + 1u) == 0u;
+    if (fits) {
+        auto put = [&](uint32_t j, float c) {
+            sh.term[base][lane] = c;
+            // Candidates past k come one place earlier in the list (rows go
+            // in ascending order).
+            const uint32_t e = base - (j > k ? 1u : 0u);
+            sh.id[j == k ? kListMax : e][lane] = (uint16_t)j;
+            ++base;
+        };
+        uint32_t i = 0u;
+        auto bits = [&](uint32_t r, uint32_t j0) {
+            if (fit)
+                split_bits(r, j0, staged_one,
+                           [&](uint32_t j, const float4& pj) { put(j, split_term(pi, sc.h2, pj.x, pj.y, pj.z)); });
+            else
+                for (; r; r &= r - 1u, ++i) {
+                    const uint32_t j = j0 + (uint32_t)__builtin_ctz(r);
+                    float c;
+                    if (i < kKept) {
+                        c = kept[i * kSplitTile];
+                    } else {
+                        const float4 pj = gathered_one(j);
+                        c = split_term(pi, sc.h2, pj.x, pj.y, pj.z);
+                    }
+                    put(j, c);
+                }
+        };
+        if (__ballot(mh != 0u)) bits(mask_ascending(mh, span, 32u), row_first(lo, hi, 2u));
+        bits(mask_ascending(m, span, 0u), row_first(lo, hi));
+    }
+    // A corner row has the fewest neighbours to list.
+    if (w == kRows - 1) {
+        float wr = 0.0f;
+        const float pk[3] = {pi.x, pi.y, pi.z};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            wr += wall_rho((pk[d] - sc.bmin[d]) * sc.inv_h);
+            wr += wall_rho((sc.wmax[d] - pk[d]) * sc.inv_h);
+        }
+        sh.wall[lane] = wr;
+    }
+    __syncthreads();
+    if (sh.over) {
+        // The first wave runs every row itself; the force pass walks masks.
+        if (w != 0) return;
+        float sum = 0.0f;
+#pragma unroll 1
+        for (int r = 0; r < kRows; ++r) {
+            split_window(rcs, sc, pi, r % 3 - 1, r / 3 - 1, lo, hi);
+            if (!active) lo = hi = 0u;
+            split_trips(gathered, pi, sc.h2, lo, hi, m, mh, [&](float c) { sum = fmaf(c * c, -c, sum); });
+        }
+        if (active) {
+            a.ncount[k] = kListOver;
+            density_finish(a, sc, k, sum, sh.wall[lane]);
+        }
+        return;
+    }
+    if (w != 0) {
+        if (!active) return;
+        const uint32_t listed = total ? total - 1u : 0u;
+        if (w == 1) a.ncount[k] = listed;
+        for (uint32_t q = (uint32_t)w - 1u; 4u * q < listed; q += (uint32_t)kRows - 1u)
+            reinterpret_cast<uint2*>(a.nlist)[(size_t)q * a.n + k] =
+                make_uint2(sh.id[4u * q][lane] | ((uint32_t)sh.id[4u * q + 1u][lane] << 16),
+                           sh.id[4u * q + 2u][lane] | ((uint32_t)sh.id[4u * q + 3u][lane] << 16));
+        return;
+    }
+    // Eight terms at a time, the next four loaded while four are added;
+    // terms past the list's end count as 0, which adds nothing.
+    float sum = 0.0f, c[4], d[4];
+    auto four = [&](uint32_t i, float* v) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = sh.term[i + u][lane];
+    };
+    auto add = [&](uint32_t i, const float* v) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float t = i + (uint32_t)u < total ? v[u] : 0.0f;
+            sum = fmaf(t * t, -t, sum);
+        }
+    };
+    four(0u, c);
+    for (uint32_t i = 0; i < total; i += 8u) {
+        four(i + 4u, d);
+        add(i, c);
+        four(min(i + 8u, kListMax + 4u), c);
+        add(i + 4u, d);
+    }
+    if (active) density_finish(a, sc, k, sum, sh.wall[lane]);
+}
+
+// Force, split form.  Four waves per 64 particles take the list in rounds of
+// 32 neighbours, eight per wave, whose records are gathered together; each
+// leaves its pairs' factors in LDS, and two waves then add them in list order
+// (force_pair's sums, one the pressure terms and one the viscosity terms)
+// while a third takes the walls.  One wave doing all of it waited for each
+// few neighbours' gathers (24k: walk 8200 of 17000 cycles, and 3900 for the
+// walls, integration and stores after it).
+constexpr uint32_t kRound = 32;
+constexpr int kForceWaves = 4;
+constexpr int kPerWave = (int)kRound / kForceWaves;
+
+struct ForceSplitShared {
+    float4 press[kRound][kSplitTile];  // s, dx, dy, dz of a pair
+    float4 visc[kRound][kSplitTile];   // vv, dvx, dvy, dvz
+    float sum[3][kSplitTile];          // the viscosity sums
+    float wall[3][kSplitTile];         // the walls' differences
+    uint32_t id[kSplitTile];
+};
+
+__global__ __launch_bounds__(64 * kForceWaves) void force_split_kernel(StepArgs a) {
+    if (a.halt && *a.halt) return;
+    __shared__ ForceSplitShared sh;
+    const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
+    const __amdgpu_buffer_rsrc_t rvel = buffer_of(a.vel_s, a.n);
+    const __amdgpu_buffer_rsrc_t rl = buffer_of(a.nlist, kListMax * a.n);
+    const uint2 ti = tile_at(a.tiles, xcd_block(blockIdx.x, gridDim.x));
+    const SceneConst sc = scene_at(a.scenes, ti.x);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t k = ti.y + lane;
+    const bool active = k < sc.p_end;
+    // Entries past a list's end hold any index; their pairs are not added.
+    auto ids = [&](uint32_t q) { return __builtin_amdgcn_raw_buffer_load_b64(rl, (int)((q * a.n + k) << 3), 0, 0); };
+    u32x2 q0 = ids(2u * (uint32_t)w), q1 = ids(2u * (uint32_t)w + 1u);
+    const float4 pi = load4(rpos, k << 4), vi = load4(rvel, k << 4);
+    const uint32_t count = active ? a.ncount[k] : 0u;
+    const uint32_t id = w == 2 && active ? a.id_s[k] : 0u;
+    float4 pj[kPerWave], vj[kPerWave];
+    auto gather = [&]() {
+        const uint32_t j[kPerWave] = {q0.x & 0xffffu, q0.x >> 16, q0.y & 0xffffu, q0.y >> 16,
+                                      q1.x & 0xffffu, q1.x >> 16, q1.y & 0xffffu, q1.y >> 16};
+#pragma unroll
+        for (int u = 0; u < kPerWave; ++u) pj[u] = load4(rpos, j[u] << 4);
+#pragma unroll
+        for (int u = 0; u < kPerWave; ++u) vj[u] = load4(rvel, j[u] << 4);
+    };
+    gather();  // before the counts are known: any index stays inside the buffers' bounds checks
+    if (__ballot(count > kListMax) != 0u) {  // the same in every wave
+        if (w != 0) return;
+        uint32_t key = 0;
+        if (active) key = force_one(a, sc, k, rpos, rvel, buffer_of(a.cstart, a.ncells + 1u));
+        finish_particle(a, ti.x, k, key, active);
+        return;
+    }
+    float f[3] = {0.f, 0.f, 0.f};
+    for (uint32_t first = 0u;; first += kRound) {
+        if (__ballot(count > first + (uint32_t)(kPerWave * w)) != 0u) {
+            if (first != 0u) {
+                q0 = ids(first / 4u + 2u * (uint32_t)w);
+                q1 = ids(first / 4u + 2u * (uint32_t)w + 1u);
+                gather();
+            }
+#pragma unroll
+            for (int u = 0; u < kPerWave; ++u) {
+                // force_pair's factors.
+                const float dx = pi.x - pj[u].x, dy = pi.y - pj[u].y, dz = pi.z - pj[u].z;
+                const float d2 = dist2(dx, dy, dz);
+                const float inv_r = __builtin_amdgcn_rsqf(fmaxf(d2, 1e-30f));
+                const float r = d2 * inv_r;
+                const float hr = sc.h - r;
+                const float s = ((pi.w + pj[u].w) * (hr * hr)) * inv_r;
+                sh.press[kPerWave * w + u][lane] = make_float4(s, dx, dy, dz);
+                sh.visc[kPerWave * w + u][lane] =
+                    make_float4(hr * vj[u].w, vj[u].x - vi.x, vj[u].y - vi.y, vj[u].z - vi.z);
+            }
+        }
+        __syncthreads();
+        const uint32_t left = count > first ? min(count - first, kRound) : 0u;
+        if (w < 2) {
+            auto chain = [&](const float4(&t)[kRound][kSplitTile]) {
+                // Four pairs at a time, the next four loaded meanwhile.
+                float4 c[4], n[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) c[u] = t[u][lane];
+#pragma unroll 2
+                for (uint32_t i = 0; i < left; i += 4u) {
+                    const uint32_t in = min(i + 4u, kRound - 4u);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) n[u] = t[in + u][lane];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        if (i + (uint32_t)u < left) {
+                            f[0] = fmaf(c[u].x, c[u].y, f[0]);
+                            f[1] = fmaf(c[u].x, c[u].z, f[1]);
+                            f[2] = fmaf(c[u].x, c[u].w, f[2]);
+                        }
+                        c[u] = n[u];
+                    }
+                }
+            };
+            if (w == 0)
+                chain(sh.press);
+            else
+                chain(sh.visc);
+        } else if (w == 2 && first == 0u) {
+            const float p[3] = {pi.x, pi.y, pi.z};
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                sh.wall[d][lane] = wall_j((p[d] - sc.bmin[d]) * sc.inv_h) - wall_j((sc.wmax[d] - p[d]) * sc.inv_h);
+            sh.id[lane] = id;
+        }
+        if (__ballot(count > first + kRound) == 0u) break;
+        __syncthreads();
+    }
+    if (w == 1) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) sh.sum[d][lane] = f[d];
+    }
+    __syncthreads();
+    if (w != 0) return;
+    uint32_t key = 0;
+    if (active) {
+        const ForceAcc acc = {f[0], f[1], f[2], sh.sum[0][lane], sh.sum[1][lane], sh.sum[2][lane]};
+        const float wj[3] = {sh.wall[0][lane], sh.wall[1][lane], sh.wall[2][lane]};
+        key = force_finish(a, sc, k, pi, vi, acc, wj, sh.id[lane]);
+    }
+    finish_particle(a, ti.x, k, key, active);
 }
 
 // Uploads come in any order, a lattice's fastest axis often across the
@@ -622,17 +1082,40 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
 // block counts them in LDS first (grids of up to kHashTiles tiles).
 constexpr uint32_t kHashTiles = 2048;
 
+// The tile sums of one block's particles: add() for every lane of the block,
+// flush() once at its end.
+struct BlockTileSums {
+    uint32_t* tsum;
+    uint32_t tiles;
+    uint32_t* local;  // kHashTiles words of LDS; null: straight to memory
+    __device__ __forceinline__ BlockTileSums(uint32_t* head, uint32_t ncells, uint32_t* lds)
+        : tsum(head + ncells), tiles((ncells + kTileCells - 1u) >> kTileShift) {
+        local = tiles <= kHashTiles ? lds : nullptr;
+        if (local) {
+            for (uint32_t i = threadIdx.x; i < tiles; i += blockDim.x) local[i] = 0u;
+            __syncthreads();
+        }
+    }
+    __device__ __forceinline__ void add(uint32_t key, bool active) {
+        if (!local)
+            add_tile_sums(tsum, key, active);
+        else if (active)
+            atomicAdd(local + (key >> kTileShift), 1u);
+    }
+    __device__ __forceinline__ void flush() {
+        if (!local) return;
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < tiles; i += blockDim.x)
+            if (local[i]) atomicAdd(tsum + i, local[i]);
+    }
+};
+
 __global__ void hash_kernel(const float4* __restrict__ pos, const float4* __restrict__ vel,
                             uint32_t* __restrict__ key0, uint32_t* __restrict__ next, uint32_t* __restrict__ head,
                             uint32_t ncells, uint32_t* __restrict__ vmax2, const SceneConst* __restrict__ scenes,
                             const uint2* __restrict__ tiles, uint32_t ntiles) {
     __shared__ uint32_t s_sum[kHashTiles];
-    const uint32_t gt = (ncells + kTileCells - 1u) >> kTileShift;
-    const bool local = gt <= kHashTiles;
-    if (local) {
-        for (uint32_t i = threadIdx.x; i < gt; i += blockDim.x) s_sum[i] = 0u;
-        __syncthreads();
-    }
+    BlockTileSums sums(head, ncells, s_sum);
     uint32_t t0, t1;
     tile_span(ntiles, t0, t1);
     for (uint32_t t = t0; t < t1; ++t) {
@@ -646,10 +1129,7 @@ __global__ void hash_kernel(const float4* __restrict__ pos, const float4* __rest
             key = cell_key(sc, p.x, p.y, p.z);
         }
         push_run(head, next, key, k, active);
-        if (!local)
-            add_tile_sums(head + ncells, key, active);
-        else if (active)
-            atomicAdd(&s_sum[key >> kTileShift], 1u);
+        sums.add(key, active);
         if (active) key0[k] = key;
         if (vmax2) {
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -657,11 +1137,33 @@ __global__ void hash_kernel(const float4* __restrict__ pos, const float4* __rest
             wave_max_v2(vmax2, ti.x, v.x, v.y, v.z, active);
         }
     }
-    if (local) {
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < gt; i += blockDim.x)
-            if (s_sum[i]) atomicAdd(head + ncells + i, s_sum[i]);
+    sums.flush();
+}
+
+// pack3, the identity ids and the hash of one scene of n particles in one
+// pass; vel_in may be null (zero velocity).
+__global__ __launch_bounds__(256) void upload_hash_kernel(const float* __restrict__ xyz, const float* __restrict__ vel_in,
+                                                          float4* __restrict__ pos, float4* __restrict__ vel,
+                                                          uint32_t* __restrict__ id, uint32_t* __restrict__ key0,
+                                                          uint32_t* __restrict__ next, uint32_t* __restrict__ head,
+                                                          uint32_t n, uint32_t ncells, SceneConst sc) {
+    __shared__ uint32_t s_sum[kHashTiles];
+    BlockTileSums sums(head, ncells, s_sum);
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool active = k < n;
+    uint32_t key = 0;
+    if (active) {
+        const float4 p = make_float4(xyz[3 * (size_t)k], xyz[3 * (size_t)k + 1], xyz[3 * (size_t)k + 2], 0.0f);
+        pos[k] = p;
+        vel[k] = vel_in ? make_float4(vel_in[3 * (size_t)k], vel_in[3 * (size_t)k + 1], vel_in[3 * (size_t)k + 2], 0.0f)
+                        : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        id[k] = k;
+        key = cell_key(sc, p.x, p.y, p.z);
+        key0[k] = key;
     }
+    push_run(head, next, key, k, active);
+    sums.add(key, active);
+    sums.flush();
 }
 
 // Neighbour sets exactly as force_one iterates them (self included).
@@ -794,6 +1296,18 @@ hipError_t launch_force(hipStream_t st, int block, uint32_t grid, const StepArgs
     return hipGetLastError();
 }
 
+hipError_t launch_density_split(hipStream_t st, const StepArgs& a) {
+    if (a.ntiles == 0) return hipSuccess;
+    hipLaunchKernelGGL(density_split_kernel, dim3(a.ntiles), dim3(64 * kRows), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_force_split(hipStream_t st, const StepArgs& a) {
+    if (a.ntiles == 0) return hipSuccess;
+    hipLaunchKernelGGL(force_split_kernel, dim3(a.ntiles), dim3(64 * kForceWaves), 0, st, a);
+    return hipGetLastError();
+}
+
 template <class K>
 static int occupancy(K kernel, int block) {
     int nb = 0;
@@ -824,6 +1338,15 @@ hipError_t launch_hash(hipStream_t st, int block, uint32_t grid, const float4* p
     if (grid == 0) return hipSuccess;
     hipLaunchKernelGGL(hash_kernel, dim3(grid), dim3(block), 0, st, pos, vel, key0, next, head, ncells, vmax2,
                        scenes, tiles, ntiles);
+    return hipGetLastError();
+}
+
+hipError_t launch_upload_hash(hipStream_t st, const float* xyz, const float* vel_in, float4* pos, float4* vel,
+                              uint32_t* id, uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t n,
+                              uint32_t ncells, const SceneConst& sc) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(upload_hash_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, st, xyz, vel_in, pos, vel, id, key0,
+                       next, head, n, ncells, sc);
     return hipGetLastError();
 }
 
