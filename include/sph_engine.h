@@ -161,7 +161,7 @@ int  sph_scene_sample_ball(uint64_t seed, const float* centre, float radius, flo
  * hipMalloc): one step of n particles whose state the caller holds in device
  * memory, enqueued on `stream` (a hipStream_t; NULL = the default stream),
  * with every intermediate in a fixed scratch array of the library (about
- * 24 MB per GPU, held until the process ends).  xyz_in, vel_in (may be NULL:
+ * 32 MB per GPU, held until the process ends).  xyz_in, vel_in (may be NULL:
  * zero velocity), xyz_out, vel_out: device arrays of 3n floats in the
  * caller's particle order.  The step and its results equal the first
  * sph_advance_steps step of a handle given the same particles and params

@@ -1230,6 +1230,14 @@ int sph_debug_step_outputs(sph_handle* h, uint32_t* keys_in, uint32_t* perm, uin
     if (rc != SPH_OK) return rc;
     const size_t n = h->n;
     hipError_t e = hipSuccess;
+    if (h->tune.sort_mode == kSortCellCount && (sorted_keys || keys_in)) {
+        uint32_t nt = 0;
+        const uint2* tl = tiles_for(h, 256, nt);
+        if (!tl) return fail(h, SPH_E_OOM, "tile table");
+        e = launch_sorted_keys(h->stream, 256, nt, h->work.pos_s.p, h->work.skey.p, h->sc_d.p, tl);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        if (e != hipSuccess) return hip_fail(h, e, "sorted keys");
+    }
     if (perm) e = hipMemcpy(perm, h->work.perm.p, n * 4, hipMemcpyDeviceToHost);
     if (e == hipSuccess && sorted_keys) e = hipMemcpy(sorted_keys, h->work.skey.p, n * 4, hipMemcpyDeviceToHost);
     if (e == hipSuccess && rho) e = hipMemcpy(rho, h->work.rho.p, n * 4, hipMemcpyDeviceToHost);

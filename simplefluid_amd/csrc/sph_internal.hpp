@@ -29,7 +29,7 @@ struct SortPlan {
     uint32_t* tmp = nullptr;          // cell-count: members of the tiles too full for LDS (n)
     uint32_t* kbuf[2] = {nullptr, nullptr};  // radix ping-pong
     uint32_t* vbuf[2] = {nullptr, nullptr};
-    uint32_t* skey = nullptr;         // sorted keys
+    uint32_t* skey = nullptr;         // radix: sorted keys
     uint32_t* perm = nullptr;         // sorted index -> state index
     uint32_t* hist = nullptr;         // radix: kMaxPasses x 256, zero on entry
     uint32_t* status = nullptr;       // radix: passes x tiles x 256
@@ -122,7 +122,7 @@ hipError_t launch_force(hipStream_t st, int block, uint32_t grid, const StepArgs
 // indices for the force pass (a particle with more is walked by its masks).
 // Same results as the other forms, bit for bit.
 constexpr uint32_t kSplitMax = 65536;   // the lists hold 16-bit indices
-constexpr uint32_t kListMax = 64;
+constexpr uint32_t kListMax = 128;
 constexpr int kSplitTile = 64;
 // Tiles up to which handles take it.  Two force blocks fit a CU, so 512 tiles
 // run at once; from there on the chip is full and its extra work shows.
@@ -141,6 +141,9 @@ hipError_t launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t value, size_t c
 // Debug: neighbour CSR as the force pass sees it.
 hipError_t launch_neighbors(hipStream_t st, int block, uint32_t grid, const StepArgs& a,
                             const uint32_t* offsets, uint32_t* counts_or_list, int fill);
+// Debug: keys of the sorted positions.
+hipError_t launch_sorted_keys(hipStream_t st, int block, uint32_t ntiles, const float4* pos_s, uint32_t* skey,
+                              const SceneConst* scenes, const uint2* tiles);
 // Original-order gather for get_*: out[3*id[k]+c] = src[k].c
 hipError_t launch_unpermute3(hipStream_t st, uint32_t n, const float4* src, const uint32_t* id,
                              float* out);

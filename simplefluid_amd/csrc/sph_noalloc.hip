@@ -57,7 +57,7 @@ struct Layout {
     static constexpr size_t total = align256(err + 4);
 };
 
-// The step's scratch on each GPU the library runs on (about 24 MB), held
+// The step's scratch on each GPU the library runs on (about 32 MB), held
 // until the process ends.  Host code reaches it only through the address
 // hipGetSymbolAddress returns on that device.
 static __device__ __align__(256) uint8_t scratch[Layout::total];

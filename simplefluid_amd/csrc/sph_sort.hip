@@ -7,10 +7,9 @@
 // each particle into its cell's chain of runs and counted particles per tile
 // of 1024 cells, so a block of cell_sort_kernel owns a tile: it takes its
 // prefix from the tile sums, counts its cells by following their chains,
-// scans the counts (cstart), lists the members cell by cell in LDS, ranks
-// each in its cell (the number of members with a smaller input index) and
-// gathers its state straight into its sorted place (pos, vel, id, key,
-// perm).  No block waits for another.
+// scans the counts (cstart), lists the members cell by cell in LDS, each
+// cell's by ascending input index, and
+// gathers its state straight into its sorted place (pos, vel, id, perm).  No block waits for another.
 // Radix sort: one histogram kernel for all 8-bit digits, then one kernel per
 // digit that ranks a tile of keys in LDS (wave64 ballot-matching of the
 // digit bits, so equal digits rank in lane order without LDS atomics) and
@@ -123,8 +122,9 @@ __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s_w, uint32
 // (22k tiles: 14 us).
 constexpr int kTileScanBlock = 1024;
 // Up to this many tiles each sort block sums the tiles before its own itself
-// (8 words per thread at most); above it tile_scan_kernel runs first.
-constexpr uint32_t kInlineTiles = 2048;
+// (24 words per thread at most; tile_scan_kernel's launch costs 5 us); above
+// it tile_scan_kernel runs first.
+constexpr uint32_t kInlineTiles = 6144;
 
 __global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __restrict__ head, uint32_t C,
                                                                    uint32_t T, const uint32_t* __restrict__ halt) {
@@ -171,7 +171,6 @@ struct CellSortArgs {
     float4* pos_out;
     float4* vel_out;
     uint32_t* id_out;
-    uint32_t* skey;
     uint32_t* perm;
     float* soa;
     uint32_t* queue;
@@ -187,7 +186,7 @@ struct CellSortArgs {
 // by the latency of its dependent steps at small sizes (tile sums and heads,
 // the links, the members' state) and by memory at large ones; one particle's
 // state is moved once.
-constexpr int kHeldLinks = 4;
+constexpr int kHeldLinks = 5;
 
 // One thread per cell up to this many tiles, where the chip waits on each
 // block's dependent steps; above it four cells per thread, where 1024-lane
@@ -208,7 +207,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     __shared__ uint32_t s_big;
     __shared__ uint32_t s_off[kTileCells + 1];
     __shared__ uint32_t s_mem[kTileMembers];
-    __shared__ uint16_t s_cell[kTileMembers];
+    __shared__ uint32_t s_unsorted;
     const uint32_t b = blockIdx.x, C = a.C;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // Tile counters of this step's persistent density and force launches.
@@ -235,22 +234,19 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     uint32_t pre;
     if (T <= kInlineTiles) {
         uint32_t x = 0;
-#pragma unroll
-        for (uint32_t e = 0; e < kInlineTiles / BLOCK; ++e) {
-            const uint32_t i = e * BLOCK + (uint32_t)tid;
-            if (i < b) x += a.head[C + i];
-        }
+#pragma unroll 8
+        for (uint32_t i = (uint32_t)tid; i < b; i += BLOCK) x += a.head[C + i];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
         if (lane == 0) s_pre[wave] = x;
-        if (tid == 0) s_big = 0u;
+        if (tid == 0) s_big = s_unsorted = 0u;
         __syncthreads();
         pre = 0u;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) pre += s_pre[w];
     } else {
         pre = a.head[C + T + b];
-        if (tid == 0) s_big = 0u;
+        if (tid == 0) s_big = s_unsorted = 0u;
         __syncthreads();
     }
     if (members == 0u) {
@@ -273,7 +269,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     auto link = [&](uint32_t run) -> uint32_t {
         return __builtin_amdgcn_raw_buffer_load_b32(rnext, (int)(run ? run_first(run) << 2 : 0xfffffffcu), 0, 0);
     };
-    auto any = [&](const uint32_t* q) -> bool {
+    auto any = [&](const uint32_t* q) __attribute__((always_inline)) -> bool {
         uint32_t o = 0;
 #pragma unroll
         for (int v = 0; v < V; ++v) o |= q[v];
@@ -306,6 +302,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
 #pragma unroll
         for (int v = 0; v < V; ++v) q[v] = r[kHeldLinks][v];
         int links = kHeldLinks;
+        if (any(q)) s_unsorted = 1u;  // longer than the registers hold (a last run may follow none: no matter)
         while (any(q)) {
             if (++links > kMaxLinks) {
                 s_big = 1u;
@@ -357,21 +354,45 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
 #pragma unroll
     for (int v = 0; v < V; ++v) s_off[V * tid + v] = off[v];
     if (tid == 0) s_off[kTileCells] = total;
-    // The members, cell by cell, in the order their runs come.
+    // The members, cell by cell.  A cell whose runs are all in registers
+    // lists them by their first particles, so its members come sorted; with a
+    // longer chain in the tile, all come as their runs do and are ranked
+    // below.
+    const bool unsorted = big || s_unsorted != 0u;
     const bool in_lds = total <= kTileMembers && !big;
     uint32_t* const tmp = a.tmp + pre;
-    if (!big) {
-        auto list = [&](const uint32_t* q) {
+    if (!unsorted) {
+        auto list = [&](auto&& put) __attribute__((always_inline)) {
+#pragma unroll
+            for (int l = 0; l < kHeldLinks; ++l) {
+                if (__ballot(any(r[l])) != 0u) {
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        const uint32_t k = run_first(r[l][v]);
+                        uint32_t at = off[v];
+#pragma unroll
+                        for (int o = 0; o < kHeldLinks; ++o)
+                            if (o != l) at += run_first(r[o][v]) < k ? run_len(r[o][v]) : 0u;
+                        const uint32_t end = k + run_len(r[l][v]);
+                        for (uint32_t t = k; t < end; ++t, ++at) put(at, t);
+                    }
+                }
+            }
+        };
+        if (in_lds)
+            list([&](uint32_t i, uint32_t k) { s_mem[i] = k; });
+        else
+            list([&](uint32_t i, uint32_t k) { tmp[i] = k; });
+    } else if (!big) {
+        auto list = [&](const uint32_t* q) __attribute__((always_inline)) {
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 const uint32_t k = run_first(q[v]), len = run_len(q[v]);
                 for (uint32_t t = 0; t < len; ++t) {
-                    if (in_lds) {
+                    if (in_lds)
                         s_mem[off[v] + t] = k + t;
-                        s_cell[off[v] + t] = (uint16_t)(V * tid + v);
-                    } else {
+                    else
                         tmp[off[v] + t] = k + t;
-                    }
                 }
                 off[v] += len;
             }
@@ -400,52 +421,77 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     }
     __threadfence_block();
     __syncthreads();
-    for (uint32_t j = (uint32_t)tid; j < total; j += BLOCK) {
-        const uint32_t k = in_lds ? s_mem[j] : tmp[j];
-        if (k >= a.n) {
-            atomicOr(a.err, 4u);
-            continue;
+    // V members per thread at a time, so that their state's loads overlap
+    // (one at a time, a full tile's 256-thread block waited for eight to
+    // sixteen loads in a row).
+    const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_in, a.n);
+    const __amdgpu_buffer_rsrc_t rvel = buffer_of(a.vel_in, a.n);
+    const __amdgpu_buffer_rsrc_t rid = buffer_of(a.id_in, a.n);
+    for (uint32_t j0 = (uint32_t)tid; j0 < total; j0 += V * BLOCK) {
+        uint32_t k[V];
+        float4 pk[V], vk[V];
+        uint32_t ik[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const uint32_t j = j0 + (uint32_t)(v * BLOCK);
+            k[v] = 0xffffffffu;
+            if (j < total) k[v] = in_lds ? s_mem[j] : tmp[j];
         }
-        const float4 pk = a.pos_in[k];
-        const float4 vk = a.vel_in[k];
-        const uint32_t ik = a.id_in[k];
-        const uint32_t c = in_lds ? (uint32_t)s_cell[j] : a.key0[k] - base;
-        if (c >= kTileCells) {
-            atomicOr(a.err, 4u);
-            continue;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            // No member: past the buffers' ends.
+            pk[v] = load4(rpos, min(k[v], a.n) << 4);
+            vk[v] = load4(rvel, min(k[v], a.n) << 4);
+            ik[v] = __builtin_amdgcn_raw_buffer_load_b32(rid, (int)(min(k[v], a.n) << 2), 0, 0);
         }
-        const uint32_t lo = s_off[c], hi = s_off[c + 1u];
-        uint32_t d = j;
-        if (hi - lo <= kMaxRankCell) {
-            d = lo;
-            if (in_lds) {
-                for (uint32_t t = lo; t < hi; ++t) d += s_mem[t] < k ? 1u : 0u;
-            } else {
-                for (uint32_t t = lo; t < hi; ++t) d += tmp[t] < k ? 1u : 0u;
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const uint32_t j = j0 + (uint32_t)(v * BLOCK);
+            if (j >= total) break;
+            if (k[v] >= a.n) {
+                atomicOr(a.err, 4u);
+                continue;
             }
-        } else {
-            // A cell this full only arises from collapsed or non-finite
-            // positions (clamped into one cell).  Ranking it costs its size
-            // per member, so it keeps the order its members were listed in
-            // (a valid permutation, not the stable one) and raises the error
-            // flag instead.
-            atomicOr(a.err, 8u);
+            uint32_t d = j;
+            if (unsorted) {
+                const uint32_t c = a.key0[k[v]] - base;
+                if (c >= kTileCells) {
+                    atomicOr(a.err, 4u);
+                    continue;
+                }
+                const uint32_t lo = s_off[c], hi = s_off[c + 1u];
+                if (hi - lo <= kMaxRankCell) {
+                    d = lo;
+                    if (in_lds) {
+#pragma unroll 4
+                        for (uint32_t t = lo; t < hi; ++t) d += s_mem[t] < k[v] ? 1u : 0u;
+                    } else {
+                        for (uint32_t t = lo; t < hi; ++t) d += tmp[t] < k[v] ? 1u : 0u;
+                    }
+                } else {
+                    // A cell this full only arises from collapsed or
+                    // non-finite positions (clamped into one cell).  Ranking
+                    // it costs its size per member, so it keeps the order its
+                    // members were listed in (a valid permutation, not the
+                    // stable one) and raises the error flag instead.
+                    atomicOr(a.err, 8u);
+                }
+            }
+            const uint32_t dst = pre + d;
+            if (dst >= a.n) {
+                atomicOr(a.err, 4u);
+                continue;
+            }
+            if (a.perm) a.perm[dst] = k[v];
+            a.pos_out[dst] = pk[v];
+            if (a.soa) {  // the planes, for the gathered density pass
+                a.soa[dst] = pk[v].x;
+                a.soa[a.n + dst] = pk[v].y;
+                a.soa[2 * (size_t)a.n + dst] = pk[v].z;
+            }
+            a.vel_out[dst] = vk[v];
+            a.id_out[dst] = ik[v];
         }
-        const uint32_t dst = pre + d;
-        if (dst >= a.n) {
-            atomicOr(a.err, 4u);
-            continue;
-        }
-        if (a.perm) a.perm[dst] = k;
-        if (a.skey) a.skey[dst] = base + c;
-        a.pos_out[dst] = pk;
-        if (a.soa) {  // the planes, for the gathered density pass
-            a.soa[dst] = pk.x;
-            a.soa[a.n + dst] = pk.y;
-            a.soa[2 * (size_t)a.n + dst] = pk.z;
-        }
-        a.vel_out[dst] = vk;
-        a.id_out[dst] = ik;
     }
 }
 
@@ -662,7 +708,6 @@ static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
     a.pos_out = sp.pos_out;
     a.vel_out = sp.vel_out;
     a.id_out = sp.id_out;
-    a.skey = sp.skey;
     a.perm = sp.perm;
     a.soa = sp.soa_out;
     a.queue = sp.queue;

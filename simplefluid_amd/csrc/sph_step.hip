@@ -650,17 +650,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
 // pass walks that list, without windows, masks or rows.
 
 constexpr uint32_t kKept = 5;        // a gathered row's terms kept in its copy's place
+constexpr uint32_t kChunk = 64;      // entries of a list in LDS at a time
 constexpr uint32_t kListOver = 0xffffu;
+template <bool V>
+struct Bool {
+    static constexpr bool value = V;
+};
 
 static_assert(kKept * kSplitTile * 4 <= sizeof(DensitySlot), "the kept terms fit a row's copy");
 
 struct SplitShared {
     DensitySlot rec[kRows];                        // the rows' copies, as planes: lanes read them in step,
                                                    // which records of 16 bytes would serve four at a time
-    float term[kListMax + 8][kSplitTile];          // the neighbours' terms, itself included
-    uint16_t id[kListMax + 4][kSplitTile];         // the neighbours; the particle itself goes to the last place
+    float term[kChunk + 4][kSplitTile];            // the neighbours' terms, itself included
+    uint16_t id[kChunk + 1][kSplitTile];           // the neighbours; the particle itself goes to the last place
     uint32_t count[3][kSplitTile];                 // neighbours per row, one byte a row (itself included)
-    uint32_t over;                                 // some row or list does not fit
+    uint32_t over;                                 // some row or list is too long
     float wall[kSplitTile];
 };
 
@@ -852,19 +857,35 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
         base = __builtin_amdgcn_sad_u8(c & before, 0u, base);
         total = __builtin_amdgcn_sad_u8(g == 2 ? c & 0xffu : c, 0u, total);
     }
-    // The list leaves the particle itself out (its term is in the sum).
     if (__ballot(total > kListMax + 1u) != 0u && lane == 0u && w == 0) sh.over = 1u;
-    const bool fits = __ballot(total > kListMax + 1u) == 0u;
-    if (fits) {
+    // A corner row has the fewest neighbours to list.
+    if (w == kRows - 1) {
+        float wr = 0.0f;
+        const float pk[3] = {pi.x, pi.y, pi.z};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            wr += wall_rho((pk[d] - sc.bmin[d]) * sc.inv_h);
+            wr += wall_rho((sc.wmax[d] - pk[d]) * sc.inv_h);
+        }
+        sh.wall[lane] = wr;
+    }
+    // Lists go through LDS kChunk entries at a time (nearly always once).
+    // The list for the force pass leaves the particle itself out; its term is
+    // in the sum.
+    const uint32_t most = wave_umax(total);
+    const uint32_t listed = total ? total - 1u : 0u;
+    float sum = 0.0f;
+    auto list = [&](uint32_t first, auto all) {
+        constexpr bool kAll = decltype(all)::value;  // every entry is in this chunk
+        uint32_t at = base - first, i = 0u;
         auto put = [&](uint32_t j, float c) {
-            sh.term[base][lane] = c;
+            if (kAll || at < kChunk) sh.term[at][lane] = c;
             // Candidates past k come one place earlier in the list (rows go
             // in ascending order).
-            const uint32_t e = base - (j > k ? 1u : 0u);
-            sh.id[j == k ? kListMax : e][lane] = (uint16_t)j;
-            ++base;
+            const uint32_t e = j == k ? kChunk : at - (j > k ? 1u : 0u);
+            if (kAll || e <= kChunk) sh.id[e][lane] = (uint16_t)j;
+            ++at;
         };
-        uint32_t i = 0u;
         auto bits = [&](uint32_t r, uint32_t j0) {
             if (fit)
                 split_bits(r, j0, staged_one,
@@ -884,67 +905,64 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
         };
         if (__ballot(mh != 0u)) bits(mask_ascending(mh, span, 32u), row_first(lo, hi, 2u));
         bits(mask_ascending(m, span, 0u), row_first(lo, hi));
-    }
-    // A corner row has the fewest neighbours to list.
-    if (w == kRows - 1) {
-        float wr = 0.0f;
-        const float pk[3] = {pi.x, pi.y, pi.z};
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            wr += wall_rho((pk[d] - sc.bmin[d]) * sc.inv_h);
-            wr += wall_rho((sc.wmax[d] - pk[d]) * sc.inv_h);
-        }
-        sh.wall[lane] = wr;
-    }
-    __syncthreads();
-    if (sh.over) {
-        // The first wave runs every row itself; the force pass walks masks.
-        if (w != 0) return;
-        float sum = 0.0f;
+    };
+    for (uint32_t first = 0u;; first += kChunk) {
+        if (most <= kChunk)
+            list(0u, Bool<true>());
+        else if (most <= kListMax + 1u)
+            list(first, Bool<false>());
+        __syncthreads();
+        if (sh.over) {
+            // The first wave runs every row itself; the force pass walks masks.
+            if (w != 0) return;
 #pragma unroll 1
-        for (int r = 0; r < kRows; ++r) {
-            split_window(rcs, sc, pi, r % 3 - 1, r / 3 - 1, lo, hi);
-            if (!active) lo = hi = 0u;
-            split_trips(gathered, pi, sc.h2, lo, hi, m, mh, [&](float c) { sum = fmaf(c * c, -c, sum); });
+            for (int r = 0; r < kRows; ++r) {
+                split_window(rcs, sc, pi, r % 3 - 1, r / 3 - 1, lo, hi);
+                if (!active) lo = hi = 0u;
+                split_trips(gathered, pi, sc.h2, lo, hi, m, mh, [&](float c) { sum = fmaf(c * c, -c, sum); });
+            }
+            if (active) {
+                a.ncount[k] = kListOver;
+                density_finish(a, sc, k, sum, sh.wall[lane]);
+            }
+            return;
         }
-        if (active) {
-            a.ncount[k] = kListOver;
-            density_finish(a, sc, k, sum, sh.wall[lane]);
-        }
-        return;
-    }
-    if (w != 0) {
-        if (!active) return;
-        const uint32_t listed = total ? total - 1u : 0u;
-        if (w == 1) a.ncount[k] = listed;
-        for (uint32_t q = (uint32_t)w - 1u; 4u * q < listed; q += (uint32_t)kRows - 1u)
-            reinterpret_cast<uint2*>(a.nlist)[(size_t)q * a.n + k] =
-                make_uint2(sh.id[4u * q][lane] | ((uint32_t)sh.id[4u * q + 1u][lane] << 16),
-                           sh.id[4u * q + 2u][lane] | ((uint32_t)sh.id[4u * q + 3u][lane] << 16));
-        return;
-    }
-    // Eight terms at a time, the next four loaded while four are added;
-    // terms past the list's end count as 0, which adds nothing.
-    float sum = 0.0f, c[4], d[4];
-    auto four = [&](uint32_t i, float* v) {
+        if (w != 0) {
+            if (active) {
+                if (w == 1 && first == 0u) a.ncount[k] = listed;
+                for (uint32_t q = (uint32_t)w - 1u; q < kChunk / 4u && first + 4u * q < listed; q += (uint32_t)kRows - 1u)
+                    reinterpret_cast<uint2*>(a.nlist)[(size_t)(first / 4u + q) * a.n + k] =
+                        make_uint2(sh.id[4u * q][lane] | ((uint32_t)sh.id[4u * q + 1u][lane] << 16),
+                                   sh.id[4u * q + 2u][lane] | ((uint32_t)sh.id[4u * q + 3u][lane] << 16));
+            }
+        } else {
+            // Eight terms at a time, the next four loaded while four are
+            // added; terms past the list's end count as 0, which adds nothing.
+            const uint32_t left = total > first ? min(total - first, kChunk) : 0u;
+            float c[4], d[4];
+            auto four = [&](uint32_t i, float* v) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = sh.term[i + u][lane];
-    };
-    auto add = [&](uint32_t i, const float* v) {
+                for (int u = 0; u < 4; ++u) v[u] = sh.term[i + u][lane];
+            };
+            auto add = [&](uint32_t i, const float* v) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float t = i + (uint32_t)u < total ? v[u] : 0.0f;
-            sum = fmaf(t * t, -t, sum);
+                for (int u = 0; u < 4; ++u) {
+                    const float t = i + (uint32_t)u < left ? v[u] : 0.0f;
+                    sum = fmaf(t * t, -t, sum);
+                }
+            };
+            four(0u, c);
+            for (uint32_t i = 0; i < left; i += 8u) {
+                four(i + 4u, d);
+                add(i, c);
+                four(min(i + 8u, kChunk), c);
+                add(i + 4u, d);
+            }
         }
-    };
-    four(0u, c);
-    for (uint32_t i = 0; i < total; i += 8u) {
-        four(i + 4u, d);
-        add(i, c);
-        four(min(i + 8u, kListMax + 4u), c);
-        add(i + 4u, d);
+        if (most <= first + kChunk) break;
+        __syncthreads();
     }
-    if (active) density_finish(a, sc, k, sum, sh.wall[lane]);
+    if (w == 0 && active) density_finish(a, sc, k, sum, sh.wall[lane]);
 }
 
 // Force, split form.  Four waves per 64 particles take the list in rounds of
@@ -1200,6 +1218,15 @@ __global__ void neighbors_kernel(StepArgs a, const uint32_t* __restrict__ offset
     }
 }
 
+// Keys of the sorted positions (the cell-count sort does not store them).
+__global__ void sorted_keys_kernel(const float4* __restrict__ pos_s, uint32_t* __restrict__ skey,
+                                   const SceneConst* __restrict__ scenes, const uint2* __restrict__ tiles) {
+    const uint2 ti = tile_at(tiles, blockIdx.x);
+    const SceneConst sc = scene_at(scenes, ti.x);
+    const uint32_t k = ti.y + threadIdx.x;
+    if (k < sc.p_end) skey[k] = cell_key(sc, pos_s[k].x, pos_s[k].y, pos_s[k].z);
+}
+
 // dt = min(dt_max, (cfl h) / (c0 + |v|max)) per scene, in this op order.
 // With a frame state: nothing once halted; else scene 0's step is added to
 // the frame time (float, as the host frame loop adds it) and a frame of at
@@ -1357,6 +1384,13 @@ hipError_t launch_neighbors(hipStream_t st, int block, uint32_t grid, const Step
         hipLaunchKernelGGL(neighbors_kernel<1>, dim3(grid), dim3(block), 0, st, a, offsets, out);
     else
         hipLaunchKernelGGL(neighbors_kernel<0>, dim3(grid), dim3(block), 0, st, a, offsets, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_sorted_keys(hipStream_t st, int block, uint32_t ntiles, const float4* pos_s, uint32_t* skey,
+                              const SceneConst* scenes, const uint2* tiles) {
+    if (ntiles == 0) return hipSuccess;
+    hipLaunchKernelGGL(sorted_keys_kernel, dim3(ntiles), dim3(block), 0, st, pos_s, skey, scenes, tiles);
     return hipGetLastError();
 }
 
