@@ -163,8 +163,9 @@ struct sph_handle {
     std::map<int, sph::DevBuf<uint2>> tiles;
     std::map<int, uint32_t> ntiles;
     sph::DevBuf<float> staging;
-    float* host_pinned = nullptr;          // 3n floats of page-locked host memory for downloads
-    size_t host_pinned_n = 0;
+    float* host_pinned = nullptr;          // page-locked host memory for downloads, one word longer than
+    size_t host_pinned_n = 0;              // host_pinned_n
+    std::vector<hipEvent_t> copy_events;   // points of a large download
     // Asynchronous frame snapshot: positions un-permuted on the step stream
     // into snap_d, copied to snap_host on copy_stream while steps continue.
     hipStream_t copy_stream = nullptr;

@@ -147,6 +147,9 @@ hipError_t launch_sorted_keys(hipStream_t st, int block, uint32_t ntiles, const 
 // Original-order gather for get_*: out[3*id[k]+c] = src[k].c
 hipError_t launch_unpermute3(hipStream_t st, uint32_t n, const float4* src, const uint32_t* id,
                              float* out);
+// Copies words of device memory and, behind them, *flag to dst (page-locked
+// host memory).
+hipError_t launch_copy_out(hipStream_t st, const uint32_t* src, size_t words, const uint32_t* flag, uint32_t* dst);
 hipError_t launch_unpermute1(hipStream_t st, uint32_t n, const float* src, const uint32_t* id,
                              float* out);
 // dst[k] = (src[3k], src[3k+1], src[3k+2], 0), or zero when src is null.

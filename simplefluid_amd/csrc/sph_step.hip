@@ -1277,6 +1277,17 @@ __global__ void unpermute3_kernel(uint32_t n, const float4* __restrict__ src,
     out[3 * (size_t)i + 2] = v.z;
 }
 
+// 16 bytes per lane (both buffers start 256-byte aligned), the rest and the
+// flag by the first lanes.
+__global__ void copy_out_kernel(const uint32_t* __restrict__ src, size_t words, const uint32_t* __restrict__ flag,
+                                uint32_t* __restrict__ dst) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t quads = words / 4;
+    if (i < quads) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    if (i < words % 4) dst[4 * quads + i] = src[4 * quads + i];
+    if (i == 0) dst[words] = *flag;
+}
+
 __global__ void unpermute1_kernel(uint32_t n, const float* __restrict__ src,
                                   const uint32_t* __restrict__ id, float* __restrict__ out) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1422,6 +1433,12 @@ hipError_t launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t value, size_t c
 hipError_t launch_unpermute3(hipStream_t st, uint32_t n, const float4* src, const uint32_t* id, float* out) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(unpermute3_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, src, id, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_out(hipStream_t st, const uint32_t* src, size_t words, const uint32_t* flag, uint32_t* dst) {
+    const size_t lanes = words / 4 > 64 ? words / 4 : 64;
+    hipLaunchKernelGGL(copy_out_kernel, dim3(blocks_for(lanes, 256)), dim3(256), 0, st, src, words, flag, dst);
     return hipGetLastError();
 }
 
