@@ -424,15 +424,20 @@ __device__ __forceinline__ void add_tile_sums(uint32_t* __restrict__ tsum, uint3
     if (r.first) atomicAdd(tsum + tile, (uint32_t)(r.end - (int)lane));
 }
 
-// Adds the wave's largest |v|^2 to arr[idx] (float bits; atomic max on the
-// bit patterns orders non-negative floats).  NaN counts as 0.  All lanes of
-// the wave must call it, with idx uniform.
-__device__ __forceinline__ void wave_max_v2(uint32_t* __restrict__ arr, uint32_t idx, float vx, float vy, float vz,
-                                            bool active) {
-    float v2 = active ? fmaxf(fmaf(vz, vz, fmaf(vy, vy, vx * vx)), 0.0f) : 0.0f;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v2 = fmaxf(v2, __shfl_xor(v2, o, 64));
-    if ((threadIdx.x & 63u) == 0u) atomicMax(arr + idx, __float_as_uint(v2));
+// |v|^2 for the CFL step; NaN counts as 0.
+__device__ __forceinline__ float speed2(float vx, float vy, float vz) {
+    return fmaxf(fmaf(vz, vz, fmaf(vy, vy, vx * vx)), 0.0f);
+}
+
+// Adds the wave's largest |v|^2 to one of kSpeedSlots words (float bits;
+// integer maxima of the bit patterns order non-negative floats), picked by
+// block: on one word the waves' atomics queue (414 of them: force pass 10.1
+// against 8.4 us).  All lanes of the wave must call it, lanes without a
+// particle with 0.
+constexpr uint32_t kSpeedSlots = 64;
+__device__ __forceinline__ void wave_max_v2(uint32_t* __restrict__ slots, float v2) {
+    const uint32_t m = wave_umax(__float_as_uint(v2));
+    if ((threadIdx.x & 63u) == 0u) atomicMax(slots + blockIdx.x % kSpeedSlots, m);
 }
 
 // Walls.  Each box face bounds a half-space of fluid at rest density; a

@@ -217,6 +217,11 @@ StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     a.ncount = h->ncount.p;
     a.acc = (h->keep_acc || w.acc.p) ? w.acc.p : nullptr;
     a.scenes = h->sc_d.p;
+    if (h->cfl) {
+        a.vmax2 = h->vmax2.p;
+        a.cfl_scene = h->sc_d.p;
+        a.dt_out = h->dt_dev.p;
+    }
     a.tiles = tiles_for(h, block, a.ntiles);
     a.n = h->n;
     a.ncells = h->ncells;
@@ -264,7 +269,7 @@ static int ensure_buffers(sph_handle* h) {
     chk(h->tickets.ensure(kMaxPasses));
     chk(h->err.ensure(1));
     chk(h->queue.ensure(kQueueWords));
-    chk(h->vmax2.ensure(h->sc_h.size()));
+    chk(h->vmax2.ensure(kSpeedSlots));
     chk(h->dt_dev.ensure(1));
     chk(h->frame.ensure(kFrameWords));
     chk(h->staging.ensure(3 * n + 1));
@@ -273,7 +278,7 @@ static int ensure_buffers(sph_handle* h) {
     chk(launch_fill_u32(h->stream, h->hist.p, 0u, kMaxPasses * 256));
     chk(launch_fill_u32(h->stream, h->err.p, 0u, 1));
     chk(launch_fill_u32(h->stream, h->queue.p, 0u, kQueueWords));
-    chk(launch_fill_u32(h->stream, h->vmax2.p, 0u, h->sc_h.size()));
+    chk(launch_fill_u32(h->stream, h->vmax2.p, 0u, kSpeedSlots));
     if (fresh_head) chk(launch_fill_u32(h->stream, h->head.p, 0u, head_words));
     chk(hipMemcpyAsync(h->sc_d.p, h->sc_h.data(), h->sc_h.size() * sizeof(SceneConst), hipMemcpyHostToDevice, h->stream));
     if (e != hipSuccess) return hip_fail(h, e, "buffer init");
@@ -298,27 +303,32 @@ static void prof_record(sph_handle* h, int slot) {
     (void)hipEventRecord(h->prof_events[idx], h->stream);
 }
 
+// New state: the chains start empty, then every particle is hashed.
+static int enqueue_hash(sph_handle* h) {
+    hipStream_t st = h->stream;
+    hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells));
+    if (e == hipSuccess && h->cfl) e = launch_fill_u32(st, h->vmax2.p, 0u, kSpeedSlots);
+    uint32_t nt = 0;
+    const uint2* tl = tiles_for(h, 256, nt);
+    if (e == hipSuccess)
+        e = launch_hash(st, 256, nt, h->pos.p, h->vel.p, h->key0.p, h->next.p, h->head.p, h->ncells,
+                        h->cfl ? h->vmax2.p : nullptr, h->sc_d.p, tl, nt);
+    if (e != hipSuccess) return hip_fail(h, e, "hash launch");
+    h->keys_valid = true;
+    return SPH_OK;
+}
+
 int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) {
     hipStream_t st = h->stream;
     if (frame) {
         if (!h->keys_valid || h->tune.sort_mode != kSortCellCount)
             return fail(h, SPH_E_INVALID, "the device frame loop needs a steady cell-count step");
-        const hipError_t ge = launch_frame_gate(st, frame);
-        if (ge != hipSuccess) return hip_fail(h, ge, "frame gate launch");
     }
     const uint8_t hashed = h->keys_valid ? 0 : 1;
     if (record_prof) prof_record(h, 0);
     if (!h->keys_valid) {
-        // New state: the chains start empty, then every particle is hashed.
-        hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells));
-        if (e == hipSuccess && h->cfl) e = launch_fill_u32(st, h->vmax2.p, 0u, h->sc_h.size());
-        uint32_t nt = 0;
-        const uint2* tl = tiles_for(h, 256, nt);
-        if (e == hipSuccess)
-            e = launch_hash(st, 256, nt, h->pos.p, h->vel.p, h->key0.p, h->next.p, h->head.p, h->ncells,
-                            h->cfl ? h->vmax2.p : nullptr, h->sc_d.p, tl, nt);
-        if (e != hipSuccess) return hip_fail(h, e, "hash launch");
-        h->keys_valid = true;
+        const int rc = enqueue_hash(h);
+        if (rc != SPH_OK) return rc;
     }
     if (record_prof) prof_record(h, 1);
     SortPlan sp;
@@ -348,7 +358,7 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     sp.pos_out = w.pos_s.p;
     const bool split = split_form(h);
     sp.soa_out = h->tune.density_staged || split ? nullptr : w.soa.p;
-    sp.halt = frame;
+    sp.frame = frame;
     sp.vel_out = w.vel_s.p;
     sp.id_out = w.id_s.p;
     hipError_t e = launch_sort_keys(st, sp);
@@ -359,32 +369,25 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     if (record_prof) prof_record(h, 3);
     if (split) {
         StepArgs a = step_args(h, w, kSplitTile);
-        a.halt = frame;
+        a.frame = frame;
         e = launch_density_split(st, a);
         if (e != hipSuccess) return hip_fail(h, e, "density launch");
     } else {
         StepArgs a = step_args(h, w, h->tune.density_block);
-        a.halt = frame;
+        a.frame = frame;
         const uint32_t grid = grid_for(h, h->tune.density_block, a.ntiles, &a.queue);
         e = launch_density(st, h->tune.density_block, grid, a, h->tune.density_staged);
         if (e != hipSuccess) return hip_fail(h, e, "density launch");
     }
     if (record_prof) prof_record(h, 4);
-    if (h->cfl) {
-        // Step length from the largest speed of the state this step starts from.
-        e = launch_cfl(st, (uint32_t)h->sc_h.size(), h->sc_d.p, h->vmax2.p, h->dt_dev.p, frame);
-        if (e != hipSuccess) return hip_fail(h, e, "cfl launch");
-    }
     if (split) {
         StepArgs a = step_args(h, w, kSplitTile);
-        a.vmax2 = h->cfl ? h->vmax2.p : nullptr;
-        a.halt = frame;
+        a.frame = frame;
         e = launch_force_split(st, a);
         if (e != hipSuccess) return hip_fail(h, e, "force launch");
     } else {
         StepArgs a = step_args(h, w, h->tune.force_block);
-        a.vmax2 = h->cfl ? h->vmax2.p : nullptr;
-        a.halt = frame;
+        a.frame = frame;
         const uint32_t grid = grid_for(h, h->tune.force_block, a.ntiles, &a.queue,
                                        force_blocks_per_cu(h->tune.force_block, h->tune.force_staged));
         e = launch_force(st, h->tune.force_block, grid, a, h->tune.force_staged);
@@ -752,8 +755,8 @@ static int step_once(sph_handle* h) {
     return enqueue_step(h, h->work, h->prof);
 }
 
-// Captures one steady step; gated: the device frame loop's step.
-// Steps in the multi-step graph.
+// Captures steady steps; gated: the device frame loop's.
+// Steps in the multi-step graphs.
 constexpr uint32_t kGraphSteps = 8;
 
 enum GraphKind { kGraphOne, kGraphMulti, kGraphFrame };
@@ -778,7 +781,7 @@ static int capture_graph(sph_handle* h, GraphKind kind = kGraphOne) {
     hipError_t e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(h, e, "begin capture");
     int rc = SPH_OK;
-    const uint32_t steps = kind == kGraphMulti ? kGraphSteps : 1u;
+    const uint32_t steps = kind == kGraphOne ? 1u : kGraphSteps;
     for (uint32_t s = 0; s < steps && rc == SPH_OK; ++s)
         rc = enqueue_step(h, h->work, false, gated ? h->frame.p : nullptr);
     hipGraph_t g = nullptr;
@@ -851,11 +854,13 @@ static int run_frame_on_device(sph_handle* h, float& frame_time, uint32_t& steps
         const int rc = capture_graph(h, kGraphFrame);
         if (rc != SPH_OK) return rc;
     }
+    // Steps come kGraphSteps to a graph; those past the frame's end are skipped.
     uint32_t batch = h->frame_steps_hint ? h->frame_steps_hint + 1 : 16;
     uint64_t launched = 0;
     uint32_t fs[kFrameWords] = {0u, 0u, 0u, 0u};
     for (;;) {
-        for (uint32_t i = 0; i < batch; ++i) {
+        batch = (batch + kGraphSteps - 1) / kGraphSteps * kGraphSteps;
+        for (uint32_t i = 0; i < batch; i += kGraphSteps) {
             e = hipGraphLaunch(h->gexec_frame, st);
             if (e != hipSuccess) return hip_fail(h, e, "graph launch");
         }
@@ -882,9 +887,9 @@ int sph_run_frame(sph_handle* h, float* frame_time_out, uint32_t* steps_out) {
     if (!h) return SPH_E_INVALID;
     float frame_time = 0.0f;
     uint32_t steps = 0;
-    if (h->cfl && h->ready && h->use_graph && !h->prof && h->keys_valid && !h->keep_acc &&
-        h->tune.sort_mode == kSortCellCount) {
-        const int rc = run_frame_on_device(h, frame_time, steps);
+    if (h->cfl && h->ready && h->use_graph && !h->prof && !h->keep_acc && h->tune.sort_mode == kSortCellCount) {
+        int rc = h->keys_valid ? SPH_OK : enqueue_hash(h);
+        if (rc == SPH_OK) rc = run_frame_on_device(h, frame_time, steps);
         if (rc != SPH_OK) return rc;
         if (frame_time_out) *frame_time_out = frame_time;
         if (steps_out) *steps_out = steps;

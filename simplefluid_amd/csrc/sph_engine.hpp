@@ -157,7 +157,7 @@ struct sph_handle {
     sph::StepBufs work;
     sph::DevBuf<uint32_t> hist, status, tickets, err, queue;
     bool cfl = false;                      // adaptive step (single scene)
-    sph::DevBuf<uint32_t> vmax2;           // per-scene max |v|^2 bits for the next step
+    sph::DevBuf<uint32_t> vmax2;           // max |v|^2 bits for the next step (kSpeedSlots words)
     sph::DevBuf<float> dt_dev;             // step length of the last step (scene 0)
     sph::DevBuf<sph::SceneConst> sc_d;
     std::map<int, sph::DevBuf<uint2>> tiles;

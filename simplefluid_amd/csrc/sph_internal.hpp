@@ -36,7 +36,7 @@ struct SortPlan {
     uint32_t* tickets = nullptr;      // radix: kMaxPasses
     uint32_t* err = nullptr;
     uint32_t* queue = nullptr;        // kQueueWords tile counters, zeroed by the sort
-    const uint32_t* halt = nullptr;   // device frame loop: non-zero word skips the step (cell-count mode)
+    uint32_t* frame = nullptr;        // device frame loop's state (cell-count mode), else null
     const float4* pos_in = nullptr;
     const float4* vel_in = nullptr;
     const uint32_t* id_in = nullptr;
@@ -84,8 +84,11 @@ struct StepArgs {
     uint32_t n;
     uint32_t ncells;
     uint32_t* queue;         // persistent launch: 8 tile counters (zeroed by the sort), else null
-    uint32_t* vmax2;         // CFL: per-scene max |v|^2 (float bits) of the new state, else null
-    const uint32_t* halt;    // device frame loop: non-zero word skips the step, else null
+    uint32_t* vmax2;         // CFL: kSpeedSlots words of max |v|^2 (float bits) of the state the step starts
+                             // from (density), of the new state (force), else null
+    SceneConst* cfl_scene;   // CFL: the scene whose dt the density pass sets from vmax2 (one scene), else null
+    float* dt_out;           // CFL: receives that dt
+    uint32_t* frame;         // device frame loop's state, else null
 };
 
 // Tile counters of the persistent density and force launches (8 each),
@@ -99,19 +102,13 @@ hipError_t launch_hash(hipStream_t st, int block, uint32_t grid, const float4* p
 hipError_t launch_upload_hash(hipStream_t st, const float* xyz, const float* vel_in, float4* pos, float4* vel,
                               uint32_t* id, uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t n,
                               uint32_t ncells, const SceneConst& sc);
-// CFL step of every scene from its max |v|^2 (scenes with cfl = 0 keep dt);
-// clears vmax2 and stores scene 0's step in *dt_out.  With a frame state
-// (below) the kernel does nothing once the frame is halted, and otherwise
-// adds scene 0's step to the frame time.
-hipError_t launch_cfl(hipStream_t st, uint32_t nscenes, SceneConst* scenes, uint32_t* vmax2, float* dt_out,
-                      uint32_t* frame);
 // Device frame loop state, 4 words: halt (steps are skipped), pending (the
 // frame reached 1/30 s in the current step), steps taken, frame time (float
-// bits).  reset zeroes them; gate, run first in each step, turns pending
-// into halt, so the step that completes the frame runs to its end.
+// bits).  reset zeroes them; the density pass adds its step and sets pending,
+// so the step that completes the frame runs to its end, and the next step's
+// sort turns pending into halt.
 constexpr int kFrameWords = 4;
 hipError_t launch_frame_reset(hipStream_t st, uint32_t* frame);
-hipError_t launch_frame_gate(hipStream_t st, uint32_t* frame);
 // staged: the density pass reads each row's candidates from LDS (same results).
 hipError_t launch_density(hipStream_t st, int block, uint32_t grid, const StepArgs& a, int staged = 0);
 // staged: the force pass reads each row's candidates from LDS (same results).

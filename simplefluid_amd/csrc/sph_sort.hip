@@ -127,8 +127,8 @@ constexpr int kTileScanBlock = 1024;
 constexpr uint32_t kInlineTiles = 6144;
 
 __global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __restrict__ head, uint32_t C,
-                                                                   uint32_t T, const uint32_t* __restrict__ halt) {
-    if (halt && *halt) return;
+                                                                   uint32_t T, const uint32_t* __restrict__ frame) {
+    if (frame && (frame[0] | frame[1])) return;
     __shared__ uint32_t s_w[kTileScanBlock / 64];
     __shared__ uint32_t s_pre[kTileScanBlock / 64];
     const uint32_t* tsum = head + C;
@@ -175,7 +175,7 @@ struct CellSortArgs {
     float* soa;
     uint32_t* queue;
     uint32_t* err;
-    const uint32_t* halt;
+    uint32_t* frame;     // device frame loop's state, or null
     int gather;          // 0: the cell-start table only (radix mode)
 };
 
@@ -198,7 +198,12 @@ constexpr uint32_t kWideTiles = 1024;
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
-    if (a.halt && *a.halt) return;
+    // A frame that is complete (pending, or halted already) skips the step;
+    // the first kernel of the step turns pending into halt for the others.
+    if (a.frame && (a.frame[0] | a.frame[1])) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.frame[0] = 1u;
+        return;
+    }
     constexpr int V = (int)kTileCells / BLOCK;
     constexpr int kWaves = BLOCK / 64;
     static_assert(V == 1 || V == 4, "one head, or four in one 16-byte load, per thread");
@@ -692,7 +697,7 @@ static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
     const uint32_t tiles = scan_tiles(sp.ncells);
     if (tiles > kInlineTiles)
         hipLaunchKernelGGL(tile_scan_kernel, dim3((tiles + kTileScanBlock - 1) / kTileScanBlock), dim3(kTileScanBlock),
-                           0, st, sp.head, sp.ncells, tiles, sp.halt);
+                           0, st, sp.head, sp.ncells, tiles, sp.frame);
     CellSortArgs a;
     a.n = sp.n;
     a.C = sp.ncells;
@@ -712,7 +717,7 @@ static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
     a.soa = sp.soa_out;
     a.queue = sp.queue;
     a.err = sp.err;
-    a.halt = sp.halt;
+    a.frame = sp.frame;
     a.gather = gather;
     if (tiles <= kWideTiles)
         hipLaunchKernelGGL(cell_sort_kernel<1024>, dim3(tiles), dim3(1024), 0, st, a);
@@ -727,7 +732,7 @@ hipError_t launch_sort_keys(hipStream_t st, const SortPlan& sp) {
         return hipGetLastError();
     }
     launch_cell_sort(st, sp, 0);
-    if (sp.halt) return hipErrorInvalidValue;  // the frame loop runs the cell-count sort only
+    if (sp.frame) return hipErrorInvalidValue;  // the frame loop runs the cell-count sort only
     const uint32_t tiles = sort_tiles(sp.n, sp.items);
     const uint32_t hist_blocks = (sp.n + kSortBlock * kHistItems - 1) / (kSortBlock * kHistItems);
     const uint32_t status_words = (uint32_t)sp.passes * tiles * kBins;

@@ -124,6 +124,7 @@ __device__ __forceinline__ void density_one(const StepArgs& a, const SceneConst&
 // floats per plane, a trip's reads of all three planes fit the 8-bit dword
 // offsets of ds_read2_b32 from one address (z at 248..251).
 constexpr uint32_t kStageD = 120;
+static_assert(kSpeedSlots == 64, "a wave reads the speed slots");
 static_assert(kStageD <= 128, "the copy into a slot takes two records per lane");
 constexpr uint32_t kPlaneD = kStageD + 4;
 struct DensitySlot {
@@ -310,6 +311,12 @@ struct ForceAcc {
     float px, py, pz, vx, vy, vz;
 };
 
+// A particle's next key and its new |v|^2.
+struct Moved {
+    uint32_t key;
+    float v2;
+};
+
 // pos.w = p/rho^2 and vel.w = 1/rho of each particle.
 __device__ __forceinline__ void force_pair(const SceneConst& sc, const float4& pi, const float4& vi,
                                            const float4& pj, const float4& vj, ForceAcc& f) {
@@ -332,7 +339,7 @@ __device__ __forceinline__ void force_pair(const SceneConst& sc, const float4& p
     f.vz = fmaf(vv, vj.z - vi.z, f.vz);
 }
 
-__device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
+__device__ __forceinline__ Moved force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                                  const float4& pi, const float4& vi, const ForceAcc& f);
 
 // The centre row's mask word (its last slot `after` slots before the row's
@@ -342,7 +349,7 @@ __device__ __forceinline__ uint32_t without_self(uint32_t word, uint32_t lo, uin
     return b < (uint32_t)kMaskBits ? word & ~(1u << b) : word;
 }
 
-__device__ __forceinline__ uint32_t force_one(const StepArgs& a, const SceneConst& sc, uint32_t k,
+__device__ __forceinline__ Moved force_one(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                               __amdgpu_buffer_rsrc_t rpos, __amdgpu_buffer_rsrc_t rvel,
                                               __amdgpu_buffer_rsrc_t rcs) {
     const float4 pi = load4(rpos, k << 4);
@@ -390,7 +397,7 @@ __device__ __forceinline__ uint32_t force_one(const StepArgs& a, const SceneCons
 
 // Integrate, clamp and stores of particle k, given its neighbours' sums, the
 // walls' differences wj and its id; returns its next key.
-__device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
+__device__ __forceinline__ Moved force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                                  const float4& pi, const float4& vi, const ForceAcc& f,
                                                  const float wj[3], uint32_t id) {
     const float cvi = sc.cV * vi.w;
@@ -427,10 +434,10 @@ __device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneC
             a.vel_out[3 * (size_t)id + d] = v[d];
         }
     }
-    return cell_key(sc, p[0], p[1], p[2]);
+    return {cell_key(sc, p[0], p[1], p[2]), speed2(v[0], v[1], v[2])};
 }
 
-__device__ __forceinline__ uint32_t force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
+__device__ __forceinline__ Moved force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                                  const float4& pi, const float4& vi, const ForceAcc& f) {
     const float pk[3] = {pi.x, pi.y, pi.z};
     float wj[3];
@@ -459,7 +466,7 @@ struct StageSlot {
 // slot.  Same pairs, same order, same arithmetic: the results are
 // force_one's bit for bit.  Every lane of the wave calls it (the copy and
 // the wave-wide bounds need them all); inactive lanes have empty windows.
-__device__ __forceinline__ uint32_t force_one_staged(const StepArgs& a, const SceneConst& sc, uint32_t k,
+__device__ __forceinline__ Moved force_one_staged(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                                      bool active, __amdgpu_buffer_rsrc_t rpos,
                                                      __amdgpu_buffer_rsrc_t rvel, __amdgpu_buffer_rsrc_t rcs,
                                                      StageSlot& slot_a, StageSlot& slot_b) {
@@ -532,12 +539,33 @@ __device__ __forceinline__ uint32_t force_one_staged(const StepArgs& a, const Sc
                 [&](uint32_t j) { force_pair(sc, pi, vi, load4(rpos, j << 4), load4(rvel, j << 4), f); });
         }
     }
-    return active ? force_finish(a, sc, k, pi, vi, f) : 0u;
+    return active ? force_finish(a, sc, k, pi, vi, f) : Moved{0u, 0.0f};
 }
 
-// The sort has read the tile sums; the density pass clears them for the
-// integrate pass.
-__device__ __forceinline__ void clear_tile_sums(const StepArgs& a) {
+// The step's bookkeeping, done by the density pass between the sort and the
+// force pass: the sort has read the tile sums, which are cleared for the
+// integrate pass, and the CFL step is set (launches of their own cost 4-6 us
+// of a 40 us step each: 26k particles).  dt = min(dt_max, (cfl h) / (c0 +
+// |v|max)), in this op order; no density reads dt.  With a frame state, the
+// step is added to the frame time (float, as the host frame loop adds it) and
+// a frame of at least 1/30 s marks pending.
+__device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
+    if (a.cfl_scene && blockIdx.x == 0 && threadIdx.x < kSpeedSlots) {  // the first wave
+        const uint32_t v2 = wave_umax(a.vmax2[threadIdx.x]);
+        a.vmax2[threadIdx.x] = 0u;
+        if (threadIdx.x == 0) {
+            SceneConst& sc = *a.cfl_scene;
+            const float dt = fminf(sc.dt_max, (sc.cfl * sc.h) / (sc.c0 + sqrtf(__uint_as_float(v2))));
+            sc.dt = dt;
+            *a.dt_out = dt;
+            if (a.frame) {
+                const float ft = __uint_as_float(a.frame[3]) + dt;
+                a.frame[3] = __float_as_uint(ft);
+                a.frame[2] += 1u;
+                if (!((double)ft < 0.0333333333)) a.frame[1] = 1u;
+            }
+        }
+    }
     if (!a.head) return;
     const uint32_t words = (a.ncells + kTileCells - 1u) >> kTileShift;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
@@ -546,23 +574,19 @@ __device__ __forceinline__ void clear_tile_sums(const StepArgs& a) {
 
 // Next step's key, its run in the cell's chain, the tile sums and the largest
 // speed (whole wave).
-__device__ __forceinline__ void finish_particle(const StepArgs& a, uint32_t scene, uint32_t k, uint32_t key,
-                                                bool active) {
+__device__ __forceinline__ void finish_particle(const StepArgs& a, uint32_t k, const Moved& to, bool active) {
+    const uint32_t key = to.key;
     if (!a.head) return;  // a single step: there is no next one
     add_tile_sums(a.head + a.ncells, key, active);
-    if (a.vmax2) {
-        float4 vn = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (active) vn = a.vel_o[k];
-        wave_max_v2(a.vmax2, scene, vn.x, vn.y, vn.z, active);
-    }
+    if (a.vmax2) wave_max_v2(a.vmax2, to.v2);
     if (active) a.key0[k] = key;
     push_run(a.head, a.next, key, k, active);  // last: it waits for its exchange's answer
 }
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void density_kernel(StepArgs a) {
-    if (a.halt && *a.halt) return;
-    clear_tile_sums(a);
+    if (a.frame && a.frame[0]) return;
+    step_bookkeeping(a);
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
     const __amdgpu_buffer_rsrc_t rx = buffer_of(a.soa, a.n);
     const __amdgpu_buffer_rsrc_t ry = buffer_of(a.soa + a.n, a.n);
@@ -580,8 +604,8 @@ __global__ __launch_bounds__(BLOCK) void density_kernel(StepArgs a) {
 // waves per SIMD: the bound fits it in 59 VGPRs without spills (65 without).
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void density_staged_kernel(StepArgs a) {
-    if (a.halt && *a.halt) return;
-    clear_tile_sums(a);
+    if (a.frame && a.frame[0]) return;
+    step_bookkeeping(a);
     __shared__ DensitySlot s_slot[BLOCK / 64];
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
     const __amdgpu_buffer_rsrc_t rcs = buffer_of(a.cstart, a.ncells + 1u);
@@ -597,7 +621,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) v
 // Six waves per SIMD (77 VGPRs, no VGPR spills).
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) void force_kernel(StepArgs a) {
-    if (a.halt && *a.halt) return;
+    if (a.frame && a.frame[0]) return;
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
     const __amdgpu_buffer_rsrc_t rvel = buffer_of(a.vel_s, a.n);
     const __amdgpu_buffer_rsrc_t rcs = buffer_of(a.cstart, a.ncells + 1u);
@@ -607,9 +631,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
         const SceneConst sc = scene_at(a.scenes, ti.x);
         const uint32_t k = ti.y + threadIdx.x;
         const bool active = k < sc.p_end;
-        uint32_t key = 0;
-        if (active) key = force_one(a, sc, k, rpos, rvel, rcs);
-        finish_particle(a, ti.x, k, key, active);
+        Moved to = {0u, 0.0f};
+        if (active) to = force_one(a, sc, k, rpos, rvel, rcs);
+        finish_particle(a, k, to, active);
     });
 }
 
@@ -618,7 +642,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
 // waves without it).
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) void force_staged_kernel(StepArgs a) {
-    if (a.halt && *a.halt) return;
+    if (a.frame && a.frame[0]) return;
     __shared__ StageSlot s_slot_a[BLOCK / 64];
     __shared__ StageSlot s_slot_b[BLOCK / 64];
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
@@ -632,8 +656,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
         const SceneConst sc = scene_at(a.scenes, ti.x);
         const uint32_t k = ti.y + threadIdx.x;
         const bool active = k < sc.p_end;
-        const uint32_t key = force_one_staged(a, sc, k, active, rpos, rvel, rcs, slot_a, slot_b);
-        finish_particle(a, ti.x, k, key, active);
+        const Moved to = force_one_staged(a, sc, k, active, rpos, rvel, rcs, slot_a, slot_b);
+        finish_particle(a, k, to, active);
     });
 }
 
@@ -779,8 +803,8 @@ __device__ __forceinline__ void split_bits(uint32_t r, uint32_t j0, G&& get, F&&
 }
 
 __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
-    if (a.halt && *a.halt) return;
-    clear_tile_sums(a);
+    if (a.frame && a.frame[0]) return;
+    step_bookkeeping(a);
     __shared__ SplitShared sh;
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
     const __amdgpu_buffer_rsrc_t rcs = buffer_of(a.cstart, a.ncells + 1u);
@@ -985,7 +1009,7 @@ struct ForceSplitShared {
 };
 
 __global__ __launch_bounds__(64 * kForceWaves) void force_split_kernel(StepArgs a) {
-    if (a.halt && *a.halt) return;
+    if (a.frame && a.frame[0]) return;
     __shared__ ForceSplitShared sh;
     const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
     const __amdgpu_buffer_rsrc_t rvel = buffer_of(a.vel_s, a.n);
@@ -1014,9 +1038,9 @@ __global__ __launch_bounds__(64 * kForceWaves) void force_split_kernel(StepArgs 
     gather();  // before the counts are known: any index stays inside the buffers' bounds checks
     if (__ballot(count > kListMax) != 0u) {  // the same in every wave
         if (w != 0) return;
-        uint32_t key = 0;
-        if (active) key = force_one(a, sc, k, rpos, rvel, buffer_of(a.cstart, a.ncells + 1u));
-        finish_particle(a, ti.x, k, key, active);
+        Moved to = {0u, 0.0f};
+        if (active) to = force_one(a, sc, k, rpos, rvel, buffer_of(a.cstart, a.ncells + 1u));
+        finish_particle(a, k, to, active);
         return;
     }
     float f[3] = {0.f, 0.f, 0.f};
@@ -1085,13 +1109,13 @@ __global__ __launch_bounds__(64 * kForceWaves) void force_split_kernel(StepArgs 
     }
     __syncthreads();
     if (w != 0) return;
-    uint32_t key = 0;
+    Moved to = {0u, 0.0f};
     if (active) {
         const ForceAcc acc = {f[0], f[1], f[2], sh.sum[0][lane], sh.sum[1][lane], sh.sum[2][lane]};
         const float wj[3] = {sh.wall[0][lane], sh.wall[1][lane], sh.wall[2][lane]};
-        key = force_finish(a, sc, k, pi, vi, acc, wj, sh.id[lane]);
+        to = force_finish(a, sc, k, pi, vi, acc, wj, sh.id[lane]);
     }
-    finish_particle(a, ti.x, k, key, active);
+    finish_particle(a, k, to, active);
 }
 
 // Uploads come in any order, a lattice's fastest axis often across the
@@ -1152,7 +1176,7 @@ __global__ void hash_kernel(const float4* __restrict__ pos, const float4* __rest
         if (vmax2) {
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
             if (active) v = vel[k];
-            wave_max_v2(vmax2, ti.x, v.x, v.y, v.z, active);
+            wave_max_v2(vmax2, speed2(v.x, v.y, v.z));
         }
     }
     sums.flush();
@@ -1227,38 +1251,8 @@ __global__ void sorted_keys_kernel(const float4* __restrict__ pos_s, uint32_t* _
     if (k < sc.p_end) skey[k] = cell_key(sc, pos_s[k].x, pos_s[k].y, pos_s[k].z);
 }
 
-// dt = min(dt_max, (cfl h) / (c0 + |v|max)) per scene, in this op order.
-// With a frame state: nothing once halted; else scene 0's step is added to
-// the frame time (float, as the host frame loop adds it) and a frame of at
-// least 1/30 s marks pending.
-__global__ void cfl_kernel(uint32_t nscenes, SceneConst* __restrict__ scenes, uint32_t* __restrict__ vmax2,
-                           float* __restrict__ dt_out, uint32_t* __restrict__ frame) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nscenes) return;
-    if (frame && frame[0]) return;
-    SceneConst& sc = scenes[s];
-    if (sc.cfl > 0.0f) {
-        const float vmax = sqrtf(__uint_as_float(vmax2[s]));
-        sc.dt = fminf(sc.dt_max, (sc.cfl * sc.h) / (sc.c0 + vmax));
-    }
-    vmax2[s] = 0u;
-    if (s == 0) {
-        *dt_out = sc.dt;
-        if (frame) {
-            const float ft = __uint_as_float(frame[3]) + sc.dt;
-            frame[3] = __float_as_uint(ft);
-            frame[2] += 1u;
-            if (!((double)ft < 0.0333333333)) frame[1] = 1u;
-        }
-    }
-}
-
 __global__ void frame_reset_kernel(uint32_t* __restrict__ frame) {
     if (threadIdx.x < (uint32_t)kFrameWords) frame[threadIdx.x] = 0u;
-}
-
-__global__ void frame_gate_kernel(uint32_t* __restrict__ frame) {
-    if (threadIdx.x == 0 && frame[1]) frame[0] = 1u;
 }
 
 __global__ void fill_u32_kernel(uint32_t* __restrict__ p, uint32_t v, size_t count) {
@@ -1405,21 +1399,8 @@ hipError_t launch_sorted_keys(hipStream_t st, int block, uint32_t ntiles, const 
     return hipGetLastError();
 }
 
-hipError_t launch_cfl(hipStream_t st, uint32_t nscenes, SceneConst* scenes, uint32_t* vmax2, float* dt_out,
-                      uint32_t* frame) {
-    if (nscenes == 0) return hipSuccess;
-    hipLaunchKernelGGL(cfl_kernel, dim3((nscenes + 255) / 256), dim3(256), 0, st, nscenes, scenes, vmax2, dt_out,
-                       frame);
-    return hipGetLastError();
-}
-
 hipError_t launch_frame_reset(hipStream_t st, uint32_t* frame) {
     hipLaunchKernelGGL(frame_reset_kernel, dim3(1), dim3(64), 0, st, frame);
-    return hipGetLastError();
-}
-
-hipError_t launch_frame_gate(hipStream_t st, uint32_t* frame) {
-    hipLaunchKernelGGL(frame_gate_kernel, dim3(1), dim3(64), 0, st, frame);
     return hipGetLastError();
 }
 
