@@ -206,8 +206,10 @@ __device__ __forceinline__ void row_window(__amdgpu_buffer_rsrc_t rcs, const Sce
 // Row masks.  The density pass tests a row's candidates [lo, hi) four at a
 // time and shifts one bit per slot into the row's mask (slots past hi shift
 // in zeros), so candidate c of a row with T groups sits at bit 4T-1-c and
-// only the last 32 slots survive.  Rows of more than 32 candidates re-test
-// the ones before with the predicate.  row_neighbors visits a row's
+// only the last 32 slots survive; the 32 slots before those go to a second
+// word of the same form (mask_hi, written and read for rows of more than 32
+// slots only, by handles with room for it).  Candidates before the words'
+// are re-tested with the predicate.  row_neighbors visits a row's
 // neighbours in ascending order: first the re-tested head, then the bits
 // from the highest (the lowest candidate) down.
 __device__ __forceinline__ uint32_t mask_span(uint32_t lo, uint32_t hi) { return (hi - lo + 3u) & ~3u; }

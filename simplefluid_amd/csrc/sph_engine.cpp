@@ -158,6 +158,16 @@ void invalidate_graph(sph_handle* h) {
     h->graph_frame = nullptr;
 }
 
+void give_back_spares(MemBudget& b) {
+    sph_handle* h = b.spares;
+    b.spares = nullptr;
+    (void)hipStreamSynchronize(h->stream);
+    invalidate_graph(h);
+    h->mask_hi.release();
+    h->nlist.release();
+    h->ncount.release();
+}
+
 uint2* tiles_for(sph_handle* h, int block, uint32_t& ntiles) {
     auto it = h->tiles.find(block);
     if (it != h->tiles.end() && it->second.p) {
@@ -213,6 +223,7 @@ StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     a.cstart = w.cstart.p;
     a.rho = w.rho.p;
     a.mask = w.mask.p;
+    a.mask_hi = h->mask_hi.p;
     a.nlist = h->nlist.p;
     a.ncount = h->ncount.p;
     a.acc = (h->keep_acc || w.acc.p) ? w.acc.p : nullptr;
@@ -245,6 +256,8 @@ int alloc_step_bufs(sph_handle* h, StepBufs& w) {
     if (e == hipSuccess) chk(launch_fill_u32(h->stream, w.tile_pre.p, 0xffffffffu, scan_tiles(h->ncells)));
     if (h->tune.sort_mode == kSortRadix)
         for (int i = 0; i < 2; ++i) { chk(w.kbuf[i].ensure(n)); chk(w.vbuf[i].ensure(n)); }
+    else
+        chk(h->tmp.ensure(n));
     chk(w.rho.ensure(n));
     chk(w.mask.ensure((size_t)kRows * n));
     if (h->keep_acc) chk(w.acc.ensure(n));
@@ -260,7 +273,6 @@ static int ensure_buffers(sph_handle* h) {
     chk(h->id.ensure(n));
     chk(h->key0.ensure(n));
     chk(h->next.ensure(n));
-    chk(h->tmp.ensure(n));
     const size_t head_words = (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells);
     const bool fresh_head = h->head.count < head_words || !h->head.p;
     chk(h->head.ensure(head_words));
@@ -284,12 +296,19 @@ static int ensure_buffers(sph_handle* h) {
     if (e != hipSuccess) return hip_fail(h, e, "buffer init");
     const int rc = alloc_step_bufs(h, h->work);
     if (rc != SPH_OK) return rc;
-    // Only speeds small steps up: a handle with no room for it does without.
+    // These only speed the step up: a handle with no room for them does
+    // without, and they are given back when another buffer needs the room.
+    h->mem.spares = nullptr;
+    if (h->mask_hi.ensure((size_t)kRows * n) != hipSuccess) {
+        h->mem.refused = 0;
+        (void)hipGetLastError();
+    }
     if (h->split_tiles <= kSplitTiles && (h->nlist.ensure((size_t)kListMax * n) != hipSuccess || h->ncount.ensure(n) != hipSuccess)) {
         h->nlist.release();
         h->mem.refused = 0;
         (void)hipGetLastError();
     }
+    if (h->mask_hi.p || h->nlist.p) h->mem.spares = h;
     return SPH_OK;
 }
 
@@ -325,6 +344,12 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
             return fail(h, SPH_E_INVALID, "the device frame loop needs a steady cell-count step");
     }
     const uint8_t hashed = h->keys_valid ? 0 : 1;
+    // Tile tables first: their allocation may give the spares back, and the
+    // step's form and both its passes have to see the same ones.
+    for (int b : {h->tune.density_block, h->tune.force_block, kSplitTile}) {
+        uint32_t nt = 0;
+        if (!tiles_for(h, b, nt)) return fail(h, SPH_E_OOM, "tile table");
+    }
     if (record_prof) prof_record(h, 0);
     if (!h->keys_valid) {
         const int rc = enqueue_hash(h);

@@ -16,7 +16,13 @@ struct MemBudget {
     uint64_t limit = 0;     // 0: no cap
     uint64_t used = 0;
     uint64_t refused = 0;   // size of the last allocation the cap refused
+    sph_handle* spares = nullptr;  // the handle, while it holds buffers it can do without
+    bool over(uint64_t bytes) const { return limit && used + bytes > limit; }
 };
+
+// Frees the buffers that only speed the step up (and the graphs that name
+// them): an allocation that does not fit beside them takes their place.
+void give_back_spares(MemBudget& b);
 
 // The budget that buffers allocated on this thread are charged to: each C-ABI
 // entry point sets it to its handle's for the duration of the call (a handle
@@ -57,11 +63,17 @@ struct DevBuf {
         if (n == 0) return hipSuccess;
         const uint64_t bytes = (uint64_t)n * sizeof(T);
         MemBudget* b = t_budget;
-        if (b && b->limit && b->used + bytes > b->limit) {
+        if (b && b->spares && b->over(bytes)) give_back_spares(*b);
+        if (b && b->over(bytes)) {
             b->refused = bytes;
             return hipErrorOutOfMemory;
         }
         hipError_t e = hipMalloc((void**)&p, bytes);
+        if (e != hipSuccess && b && b->spares) {
+            (void)hipGetLastError();
+            give_back_spares(*b);
+            e = hipMalloc((void**)&p, bytes);
+        }
         if (e != hipSuccess) { p = nullptr; return e; }
         count = n;
         owner = b;
@@ -151,8 +163,9 @@ struct sph_handle {
     // State (state order) and per-step buffers.
     sph::DevBuf<float4> pos, vel;
     sph::DevBuf<uint32_t> id, key0, next, head;
-    sph::DevBuf<uint16_t> nlist;           // split form's neighbour lists (left out under a memory limit
-    sph::DevBuf<uint32_t> ncount;          // they do not fit)
+    sph::DevBuf<uint16_t> nlist;           // spares: the split form's neighbour lists and
+    sph::DevBuf<uint32_t> ncount;          // their lengths,
+    sph::DevBuf<uint32_t> mask_hi;         // second mask words
     sph::DevBuf<uint32_t> tmp;             // cell-count sort: members of the tiles too full for LDS
     sph::StepBufs work;
     sph::DevBuf<uint32_t> hist, status, tickets, err, queue;

@@ -73,6 +73,7 @@ struct StepArgs {
     const uint32_t* cstart;  // cell-start table of this step
     float* rho;
     uint32_t* mask;
+    uint32_t* mask_hi;       // the 32 slots before mask's, rows of more than 32 slots; or null
     uint16_t* nlist;         // split form: neighbour lists, else null
     uint32_t* ncount;        // split form: their lengths
     float* xyz_out;          // state out in original order too (3 n floats each), or null

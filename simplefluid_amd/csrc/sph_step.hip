@@ -89,21 +89,30 @@ __device__ __forceinline__ void density_one(const StepArgs& a, const SceneConst&
         uint32_t m = 0u;
         const uint32_t cnt = hi[row] - lo[row];
         uint32_t off = lo[row] << 2;
-        const uint32_t full_end = off + ((cnt & ~3u) << 2);
         // Slots past the row end shift in zero bits (past the array end the
         // buffer returns 0).  Each trip's planes are loaded while the trip
         // before is tested, so a lane has two trips' loads in flight.
-        if (off != full_end) {
-            float4 X = load4(rx, off), Y = load4(ry, off), Z = load4(rz, off);
-            for (off += 16u; off != full_end; off += 16u) {
-                const float4 Xn = load4(rx, off), Yn = load4(ry, off), Zn = load4(rz, off);
+        auto trips = [&](uint32_t end) __attribute__((always_inline)) {
+            if (off != end) {
+                float4 X = load4(rx, off), Y = load4(ry, off), Z = load4(rz, off);
+                for (off += 16u; off != end; off += 16u) {
+                    const float4 Xn = load4(rx, off), Yn = load4(ry, off), Zn = load4(rz, off);
+                    density_trip<true>(pi, h2, X, Y, Z, 4, sum, m);
+                    X = Xn;
+                    Y = Yn;
+                    Z = Zn;
+                }
                 density_trip<true>(pi, h2, X, Y, Z, 4, sum, m);
-                X = Xn;
-                Y = Yn;
-                Z = Zn;
             }
-            density_trip<true>(pi, h2, X, Y, Z, 4, sum, m);
+        };
+        if (a.mask_hi) {
+            const uint32_t jm = row_first(lo[row], hi[row]);
+            if (jm != lo[row]) {
+                trips(jm << 2);
+                a.mask_hi[(size_t)row * a.n + k] = m;
+            }
         }
+        trips((lo[row] + (cnt & ~3u)) << 2);
         const int rem = (int)(cnt & 3u);
         if (rem > 0) density_trip<false>(pi, h2, load4(rx, off), load4(ry, off), load4(rz, off), rem, sum, m);
         a.mask[(size_t)row * a.n + k] = m;
@@ -273,6 +282,15 @@ __device__ __forceinline__ void density_one_staged(const StepArgs& a, const Scen
             // loop's exit test.
             const float* p = slot.v + (lo[row] - ulo);
             const float* const full_end = p + (cnt & ~3u);
+            if (a.mask_hi) {
+                const uint32_t jm = row_first(lo[row], hi[row]);
+                if (jm != lo[row]) {
+                    const float* const mid = slot.v + (jm - ulo);
+                    for (; p != mid; p += 4)
+                        density_trip<true>(pi, h2, slot_quad(p, 0), slot_quad(p, 1), slot_quad(p, 2), 4, sum, m);
+                    a.mask_hi[(size_t)row * a.n + k] = m;
+                }
+            }
             for (; p != full_end; p += 4)
                 density_trip<true>(pi, h2, slot_quad(p, 0), slot_quad(p, 1), slot_quad(p, 2), 4, sum, m);
             const int rem = (int)(cnt & 3u);
@@ -283,8 +301,10 @@ __device__ __forceinline__ void density_one_staged(const StepArgs& a, const Scen
             // Past the buffer end the records read as zeros, as the planes do.
             uint32_t j = lo[row];
             const uint32_t full_end = j + (cnt & ~3u);
+            const uint32_t jm = row_first(lo[row], hi[row]);
             float4 X, Y, Z;
             for (; j != full_end; j += 4u) {
+                if (j == jm && jm != lo[row] && a.mask_hi) a.mask_hi[(size_t)row * a.n + k] = m;
                 load_quad(rpos, j, X, Y, Z);
                 density_trip<true>(pi, h2, X, Y, Z, 4, sum, m);
             }
@@ -349,6 +369,48 @@ __device__ __forceinline__ uint32_t without_self(uint32_t word, uint32_t lo, uin
     return b < (uint32_t)kMaskBits ? word & ~(1u << b) : word;
 }
 
+// One row's pairs in ascending order of candidates: the re-tested ones before
+// the masks', the second word's, the mask m's.  pos(j), vel(j): candidate j's
+// records; walk(r, j0): the pairs of the bits of r (bit i: candidate j0 + i).
+template <class P, class V, class W>
+__device__ __forceinline__ void force_row(const StepArgs& a, const SceneConst& sc, uint32_t k, int row, uint32_t lo,
+                                          uint32_t hi, uint32_t m, const float4& pi, const float4& vi, ForceAcc& f,
+                                          P&& pos, V&& vel, W&& walk) {
+    const uint32_t span = mask_span(lo, hi);
+    if (span > 32u) {
+        uint32_t mh = a.mask_hi ? a.mask_hi[(size_t)row * a.n + k] : 0u;
+        if (row == 4) mh = without_self(mh, lo, hi, k, 32u);
+        const uint32_t j1 = row_first(lo, hi, a.mask_hi ? 2u : 1u);
+        for (uint32_t j = lo; j < j1; ++j) {
+            const float4 pj = pos(j);
+            if (j != k && dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z) < sc.h2)
+                force_pair(sc, pi, vi, pj, vel(j), f);
+        }
+        walk(mask_ascending(mh, span, 32u), row_first(lo, hi, 2u));
+    }
+    walk(mask_ascending(m, span, 0u), row_first(lo, hi));
+}
+
+// The walk over records in global memory: each one's are loaded while the one
+// before is summed, so a lane has two neighbours' loads in flight; unrolled
+// twice, the two register sets swap roles instead of being copied.
+__device__ __forceinline__ void walk_gathered(const SceneConst& sc, __amdgpu_buffer_rsrc_t rpos,
+                                              __amdgpu_buffer_rsrc_t rvel, const float4& pi, const float4& vi,
+                                              uint32_t r, uint32_t j0, ForceAcc& f) {
+    if (!r) return;
+    uint32_t j = j0 + (uint32_t)__builtin_ctz(r);
+    float4 pj = load4(rpos, j << 4), vj = load4(rvel, j << 4);
+#pragma unroll 2
+    for (r &= r - 1u; r; r &= r - 1u) {
+        j = j0 + (uint32_t)__builtin_ctz(r);
+        const float4 pn = load4(rpos, j << 4), vn = load4(rvel, j << 4);
+        force_pair(sc, pi, vi, pj, vj, f);
+        pj = pn;
+        vj = vn;
+    }
+    force_pair(sc, pi, vi, pj, vj, f);
+}
+
 __device__ __forceinline__ Moved force_one(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                               __amdgpu_buffer_rsrc_t rpos, __amdgpu_buffer_rsrc_t rvel,
                                               __amdgpu_buffer_rsrc_t rcs) {
@@ -365,32 +427,10 @@ __device__ __forceinline__ Moved force_one(const StepArgs& a, const SceneConst& 
     ForceAcc f = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int row = 0; row < kRows; ++row) {
-        const uint32_t span = mask_span(lo[row], hi[row]);
-        const uint32_t j0 = row_first(lo[row], hi[row]);
-        for (uint32_t j = lo[row]; j < j0; ++j) {
-            const float4 pj = load4(rpos, j << 4);
-            if (j != k && dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z) < sc.h2)
-                force_pair(sc, pi, vi, pj, load4(rvel, j << 4), f);
-        }
-        // The mask's neighbours in ascending order (bit i: candidate j0 + i),
-        // each one's records loaded while the one before is summed, so a
-        // lane has two neighbours' loads in flight; unrolled twice, the two
-        // register sets swap roles instead of being copied.
-        uint32_t r = __builtin_bitreverse32(mk[row]);
-        if (span - 1u < 31u) r >>= 32u - span;
-        if (r) {
-            uint32_t j = j0 + (uint32_t)__builtin_ctz(r);
-            float4 pj = load4(rpos, j << 4), vj = load4(rvel, j << 4);
-#pragma unroll 2
-            for (r &= r - 1u; r; r &= r - 1u) {
-                j = j0 + (uint32_t)__builtin_ctz(r);
-                const float4 pn = load4(rpos, j << 4), vn = load4(rvel, j << 4);
-                force_pair(sc, pi, vi, pj, vj, f);
-                pj = pn;
-                vj = vn;
-            }
-            force_pair(sc, pi, vi, pj, vj, f);
-        }
+        force_row(
+            a, sc, k, row, lo[row], hi[row], mk[row], pi, vi, f, [&](uint32_t j) { return load4(rpos, j << 4); },
+            [&](uint32_t j) { return load4(rvel, j << 4); },
+            [&](uint32_t r, uint32_t j0) { walk_gathered(sc, rpos, rvel, pi, vi, r, j0, f); });
     }
     return force_finish(a, sc, k, pi, vi, f);
 }
@@ -451,9 +491,14 @@ __device__ __forceinline__ Moved force_finish(const StepArgs& a, const SceneCons
 // one sorted range of about 64 + 2 chords of particles when the wave sits in
 // one y/z column (73 on average on the 1M dam break, 99 at the 99th
 // percentile of the 4.4M sphere drop); a wider range (a wave across two
-// columns) is walked from global memory as in force_one.  A wave has two
-// slots, one filled while the other is walked.
-constexpr uint32_t kStage = 96;
+// columns, or a dense state) is walked from global memory.  A wave has two
+// slots, one filled while the other is walked.  104 is the most that leaves
+// room for 24 waves a CU, six per SIMD (159.7 of 160 KB); against 96 the
+// force pass takes 117 for 130 us on the collapsed 1M dam break (alike, 72 to
+// 77, on the fresh one), 185 for 191 on 96 scenes of 20k, 336 for 347 on the
+// 4.4M drop.  Wider rows copied piece by piece
+// through the slot: 102 to 169 spilled registers, 76 and 410 us.
+constexpr uint32_t kStage = 104;
 static_assert(kStage <= 128, "the copy into a slot takes two records per lane");
 struct StageSlot {
     float4 pos[kStage];
@@ -518,25 +563,28 @@ __device__ __forceinline__ Moved force_one_staged(const StepArgs& a, const Scene
         if (ulo >= uhi) continue;
         if (fit) {
             // Entry j of the row sits at slot.pos[j - ulo], its velocity
-            // kStage records further on; the mask's entries from row_first.
+            // kStage records further on.
             const float4* base = slot.pos - ulo;
-            const float4* bm = slot.pos + (row_first(lo[row], hi[row]) - ulo);
-            row_neighbors_from(
-                lo[row], hi[row], mk[row],
-                [&](uint32_t j) {
-                    const float4 pj = base[j];
-                    return j != k && dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z) < sc.h2;
-                },
-                [&](uint32_t j) { force_pair(sc, pi, vi, base[j], base[j + kStage], f); },
-                [&](uint32_t i) { force_pair(sc, pi, vi, bm[i], bm[i + kStage], f); });
+            force_row(
+                a, sc, k, row, lo[row], hi[row], mk[row], pi, vi, f, [&](uint32_t j) { return base[j]; },
+                [&](uint32_t j) { return base[j + kStage]; },
+                [&](uint32_t r, uint32_t j0) {
+                    const float4* bm = base + j0;
+                    for (; r; r &= r - 1u) {
+                        const uint32_t i = (uint32_t)__builtin_ctz(r);
+                        force_pair(sc, pi, vi, bm[i], bm[i + kStage], f);
+                    }
+                });
         } else {
-            row_neighbors(
-                lo[row], hi[row], mk[row],
-                [&](uint32_t j) {
-                    const float4 pj = load4(rpos, j << 4);
-                    return j != k && dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z) < sc.h2;
-                },
-                [&](uint32_t j) { force_pair(sc, pi, vi, load4(rpos, j << 4), load4(rvel, j << 4), f); });
+            force_row(
+                a, sc, k, row, lo[row], hi[row], mk[row], pi, vi, f, [&](uint32_t j) { return load4(rpos, j << 4); },
+                [&](uint32_t j) { return load4(rvel, j << 4); },
+                [&](uint32_t r, uint32_t j0) {
+                    for (; r; r &= r - 1u) {
+                        const uint32_t j = j0 + (uint32_t)__builtin_ctz(r);
+                        force_pair(sc, pi, vi, load4(rpos, j << 4), load4(rvel, j << 4), f);
+                    }
+                });
         }
     }
     return active ? force_finish(a, sc, k, pi, vi, f) : Moved{0u, 0.0f};
@@ -618,7 +666,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) v
     });
 }
 
-// Six waves per SIMD (77 VGPRs, no VGPR spills).
+// Bound by its gathers: two records per neighbour, in a chain.  Six waves per
+// SIMD (80 VGPRs, no VGPR spills).  With the second mask word read instead of
+// the candidates before the mask's re-tested: 197k 37.5 -> 34.9 us, 65k
+// collapsed 31.9 -> 25.0.
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) void force_kernel(StepArgs a) {
     if (a.frame && a.frame[0]) return;
@@ -637,9 +688,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
     });
 }
 
-// force_kernel with the rows staged in LDS (two 3 KB slots per wave).  Six
-// waves per SIMD: the bound fits it in 80 VGPRs (one spilled; 82 and five
-// waves without it).
+// force_kernel with the rows staged in LDS (two 3.25 KB slots per wave).  Bound
+// by latency, of LDS reads in a chain per neighbour and of a row's copy.  Six
+// waves per SIMD: the bound fits it in 80 VGPRs (nine spilled).  With the
+// second mask word: the 1M dam break 74.4 -> 71.7 us fresh, 149 -> 117
+// collapsed (a quarter of its rows over 32 candidates), 96 scenes of 20k
+// 198 -> 185, the 4.4M drop 347 -> 336.
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) void force_staged_kernel(StepArgs a) {
     if (a.frame && a.frame[0]) return;
@@ -865,8 +919,11 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
                 ++nkept;
             }
         });
-    if (active) a.mask[(size_t)w * a.n + k] = m;
     const uint32_t span = mask_span(lo, hi);
+    if (active) {
+        a.mask[(size_t)w * a.n + k] = m;
+        if (a.mask_hi && span > 32u) a.mask_hi[(size_t)w * a.n + k] = mh;
+    }
     if (span <= 32u) mh = 0u;
     const uint32_t cnt = (uint32_t)__popc(m) + (uint32_t)__popc(mh);
     reinterpret_cast<uint8_t*>(sh.count)[(((uint32_t)w >> 2) * kSplitTile + lane) * 4u + ((uint32_t)w & 3u)] = (uint8_t)cnt;

@@ -65,3 +65,41 @@ def test_small_handles_form_equals_the_others(name):
     for other in got[1:]:
         for a, b in zip(got[0], other):
             assert np.array_equal(a, b), name
+
+
+@pytest.mark.parametrize("name", ["n1", "dense", "denser"])
+def test_spare_buffers_give_way(name):
+    """The neighbour lists and second mask words are left out where a memory
+    cap has no room for them, and given back to an allocation that needs the
+    room; the steps stay the same bit for bit either way, in every form."""
+    from simplefluid_amd import engine as E
+    params, pos, xsub = scenes(E)[name]
+    x = pos[0]
+
+    def run(limit, form, rollout):
+        e = E.Engine(params[0])
+        e.set_device_memory_limit(limit)
+        e.set_cell_subdivision(xsub)
+        e.set_particles(x)
+        e.make_ready()
+        if form is not None:
+            e.set_tuning(**form)
+        e.advance_steps(2)
+        used = e.device_memory_used()
+        if rollout:
+            e.rollout_forward(2)
+        e.advance_steps(2)
+        out = (e.get_particles(), e.get_velocity(), used, e.device_memory_used())
+        e.close()
+        return out
+
+    spares = len(x) * (9 * 4 + 128 * 2 + 4)
+    for form in (None,) + FORMS:
+        full = run(0, form, False)
+        bare = run(full[2] - spares, form, False)
+        assert bare[2] == full[2] - spares
+        taped = run(0, form, True)
+        tight = run(taped[3] - 4, form, True)
+        assert tight[3] == taped[3] - spares
+        for a, b in ((full, bare), (taped, tight)):
+            assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), (name, form)
