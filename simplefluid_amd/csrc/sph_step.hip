@@ -730,6 +730,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
 constexpr uint32_t kKept = 5;        // a gathered row's terms kept in its copy's place
 constexpr uint32_t kChunk = 64;      // entries of a list in LDS at a time
 constexpr uint32_t kListOver = 0xffffu;
+constexpr uint32_t kRowOver = 255u;
+static_assert(kRowOver > kListMax + 1u, "such a row's particle is over its list's length too");
 template <bool V>
 struct Bool {
     static constexpr bool value = V;
@@ -743,7 +745,6 @@ struct SplitShared {
     float term[kChunk + 4][kSplitTile];            // the neighbours' terms, itself included
     uint16_t id[kChunk + 1][kSplitTile];           // the neighbours; the particle itself goes to the last place
     uint32_t count[3][kSplitTile];                 // neighbours per row, one byte a row (itself included)
-    uint32_t over;                                 // some row or list is too long
     float wall[kSplitTile];
 };
 
@@ -872,7 +873,6 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
     uint32_t lo, hi;
     split_window(rcs, sc, pi, w % 3 - 1, w / 3 - 1, lo, hi);
     if (!active) lo = hi = 0u;
-    if (threadIdx.x == 0) sh.over = 0u;
     // The row's union of windows.
     const bool has = hi > lo;
     const uint32_t ulo = wave_umin(has ? lo : 0xffffffffu);
@@ -925,9 +925,9 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
         if (a.mask_hi && span > 32u) a.mask_hi[(size_t)w * a.n + k] = mh;
     }
     if (span <= 32u) mh = 0u;
-    const uint32_t cnt = (uint32_t)__popc(m) + (uint32_t)__popc(mh);
+    // A row the two words do not cover counts as more than any list holds.
+    const uint32_t cnt = span > 64u ? kRowOver : (uint32_t)__popc(m) + (uint32_t)__popc(mh);
     reinterpret_cast<uint8_t*>(sh.count)[(((uint32_t)w >> 2) * kSplitTile + lane) * 4u + ((uint32_t)w & 3u)] = (uint8_t)cnt;
-    if (__ballot(span > 64u) != 0u && lane == 0u) sh.over = 1u;
     __syncthreads();
     // Where this row's neighbours go in the list, and how many there are.
     uint32_t base = 0u, total = 0u;
@@ -938,7 +938,6 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
         base = __builtin_amdgcn_sad_u8(c & before, 0u, base);
         total = __builtin_amdgcn_sad_u8(g == 2 ? c & 0xffu : c, 0u, total);
     }
-    if (__ballot(total > kListMax + 1u) != 0u && lane == 0u && w == 0) sh.over = 1u;
     // A corner row has the fewest neighbours to list.
     if (w == kRows - 1) {
         float wr = 0.0f;
@@ -953,7 +952,8 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
     // Lists go through LDS kChunk entries at a time (nearly always once).
     // The list for the force pass leaves the particle itself out; its term is
     // in the sum.
-    const uint32_t most = wave_umax(total);
+    const uint32_t most = wave_umax(total);  // the same in every wave, and so is the branch on it
+    const bool over = most > kListMax + 1u;
     const uint32_t listed = total ? total - 1u : 0u;
     float sum = 0.0f;
     auto list = [&](uint32_t first, auto all) {
@@ -990,10 +990,10 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
     for (uint32_t first = 0u;; first += kChunk) {
         if (most <= kChunk)
             list(0u, Bool<true>());
-        else if (most <= kListMax + 1u)
+        else if (!over)
             list(first, Bool<false>());
         __syncthreads();
-        if (sh.over) {
+        if (over) {
             // The first wave runs every row itself; the force pass walks masks.
             if (w != 0) return;
 #pragma unroll 1
