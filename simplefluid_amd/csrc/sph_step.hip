@@ -32,6 +32,12 @@ __device__ __forceinline__ uint32_t push_sign(uint32_t m, float c) {
     return __builtin_amdgcn_alignbit(m, __float_as_uint(c), 31u);
 }
 
+// A trip pushes four bits into m; those it pushes out go on into mh, which so
+// holds the 32 slots before m's at the row's end (one funnel shift a trip).
+__device__ __forceinline__ uint32_t push_out(uint32_t mh, uint32_t m) {
+    return __builtin_amdgcn_alignbit(mh, m, 28u);
+}
+
 // Candidates come from the x, y, z planes: one 16-byte load per plane gives
 // four consecutive candidates (three loads per trip instead of four, which
 // relieves the texture address units this pass otherwise saturates).
@@ -39,7 +45,8 @@ __device__ __forceinline__ uint32_t push_sign(uint32_t m, float c) {
 // partial trip masks the slots past its end.
 template <bool FULL>
 __device__ __forceinline__ void density_trip(const float4& pi, float h2, const float4& X, const float4& Y,
-                                             const float4& Z, int rem, float& sum, uint32_t& m) {
+                                             const float4& Z, int rem, float& sum, uint32_t& m, uint32_t& mh) {
+    mh = push_out(mh, m);
     const float xs[4] = {X.x, X.y, X.z, X.w}, ys[4] = {Y.x, Y.y, Y.z, Y.w}, zs[4] = {Z.x, Z.y, Z.z, Z.w};
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -86,35 +93,27 @@ __device__ __forceinline__ void density_one(const StepArgs& a, const SceneConst&
     float sum = 0.0f;
 #pragma unroll
     for (int row = 0; row < kRows; ++row) {
-        uint32_t m = 0u;
+        uint32_t m = 0u, mh = 0u;
         const uint32_t cnt = hi[row] - lo[row];
         uint32_t off = lo[row] << 2;
+        const uint32_t full_end = (lo[row] + (cnt & ~3u)) << 2;
         // Slots past the row end shift in zero bits (past the array end the
         // buffer returns 0).  Each trip's planes are loaded while the trip
         // before is tested, so a lane has two trips' loads in flight.
-        auto trips = [&](uint32_t end) __attribute__((always_inline)) {
-            if (off != end) {
-                float4 X = load4(rx, off), Y = load4(ry, off), Z = load4(rz, off);
-                for (off += 16u; off != end; off += 16u) {
-                    const float4 Xn = load4(rx, off), Yn = load4(ry, off), Zn = load4(rz, off);
-                    density_trip<true>(pi, h2, X, Y, Z, 4, sum, m);
-                    X = Xn;
-                    Y = Yn;
-                    Z = Zn;
-                }
-                density_trip<true>(pi, h2, X, Y, Z, 4, sum, m);
+        if (off != full_end) {
+            float4 X = load4(rx, off), Y = load4(ry, off), Z = load4(rz, off);
+            for (off += 16u; off != full_end; off += 16u) {
+                const float4 Xn = load4(rx, off), Yn = load4(ry, off), Zn = load4(rz, off);
+                density_trip<true>(pi, h2, X, Y, Z, 4, sum, m, mh);
+                X = Xn;
+                Y = Yn;
+                Z = Zn;
             }
-        };
-        if (a.mask_hi) {
-            const uint32_t jm = row_first(lo[row], hi[row]);
-            if (jm != lo[row]) {
-                trips(jm << 2);
-                a.mask_hi[(size_t)row * a.n + k] = m;
-            }
+            density_trip<true>(pi, h2, X, Y, Z, 4, sum, m, mh);
         }
-        trips((lo[row] + (cnt & ~3u)) << 2);
         const int rem = (int)(cnt & 3u);
-        if (rem > 0) density_trip<false>(pi, h2, load4(rx, off), load4(ry, off), load4(rz, off), rem, sum, m);
+        if (rem > 0) density_trip<false>(pi, h2, load4(rx, off), load4(ry, off), load4(rz, off), rem, sum, m, mh);
+        if (cnt > 32u && a.mask_hi) a.mask_hi[(size_t)row * a.n + k] = mh;
         a.mask[(size_t)row * a.n + k] = m;
     }
     // The walls' half-space fluid, faces in the order x-, x+, y-, y+, z-, z+.
@@ -257,7 +256,7 @@ __device__ __forceinline__ void density_one_staged(const StepArgs& a, const Scen
     fetch(0);
 #pragma unroll
     for (int row = 0; row < kRows; ++row) {
-        uint32_t m = 0u;
+        uint32_t m = 0u, mh = 0u;
         const uint32_t cnt = hi[row] - lo[row];
         const bool has = cnt > 0u;
         const uint32_t ulo = nlo, uhi = nhi;
@@ -282,38 +281,28 @@ __device__ __forceinline__ void density_one_staged(const StepArgs& a, const Scen
             // loop's exit test.
             const float* p = slot.v + (lo[row] - ulo);
             const float* const full_end = p + (cnt & ~3u);
-            if (a.mask_hi) {
-                const uint32_t jm = row_first(lo[row], hi[row]);
-                if (jm != lo[row]) {
-                    const float* const mid = slot.v + (jm - ulo);
-                    for (; p != mid; p += 4)
-                        density_trip<true>(pi, h2, slot_quad(p, 0), slot_quad(p, 1), slot_quad(p, 2), 4, sum, m);
-                    a.mask_hi[(size_t)row * a.n + k] = m;
-                }
-            }
             for (; p != full_end; p += 4)
-                density_trip<true>(pi, h2, slot_quad(p, 0), slot_quad(p, 1), slot_quad(p, 2), 4, sum, m);
+                density_trip<true>(pi, h2, slot_quad(p, 0), slot_quad(p, 1), slot_quad(p, 2), 4, sum, m, mh);
             const int rem = (int)(cnt & 3u);
             if (rem > 0)
-                density_trip<false>(pi, h2, slot_quad(p, 0), slot_quad(p, 1), slot_quad(p, 2), rem, sum, m);
+                density_trip<false>(pi, h2, slot_quad(p, 0), slot_quad(p, 1), slot_quad(p, 2), rem, sum, m, mh);
             wave_lds_sync();
         } else if (has) {
             // Past the buffer end the records read as zeros, as the planes do.
             uint32_t j = lo[row];
             const uint32_t full_end = j + (cnt & ~3u);
-            const uint32_t jm = row_first(lo[row], hi[row]);
             float4 X, Y, Z;
             for (; j != full_end; j += 4u) {
-                if (j == jm && jm != lo[row] && a.mask_hi) a.mask_hi[(size_t)row * a.n + k] = m;
                 load_quad(rpos, j, X, Y, Z);
-                density_trip<true>(pi, h2, X, Y, Z, 4, sum, m);
+                density_trip<true>(pi, h2, X, Y, Z, 4, sum, m, mh);
             }
             const int rem = (int)(cnt & 3u);
             if (rem > 0) {
                 load_quad(rpos, j, X, Y, Z);
-                density_trip<false>(pi, h2, X, Y, Z, rem, sum, m);
+                density_trip<false>(pi, h2, X, Y, Z, rem, sum, m, mh);
             }
         }
+        if (cnt > 32u && a.mask_hi) a.mask_hi[(size_t)row * a.n + k] = mh;
         if (active) a.mask[(size_t)row * a.n + k] = m;
     }
     if (!active) return;
@@ -788,10 +777,10 @@ __device__ __forceinline__ void split_trips(G&& quad, const float4& pi, float h2
                                             uint32_t& m, uint32_t& mh, F&& f) {
     m = 0u;
     mh = 0u;
-    const bool two = __ballot(mask_span(lo, hi) > 32u) != 0u;
     if (lo >= hi) return;
     Quad cur, nxt;
     auto test = [&](const Quad& q, uint32_t left) {
+        mh = push_out(mh, m);
         const float xs[4] = {q.X.x, q.X.y, q.X.z, q.X.w}, ys[4] = {q.Y.x, q.Y.y, q.Y.z, q.Y.w},
                     zs[4] = {q.Z.x, q.Z.y, q.Z.z, q.Z.w};
 #pragma unroll
@@ -806,18 +795,6 @@ __device__ __forceinline__ void split_trips(G&& quad, const float4& pi, float h2
     uint32_t j = lo;
     const uint32_t full_end = lo + ((hi - lo) & ~3u);
     quad(j, cur);
-    if (two) {
-        const uint32_t jm = row_first(lo, hi);
-        for (; j != full_end; j += 4u) {
-            if (j == jm) mh = m;
-            quad(j + 4u, nxt);
-            test(cur, 4u);
-            cur = nxt;
-        }
-        if (j == jm) mh = m;
-        if (j != hi) test(cur, hi - j);
-        return;
-    }
     // The next trip's records load while this one's are tested, the two
     // register sets in turn.
     for (;;) {
@@ -924,7 +901,6 @@ __global__ __launch_bounds__(64 * kRows) void density_split_kernel(StepArgs a) {
         a.mask[(size_t)w * a.n + k] = m;
         if (a.mask_hi && span > 32u) a.mask_hi[(size_t)w * a.n + k] = mh;
     }
-    if (span <= 32u) mh = 0u;
     // A row the two words do not cover counts as more than any list holds.
     const uint32_t cnt = span > 64u ? kRowOver : (uint32_t)__popc(m) + (uint32_t)__popc(mh);
     reinterpret_cast<uint8_t*>(sh.count)[(((uint32_t)w >> 2) * kSplitTile + lane) * 4u + ((uint32_t)w & 3u)] = (uint8_t)cnt;
