@@ -8,7 +8,7 @@
 //   key0            uint32 x N   cell key of the state positions (written by integrate)
 //   head            uint32 x C+2T per cell, the newest run of particles that entered it
 //                                (0: none; built by the integrate pass, cleared by the
-//                                sort), then particles per tile of 1024 cells, then the
+//                                sort), then particles per tile of cells, then the
 //                                exclusive scan of the tile sums
 //   next            uint32 x N   per run (at its first particle), the cell's run before it
 //   radix ping-pong 2 x (uint32 key + uint32 value) x N (radix mode)
@@ -358,10 +358,15 @@ __device__ __forceinline__ uint32_t cell_key(const SceneConst& sc, float x, floa
     return sc.cell_offset + ((uint32_t)cz * (uint32_t)sc.G[1] + (uint32_t)cy) * (uint32_t)sc.G[0] + (uint32_t)cx;
 }
 
-// Cells per tile of the sort (1024): the integrate pass also sums particles
-// per tile, so every sort block finds its prefix without waiting.
-constexpr uint32_t kTileShift = 10;
-constexpr uint32_t kTileCells = 1u << kTileShift;
+// Cells per tile of the sort, as a shift: the integrate pass also sums
+// particles per tile, so every sort block finds its prefix without waiting.
+constexpr uint32_t kTileShiftMax = 10;
+__host__ __device__ constexpr uint32_t tile_shift(uint32_t ncells) {
+    return ncells <= (1u << 17) ? 8u : ncells <= (1u << 19) ? 9u : kTileShiftMax;
+}
+__host__ __device__ constexpr uint32_t scan_tiles(uint32_t ncells) {
+    return (ncells + (1u << tile_shift(ncells)) - 1u) >> tile_shift(ncells);
+}
 
 // Runs.  A cell's members are kept as a chain of runs: consecutive particles
 // of one wave with the same key, at most 15 of them so that a run packs into
@@ -412,8 +417,9 @@ __device__ __forceinline__ void push_run(uint32_t* __restrict__ head, uint32_t* 
 
 // Adds the wave's particles to their tiles' sums: one atomic per run of
 // lanes in one tile, or one in all where the wave has a single tile.
-__device__ __forceinline__ void add_tile_sums(uint32_t* __restrict__ tsum, uint32_t key, bool active) {
-    const uint32_t lane = threadIdx.x & 63u, tile = key >> kTileShift;
+__device__ __forceinline__ void add_tile_sums(uint32_t* __restrict__ tsum, uint32_t shift, uint32_t key,
+                                              bool active) {
+    const uint32_t lane = threadIdx.x & 63u, tile = key >> shift;
     const uint64_t act = __ballot(active);
     if (act == 0u) return;
     const uint32_t first = (uint32_t)__builtin_ctzll(act);

@@ -48,9 +48,8 @@ struct SortPlan {
 };
 
 uint32_t sort_tiles(uint32_t n, int items);
-// Tiles of 1024 cells.  head holds C chain heads, then T = scan_tiles(C)
-// per-tile sums, then their exclusive scan (T words).
-uint32_t scan_tiles(uint32_t ncells);
+// head holds C chain heads, then T = scan_tiles(C) per-tile sums, then their
+// exclusive scan (T words).
 int sort_key_passes(uint32_t ncells);
 // Cell-start table and the sort; cell-count mode gathers the state too ...
 hipError_t launch_sort_keys(hipStream_t st, const SortPlan& sp);

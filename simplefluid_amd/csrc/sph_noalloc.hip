@@ -29,7 +29,9 @@ constexpr uint32_t kMaxParticles = 65536;
 constexpr uint32_t kMaxCells = 1u << 20;
 constexpr uint32_t kMaxTiles = kMaxParticles / kSplitTile;
 static_assert(kMaxParticles <= kSplitMax, "the step runs in the split form");
-constexpr uint32_t kScanTilesMax = (kMaxCells + kTileCells - 1u) / kTileCells;
+constexpr uint32_t kScanTilesMax = 1024;
+static_assert(scan_tiles(kMaxCells) <= kScanTilesMax && scan_tiles(1u << 19) <= kScanTilesMax &&
+              scan_tiles(1u << 17) <= kScanTilesMax, "the most tiles of each tile size");
 
 // Byte offsets of the arrays inside the scratch, each 256-byte aligned.
 constexpr size_t align256(size_t x) { return (x + 255u) & ~(size_t)255u; }
@@ -74,7 +76,7 @@ __global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint8_t* __
         *reinterpret_cast<SceneConst*>(base + Layout::scene) = sc;
         *reinterpret_cast<uint32_t*>(base + Layout::err) = 0u;
     }
-    const uint32_t T = (ncells + kTileCells - 1u) >> kTileShift;
+    const uint32_t T = scan_tiles(ncells);
     uint32_t* head = reinterpret_cast<uint32_t*>(base + Layout::head);
     // Whole 16-byte words; the scratch behind the last tile sum is unused.
     for (uint32_t w = i; w < (ncells + 2u * T + 3u) / 4u; w += stride)

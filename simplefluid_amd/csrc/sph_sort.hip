@@ -196,7 +196,7 @@ constexpr int kHeldLinks = 5;
 // 23.1 us.
 constexpr uint32_t kWideTiles = 1024;
 
-template <int BLOCK>
+template <int BLOCK, int V>
 __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     // A frame that is complete (pending, or halted already) skips the step;
     // the first kernel of the step turns pending into halt for the others.
@@ -204,21 +204,22 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
         if (blockIdx.x == 0 && threadIdx.x == 0) a.frame[0] = 1u;
         return;
     }
-    constexpr int V = (int)kTileCells / BLOCK;
+    constexpr uint32_t kCells = (uint32_t)(BLOCK * V);
+    constexpr uint32_t kMembers = kCells * 8u < kTileMembers ? kCells * 8u : kTileMembers;
     constexpr int kWaves = BLOCK / 64;
     static_assert(V == 1 || V == 4, "one head, or four in one 16-byte load, per thread");
     __shared__ uint32_t s_w[kWaves];
     __shared__ uint32_t s_pre[kWaves];
     __shared__ uint32_t s_big;
-    __shared__ uint32_t s_off[kTileCells + 1];
-    __shared__ uint32_t s_mem[kTileMembers];
+    __shared__ uint32_t s_off[kCells + 1];
+    __shared__ uint32_t s_mem[kMembers];
     __shared__ uint32_t s_unsorted;
     const uint32_t b = blockIdx.x, C = a.C;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // Tile counters of this step's persistent density and force launches.
     if (b == 0 && tid < kQueueWords && a.queue) a.queue[tid] = 0u;
-    const uint32_t T = (C + kTileCells - 1u) >> kTileShift;
-    const uint32_t base = b << kTileShift;
+    const uint32_t T = gridDim.x;
+    const uint32_t base = b * kCells;
     const uint32_t i0 = base + (uint32_t)(V * tid);
     uint32_t r[kHeldLinks + 1][V];
     const bool whole = i0 + (uint32_t)V <= C;
@@ -324,11 +325,11 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     const bool big = s_big != 0u;
     if (big) {
         // Count by scanning all keys (s_off as the counters).
-        for (uint32_t i = (uint32_t)tid; i < kTileCells; i += BLOCK) s_off[i] = 0u;
+        for (uint32_t i = (uint32_t)tid; i < kCells; i += BLOCK) s_off[i] = 0u;
         __syncthreads();
         for (uint32_t k = (uint32_t)tid; k < a.n; k += BLOCK) {
             const uint32_t c = a.key0[k] - base;
-            if (c < kTileCells) atomicAdd(&s_off[c], 1u);
+            if (c < kCells) atomicAdd(&s_off[c], 1u);
         }
         __syncthreads();
 #pragma unroll
@@ -358,13 +359,13 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     }
 #pragma unroll
     for (int v = 0; v < V; ++v) s_off[V * tid + v] = off[v];
-    if (tid == 0) s_off[kTileCells] = total;
+    if (tid == 0) s_off[kCells] = total;
     // The members, cell by cell.  A cell whose runs are all in registers
     // lists them by their first particles, so its members come sorted; with a
     // longer chain in the tile, all come as their runs do and are ranked
     // below.
     const bool unsorted = big || s_unsorted != 0u;
-    const bool in_lds = total <= kTileMembers && !big;
+    const bool in_lds = total <= kMembers && !big;
     uint32_t* const tmp = a.tmp + pre;
     if (!unsorted) {
         auto list = [&](auto&& put) __attribute__((always_inline)) {
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
         __syncthreads();
         for (uint32_t k = (uint32_t)tid; k < a.n; k += BLOCK) {
             const uint32_t c = a.key0[k] - base;
-            if (c < kTileCells) tmp[atomicAdd(&s_off[c], 1u)] = k;
+            if (c < kCells) tmp[atomicAdd(&s_off[c], 1u)] = k;
         }
         __syncthreads();
         // The counters ended at the next cell's start.
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
             uint32_t d = j;
             if (unsorted) {
                 const uint32_t c = a.key0[k[v]] - base;
-                if (c >= kTileCells) {
+                if (c >= kCells) {
                     atomicOr(a.err, 4u);
                     continue;
                 }
@@ -685,13 +686,13 @@ uint32_t sort_tiles(uint32_t n, int items) {
     return (n + tile - 1) / tile;
 }
 
-uint32_t scan_tiles(uint32_t C) { return (C + kTileCells - 1u) >> kTileShift; }
-
 int sort_key_passes(uint32_t ncells) {
     int bits = 1;
     while (bits < 32 && (1ull << bits) < (uint64_t)ncells) ++bits;
     return (bits + 7) / 8;
 }
+
+#define SPH_CELL_SORT(block, v) HIP_KERNEL_NAME(cell_sort_kernel<block, v>)
 
 static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
     const uint32_t tiles = scan_tiles(sp.ncells);
@@ -719,10 +720,15 @@ static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
     a.err = sp.err;
     a.frame = sp.frame;
     a.gather = gather;
-    if (tiles <= kWideTiles)
-        hipLaunchKernelGGL(cell_sort_kernel<1024>, dim3(tiles), dim3(1024), 0, st, a);
+    const uint32_t shift = tile_shift(sp.ncells);
+    if (shift == 8u)
+        hipLaunchKernelGGL(SPH_CELL_SORT(256, 1), dim3(tiles), dim3(256), 0, st, a);
+    else if (shift == 9u)
+        hipLaunchKernelGGL(SPH_CELL_SORT(512, 1), dim3(tiles), dim3(512), 0, st, a);
+    else if (tiles <= kWideTiles)
+        hipLaunchKernelGGL(SPH_CELL_SORT(1024, 1), dim3(tiles), dim3(1024), 0, st, a);
     else
-        hipLaunchKernelGGL(cell_sort_kernel<256>, dim3(tiles), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(SPH_CELL_SORT(256, 4), dim3(tiles), dim3(256), 0, st, a);
 }
 
 hipError_t launch_sort_keys(hipStream_t st, const SortPlan& sp) {

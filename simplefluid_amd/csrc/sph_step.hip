@@ -604,7 +604,7 @@ __device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
         }
     }
     if (!a.head) return;
-    const uint32_t words = (a.ncells + kTileCells - 1u) >> kTileShift;
+    const uint32_t words = scan_tiles(a.ncells);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
         a.head[a.ncells + i] = 0u;
 }
@@ -614,7 +614,7 @@ __device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
 __device__ __forceinline__ void finish_particle(const StepArgs& a, uint32_t k, const Moved& to, bool active) {
     const uint32_t key = to.key;
     if (!a.head) return;  // a single step: there is no next one
-    add_tile_sums(a.head + a.ncells, key, active);
+    add_tile_sums(a.head + a.ncells, tile_shift(a.ncells), key, active);
     if (a.vmax2) wave_max_v2(a.vmax2, to.v2);
     if (active) a.key0[k] = key;
     push_run(a.head, a.next, key, k, active);  // last: it waits for its exchange's answer
@@ -1161,10 +1161,10 @@ constexpr uint32_t kHashTiles = 2048;
 // flush() once at its end.
 struct BlockTileSums {
     uint32_t* tsum;
-    uint32_t tiles;
+    uint32_t shift, tiles;
     uint32_t* local;  // kHashTiles words of LDS; null: straight to memory
     __device__ __forceinline__ BlockTileSums(uint32_t* head, uint32_t ncells, uint32_t* lds)
-        : tsum(head + ncells), tiles((ncells + kTileCells - 1u) >> kTileShift) {
+        : tsum(head + ncells), shift(tile_shift(ncells)), tiles(scan_tiles(ncells)) {
         local = tiles <= kHashTiles ? lds : nullptr;
         if (local) {
             for (uint32_t i = threadIdx.x; i < tiles; i += blockDim.x) local[i] = 0u;
@@ -1173,9 +1173,9 @@ struct BlockTileSums {
     }
     __device__ __forceinline__ void add(uint32_t key, bool active) {
         if (!local)
-            add_tile_sums(tsum, key, active);
+            add_tile_sums(tsum, shift, key, active);
         else if (active)
-            atomicAdd(local + (key >> kTileShift), 1u);
+            atomicAdd(local + (key >> shift), 1u);
     }
     __device__ __forceinline__ void flush() {
         if (!local) return;
