@@ -360,9 +360,15 @@ __device__ __forceinline__ uint32_t cell_key(const SceneConst& sc, float x, floa
 
 // Cells per tile of the sort, as a shift: the integrate pass also sums
 // particles per tile, so every sort block finds its prefix without waiting.
+// A tile's block moves its particles alone, so small grids take small tiles:
+// a fluid settled over the floor of a 500k-cell grid fills 50 tiles of 1024
+// cells, up to 1,700 particles each (49k particles: sort 10.9 us, 9.8 with
+// tiles of 512, 9.2 with 256; DoubleDambreak at resolution 24, 55k cells:
+// frame 8.06 ms, 7.76 with 256).  Above 2^20 cells more tiles cost
+// more in the sums each block adds up than their balance gives.
 constexpr uint32_t kTileShiftMax = 10;
 __host__ __device__ constexpr uint32_t tile_shift(uint32_t ncells) {
-    return ncells <= (1u << 17) ? 8u : ncells <= (1u << 19) ? 9u : kTileShiftMax;
+    return ncells <= (1u << 19) ? 8u : ncells <= (1u << 20) ? 9u : kTileShiftMax;
 }
 __host__ __device__ constexpr uint32_t scan_tiles(uint32_t ncells) {
     return (ncells + (1u << tile_shift(ncells)) - 1u) >> tile_shift(ncells);

@@ -29,9 +29,9 @@ constexpr uint32_t kMaxParticles = 65536;
 constexpr uint32_t kMaxCells = 1u << 20;
 constexpr uint32_t kMaxTiles = kMaxParticles / kSplitTile;
 static_assert(kMaxParticles <= kSplitMax, "the step runs in the split form");
-constexpr uint32_t kScanTilesMax = 1024;
-static_assert(scan_tiles(kMaxCells) <= kScanTilesMax && scan_tiles(1u << 19) <= kScanTilesMax &&
-              scan_tiles(1u << 17) <= kScanTilesMax, "the most tiles of each tile size");
+constexpr uint32_t kScanTilesMax = 2048;
+static_assert(scan_tiles(kMaxCells) <= kScanTilesMax && scan_tiles(1u << 19) <= kScanTilesMax,
+              "the most tiles of each tile size");
 
 // Byte offsets of the arrays inside the scratch, each 256-byte aligned.
 constexpr size_t align256(size_t x) { return (x + 255u) & ~(size_t)255u; }

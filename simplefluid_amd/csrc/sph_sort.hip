@@ -5,7 +5,7 @@
 //
 // Cell-count sort (default): one kernel.  The integrate pass already linked
 // each particle into its cell's chain of runs and counted particles per tile
-// of 1024 cells, so a block of cell_sort_kernel owns a tile: it takes its
+// of cells, so a block of cell_sort_kernel owns a tile: it takes its
 // prefix from the tile sums, counts its cells by following their chains,
 // scans the counts (cstart), lists the members cell by cell in LDS, each
 // cell's by ascending input index, and
@@ -150,7 +150,8 @@ __global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __r
 // Members a cell may hold for the stable in-cell rank (a member's rank scans
 // its cell).  Rest-density fluid holds a few per cell.
 constexpr uint32_t kMaxRankCell = 1024;
-// Members of a tile listed in LDS; a fuller tile lists them in global memory.
+// Members of a tile listed in LDS, at most eight per cell; a fuller tile lists
+// them in global memory.
 constexpr uint32_t kTileMembers = 4096;
 // Links of one cell followed in its chain; a longer chain (a pile of
 // particles in one cell, or an upload in random order of a very full one)
@@ -179,7 +180,7 @@ struct CellSortArgs {
     int gather;          // 0: the cell-start table only (radix mode)
 };
 
-// Block b sorts the particles of cells [1024 b, 1024 (b + 1)).  Thread t owns
+// Block b sorts the particles of tile b, of BLOCK V cells.  Thread t owns
 // V consecutive cells; their chains are followed together, so a wave waits
 // once per link for the longest chain among its cells, and the first
 // kHeldLinks links stay in registers for the listing.  The kernel is bound
@@ -188,14 +189,12 @@ struct CellSortArgs {
 // state is moved once.
 constexpr int kHeldLinks = 5;
 
-// One thread per cell up to this many tiles, where the chip waits on each
-// block's dependent steps; above it four cells per thread, where 1024-lane
-// blocks only hold up each other's phases.  Measured, 1024 against 256
-// threads: DoubleDambreak at resolution 24 (54 tiles) 7.0 against 11.5 us,
-// 65k dam break (489 tiles) 7.8 against 11.3 us, 1M (2013 tiles) 29.2 against
-// 23.1 us.
-constexpr uint32_t kWideTiles = 1024;
-
+// One thread per cell for tiles of up to 512 cells (grids of up to 2^20),
+// where the chip waits on each block's dependent steps; four cells per thread
+// for tiles of 1024, where 1024-lane blocks only hold up each other's phases.
+// Measured at 1024 cells, one against four: DoubleDambreak at resolution 24
+// (54 tiles) 7.0 against 11.5 us, 65k dam break (489 tiles) 7.8 against 11.3
+// us, 1M (2013 tiles) 29.2 against 23.1 us.
 template <int BLOCK, int V>
 __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     // A frame that is complete (pending, or halted already) skips the step;
@@ -206,6 +205,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     }
     constexpr uint32_t kCells = (uint32_t)(BLOCK * V);
     constexpr uint32_t kMembers = kCells * 8u < kTileMembers ? kCells * 8u : kTileMembers;
+    static_assert(kCells <= 1u << kTileShiftMax, "a tile");
     constexpr int kWaves = BLOCK / 64;
     static_assert(V == 1 || V == 4, "one head, or four in one 16-byte load, per thread");
     __shared__ uint32_t s_w[kWaves];
@@ -725,8 +725,6 @@ static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
         hipLaunchKernelGGL(SPH_CELL_SORT(256, 1), dim3(tiles), dim3(256), 0, st, a);
     else if (shift == 9u)
         hipLaunchKernelGGL(SPH_CELL_SORT(512, 1), dim3(tiles), dim3(512), 0, st, a);
-    else if (tiles <= kWideTiles)
-        hipLaunchKernelGGL(SPH_CELL_SORT(1024, 1), dim3(tiles), dim3(1024), 0, st, a);
     else
         hipLaunchKernelGGL(SPH_CELL_SORT(256, 4), dim3(tiles), dim3(256), 0, st, a);
 }

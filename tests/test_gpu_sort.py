@@ -1,6 +1,6 @@
 """The cell-count sort at its edges, against numpy's stable sort of the same
 keys: tiles fuller than the LDS list, cells whose chain of runs is longer than
-the sort follows, both tile widths, partial last tiles, and grids of more
+the sort follows, all tile sizes, partial last tiles, and grids of more
 tiles than a block sums itself.  Permutation, sorted keys and cell table are
 whole numbers and compared exactly."""
 import numpy as np
@@ -37,9 +37,11 @@ def scenes():
     # 1,025 cells: a last tile of one cell.
     out["last_tile_of_one"] = lambda E: (params(E, (0.999 * 41 * 0.02, 0.999 * 5 * 0.02, 0.999 * 5 * 0.02)),
                                          rng.uniform(0.0, 1.0, (3000, 3)) * (0.8, 0.09, 0.09) + 0.005, 1)
-    # More than 1024 tiles (four cells per thread) ...
+    # Between 2^19 and 2^20 cells (tiles of 512) ...
+    out["middle"] = lambda E: (params(E, (1.4, 1.1, 1.3)), rng.uniform(0.1, 1.0, (20000, 3)), 4)
+    # ... more than 2^20 (tiles of 1024, four cells per thread) ...
     out["narrow"] = lambda E: (params(E, (2.0, 1.1, 1.3)), rng.uniform(0.1, 1.0, (20000, 3)), 4)
-    # ... and more than 2048 (the tile sums are scanned by their own kernel).
+    # ... and more than 6144 tiles (their sums are scanned by their own kernel).
     out["scanned_tiles"] = lambda E: (params(E, (3.0, 3.0, 3.0)), rng.uniform(0.01, 2.99, (30000, 3)), 4)
     return out
 
