@@ -110,48 +110,62 @@ __global__ void adj_integrate_kernel(AdjArgs a) {
     }
 }
 
-// Per-particle sums of the adjoint force pass.
+// Per-particle sums of the adjoint force pass, without their constant factors
+// (adj_force_finish applies those): g without cP, h without -cV q_i, Pb
+// without cP, qb without cV.
 struct AdjForceAcc {
     float gx, gy, gz, hx, hy, hz, Pb, qb, Ax, Ay, Az;
 };
 
-// One neighbour's terms of the adjoint force pass (pos.w = p/rho^2, vel.w = 1/rho).
+__device__ __forceinline__ float dot3(float ax, float ay, float az, float bx, float by, float bz) {
+    return fmaf(az, bz, fmaf(ay, by, ax * bx));
+}
+
+// One neighbour's terms of the adjoint force pass (pos.w = p/rho^2, vel.w =
+// 1/rho); vp = cV q_i / cP.  The passes are bound by this arithmetic: a wave
+// walks each row for as long as its longest lane, some 58 pairs a lane where
+// 32 count, at four cycles an instruction.  With multiply-adds and the sums'
+// constants taken out it has 53 instructions where it had 78: staged force
+// pass of 16 x 32k particles 72.1 -> 63.8 us, gathered of 7k 23.5 -> 21.0.
 __device__ __forceinline__ void adj_force_pair(const SceneConst& sc, const float4& pi, const float4& vi,
-                                               const float4& abi, const float4& pj, const float4& vj,
+                                               const float4& abi, float vp, const float4& pj, const float4& vj,
                                                const float4& abj, AdjForceAcc& c) {
-    const float Pi = pi.w, qi = vi.w;
     const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
     const float d2 = dist2(rx, ry, rz);
     const float inv_r = d2 > 0.0f ? __builtin_amdgcn_rsqf(d2) : 0.0f;
-    const float dd = d2 * inv_r;
-    const float hr = sc.h - dd;
+    const float hr = fmaf(-d2, inv_r, sc.h);
     const float tt = sc.h2 - d2;
     const float phi = hr * hr * inv_r;
     const float dphi_r = -tt * inv_r * inv_r * inv_r;
+    const float w = hr * vj.w;
     const float dax = abi.x - abj.x, day = abi.y - abj.y, daz = abi.z - abj.z;
     const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
-    const float PP = sc.cP * (Pi + pj.w);
-    const float dar = dax * rx + day * ry + daz * rz;
-    const float dav = dax * dvx + day * dvy + daz * dvz;
-    const float cq = sc.cV * qi * vj.w;
-    const float coefr = PP * dphi_r * dar - cq * inv_r * dav;
-    c.gx += PP * phi * dax + coefr * rx;
-    c.gy += PP * phi * day + coefr * ry;
-    c.gz += PP * phi * daz + coefr * rz;
-    c.hx -= cq * hr * dax;
-    c.hy -= cq * hr * day;
-    c.hz -= cq * hr * daz;
-    c.Pb += sc.cP * phi * dar;
-    c.qb += sc.cV * vj.w * hr * dav;
-    c.Ax += hr * vj.w * dvx;
-    c.Ay += hr * vj.w * dvy;
-    c.Az += hr * vj.w * dvz;
+    const float PP = pi.w + pj.w;
+    const float dar = dot3(dax, day, daz, rx, ry, rz);
+    const float dav = dot3(dax, day, daz, dvx, dvy, dvz);
+    const float coefr = fmaf(PP * dphi_r, dar, -((vp * vj.w) * inv_r) * dav);
+    const float pphi = PP * phi;
+    c.gx = fmaf(coefr, rx, fmaf(pphi, dax, c.gx));
+    c.gy = fmaf(coefr, ry, fmaf(pphi, day, c.gy));
+    c.gz = fmaf(coefr, rz, fmaf(pphi, daz, c.gz));
+    c.hx = fmaf(w, dax, c.hx);
+    c.hy = fmaf(w, day, c.hy);
+    c.hz = fmaf(w, daz, c.hz);
+    c.Pb = fmaf(phi, dar, c.Pb);
+    c.qb = fmaf(w, dav, c.qb);
+    c.Ax = fmaf(w, dvx, c.Ax);
+    c.Ay = fmaf(w, dvy, c.Ay);
+    c.Az = fmaf(w, dvz, c.Az);
 }
+
+// Factor of the viscosity terms against the pressure terms' cP.
+__device__ __forceinline__ float visc_ratio(const SceneConst& sc, const float4& vi) { return (sc.cV * vi.w) / sc.cP; }
 
 // The EOS reverse and the stores of particle k; returns its (dL/dB, dL/dmu) terms.
 __device__ __forceinline__ double2 adj_force_finish(const AdjArgs& a, const SceneConst& sc, uint32_t k,
                                                     const float4& vi, const float4& abi, const AdjForceAcc& c) {
     const float qi = vi.w;
+    const float Pb = fmaf(sc.cP, c.Pb, abi.w), qb = sc.cV * c.qb, cvq = sc.cV * qi;
     // EOS derivatives (clamped Tait, exponent 7).
     const float rho = a.rho[k];
     const float x = rho * sc.inv_rho0;
@@ -161,12 +175,12 @@ __device__ __forceinline__ double2 adj_force_finish(const AdjArgs& a, const Scen
     const float p = praw * sgn;
     const float dp_drho = sgn * sc.B * 7.0f * x6 * sc.inv_rho0;
     const float dp_dB = sgn * (x7 - 1.0f);
-    a.rhobar[k] = c.Pb * (dp_drho * qi * qi - 2.0f * p * qi * qi * qi) - c.qb * qi * qi;
-    const float bpart = c.Pb * qi * qi * dp_dB;
+    a.rhobar[k] = Pb * (dp_drho * qi * qi - 2.0f * p * qi * qi * qi) - qb * qi * qi;
+    const float bpart = Pb * qi * qi * dp_dB;
     const float mpart = sc.cP * qi * (abi.x * c.Ax + abi.y * c.Ay + abi.z * c.Az);
     float4 xs = a.xs[k], vs = a.vs[k];
-    xs.x += c.gx; xs.y += c.gy; xs.z += c.gz;
-    vs.x += c.hx; vs.y += c.hy; vs.z += c.hz;
+    xs.x = fmaf(sc.cP, c.gx, xs.x); xs.y = fmaf(sc.cP, c.gy, xs.y); xs.z = fmaf(sc.cP, c.gz, xs.z);
+    vs.x = fmaf(-cvq, c.hx, vs.x); vs.y = fmaf(-cvq, c.hy, vs.y); vs.z = fmaf(-cvq, c.hz, vs.z);
     a.xs[k] = xs;
     a.vs[k] = vs;
     return make_double2((double)bpart, (double)mpart);
@@ -175,9 +189,10 @@ __device__ __forceinline__ double2 adj_force_finish(const AdjArgs& a, const Scen
 // One particle of the adjoint force pass; returns its (dL/dB, dL/dmu) terms.
 __device__ __forceinline__ double2 adj_force_one(const AdjArgs& a, const SceneConst& sc, uint32_t k) {
     const float4 pi = a.pos_s[k], vi = a.vel_s[k], abi = a.abar[k];
-    AdjForceAcc c = {0, 0, 0, 0, 0, 0, abi.w, 0, 0, 0, 0};
+    AdjForceAcc c = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const float vp = visc_ratio(sc, vi);
     for_each_neighbor(a, sc, k, pi, [&](uint32_t j) {
-        adj_force_pair(sc, pi, vi, abi, a.pos_s[j], a.vel_s[j], a.abar[j], c);
+        adj_force_pair(sc, pi, vi, abi, vp, a.pos_s[j], a.vel_s[j], a.abar[j], c);
     });
     return adj_force_finish(a, sc, k, vi, abi, c);
 }
@@ -226,7 +241,8 @@ __device__ __forceinline__ double2 adj_force_one_staged(const AdjArgs& a, const 
     const float4 pi = a.pos_s[kv], vi = a.vel_s[kv], abi = a.abar[kv];
     AdjRows r;
     adj_rows(a, sc, k, active, pi, r);
-    AdjForceAcc c = {0, 0, 0, 0, 0, 0, abi.w, 0, 0, 0, 0};
+    AdjForceAcc c = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const float vp = visc_ratio(sc, vi);
     const uint32_t lane = threadIdx.x & 63u;
 #pragma unroll
     for (int row = 0; row < kRows; ++row) {
@@ -270,10 +286,10 @@ __device__ __forceinline__ double2 adj_force_one_staged(const AdjArgs& a, const 
                 },
                 [&](uint32_t j) {
                     const uint32_t e = j - ulo;
-                    adj_force_pair(sc, pi, vi, abi, slot.pos[e], slot.vel[e], slot.abar[e], c);
+                    adj_force_pair(sc, pi, vi, abi, vp, slot.pos[e], slot.vel[e], slot.abar[e], c);
                 },
                 [&](uint32_t i) {
-                    adj_force_pair(sc, pi, vi, abi, slot.pos[e0 + i], slot.vel[e0 + i], slot.abar[e0 + i], c);
+                    adj_force_pair(sc, pi, vi, abi, vp, slot.pos[e0 + i], slot.vel[e0 + i], slot.abar[e0 + i], c);
                 });
             wave_lds_sync();
         } else {
@@ -283,7 +299,7 @@ __device__ __forceinline__ double2 adj_force_one_staged(const AdjArgs& a, const 
                     const float4 pj = a.pos_s[j];
                     return j != k && dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z) < sc.h2;
                 },
-                [&](uint32_t j) { adj_force_pair(sc, pi, vi, abi, a.pos_s[j], a.vel_s[j], a.abar[j], c); });
+                [&](uint32_t j) { adj_force_pair(sc, pi, vi, abi, vp, a.pos_s[j], a.vel_s[j], a.abar[j], c); });
         }
     }
     return active ? adj_force_finish(a, sc, k, vi, abi, c) : make_double2(0.0, 0.0);
@@ -355,15 +371,16 @@ __global__ __launch_bounds__(256) void adj_force_staged_kernel(AdjArgs a) {
     }
 }
 
-// One neighbour's term of the adjoint density pass.
+// One neighbour's term of the adjoint density pass, without its factor -6 cD
+// (adj_density_finish applies it).
 __device__ __forceinline__ void adj_density_pair(const SceneConst& sc, const float4& pi, float rbi, const float4& pj,
                                                  float rbj, float& gx, float& gy, float& gz) {
     const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
     const float tt = sc.h2 - dist2(rx, ry, rz);
-    const float s = -6.0f * sc.cD * tt * tt * (rbi + rbj);
-    gx += s * rx;
-    gy += s * ry;
-    gz += s * rz;
+    const float s = (tt * tt) * (rbi + rbj);
+    gx = fmaf(s, rx, gx);
+    gy = fmaf(s, ry, gy);
+    gz = fmaf(s, rz, gz);
 }
 
 // The walls' density reverse, and the adjoints of particle k scattered back
@@ -377,9 +394,10 @@ __device__ __forceinline__ void adj_density_finish(const AdjArgs& a, const Scene
         const float ul = (pk[d] - sc.bmin[d]) * sc.inv_h, uh = (sc.wmax[d] - pk[d]) * sc.inv_h;
         gw[d] = (rbi * sc.rho0) * (sc.inv_h * (wall_rho_du(ul) - wall_rho_du(uh)));
     }
-    gx += gw[0];
-    gy += gw[1];
-    gz += gw[2];
+    const float cg = -6.0f * sc.cD;
+    gx = fmaf(cg, gx, gw[0]);
+    gy = fmaf(cg, gy, gw[1]);
+    gz = fmaf(cg, gz, gw[2]);
     float4 xs = a.xs[k];
     xs.x += gx; xs.y += gy; xs.z += gz;
     const uint32_t src = a.perm[k];
