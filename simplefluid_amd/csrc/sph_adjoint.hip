@@ -16,7 +16,8 @@
 //                  with da = abar_i - abar_j, dv = v_j - v_i, phi = hr^2/d,
 //                  phi'/d = -t/d^3, psi' = -1; per-particle dL/dB and dL/dmu terms
 //   adj_density:   xbar_i += sum -6 cD t^2 (rhobar_i + rhobar_j) r, then
-//                  scatter both adjoints back to the step's input order.
+//                  scatter both adjoints back to the step's input order, through
+//                  adj_integrate of the step before
 // Walls, per axis d (u_lo = (x_d - box_min_d)/h, u_hi = (box_max_d - x_d)/h;
 // forward: rho_i += rho0 wall_rho(u), a_i,d += cW P_i (wall_j(u_lo) - wall_j(u_hi))):
 //   adj_integrate: xbar_i,d += cW P_i abar_i,d (wall_j'(u_lo) + wall_j'(u_hi)) / h,
@@ -65,6 +66,48 @@ __device__ __forceinline__ void for_each_neighbor(const AdjArgs& a, const SceneC
     }
 }
 
+// The reverse of clamp and symplectic Euler for output k of a step whose sorted
+// state is x0, v0 and acceleration ac: xb, vb the adjoint of that output; writes
+// what the step's force pass starts from.
+__device__ __forceinline__ void adj_integrate_one(const AdjArgs& a, const SceneConst& sc, uint32_t k, const float4& x0,
+                                                  const float4& v0, const float4& ac, const float4& xb,
+                                                  const float4& vb) {
+    const float xa[3] = {x0.x, x0.y, x0.z}, va[3] = {v0.x, v0.y, v0.z}, aa[3] = {ac.x, ac.y, ac.z};
+    const float xba[3] = {xb.x, xb.y, xb.z}, vba[3] = {vb.x, vb.y, vb.z};
+    float xo[3], vo[3], ab[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float v1 = va[d] + sc.dt * aa[d];
+        const float xt = xa[d] + sc.dt * v1;
+        float xbt = xba[d], vb1 = vba[d];
+        if (xt < sc.lo[d]) {
+            xbt = 0.0f;
+            if (v1 < 0.0f) vb1 = -sc.e * vb1;
+        } else if (xt > sc.hi[d]) {
+            xbt = 0.0f;
+            if (v1 > 0.0f) vb1 = -sc.e * vb1;
+        }
+        vb1 += sc.dt * xbt;
+        xo[d] = xbt;
+        vo[d] = vb1;
+        ab[d] = sc.dt * vb1;
+    }
+    // Walls: their pressure term depends on this particle alone, so its
+    // reverse (Pbar share in abar.w, xbar here) is elementwise.
+    float pw = 0.0f;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float ul = (xa[d] - sc.bmin[d]) * sc.inv_h, uh = (sc.wmax[d] - xa[d]) * sc.inv_h;
+        pw += sc.cW * ab[d] * (wall_j(ul) - wall_j(uh));
+        xo[d] += ((sc.cW * x0.w) * ab[d]) * (sc.inv_h * (wall_j_du(ul) + wall_j_du(uh)));
+    }
+    a.xbar_o[k] = make_float4(xo[0], xo[1], xo[2], 0.0f);
+    a.vbar_o[k] = make_float4(vo[0], vo[1], vo[2], 0.0f);
+    a.abar[k] = make_float4(ab[0], ab[1], ab[2], pw);
+}
+
+// The last step of a segment (the others' is done by the density pass of the
+// step after them).
 __global__ void adj_integrate_kernel(AdjArgs a) {
     uint32_t t0, t1;
     tile_span(a.ntiles, t0, t1);
@@ -73,40 +116,7 @@ __global__ void adj_integrate_kernel(AdjArgs a) {
         const SceneConst sc = scene_at(a.scenes, ti.x);
         const uint32_t k = ti.y + threadIdx.x;
         if (k >= sc.p_end) continue;
-        const float4 x0 = a.pos_s[k], v0 = a.vel_s[k], ac = a.acc[k];
-        const float4 xb = a.xbar[k], vb = a.vbar[k];
-        const float xa[3] = {x0.x, x0.y, x0.z}, va[3] = {v0.x, v0.y, v0.z}, aa[3] = {ac.x, ac.y, ac.z};
-        const float xba[3] = {xb.x, xb.y, xb.z}, vba[3] = {vb.x, vb.y, vb.z};
-        float xo[3], vo[3], ab[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const float v1 = va[d] + sc.dt * aa[d];
-            const float xt = xa[d] + sc.dt * v1;
-            float xbt = xba[d], vb1 = vba[d];
-            if (xt < sc.lo[d]) {
-                xbt = 0.0f;
-                if (v1 < 0.0f) vb1 = -sc.e * vb1;
-            } else if (xt > sc.hi[d]) {
-                xbt = 0.0f;
-                if (v1 > 0.0f) vb1 = -sc.e * vb1;
-            }
-            vb1 += sc.dt * xbt;
-            xo[d] = xbt;
-            vo[d] = vb1;
-            ab[d] = sc.dt * vb1;
-        }
-        // Walls: their pressure term depends on this particle alone, so its
-        // reverse (Pbar share in abar.w, xbar here) is elementwise.
-        float pw = 0.0f;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const float ul = (xa[d] - sc.bmin[d]) * sc.inv_h, uh = (sc.wmax[d] - xa[d]) * sc.inv_h;
-            pw += sc.cW * ab[d] * (wall_j(ul) - wall_j(uh));
-            xo[d] += ((sc.cW * x0.w) * ab[d]) * (sc.inv_h * (wall_j_du(ul) + wall_j_du(uh)));
-        }
-        a.xs[k] = make_float4(xo[0], xo[1], xo[2], 0.0f);
-        a.vs[k] = make_float4(vo[0], vo[1], vo[2], 0.0f);
-        a.abar[k] = make_float4(ab[0], ab[1], ab[2], pw);
+        adj_integrate_one(a, sc, k, a.pos_s[k], a.vel_s[k], a.acc[k], a.xbar[k], a.vbar[k]);
     }
 }
 
@@ -178,11 +188,11 @@ __device__ __forceinline__ double2 adj_force_finish(const AdjArgs& a, const Scen
     a.rhobar[k] = Pb * (dp_drho * qi * qi - 2.0f * p * qi * qi * qi) - qb * qi * qi;
     const float bpart = Pb * qi * qi * dp_dB;
     const float mpart = sc.cP * qi * (abi.x * c.Ax + abi.y * c.Ay + abi.z * c.Az);
-    float4 xs = a.xs[k], vs = a.vs[k];
+    float4 xs = a.xbar[k], vs = a.vbar[k];
     xs.x = fmaf(sc.cP, c.gx, xs.x); xs.y = fmaf(sc.cP, c.gy, xs.y); xs.z = fmaf(sc.cP, c.gz, xs.z);
     vs.x = fmaf(-cvq, c.hx, vs.x); vs.y = fmaf(-cvq, c.hy, vs.y); vs.z = fmaf(-cvq, c.hz, vs.z);
-    a.xs[k] = xs;
-    a.vs[k] = vs;
+    a.xbar[k] = xs;
+    a.vbar[k] = vs;
     return make_double2((double)bpart, (double)mpart);
 }
 
@@ -384,7 +394,10 @@ __device__ __forceinline__ void adj_density_pair(const SceneConst& sc, const flo
 }
 
 // The walls' density reverse, and the adjoints of particle k scattered back
-// to the step's input order.
+// to the step's input order: the step before's output, whose integration is
+// reversed right away where that step is on the tape (a pass of its own read
+// and wrote 64 bytes a particle more and took 13 us for 16 x 32k particles, 5
+// for 7k).
 __device__ __forceinline__ void adj_density_finish(const AdjArgs& a, const SceneConst& sc, uint32_t k,
                                                    const float4& pi, float rbi, float gx, float gy, float gz) {
     const float pk[3] = {pi.x, pi.y, pi.z};
@@ -398,11 +411,16 @@ __device__ __forceinline__ void adj_density_finish(const AdjArgs& a, const Scene
     gx = fmaf(cg, gx, gw[0]);
     gy = fmaf(cg, gy, gw[1]);
     gz = fmaf(cg, gz, gw[2]);
-    float4 xs = a.xs[k];
-    xs.x += gx; xs.y += gy; xs.z += gz;
     const uint32_t src = a.perm[k];
-    a.xbar[src] = xs;
-    a.vbar[src] = a.vs[k];
+    float4 xs = a.xbar[k];
+    const float4 vs = a.vbar[k];
+    xs.x += gx; xs.y += gy; xs.z += gz;
+    if (a.pos_p) {
+        adj_integrate_one(a, sc, src, a.pos_p[src], a.vel_p[src], a.acc_p[src], xs, vs);
+    } else {
+        a.xbar_o[src] = xs;
+        a.vbar_o[src] = vs;
+    }
 }
 
 // adj_density_kernel with the rows staged in LDS (1.9 KB per wave).

@@ -161,10 +161,13 @@ struct AdjArgs {
     const uint32_t* mask;
     const uint32_t* cstart;
     const uint32_t* perm;
-    float4* xbar;            // in: adjoint of the step output; out: of its input
-    float4* vbar;
-    float4* xs;
-    float4* vs;
+    const float4* pos_p;     // the same of the step before, whose integration the density pass reverses too,
+    const float4* vel_p;     // or null
+    const float4* acc_p;
+    float4* xbar;            // adjoint: of the step's output (integrate), then of its sorted state (force,
+    float4* vbar;            // density)
+    float4* xbar_o;          // integrate: of the step's sorted state; density: of its input, or of the sorted
+    float4* vbar_o;          // state of the step before
     float4* abar;
     float* rhobar;
     double2* tile_acc;       // per tile: running (dL/dB, dL/dmu) sums over the reverse steps

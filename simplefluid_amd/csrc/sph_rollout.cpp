@@ -135,6 +135,9 @@ int sph_rollout_backward(sph_handle* h, const float* dL_dx_final, float* dL_dB, 
     if (e != hipSuccess) return hip_fail(h, e, "adjoint seed");
 
     const uint32_t grid = ntiles;  // one block per tile
+    // The adjoint moves between two pairs of buffers: xb, vb hold it, each
+    // pass that reorders it or starts from it writes the other pair.
+    float4 *xb = R.xbar.p, *vb = R.vbar.p, *xo = R.xs.p, *vo = R.vs.p;
     for (int seg = (int)R.nseg - 1; seg >= 0; --seg) {
         const uint32_t len = std::min(R.every, R.steps - (uint32_t)seg * R.every);
         if (seg == (int)R.nseg - 1 && R.last_taped) {
@@ -153,20 +156,36 @@ int sph_rollout_backward(sph_handle* h, const float* dL_dx_final, float* dL_dB, 
             std::memset(&a, 0, sizeof(a));
             a.pos_s = w.pos_s.p; a.vel_s = w.vel_s.p; a.acc = w.acc.p; a.rho = w.rho.p;
             a.mask = w.mask.p; a.cstart = w.cstart.p; a.perm = w.perm.p;
-            a.xbar = R.xbar.p; a.vbar = R.vbar.p; a.xs = R.xs.p; a.vs = R.vs.p; a.abar = R.abar.p;
-            a.rhobar = R.rhobar.p; a.tile_acc = R.tile_acc.p;
+            a.abar = R.abar.p; a.rhobar = R.rhobar.p; a.tile_acc = R.tile_acc.p;
             a.scenes = h->sc_d.p; a.tiles = tiles; a.ntiles = ntiles; a.n = (uint32_t)n; a.ncells = h->ncells;
-            chk(launch_adj_integrate(st, 256, grid, a));
+            auto pairs = [&] {
+                a.xbar = xb; a.vbar = vb; a.xbar_o = xo; a.vbar_o = vo;
+            };
+            auto swap = [&] {
+                std::swap(xb, xo);
+                std::swap(vb, vo);
+            };
+            if (t == (int)len - 1) {
+                pairs();
+                chk(launch_adj_integrate(st, 256, grid, a));
+                swap();
+            }
+            if (t > 0) {
+                StepBufs& p = *R.tape[t - 1];
+                a.pos_p = p.pos_s.p; a.vel_p = p.vel_s.p; a.acc_p = p.acc.p;
+            }
+            pairs();
             // The reverse walk takes the forward force pass's form.
             chk(launch_adj_force(st, 256, grid, a, h->tune.force_staged));
             chk(launch_adj_density(st, 256, grid, a, h->tune.force_staged));
+            swap();
             if (e != hipSuccess) return hip_fail(h, e, "adjoint launch");
         }
     }
     chk(launch_scene_tile_sums(st, ns, R.tile_first.p, R.tile_acc.p, R.gB.p, R.gmu.p));
     // vbar is now in the initial state's order (checkpoint 0's ids).
     if (dL_dv0) {
-        chk(launch_unpermute3(st, (uint32_t)n, R.vbar.p, R.ck_id.p, R.gbuf.p));
+        chk(launch_unpermute3(st, (uint32_t)n, vb, R.ck_id.p, R.gbuf.p));
         chk(hipMemcpyAsync(dL_dv0, R.gbuf.p, 3 * n * sizeof(float), hipMemcpyDeviceToHost, st));
     }
     std::vector<double> gb(ns), gm(ns);
