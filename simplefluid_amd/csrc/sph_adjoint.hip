@@ -69,9 +69,19 @@ __device__ __forceinline__ void for_each_neighbor(const AdjArgs& a, const SceneC
 // The reverse of clamp and symplectic Euler for output k of a step whose sorted
 // state is x0, v0 and acceleration ac: xb, vb the adjoint of that output; writes
 // what the step's force pass starts from.
+// (wj, wd: the walls' differences and slopes at x0, adj_walls).
+__device__ __forceinline__ void adj_walls(const SceneConst& sc, const float4& x0, float wj[3], float wd[3]) {
+    const float xa[3] = {x0.x, x0.y, x0.z};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float ul = (xa[d] - sc.bmin[d]) * sc.inv_h, uh = (sc.wmax[d] - xa[d]) * sc.inv_h;
+        wj[d] = wall_j(ul) - wall_j(uh);
+        wd[d] = sc.inv_h * (wall_j_du(ul) + wall_j_du(uh));
+    }
+}
 __device__ __forceinline__ void adj_integrate_one(const AdjArgs& a, const SceneConst& sc, uint32_t k, const float4& x0,
                                                   const float4& v0, const float4& ac, const float4& xb,
-                                                  const float4& vb) {
+                                                  const float4& vb, const float wj[3], const float wd[3]) {
     const float xa[3] = {x0.x, x0.y, x0.z}, va[3] = {v0.x, v0.y, v0.z}, aa[3] = {ac.x, ac.y, ac.z};
     const float xba[3] = {xb.x, xb.y, xb.z}, vba[3] = {vb.x, vb.y, vb.z};
     float xo[3], vo[3], ab[3];
@@ -97,9 +107,8 @@ __device__ __forceinline__ void adj_integrate_one(const AdjArgs& a, const SceneC
     float pw = 0.0f;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const float ul = (xa[d] - sc.bmin[d]) * sc.inv_h, uh = (sc.wmax[d] - xa[d]) * sc.inv_h;
-        pw += sc.cW * ab[d] * (wall_j(ul) - wall_j(uh));
-        xo[d] += ((sc.cW * x0.w) * ab[d]) * (sc.inv_h * (wall_j_du(ul) + wall_j_du(uh)));
+        pw += sc.cW * ab[d] * wj[d];
+        xo[d] += ((sc.cW * x0.w) * ab[d]) * wd[d];
     }
     a.xbar_o[k] = make_float4(xo[0], xo[1], xo[2], 0.0f);
     a.vbar_o[k] = make_float4(vo[0], vo[1], vo[2], 0.0f);
@@ -116,7 +125,10 @@ __global__ void adj_integrate_kernel(AdjArgs a) {
         const SceneConst sc = scene_at(a.scenes, ti.x);
         const uint32_t k = ti.y + threadIdx.x;
         if (k >= sc.p_end) continue;
-        adj_integrate_one(a, sc, k, a.pos_s[k], a.vel_s[k], a.acc[k], a.xbar[k], a.vbar[k]);
+        const float4 x0 = a.pos_s[k];
+        float wj[3], wd[3];
+        adj_walls(sc, x0, wj, wd);
+        adj_integrate_one(a, sc, k, x0, a.vel_s[k], a.acc[k], a.xbar[k], a.vbar[k], wj, wd);
     }
 }
 
@@ -137,47 +149,71 @@ __device__ __forceinline__ float dot3(float ax, float ay, float az, float bx, fl
 // 32 count, at four cycles an instruction.  With multiply-adds and the sums'
 // constants taken out it has 53 instructions where it had 78: staged force
 // pass of 16 x 32k particles 72.1 -> 63.8 us, gathered of 7k 23.5 -> 21.0.
-__device__ __forceinline__ void adj_force_pair(const SceneConst& sc, const float4& pi, const float4& vi,
-                                               const float4& abi, float vp, const float4& pj, const float4& vj,
-                                               const float4& abj, AdjForceAcc& c) {
-    const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
-    const float d2 = dist2(rx, ry, rz);
+struct AdjFactors {
+    float coefr, rx, ry, rz, pphi, dax, day, daz, w, dvx, dvy, dvz, phi, dar, dav;
+};
+__device__ __forceinline__ AdjFactors adj_force_factors(const SceneConst& sc, const float4& pi, const float4& vi,
+                                                        const float4& abi, float vp, const float4& pj,
+                                                        const float4& vj, const float4& abj) {
+    AdjFactors f;
+    f.rx = pi.x - pj.x, f.ry = pi.y - pj.y, f.rz = pi.z - pj.z;
+    const float d2 = dist2(f.rx, f.ry, f.rz);
     const float inv_r = d2 > 0.0f ? __builtin_amdgcn_rsqf(d2) : 0.0f;
     const float hr = fmaf(-d2, inv_r, sc.h);
     const float tt = sc.h2 - d2;
-    const float phi = hr * hr * inv_r;
+    f.phi = hr * hr * inv_r;
     const float dphi_r = -tt * inv_r * inv_r * inv_r;
-    const float w = hr * vj.w;
-    const float dax = abi.x - abj.x, day = abi.y - abj.y, daz = abi.z - abj.z;
-    const float dvx = vj.x - vi.x, dvy = vj.y - vi.y, dvz = vj.z - vi.z;
+    f.w = hr * vj.w;
+    f.dax = abi.x - abj.x, f.day = abi.y - abj.y, f.daz = abi.z - abj.z;
+    f.dvx = vj.x - vi.x, f.dvy = vj.y - vi.y, f.dvz = vj.z - vi.z;
     const float PP = pi.w + pj.w;
-    const float dar = dot3(dax, day, daz, rx, ry, rz);
-    const float dav = dot3(dax, day, daz, dvx, dvy, dvz);
-    const float coefr = fmaf(PP * dphi_r, dar, -((vp * vj.w) * inv_r) * dav);
-    const float pphi = PP * phi;
-    c.gx = fmaf(coefr, rx, fmaf(pphi, dax, c.gx));
-    c.gy = fmaf(coefr, ry, fmaf(pphi, day, c.gy));
-    c.gz = fmaf(coefr, rz, fmaf(pphi, daz, c.gz));
-    c.hx = fmaf(w, dax, c.hx);
-    c.hy = fmaf(w, day, c.hy);
-    c.hz = fmaf(w, daz, c.hz);
-    c.Pb = fmaf(phi, dar, c.Pb);
-    c.qb = fmaf(w, dav, c.qb);
-    c.Ax = fmaf(w, dvx, c.Ax);
-    c.Ay = fmaf(w, dvy, c.Ay);
-    c.Az = fmaf(w, dvz, c.Az);
+    f.dar = dot3(f.dax, f.day, f.daz, f.rx, f.ry, f.rz);
+    f.dav = dot3(f.dax, f.day, f.daz, f.dvx, f.dvy, f.dvz);
+    f.coefr = fmaf(PP * dphi_r, f.dar, -((vp * vj.w) * inv_r) * f.dav);
+    f.pphi = PP * f.phi;
+    return f;
+}
+__device__ __forceinline__ void adj_force_pair(const SceneConst& sc, const float4& pi, const float4& vi,
+                                               const float4& abi, float vp, const float4& pj, const float4& vj,
+                                               const float4& abj, AdjForceAcc& c) {
+    const AdjFactors f = adj_force_factors(sc, pi, vi, abi, vp, pj, vj, abj);
+    c.gx = fmaf(f.coefr, f.rx, fmaf(f.pphi, f.dax, c.gx));
+    c.gy = fmaf(f.coefr, f.ry, fmaf(f.pphi, f.day, c.gy));
+    c.gz = fmaf(f.coefr, f.rz, fmaf(f.pphi, f.daz, c.gz));
+    c.hx = fmaf(f.w, f.dax, c.hx);
+    c.hy = fmaf(f.w, f.day, c.hy);
+    c.hz = fmaf(f.w, f.daz, c.hz);
+    c.Pb = fmaf(f.phi, f.dar, c.Pb);
+    c.qb = fmaf(f.w, f.dav, c.qb);
+    c.Ax = fmaf(f.w, f.dvx, c.Ax);
+    c.Ay = fmaf(f.w, f.dvy, c.Ay);
+    c.Az = fmaf(f.w, f.dvz, c.Az);
 }
 
 // Factor of the viscosity terms against the pressure terms' cP.
 __device__ __forceinline__ float visc_ratio(const SceneConst& sc, const float4& vi) { return (sc.cV * vi.w) / sc.cP; }
 
-// The EOS reverse and the stores of particle k; returns its (dL/dB, dL/dmu) terms.
-__device__ __forceinline__ double2 adj_force_finish(const AdjArgs& a, const SceneConst& sc, uint32_t k,
-                                                    const float4& vi, const float4& abi, const AdjForceAcc& c) {
-    const float qi = vi.w;
-    const float Pb = fmaf(sc.cP, c.Pb, abi.w), qb = sc.cV * c.qb, cvq = sc.cV * qi;
+// The sums' ends: the position adjoint ...
+__device__ __forceinline__ float4 adj_finish_x(const SceneConst& sc, float4 xs, float gx, float gy, float gz) {
+    xs.x = fmaf(sc.cP, gx, xs.x); xs.y = fmaf(sc.cP, gy, xs.y); xs.z = fmaf(sc.cP, gz, xs.z);
+    return xs;
+}
+// ... the velocity adjoint, ...
+__device__ __forceinline__ float4 adj_finish_v(const SceneConst& sc, float4 vs, float qi, float hx, float hy, float hz) {
+    const float cvq = sc.cV * qi;
+    vs.x = fmaf(-cvq, hx, vs.x); vs.y = fmaf(-cvq, hy, vs.y); vs.z = fmaf(-cvq, hz, vs.z);
+    return vs;
+}
+// ... the dL/dmu term, ...
+__device__ __forceinline__ float adj_finish_mu(const SceneConst& sc, float qi, const float4& abi, float Ax, float Ay,
+                                               float Az) {
+    return sc.cP * qi * (abi.x * Ax + abi.y * Ay + abi.z * Az);
+}
+// ... and the EOS reverse: the density adjoint and the dL/dB term.
+__device__ __forceinline__ float adj_finish_rho(const SceneConst& sc, float rho, float qi, const float4& abi, float Pbs,
+                                                float qbs, float& rhobar) {
+    const float Pb = fmaf(sc.cP, Pbs, abi.w), qb = sc.cV * qbs;
     // EOS derivatives (clamped Tait, exponent 7).
-    const float rho = a.rho[k];
     const float x = rho * sc.inv_rho0;
     const float x2 = x * x, x4 = x2 * x2, x6 = x4 * x2, x7 = x6 * x;
     const float praw = sc.B * (x7 - 1.0f);
@@ -185,14 +221,19 @@ __device__ __forceinline__ double2 adj_force_finish(const AdjArgs& a, const Scen
     const float p = praw * sgn;
     const float dp_drho = sgn * sc.B * 7.0f * x6 * sc.inv_rho0;
     const float dp_dB = sgn * (x7 - 1.0f);
-    a.rhobar[k] = Pb * (dp_drho * qi * qi - 2.0f * p * qi * qi * qi) - qb * qi * qi;
-    const float bpart = Pb * qi * qi * dp_dB;
-    const float mpart = sc.cP * qi * (abi.x * c.Ax + abi.y * c.Ay + abi.z * c.Az);
-    float4 xs = a.xbar[k], vs = a.vbar[k];
-    xs.x = fmaf(sc.cP, c.gx, xs.x); xs.y = fmaf(sc.cP, c.gy, xs.y); xs.z = fmaf(sc.cP, c.gz, xs.z);
-    vs.x = fmaf(-cvq, c.hx, vs.x); vs.y = fmaf(-cvq, c.hy, vs.y); vs.z = fmaf(-cvq, c.hz, vs.z);
-    a.xbar[k] = xs;
-    a.vbar[k] = vs;
+    rhobar = Pb * (dp_drho * qi * qi - 2.0f * p * qi * qi * qi) - qb * qi * qi;
+    return Pb * qi * qi * dp_dB;
+}
+
+// The stores of particle k; returns its (dL/dB, dL/dmu) terms.
+__device__ __forceinline__ double2 adj_force_finish(const AdjArgs& a, const SceneConst& sc, uint32_t k,
+                                                    const float4& vi, const float4& abi, const AdjForceAcc& c) {
+    float rhobar;
+    const float bpart = adj_finish_rho(sc, a.rho[k], vi.w, abi, c.Pb, c.qb, rhobar);
+    a.rhobar[k] = rhobar;
+    const float mpart = adj_finish_mu(sc, vi.w, abi, c.Ax, c.Ay, c.Az);
+    a.xbar[k] = adj_finish_x(sc, a.xbar[k], c.gx, c.gy, c.gz);
+    a.vbar[k] = adj_finish_v(sc, a.vbar[k], vi.w, c.hx, c.hy, c.hz);
     return make_double2((double)bpart, (double)mpart);
 }
 
@@ -381,13 +422,17 @@ __global__ __launch_bounds__(256) void adj_force_staged_kernel(AdjArgs a) {
     }
 }
 
+__device__ __forceinline__ float adj_density_factor(const SceneConst& sc, float rx, float ry, float rz, float rbi,
+                                                    float rbj) {
+    const float tt = sc.h2 - dist2(rx, ry, rz);
+    return (tt * tt) * (rbi + rbj);
+}
 // One neighbour's term of the adjoint density pass, without its factor -6 cD
 // (adj_density_finish applies it).
 __device__ __forceinline__ void adj_density_pair(const SceneConst& sc, const float4& pi, float rbi, const float4& pj,
                                                  float rbj, float& gx, float& gy, float& gz) {
     const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
-    const float tt = sc.h2 - dist2(rx, ry, rz);
-    const float s = (tt * tt) * (rbi + rbj);
+    const float s = adj_density_factor(sc, rx, ry, rz, rbi, rbj);
     gx = fmaf(s, rx, gx);
     gy = fmaf(s, ry, gy);
     gz = fmaf(s, rz, gz);
@@ -398,29 +443,51 @@ __device__ __forceinline__ void adj_density_pair(const SceneConst& sc, const flo
 // reversed right away where that step is on the tape (a pass of its own read
 // and wrote 64 bytes a particle more and took 13 us for 16 x 32k particles, 5
 // for 7k).
-__device__ __forceinline__ void adj_density_finish(const AdjArgs& a, const SceneConst& sc, uint32_t k,
-                                                   const float4& pi, float rbi, float gx, float gy, float gz) {
+struct AdjMove {
+    uint32_t src;
+    float4 xs, vs, x0, v0, ac;
+};
+__device__ __forceinline__ AdjMove adj_move(const AdjArgs& a, uint32_t k) {
+    AdjMove m;
+    m.src = a.perm[k];
+    m.xs = a.xbar[k];
+    m.vs = a.vbar[k];
+    m.x0 = m.v0 = m.ac = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (a.pos_p) {
+        m.x0 = a.pos_p[m.src];
+        m.v0 = a.vel_p[m.src];
+        m.ac = a.acc_p[m.src];
+    }
+    return m;
+}
+__device__ __forceinline__ void adj_density_walls(const SceneConst& sc, const float4& pi, float rbi, float gw[3]) {
     const float pk[3] = {pi.x, pi.y, pi.z};
-    float gw[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const float ul = (pk[d] - sc.bmin[d]) * sc.inv_h, uh = (sc.wmax[d] - pk[d]) * sc.inv_h;
         gw[d] = (rbi * sc.rho0) * (sc.inv_h * (wall_rho_du(ul) - wall_rho_du(uh)));
     }
+}
+__device__ __forceinline__ void adj_scatter(const AdjArgs& a, const SceneConst& sc, AdjMove& m, float gx, float gy,
+                                            float gz, const float gw[3], const float wj[3], const float wd[3]) {
     const float cg = -6.0f * sc.cD;
-    gx = fmaf(cg, gx, gw[0]);
-    gy = fmaf(cg, gy, gw[1]);
-    gz = fmaf(cg, gz, gw[2]);
-    const uint32_t src = a.perm[k];
-    float4 xs = a.xbar[k];
-    const float4 vs = a.vbar[k];
-    xs.x += gx; xs.y += gy; xs.z += gz;
+    m.xs.x += fmaf(cg, gx, gw[0]);
+    m.xs.y += fmaf(cg, gy, gw[1]);
+    m.xs.z += fmaf(cg, gz, gw[2]);
     if (a.pos_p) {
-        adj_integrate_one(a, sc, src, a.pos_p[src], a.vel_p[src], a.acc_p[src], xs, vs);
+        adj_integrate_one(a, sc, m.src, m.x0, m.v0, m.ac, m.xs, m.vs, wj, wd);
     } else {
-        a.xbar_o[src] = xs;
-        a.vbar_o[src] = vs;
+        a.xbar_o[m.src] = m.xs;
+        a.vbar_o[m.src] = m.vs;
     }
+}
+__device__ __forceinline__ void adj_density_finish(const AdjArgs& a, const SceneConst& sc, uint32_t k,
+                                                   const float4& pi, float rbi, float gx, float gy, float gz) {
+    float gw[3], wj[3], wd[3];
+    adj_density_walls(sc, pi, rbi, gw);
+    AdjMove m = adj_move(a, k);
+    adj_walls(sc, m.x0, wj, wd);
+    adj_scatter(a, sc, m, gx, gy, gz, gw, wj, wd);
 }
 
 // adj_density_kernel with the rows staged in LDS (1.9 KB per wave).
@@ -516,6 +583,298 @@ __global__ void adj_density_kernel(AdjArgs a) {
     }
 }
 
+// ------------------------------------------------------------- split form
+//
+// As in the forward step, a small handle's pass lasts as long as one wave's
+// chain (7k particles, 113 waves: force 21.0 us, density 13.5; in this form
+// 7.8 and 5.5, bound by the latency of the windows, the gathers and the
+// in-order sums one after the other).  Force: nine
+// waves per 64 particles list the neighbours, one row each, from the step's
+// masks; eight of them gather the pairs of kAdjRound list entries and leave
+// their factors in LDS; then three waves add them in list order, each its
+// share of the sums, and finish that share.  The density pass takes the list
+// over, four waves per 64 particles.  The sums' order and arithmetic are the
+// other forms', bit for bit.
+constexpr int kAdjRound = 16;  // two blocks of 77 KB fit a CU
+
+struct AdjForceShared {
+    float4 f1[kAdjRound][kSplitTile];    // coefr, r
+    float4 f2[kAdjRound][kSplitTile];    // (P_i + P_j) phi, da
+    float4 f3[kAdjRound][kSplitTile];    // w, dv
+    float2 f4[kAdjRound][kSplitTile];    // phi, da.r
+    float f5[kAdjRound][kSplitTile];     // da.dv
+    uint16_t id[kListMax][kSplitTile];   // the neighbours, without the particle itself
+    uint32_t count[3][kSplitTile];       // neighbours per row, one byte a row
+};
+static_assert(2 * sizeof(AdjForceShared) <= 160 * 1024, "two blocks per CU");
+
+__global__ __launch_bounds__(64 * kRows) void adj_force_split_kernel(AdjArgs a) {
+    __shared__ AdjForceShared sh;
+    const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
+    const __amdgpu_buffer_rsrc_t rvel = buffer_of(a.vel_s, a.n);
+    const __amdgpu_buffer_rsrc_t rab = buffer_of((const float4*)a.abar, a.n);
+    const __amdgpu_buffer_rsrc_t rcs = buffer_of(a.cstart, a.ncells + 1u);
+    const uint2 ti = tile_at(a.tiles, xcd_block(blockIdx.x, gridDim.x));
+    const SceneConst sc = scene_at(a.scenes, ti.x);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t k = ti.y + lane;
+    const bool active = k < sc.p_end;
+    // Zeros past the buffers' ends.
+    const float4 pi = load4(rpos, k << 4), vi = load4(rvel, k << 4), abi = load4(rab, k << 4);
+    uint32_t m = active ? a.mask[(size_t)w * a.n + k] : 0u;
+    // What the finishing waves add their sums to.
+    float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (active) {
+        if (w == 0) own = a.xbar[k];
+        if (w == 1) own = a.vbar[k];
+        if (w == 2) own.x = a.rho[k];
+    }
+    uint32_t lo, hi;
+    split_window(rcs, sc, pi, w % 3 - 1, w / 3 - 1, lo, hi);
+    if (!active) lo = hi = 0u;
+    if (w == 4 && active) m = without_self(m, lo, hi, k, 0u);
+    // The mask's slots as ascending bits, and the 32 before them, tested again.
+    const uint32_t span = mask_span(lo, hi);
+    const uint32_t j1 = row_first(lo, hi, 2u), j0 = row_first(lo, hi);
+    const uint32_t r = mask_ascending(m, span, 0u);
+    uint32_t rh = 0u;
+    for (uint32_t j = j1; j < j0; ++j) {
+        const float4 pj = load4(rpos, j << 4);
+        if (j != k && dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z) < sc.h2) rh |= 1u << (j - j1);
+    }
+    const uint32_t cnt = span > 64u ? kRowOver : (uint32_t)__popc(r) + (uint32_t)__popc(rh);
+    reinterpret_cast<uint8_t*>(sh.count)[(((uint32_t)w >> 2) * kSplitTile + lane) * 4u + ((uint32_t)w & 3u)] = (uint8_t)cnt;
+    __syncthreads();
+    uint32_t at = 0u, total = 0u;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+        const uint32_t c = sh.count[g][lane];
+        const uint32_t before = w >= 4 * g + 4 ? 0xffffffffu : w > 4 * g ? (1u << (8 * (w - 4 * g))) - 1u : 0u;
+        at = __builtin_amdgcn_sad_u8(c & before, 0u, at);
+        total = __builtin_amdgcn_sad_u8(g == 2 ? c & 0xffu : c, 0u, total);
+    }
+    const uint32_t most = wave_umax(total);  // the same in every wave
+    if (most > kListMax) {
+        if (w == 0 && active) {
+            a.ncount[k] = kListOver;
+            a.part[k] = adj_force_one(a, sc, k);
+        }
+        return;
+    }
+    for (uint32_t q = rh; q; q &= q - 1u) sh.id[at++][lane] = (uint16_t)(j1 + (uint32_t)__builtin_ctz(q));
+    for (uint32_t q = r; q; q &= q - 1u) sh.id[at++][lane] = (uint16_t)(j0 + (uint32_t)__builtin_ctz(q));
+    __syncthreads();
+    const float vp = visc_ratio(sc, vi);
+    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f, s4 = 0.f, s5 = 0.f;
+    for (uint32_t first = 0u;; first += kAdjRound) {
+        if (w < 8) {
+            const uint32_t e = 2u * (uint32_t)w;
+            if (__ballot(total > first + e) != 0u) {
+                float4 pj[2], vj[2], bj[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const uint32_t i = first + e + (uint32_t)u;
+                    const uint32_t j = i < total ? (uint32_t)sh.id[i][lane] : k;  // past the list: not added
+                    pj[u] = load4(rpos, j << 4);
+                    vj[u] = load4(rvel, j << 4);
+                    bj[u] = load4(rab, j << 4);
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const AdjFactors f = adj_force_factors(sc, pi, vi, abi, vp, pj[u], vj[u], bj[u]);
+                    sh.f1[e + (uint32_t)u][lane] = make_float4(f.coefr, f.rx, f.ry, f.rz);
+                    sh.f2[e + (uint32_t)u][lane] = make_float4(f.pphi, f.dax, f.day, f.daz);
+                    sh.f3[e + (uint32_t)u][lane] = make_float4(f.w, f.dvx, f.dvy, f.dvz);
+                    sh.f4[e + (uint32_t)u][lane] = make_float2(f.phi, f.dar);
+                    sh.f5[e + (uint32_t)u][lane] = f.dav;
+                }
+            }
+        } else if (first == 0u && active) {
+            // The list, for the density pass.
+            a.ncount[k] = total;
+            for (uint32_t q = 0; 4u * q < total; ++q)
+                reinterpret_cast<uint2*>(a.nlist)[(size_t)q * a.n + k] =
+                    make_uint2(sh.id[4u * q][lane] | ((uint32_t)sh.id[4u * q + 1u][lane] << 16),
+                               sh.id[4u * q + 2u][lane] | ((uint32_t)sh.id[4u * q + 3u][lane] << 16));
+        }
+        __syncthreads();
+        const uint32_t left = total > first ? min(total - first, (uint32_t)kAdjRound) : 0u;
+        if (w == 0) {
+#pragma unroll 4
+            for (uint32_t i = 0; i < left; ++i) {
+                const float4 f1 = sh.f1[i][lane], f2 = sh.f2[i][lane];
+                s0 = fmaf(f1.x, f1.y, fmaf(f2.x, f2.y, s0));
+                s1 = fmaf(f1.x, f1.z, fmaf(f2.x, f2.z, s1));
+                s2 = fmaf(f1.x, f1.w, fmaf(f2.x, f2.w, s2));
+            }
+        } else if (w == 1) {
+#pragma unroll 4
+            for (uint32_t i = 0; i < left; ++i) {
+                const float4 f2 = sh.f2[i][lane], f3 = sh.f3[i][lane];
+                s0 = fmaf(f3.x, f2.y, s0);
+                s1 = fmaf(f3.x, f2.z, s1);
+                s2 = fmaf(f3.x, f2.w, s2);
+                s3 = fmaf(f3.x, f3.y, s3);
+                s4 = fmaf(f3.x, f3.z, s4);
+                s5 = fmaf(f3.x, f3.w, s5);
+            }
+        } else if (w == 2) {
+#pragma unroll 4
+            for (uint32_t i = 0; i < left; ++i) {
+                const float2 f4 = sh.f4[i][lane];
+                s0 = fmaf(f4.x, f4.y, s0);
+                s1 = fmaf(sh.f3[i][lane].x, sh.f5[i][lane], s1);
+            }
+        }
+        if (most <= first + (uint32_t)kAdjRound) break;
+        __syncthreads();
+    }
+    if (!active) return;
+    double* const part = reinterpret_cast<double*>(a.part + k);
+    if (w == 0) a.xbar[k] = adj_finish_x(sc, own, s0, s1, s2);
+    if (w == 1) {
+        a.vbar[k] = adj_finish_v(sc, own, vi.w, s0, s1, s2);
+        part[1] = (double)adj_finish_mu(sc, vi.w, abi, s3, s4, s5);
+    }
+    if (w == 2) {
+        float rhobar;
+        part[0] = (double)adj_finish_rho(sc, own.x, vi.w, abi, s0, s1, rhobar);
+        a.rhobar[k] = rhobar;
+    }
+}
+
+constexpr uint32_t kAdjDensityRound = 32;
+constexpr int kAdjDensityWaves = 4;
+constexpr int kAdjPerWave = (int)kAdjDensityRound / kAdjDensityWaves;
+
+struct AdjDensityShared {
+    float4 f[kAdjDensityRound][kSplitTile];  // s, r
+    float gw[3][kSplitTile];                 // the walls' density term
+    float wj[3][kSplitTile], wd[3][kSplitTile];
+};
+
+__global__ __launch_bounds__(64 * kAdjDensityWaves) void adj_density_split_kernel(AdjArgs a) {
+    __shared__ AdjDensityShared sh;
+    const __amdgpu_buffer_rsrc_t rpos = buffer_of(a.pos_s, a.n);
+    const __amdgpu_buffer_rsrc_t rrb = buffer_of((const float*)a.rhobar, a.n);
+    const __amdgpu_buffer_rsrc_t rl = buffer_of((const uint16_t*)a.nlist, kListMax * a.n);
+    const uint2 ti = tile_at(a.tiles, xcd_block(blockIdx.x, gridDim.x));
+    const SceneConst sc = scene_at(a.scenes, ti.x);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t k = ti.y + lane;
+    const bool active = k < sc.p_end;
+    // Entries past a list's end hold any index; their pairs are not added.
+    auto ids = [&](uint32_t q) { return __builtin_amdgcn_raw_buffer_load_b64(rl, (int)((q * a.n + k) << 3), 0, 0); };
+    u32x2 q0 = ids(2u * (uint32_t)w), q1 = ids(2u * (uint32_t)w + 1u);
+    const float4 pi = load4(rpos, k << 4);
+    const float rbi = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rrb, (int)(k << 2), 0, 0));
+    const uint32_t count = active ? a.ncount[k] : 0u;
+    float4 pj[kAdjPerWave];
+    float rj[kAdjPerWave];
+    auto gather = [&]() {
+        const uint32_t j[kAdjPerWave] = {q0.x & 0xffffu, q0.x >> 16, q0.y & 0xffffu, q0.y >> 16,
+                                         q1.x & 0xffffu, q1.x >> 16, q1.y & 0xffffu, q1.y >> 16};
+#pragma unroll
+        for (int u = 0; u < kAdjPerWave; ++u) {
+            pj[u] = load4(rpos, j[u] << 4);
+            rj[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rrb, (int)(j[u] << 2), 0, 0));
+        }
+    };
+    gather();  // before the counts are known: any index stays inside the buffers' bounds checks
+    AdjMove mv;
+    if (w == 0 && active) mv = adj_move(a, k);
+    if (w == 3 && ((ti.y - sc.p_begin) & 255u) == 0u) {
+        // The step's terms of 256 particles into their tile's running sums,
+        // added in adj_force_kernel's tree.
+        double2 p[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+            p[i] = make_double2(0.0, 0.0);
+            if (k + 64u * i < sc.p_end) p[i] = a.part[k + 64u * i];
+        }
+        double x = (p[0].x + p[2].x) + (p[1].x + p[3].x), y = (p[0].y + p[2].y) + (p[1].y + p[3].y);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            x += __shfl_down(x, o, 64);
+            y += __shfl_down(y, o, 64);
+        }
+        if (lane == 0u) {
+            const uint32_t t = a.tile_first[ti.x] + ((ti.y - sc.p_begin) >> 8);
+            double2 acc = a.tile_acc[t];
+            acc.x += x;
+            acc.y += y;
+            a.tile_acc[t] = acc;
+        }
+    }
+    if (__ballot(count > kListMax) != 0u) {  // the same in every wave
+        if (w == 0 && active) {
+            float gx = 0.f, gy = 0.f, gz = 0.f;
+            for_each_neighbor(a, sc, k, pi, [&](uint32_t j) {
+                adj_density_pair(sc, pi, rbi, a.pos_s[j], a.rhobar[j], gx, gy, gz);
+            });
+            adj_density_finish(a, sc, k, pi, rbi, gx, gy, gz);
+        }
+        return;
+    }
+    float gx = 0.f, gy = 0.f, gz = 0.f;
+    for (uint32_t first = 0u;; first += kAdjDensityRound) {
+        if (__ballot(count > first + (uint32_t)(kAdjPerWave * w)) != 0u) {
+            if (first != 0u) {
+                q0 = ids(first / 4u + 2u * (uint32_t)w);
+                q1 = ids(first / 4u + 2u * (uint32_t)w + 1u);
+                gather();
+            }
+#pragma unroll
+            for (int u = 0; u < kAdjPerWave; ++u) {
+                const float rx = pi.x - pj[u].x, ry = pi.y - pj[u].y, rz = pi.z - pj[u].z;
+                sh.f[kAdjPerWave * w + u][lane] =
+                    make_float4(adj_density_factor(sc, rx, ry, rz, rbi, rj[u]), rx, ry, rz);
+            }
+        }
+        if (first == 0u && active) {
+            float t[3], u[3];
+            if (w == 1) {
+                adj_density_walls(sc, pi, rbi, t);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) sh.gw[d][lane] = t[d];
+            } else if (w == 2 && a.pos_p) {
+                adj_walls(sc, a.pos_p[a.perm[k]], t, u);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    sh.wj[d][lane] = t[d];
+                    sh.wd[d][lane] = u[d];
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t left = count > first ? min(count - first, kAdjDensityRound) : 0u;
+        if (w == 0) {
+#pragma unroll 4
+            for (uint32_t i = 0; i < left; ++i) {
+                const float4 f = sh.f[i][lane];
+                gx = fmaf(f.x, f.y, gx);
+                gy = fmaf(f.x, f.z, gy);
+                gz = fmaf(f.x, f.w, gz);
+            }
+        }
+        if (__ballot(count > first + kAdjDensityRound) == 0u) break;
+        __syncthreads();
+    }
+    if (w != 0 || !active) return;
+    const float gw[3] = {sh.gw[0][lane], sh.gw[1][lane], sh.gw[2][lane]};
+    float wj[3] = {0.f, 0.f, 0.f}, wd[3] = {0.f, 0.f, 0.f};
+    if (a.pos_p) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            wj[d] = sh.wj[d][lane];
+            wd[d] = sh.wd[d][lane];
+        }
+    }
+    adj_scatter(a, sc, mv, gx, gy, gz, gw, wj, wd);
+}
+
 // Per-scene totals of the per-tile accumulators: block s sums tiles
 // [tile_first[s], tile_first[s + 1]) in a fixed order (threads stride, then
 // a tree), so the result is the same run to run.
@@ -581,6 +940,18 @@ hipError_t launch_adj_density(hipStream_t st, int block, uint32_t grid, const Ad
         hipLaunchKernelGGL(adj_density_staged_kernel, dim3(grid), dim3(block), 0, st, a);
     else
         hipLaunchKernelGGL(adj_density_kernel, dim3(grid), dim3(block), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_adj_force_split(hipStream_t st, const AdjArgs& a) {
+    if (a.ntiles == 0) return hipSuccess;
+    hipLaunchKernelGGL(adj_force_split_kernel, dim3(a.ntiles), dim3(64 * kRows), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_adj_density_split(hipStream_t st, const AdjArgs& a) {
+    if (a.ntiles == 0) return hipSuccess;
+    hipLaunchKernelGGL(adj_density_split_kernel, dim3(a.ntiles), dim3(64 * kAdjDensityWaves), 0, st, a);
     return hipGetLastError();
 }
 

@@ -203,6 +203,30 @@ __device__ __forceinline__ void row_window(__amdgpu_buffer_rsrc_t rcs, const Sce
     chord_window(rcs, sc, g.fx, w2, g.row0 + (uint32_t)(dz * sc.G[1] + dy) * (uint32_t)sc.G[0], lo, hi);
 }
 
+// The window of one row (dy, dz) of a particle: row_geom and row_window for
+// that row alone.
+__device__ __forceinline__ void split_window(__amdgpu_buffer_rsrc_t rcs, const SceneConst& sc, const float4& p, int dy,
+                                             int dz, uint32_t& lo, uint32_t& hi) {
+    const float fx = (p.x - sc.bmin[0]) * sc.inv_csx;
+    const float f[2] = {(p.y - sc.bmin[1]) * sc.inv_cs, (p.z - sc.bmin[2]) * sc.inv_cs};
+    const int d[2] = {dy, dz};
+    int c[2];
+    float q[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        c[i] = (int)fminf(fmaxf(f[i], 0.0f), (float)(sc.G[i + 1] - 1));
+        const float m = 0.0009765625f;
+        const float r = fminf(fmaxf(f[i] - (float)c[i], 0.0f), 1.0f);
+        const float near = fmaxf((d[i] < 0 ? r : 1.0f - r) - m, 0.0f);
+        const bool in = d[i] < 0 ? c[i] > 0 : c[i] < sc.G[i + 1] - 1;
+        q[i] = d[i] == 0 ? 0.0f : in ? near * near : 4.0f;
+    }
+    lo = hi = 0u;
+    if (!(__builtin_isfinite(p.x) && __builtin_isfinite(p.y) && __builtin_isfinite(p.z))) return;
+    const uint32_t row = ((uint32_t)(c[1] + dz) * (uint32_t)sc.G[1] + (uint32_t)(c[0] + dy)) * (uint32_t)sc.G[0];
+    chord_window(rcs, sc, fx, sc.hc2 - (q[0] + q[1]), sc.cell_offset + row, lo, hi);
+}
+
 // Row masks.  The density pass tests a row's candidates [lo, hi) four at a
 // time and shifts one bit per slot into the row's mask (slots past hi shift
 // in zeros), so candidate c of a row with T groups sits at bit 4T-1-c and
@@ -253,6 +277,13 @@ __device__ __forceinline__ uint32_t mask_ascending(uint32_t word, uint32_t span,
     const uint32_t slots = span - after;
     if (slots - 1u < 31u) r >>= 32u - slots;
     return r;
+}
+
+// The centre row's mask word (its last slot `after` slots before the row's
+// end) without particle k's own bit.
+__device__ __forceinline__ uint32_t without_self(uint32_t word, uint32_t lo, uint32_t hi, uint32_t k, uint32_t after) {
+    const uint32_t b = mask_bit(lo, hi, k) - after;
+    return b < (uint32_t)kMaskBits ? word & ~(1u << b) : word;
 }
 
 // row_neighbors with the mask's visits given as offsets: g(i) for candidate

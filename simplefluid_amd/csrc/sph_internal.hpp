@@ -121,6 +121,9 @@ hipError_t launch_force(hipStream_t st, int block, uint32_t grid, const StepArgs
 constexpr uint32_t kSplitMax = 65536;   // the lists hold 16-bit indices
 constexpr uint32_t kListMax = 128;
 constexpr int kSplitTile = 64;
+constexpr uint32_t kListOver = 0xffffu;  // the length of a list that is too long
+constexpr uint32_t kRowOver = 255u;      // the count of a row longer than two mask words
+static_assert(kRowOver > kListMax + 1u, "such a row's particle is over its list's length too");
 // Tiles up to which handles take it.  Two force blocks fit a CU, so 512 tiles
 // run at once; from there on the chip is full and its extra work shows.
 // Measured per step, the split form against the best of the others: 512
@@ -171,6 +174,13 @@ struct AdjArgs {
     float4* abar;
     float* rhobar;
     double2* tile_acc;       // per tile: running (dL/dB, dL/dmu) sums over the reverse steps
+    // Split form: the particles' (dL/dB, dL/dmu) terms of the step, which the
+    // density pass adds up in tiles of 256, each scene's first one, and the
+    // neighbour lists (force to density) and their lengths.
+    double2* part;
+    const uint32_t* tile_first;
+    uint16_t* nlist;
+    uint32_t* ncount;
     const SceneConst* scenes;
     const uint2* tiles;
     uint32_t ntiles;
@@ -182,6 +192,9 @@ hipError_t launch_adj_integrate(hipStream_t st, int block, uint32_t grid, const 
 // staged: each row's candidates read from LDS (same results; whole waves only).
 hipError_t launch_adj_force(hipStream_t st, int block, uint32_t grid, const AdjArgs& a, int staged = 0);
 hipError_t launch_adj_density(hipStream_t st, int block, uint32_t grid, const AdjArgs& a, int staged = 0);
+// The split form of both, over tiles of kSplitTile particles: same results.
+hipError_t launch_adj_force_split(hipStream_t st, const AdjArgs& a);
+hipError_t launch_adj_density_split(hipStream_t st, const AdjArgs& a);
 // Per-scene totals of the tile accumulators in a fixed order: scene s sums
 // tiles [tile_first[s], tile_first[s + 1]) into acc_a[s], acc_b[s].
 hipError_t launch_scene_tile_sums(hipStream_t st, uint32_t nscenes, const uint32_t* tile_first,

@@ -116,7 +116,9 @@ int sph_rollout_backward(sph_handle* h, const float* dL_dx_final, float* dL_dB, 
     chk(R.gbuf.ensure(3 * n + 1));
     uint32_t ntiles = 0;
     const uint2* tiles = tiles_for(h, 256, ntiles);  // tiles of 256 particles, scene by scene
-    if (!tiles) return fail(h, SPH_E_OOM, "tile table");
+    uint32_t n_split = 0;
+    const uint2* split_tiles = tiles_for(h, kSplitTile, n_split);
+    if (!tiles || !split_tiles) return fail(h, SPH_E_OOM, "tile table");
     // First tile of each scene, as the tile table lists them.
     std::vector<uint32_t> first(ns + 1, 0);
     for (uint32_t s = 0; s < ns; ++s)
@@ -176,8 +178,21 @@ int sph_rollout_backward(sph_handle* h, const float* dL_dx_final, float* dL_dB, 
             }
             pairs();
             // The reverse walk takes the forward force pass's form.
-            chk(launch_adj_force(st, 256, grid, a, h->tune.force_staged));
-            chk(launch_adj_density(st, 256, grid, a, h->tune.force_staged));
+            if (split_form(h)) {
+                a.tiles = split_tiles;
+                a.ntiles = n_split;
+                a.nlist = h->nlist.p;
+                a.ncount = h->ncount.p;
+                a.tile_first = R.tile_first.p;
+                // This step's acceleration has been used: its room holds the
+                // particles' parameter terms.
+                a.part = reinterpret_cast<double2*>(w.acc.p);
+                chk(launch_adj_force_split(st, a));
+                chk(launch_adj_density_split(st, a));
+            } else {
+                chk(launch_adj_force(st, 256, grid, a, h->tune.force_staged));
+                chk(launch_adj_density(st, 256, grid, a, h->tune.force_staged));
+            }
             swap();
             if (e != hipSuccess) return hip_fail(h, e, "adjoint launch");
         }

@@ -351,13 +351,6 @@ __device__ __forceinline__ void force_pair(const SceneConst& sc, const float4& p
 __device__ __forceinline__ Moved force_finish(const StepArgs& a, const SceneConst& sc, uint32_t k,
                                                  const float4& pi, const float4& vi, const ForceAcc& f);
 
-// The centre row's mask word (its last slot `after` slots before the row's
-// end) without particle k's own bit.
-__device__ __forceinline__ uint32_t without_self(uint32_t word, uint32_t lo, uint32_t hi, uint32_t k, uint32_t after) {
-    const uint32_t b = mask_bit(lo, hi, k) - after;
-    return b < (uint32_t)kMaskBits ? word & ~(1u << b) : word;
-}
-
 // One row's pairs in ascending order of candidates: the re-tested ones before
 // the masks', the second word's, the mask m's.  pos(j), vel(j): candidate j's
 // records; walk(r, j0): the pairs of the bits of r (bit i: candidate j0 + i).
@@ -718,9 +711,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) v
 
 constexpr uint32_t kKept = 5;        // a gathered row's terms kept in its copy's place
 constexpr uint32_t kChunk = 64;      // entries of a list in LDS at a time
-constexpr uint32_t kListOver = 0xffffu;
-constexpr uint32_t kRowOver = 255u;
-static_assert(kRowOver > kListMax + 1u, "such a row's particle is over its list's length too");
 template <bool V>
 struct Bool {
     static constexpr bool value = V;
@@ -736,30 +726,6 @@ struct SplitShared {
     uint32_t count[3][kSplitTile];                 // neighbours per row, one byte a row (itself included)
     float wall[kSplitTile];
 };
-
-// The window of one row (dy, dz) of a particle: row_geom and row_window for
-// that row alone.
-__device__ __forceinline__ void split_window(__amdgpu_buffer_rsrc_t rcs, const SceneConst& sc, const float4& p, int dy,
-                                             int dz, uint32_t& lo, uint32_t& hi) {
-    const float fx = (p.x - sc.bmin[0]) * sc.inv_csx;
-    const float f[2] = {(p.y - sc.bmin[1]) * sc.inv_cs, (p.z - sc.bmin[2]) * sc.inv_cs};
-    const int d[2] = {dy, dz};
-    int c[2];
-    float q[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        c[i] = (int)fminf(fmaxf(f[i], 0.0f), (float)(sc.G[i + 1] - 1));
-        const float m = 0.0009765625f;
-        const float r = fminf(fmaxf(f[i] - (float)c[i], 0.0f), 1.0f);
-        const float near = fmaxf((d[i] < 0 ? r : 1.0f - r) - m, 0.0f);
-        const bool in = d[i] < 0 ? c[i] > 0 : c[i] < sc.G[i + 1] - 1;
-        q[i] = d[i] == 0 ? 0.0f : in ? near * near : 4.0f;
-    }
-    lo = hi = 0u;
-    if (!(__builtin_isfinite(p.x) && __builtin_isfinite(p.y) && __builtin_isfinite(p.z))) return;
-    const uint32_t row = ((uint32_t)(c[1] + dz) * (uint32_t)sc.G[1] + (uint32_t)(c[0] + dy)) * (uint32_t)sc.G[0];
-    chord_window(rcs, sc, fx, sc.hc2 - (q[0] + q[1]), sc.cell_offset + row, lo, hi);
-}
 
 // One candidate's term c = min(d^2 - h^2, 0), formed as density_trip forms it.
 __device__ __forceinline__ float split_term(const float4& pi, float h2, float x, float y, float z) {
