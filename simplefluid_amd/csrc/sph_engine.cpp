@@ -249,11 +249,15 @@ int alloc_step_bufs(sph_handle* h, StepBufs& w) {
     chk(w.id_s.ensure(n));
     chk(w.skey.ensure(n));
     chk(w.perm.ensure(n));
+    // A table that is new or held another grid's cells: every tile is
+    // rewritten at the next sort.
+    const uint32_t T = scan_tiles(h->ncells);
+    const bool stale = w.cstart.count < (size_t)h->ncells + 1 || w.tile_pre.count < T || w.tile_cells != h->ncells;
+    w.tile_cells = 0;
     chk(w.cstart.ensure((size_t)h->ncells + 1));
-    // The table's contents are for another grid (or none) now: every tile
-    // is rewritten at the next scan.
-    chk(w.tile_pre.ensure(scan_tiles(h->ncells)));
-    if (e == hipSuccess) chk(launch_fill_u32(h->stream, w.tile_pre.p, 0xffffffffu, scan_tiles(h->ncells)));
+    chk(w.tile_pre.ensure(T));
+    if (e == hipSuccess && stale) chk(launch_fill_u32(h->stream, w.tile_pre.p, 0xffffffffu, T));
+    if (e == hipSuccess) w.tile_cells = h->ncells;
     if (h->tune.sort_mode == kSortRadix)
         for (int i = 0; i < 2; ++i) { chk(w.kbuf[i].ensure(n)); chk(w.vbuf[i].ensure(n)); }
     else

@@ -91,6 +91,7 @@ struct StepBufs {
     DevBuf<uint32_t> skey, perm;   // sorted keys, sorted index -> state index
     DevBuf<uint32_t> cstart;       // C + 1 lower-bound cell-start table
     DevBuf<uint32_t> tile_pre;     // per tile of cstart: prefix held by an empty tile, or ~0u
+    uint32_t tile_cells = 0;       // cells of the grid tile_pre describes cstart for
     DevBuf<uint32_t> kbuf[2], vbuf[2];  // radix ping-pong (radix mode only)
     DevBuf<float> rho;
     DevBuf<uint32_t> mask;

@@ -152,6 +152,9 @@ hipError_t launch_unpermute3(hipStream_t st, uint32_t n, const float4* src, cons
 hipError_t launch_copy_out(hipStream_t st, const uint32_t* src, size_t words, const uint32_t* flag, uint32_t* dst);
 hipError_t launch_unpermute1(hipStream_t st, uint32_t n, const float* src, const uint32_t* id,
                              float* out);
+// Copies a state: n positions, velocities and ids.
+hipError_t launch_copy_state(hipStream_t st, uint32_t n, float4* dp, float4* dv, uint32_t* di, const float4* sp,
+                             const float4* sv, const uint32_t* si);
 // dst[k] = (src[3k], src[3k+1], src[3k+2], 0), or zero when src is null.
 hipError_t launch_pack3(hipStream_t st, uint32_t n, const float* src, float4* dst);
 

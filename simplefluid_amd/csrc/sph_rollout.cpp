@@ -15,11 +15,7 @@ namespace {
 
 hipError_t copy_state(sph_handle* h, float4* dp, float4* dv, uint32_t* di, const float4* sp, const float4* sv,
                       const uint32_t* si) {
-    const size_t n = h->n;
-    hipError_t e = hipMemcpyAsync(dp, sp, n * sizeof(float4), hipMemcpyDeviceToDevice, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dv, sv, n * sizeof(float4), hipMemcpyDeviceToDevice, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(di, si, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, h->stream);
-    return e;
+    return launch_copy_state(h->stream, h->n, dp, dv, di, sp, sv, si);
 }
 
 hipError_t save_checkpoint(sph_handle* h, RolloutState& R, uint32_t slot) {
