@@ -356,6 +356,41 @@ __device__ __forceinline__ double2 adj_force_one_staged(const AdjArgs& a, const 
     return active ? adj_force_finish(a, sc, k, vi, abi, c) : make_double2(0.0, 0.0);
 }
 
+// Adds the terms of a tile of blockDim.x particles to its running sums, in
+// the order of a tree over the lanes (halves of the tile first): its halves
+// above a wave by wave 0, the wave by shuffles.  One barrier, where the tree
+// in LDS had nine (the second one only for a block with another tile to go).
+__device__ __forceinline__ void add_wave_terms(double2* __restrict__ acc, double x, double y) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        x += __shfl_down(x, o, 64);
+        y += __shfl_down(y, o, 64);
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        double2 sum = *acc;
+        sum.x += x;
+        sum.y += y;
+        *acc = sum;
+    }
+}
+__device__ __forceinline__ void add_tile_terms(const AdjArgs& a, uint32_t t, double2 part, double2* red) {
+    red[threadIdx.x] = part;
+    __syncthreads();
+    if (threadIdx.x < 64u) {
+        double x = part.x, y = part.y;
+        const uint32_t i = threadIdx.x;
+        if (blockDim.x == 256u) {
+            x = (x + red[i + 128u].x) + (red[i + 64u].x + red[i + 192u].x);
+            y = (y + red[i + 128u].y) + (red[i + 64u].y + red[i + 192u].y);
+        } else if (blockDim.x == 128u) {
+            x += red[i + 64u].x;
+            y += red[i + 64u].y;
+        }
+        add_wave_terms(a.tile_acc + t, x, y);
+    }
+    __syncthreads();
+}
+
 // Eight waves per SIMD (64 VGPRs, a 36-byte spill): the backward pass was
 // 3 % faster than without the bound (47.0 against 48.3 ms, 16 x 32k
 // particles x 200 steps, with the walls' reverse still in this kernel).
@@ -371,22 +406,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
         const uint32_t k = ti.y + threadIdx.x;
         double2 part = make_double2(0.0, 0.0);
         if (k < sc.p_end) part = adj_force_one(a, sc, k);
-        red[threadIdx.x] = part;
-        __syncthreads();
-        for (uint32_t o = blockDim.x >> 1; o > 0; o >>= 1) {
-            if (threadIdx.x < o) {
-                red[threadIdx.x].x += red[threadIdx.x + o].x;
-                red[threadIdx.x].y += red[threadIdx.x + o].y;
-            }
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-            double2 acc = a.tile_acc[t];
-            acc.x += red[0].x;
-            acc.y += red[0].y;
-            a.tile_acc[t] = acc;
-        }
-        __syncthreads();
+        add_tile_terms(a, t, part, red);
     }
 }
 
@@ -403,22 +423,7 @@ __global__ __launch_bounds__(256) void adj_force_staged_kernel(AdjArgs a) {
         const uint32_t k = ti.y + threadIdx.x;
         const bool active = k < sc.p_end;
         const double2 part = adj_force_one_staged(a, sc, k, active, active ? k : ti.y, slot);
-        red[threadIdx.x] = part;
-        __syncthreads();
-        for (uint32_t o = blockDim.x >> 1; o > 0; o >>= 1) {
-            if (threadIdx.x < o) {
-                red[threadIdx.x].x += red[threadIdx.x + o].x;
-                red[threadIdx.x].y += red[threadIdx.x + o].y;
-            }
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-            double2 acc = a.tile_acc[t];
-            acc.x += red[0].x;
-            acc.y += red[0].y;
-            a.tile_acc[t] = acc;
-        }
-        __syncthreads();
+        add_tile_terms(a, t, part, red);
     }
 }
 
@@ -787,7 +792,7 @@ __global__ __launch_bounds__(64 * kAdjDensityWaves) void adj_density_split_kerne
     if (w == 0 && active) mv = adj_move(a, k);
     if (w == 3 && ((ti.y - sc.p_begin) & 255u) == 0u) {
         // The step's terms of 256 particles into their tile's running sums,
-        // added in adj_force_kernel's tree.
+        // added in add_tile_terms' order.
         double2 p[4];
 #pragma unroll
         for (uint32_t i = 0; i < 4u; ++i) {
@@ -795,18 +800,7 @@ __global__ __launch_bounds__(64 * kAdjDensityWaves) void adj_density_split_kerne
             if (k + 64u * i < sc.p_end) p[i] = a.part[k + 64u * i];
         }
         double x = (p[0].x + p[2].x) + (p[1].x + p[3].x), y = (p[0].y + p[2].y) + (p[1].y + p[3].y);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            x += __shfl_down(x, o, 64);
-            y += __shfl_down(y, o, 64);
-        }
-        if (lane == 0u) {
-            const uint32_t t = a.tile_first[ti.x] + ((ti.y - sc.p_begin) >> 8);
-            double2 acc = a.tile_acc[t];
-            acc.x += x;
-            acc.y += y;
-            a.tile_acc[t] = acc;
-        }
+        add_wave_terms(a.tile_acc + (a.tile_first[ti.x] + ((ti.y - sc.p_begin) >> 8)), x, y);
     }
     if (__ballot(count > kListMax) != 0u) {  // the same in every wave
         if (w == 0 && active) {
@@ -923,9 +917,8 @@ hipError_t launch_adj_integrate(hipStream_t st, int block, uint32_t grid, const 
 
 hipError_t launch_adj_force(hipStream_t st, int block, uint32_t grid, const AdjArgs& a, int staged) {
     if (grid == 0) return hipSuccess;
-    // __launch_bounds__(256), and the per-tile tree wants a power of two;
-    // the staged form also wants whole waves.
-    if (block > 256 || (block & (block - 1)) || (staged && block < 64)) return hipErrorInvalidValue;
+    // __launch_bounds__(256), and whole waves whose terms add_tile_terms adds.
+    if (block != 64 && block != 128 && block != 256) return hipErrorInvalidValue;
     if (staged)
         hipLaunchKernelGGL(adj_force_staged_kernel, dim3(grid), dim3(block), 0, st, a);
     else
