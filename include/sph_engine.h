@@ -236,7 +236,8 @@ int  sph_autotune(sph_handle* h);
  * candidates in LDS (clear: it gathers them from global memory), bit 2 the
  * same for the density pass.  A handle of at most 40,960 particles (640 tiles
  * of 64, scene by scene) runs density and force in a form of its own that
- * none of these shape, until sph_set_tuning asks for the forms above.  Every
+ * none of these shape, until sph_set_tuning asks for the forms above; one of
+ * 131,072 particles or more stages both until it is tuned or set.  Every
  * choice gives the same results bit for bit.                                */
 int  sph_get_tuning(const sph_handle* h, int* cfg5);
 int  sph_set_tuning(sph_handle* h, const int* cfg5);

@@ -96,7 +96,9 @@ extern "C" int sph_autotune(sph_handle* h) {
 
     const int blocks[] = {64, 128, 256, 512};
     const int items[] = {4, 8, 12, 16};
+    const Tuning before = h->tune;
     Tuning best = h->tune;
+    best.by_size = 0;
     double ms[SPH_NUM_PASSES];
     int rc = SPH_OK;
     // Density and force blocks, then reorder block, then sort items.
@@ -152,7 +154,7 @@ extern "C" int sph_autotune(sph_handle* h) {
         }
         best.density_staged = best_v;
     }
-    h->tune = best;
+    h->tune = rc == SPH_OK ? best : before;
     h->prof = prof_was;
     const hipError_t re = restore();
     invalidate_graph(h);

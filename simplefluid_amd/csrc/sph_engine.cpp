@@ -386,7 +386,7 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     sp.id_in = h->id.p;
     sp.pos_out = w.pos_s.p;
     const bool split = split_form(h);
-    sp.soa_out = h->tune.density_staged || split ? nullptr : w.soa.p;
+    sp.soa_out = density_staged(h) || split ? nullptr : w.soa.p;
     sp.frame = frame;
     sp.vel_out = w.vel_s.p;
     sp.id_out = w.id_s.p;
@@ -405,7 +405,7 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
         StepArgs a = step_args(h, w, h->tune.density_block);
         a.frame = frame;
         const uint32_t grid = grid_for(h, h->tune.density_block, a.ntiles, &a.queue);
-        e = launch_density(st, h->tune.density_block, grid, a, h->tune.density_staged);
+        e = launch_density(st, h->tune.density_block, grid, a, density_staged(h));
         if (e != hipSuccess) return hip_fail(h, e, "density launch");
     }
     if (record_prof) prof_record(h, 4);
@@ -418,8 +418,8 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
         StepArgs a = step_args(h, w, h->tune.force_block);
         a.frame = frame;
         const uint32_t grid = grid_for(h, h->tune.force_block, a.ntiles, &a.queue,
-                                       force_blocks_per_cu(h->tune.force_block, h->tune.force_staged));
-        e = launch_force(st, h->tune.force_block, grid, a, h->tune.force_staged);
+                                       force_blocks_per_cu(h->tune.force_block, force_staged(h)));
+        e = launch_force(st, h->tune.force_block, grid, a, force_staged(h));
         if (e != hipSuccess) return hip_fail(h, e, "force launch");
     }
     if (record_prof) {
@@ -806,7 +806,7 @@ static int capture_graph(sph_handle* h, GraphKind kind = kGraphOne) {
         uint32_t nt = 0;
         if (!tiles_for(h, b, nt)) return fail(h, SPH_E_OOM, "tile table");
     }
-    (void)force_blocks_per_cu(h->tune.force_block, h->tune.force_staged);  // runtime query, outside capture
+    (void)force_blocks_per_cu(h->tune.force_block, force_staged(h));  // runtime query, outside capture
     hipError_t e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(h, e, "begin capture");
     int rc = SPH_OK;
@@ -1231,6 +1231,7 @@ int sph_set_tuning(sph_handle* h, const int* cfg) {
     h->tune.persistent = cfg[4] & 1;
     h->tune.force_staged = (cfg[4] >> 1) & 1;
     h->tune.density_staged = (cfg[4] >> 2) & 1;
+    h->tune.by_size = 0;
     h->tune.split = 0;
     invalidate_graph(h);
     return SPH_OK;

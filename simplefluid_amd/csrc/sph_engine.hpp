@@ -106,6 +106,8 @@ struct Tuning {
     int persistent = 0;   // density and force: 0 one block per tile, 1 persistent blocks over tile queues
     int force_staged = 0; // force: 1 each row's candidates staged in LDS, 0 gathered from global memory
     int density_staged = 0;  // density: the same choice
+    int by_size = 1;      // 1 force and density are staged by the handle's size (staged_form), 0 as the two fields
+                          // above say (sph_set_tuning, sph_autotune)
     int split = 1;        // density and force: 1 the split form where it applies (split_form), 0 the forms above
                           // (sph_set_tuning)
     int sort_mode = kSortCellCount;
@@ -240,6 +242,20 @@ uint32_t grid_for(sph_handle* h, int block, uint32_t ntiles, uint32_t** queue, i
 // Density and force run in the split form: few enough tiles, its lists
 // allocated, and no other form asked for (sph_set_tuning).
 bool split_form(const sph_handle* h);
+// Particles from which a handle no one has tuned stages density and force.
+// Below, a wave's copies and bounds cost more than its gathers, whose records
+// are in cache.  Measured per step, gathered against staged, fresh and after
+// 2,500 steps: 47k 43.0 / 49.1 against 45.3 / 49.6 us, 104k 53.0 / 55.7
+// against 52.6 / 53.9, 50 scenes of 2.4k 69.0 / 73.9 against 71.4 / 78.4, 176k
+// 64.5 / 74.6 against 62.2 / 69.7, 40 scenes of 25k 236.7 / 302.0 against
+// 186.7 / 238.0, 1M 216.8 / 322.8 against 167.0 / 233.2.
+constexpr uint32_t kStagedFrom = 1u << 17;
+inline int force_staged(const sph_handle* h) {
+    return h->tune.by_size ? h->n >= kStagedFrom : h->tune.force_staged;
+}
+inline int density_staged(const sph_handle* h) {
+    return h->tune.by_size ? h->n >= kStagedFrom : h->tune.density_staged;
+}
 StepArgs step_args(sph_handle* h, StepBufs& w, int block);
 // Enqueue one step reading/writing the state buffers with intermediates in w.
 // frame: device frame state (every kernel of the step skips once it is

@@ -186,8 +186,8 @@ int sph_rollout_backward(sph_handle* h, const float* dL_dx_final, float* dL_dB, 
                 chk(launch_adj_force_split(st, a));
                 chk(launch_adj_density_split(st, a));
             } else {
-                chk(launch_adj_force(st, 256, grid, a, h->tune.force_staged));
-                chk(launch_adj_density(st, 256, grid, a, h->tune.force_staged));
+                chk(launch_adj_force(st, 256, grid, a, force_staged(h)));
+                chk(launch_adj_density(st, 256, grid, a, force_staged(h)));
             }
             swap();
             if (e != hipSuccess) return hip_fail(h, e, "adjoint launch");
