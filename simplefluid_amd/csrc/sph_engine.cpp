@@ -468,6 +468,26 @@ int check_device_error(sph_handle* h) {
     return report_device_error(h, flag);
 }
 
+// Waits for a kernel that wrote `words` words and the error flag to the
+// page-locked buffer; e: its launch's result.
+static int wait_words(sph_handle* h, size_t words, hipError_t e) {
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return hip_fail(h, e, "download");
+    uint32_t flag;
+    std::memcpy(&flag, h->host_pinned + words, sizeof(flag));
+    return report_device_error(h, flag);
+}
+
+// A few particles' values in original order, in one launch.
+static int read_small(sph_handle* h, const float4* src4, const float* src1, float* out) {
+    const size_t words = (size_t)h->n * (src4 ? 3 : 1);
+    int rc = host_words(h, words);
+    if (rc != SPH_OK) return rc;
+    rc = wait_words(h, words, launch_read_small(h->stream, h->n, src4, src1, h->id.p, h->err.p, h->host_pinned));
+    if (rc == SPH_OK) std::memcpy(out, h->host_pinned, words * sizeof(float));
+    return rc;
+}
+
 // Copies `words` words of device memory to the page-locked buffer, the error
 // flag behind them, waits, and hands them to use(first, count) in pieces, on
 // this thread or on helpers.  One launch and one wait where the data is
@@ -483,13 +503,9 @@ static int download(sph_handle* h, const void* src, size_t words, Use&& use) {
     if (rc != SPH_OK) return rc;
     constexpr size_t kSmall = (size_t)1 << 19;  // words: 2 MB
     if (words <= kSmall) {
-        hipError_t e = launch_copy_out(h->stream, static_cast<const uint32_t*>(src), words, h->err.p,
-                                       reinterpret_cast<uint32_t*>(h->host_pinned));
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-        if (e != hipSuccess) return hip_fail(h, e, "download");
-        uint32_t flag;
-        std::memcpy(&flag, h->host_pinned + words, sizeof(flag));
-        rc = report_device_error(h, flag);
+        const hipError_t e = launch_copy_out(h->stream, static_cast<const uint32_t*>(src), words, h->err.p,
+                                             reinterpret_cast<uint32_t*>(h->host_pinned));
+        rc = wait_words(h, words, e);
         if (rc == SPH_OK) use((size_t)0, words);
         return rc;
     }
@@ -980,6 +996,7 @@ static int fetch3(sph_handle* h, const float4* src, float* out) {
     if (!h || !out) return SPH_E_INVALID;
     if (!h->has_particles) return fail(h, SPH_E_NOT_READY, "no particles set");
     if (h->n == 0) return SPH_OK;
+    if (h->n <= kReadSmall) return read_small(h, src, nullptr, out);
     const hipError_t e = launch_unpermute3(h->stream, h->n, src, h->id.p, h->staging.p);
     if (e != hipSuccess) return hip_fail(h, e, "particle download");
     return download(h, h->staging.p, 3 * (size_t)h->n,
@@ -1000,6 +1017,7 @@ int sph_get_density(sph_handle* h, float* rho_out) {
     if (!h || !rho_out) return SPH_E_INVALID;
     if (!h->has_step) return fail(h, SPH_E_NOT_READY, "no step has run");
     // Density is in the last step's sorted order, which is the state order.
+    if (h->n && h->n <= kReadSmall) return read_small(h, nullptr, h->work.rho.p, rho_out);
     hipError_t e = launch_unpermute1(h->stream, h->n, h->work.rho.p, h->id.p, h->staging.p);
     if (e != hipSuccess) return hip_fail(h, e, "density download");
     return download(h, h->staging.p, h->n,

@@ -150,6 +150,13 @@ hipError_t launch_unpermute3(hipStream_t st, uint32_t n, const float4* src, cons
 // Copies words of device memory and, behind them, *flag to dst (page-locked
 // host memory).
 hipError_t launch_copy_out(hipStream_t st, const uint32_t* src, size_t words, const uint32_t* flag, uint32_t* dst);
+// x, y, z of src4, or src1 where that is null, in original order, then *flag, to
+// dst (page-locked host memory), for at most kReadSmall particles: one block,
+// which puts them in order in LDS (40 KB, and from there on one CU's writes
+// over the bus take longer than the launch they save).
+constexpr uint32_t kReadSmall = 3400;
+hipError_t launch_read_small(hipStream_t st, uint32_t n, const float4* src4, const float* src1, const uint32_t* id,
+                             const uint32_t* flag, float* dst);
 hipError_t launch_unpermute1(hipStream_t st, uint32_t n, const float* src, const uint32_t* id,
                              float* out);
 // Copies a state: n positions, velocities and ids.

@@ -1281,6 +1281,29 @@ __global__ void copy_out_kernel(const uint32_t* __restrict__ src, size_t words, 
     if (i == 0) dst[words] = *flag;
 }
 
+__global__ __launch_bounds__(1024) void read_small_kernel(uint32_t n, const float4* __restrict__ src4,
+                                                          const float* __restrict__ src1,
+                                                          const uint32_t* __restrict__ id,
+                                                          const uint32_t* __restrict__ flag, float* __restrict__ dst) {
+    __shared__ float s[3 * kReadSmall];
+    for (uint32_t k = threadIdx.x; k < n; k += 1024u) {
+        const uint32_t i = id[k];
+        if (i >= n) continue;
+        if (src4) {
+            const float4 v = src4[k];
+            s[3u * i] = v.x;
+            s[3u * i + 1u] = v.y;
+            s[3u * i + 2u] = v.z;
+        } else {
+            s[i] = src1[k];
+        }
+    }
+    __syncthreads();
+    const uint32_t words = src4 ? 3u * n : n;
+    for (uint32_t i = threadIdx.x; i < words; i += 1024u) dst[i] = s[i];
+    if (threadIdx.x == 0) reinterpret_cast<uint32_t*>(dst)[words] = *flag;
+}
+
 __global__ void unpermute1_kernel(uint32_t n, const float* __restrict__ src,
                                   const uint32_t* __restrict__ id, float* __restrict__ out) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1431,6 +1454,13 @@ hipError_t launch_unpermute3(hipStream_t st, uint32_t n, const float4* src, cons
 hipError_t launch_copy_out(hipStream_t st, const uint32_t* src, size_t words, const uint32_t* flag, uint32_t* dst) {
     const size_t lanes = words / 4 > 64 ? words / 4 : 64;
     hipLaunchKernelGGL(copy_out_kernel, dim3(blocks_for(lanes, 256)), dim3(256), 0, st, src, words, flag, dst);
+    return hipGetLastError();
+}
+
+hipError_t launch_read_small(hipStream_t st, uint32_t n, const float4* src4, const float* src1, const uint32_t* id,
+                             const uint32_t* flag, float* dst) {
+    if (n == 0 || n > kReadSmall) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(read_small_kernel, dim3(1), dim3(1024), 0, st, n, src4, src1, id, flag, dst);
     return hipGetLastError();
 }
 

@@ -10,6 +10,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+READ = 3400  # particles whose order one block restores
 SMALL = (1 << 19) // 3  # particles whose 3n words are the most one piece takes
 
 
@@ -24,7 +25,7 @@ def upload(n, seed):
     return e, x, v
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 85, SMALL, SMALL + 1, 700_001, 3_000_000])
+@pytest.mark.parametrize("n", [1, 2, 3, 85, READ, READ + 1, SMALL, SMALL + 1, 700_001, 3_000_000])
 def test_downloads_return_what_was_uploaded(n):
     e, x, v = upload(n, n)
     for _ in range(2):
