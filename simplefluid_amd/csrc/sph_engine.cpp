@@ -163,9 +163,9 @@ void give_back_spares(MemBudget& b) {
     b.spares = nullptr;
     (void)hipStreamSynchronize(h->stream);
     invalidate_graph(h);
-    h->mask_hi.release();
-    h->nlist.release();
-    h->ncount.release();
+    h->spare.release();
+    h->mask_hi = h->ncount = nullptr;
+    h->nlist = nullptr;
 }
 
 uint2* tiles_for(sph_handle* h, int block, uint32_t& ntiles) {
@@ -204,7 +204,7 @@ uint32_t grid_for(sph_handle* h, int block, uint32_t ntiles, uint32_t** queue, i
 }
 
 bool split_form(const sph_handle* h) {
-    return h->tune.split && h->split_tiles <= kSplitTiles && h->nlist.p && h->ncount.p;
+    return h->tune.split && h->split_tiles <= kSplitTiles && h->nlist;
 }
 
 StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
@@ -223,9 +223,9 @@ StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     a.cstart = w.cstart.p;
     a.rho = w.rho.p;
     a.mask = w.mask.p;
-    a.mask_hi = h->mask_hi.p;
-    a.nlist = h->nlist.p;
-    a.ncount = h->ncount.p;
+    a.mask_hi = h->mask_hi;
+    a.nlist = h->nlist;
+    a.ncount = h->ncount;
     a.acc = (h->keep_acc || w.acc.p) ? w.acc.p : nullptr;
     a.scenes = h->sc_d.p;
     if (h->cfl) {
@@ -303,16 +303,23 @@ static int ensure_buffers(sph_handle* h) {
     // These only speed the step up: a handle with no room for them does
     // without, and they are given back when another buffer needs the room.
     h->mem.spares = nullptr;
-    if (h->mask_hi.ensure((size_t)kRows * n) != hipSuccess) {
+    h->mask_hi = h->ncount = nullptr;
+    h->nlist = nullptr;
+    static_assert(kListMax % 2 == 0, "lists of whole words");
+    const size_t list_words = h->split_tiles <= kSplitTiles ? (kListMax / 2 + 1) * n : 0;
+    for (const size_t words : {list_words, (size_t)0}) {  // without the lists where only the masks fit
+        if (h->spare.ensure(words + (size_t)kRows * n) == hipSuccess) {
+            if (words) {
+                h->nlist = reinterpret_cast<uint16_t*>(h->spare.p);
+                h->ncount = h->spare.p + (kListMax / 2) * n;
+            }
+            h->mask_hi = h->spare.p ? h->spare.p + words : nullptr;
+            h->mem.spares = h->spare.p ? h : nullptr;
+            break;
+        }
         h->mem.refused = 0;
         (void)hipGetLastError();
     }
-    if (h->split_tiles <= kSplitTiles && (h->nlist.ensure((size_t)kListMax * n) != hipSuccess || h->ncount.ensure(n) != hipSuccess)) {
-        h->nlist.release();
-        h->mem.refused = 0;
-        (void)hipGetLastError();
-    }
-    if (h->mask_hi.p || h->nlist.p) h->mem.spares = h;
     return SPH_OK;
 }
 

@@ -166,9 +166,10 @@ struct sph_handle {
     // State (state order) and per-step buffers.
     sph::DevBuf<float4> pos, vel;
     sph::DevBuf<uint32_t> id, key0, next, head;
-    sph::DevBuf<uint16_t> nlist;           // spares: the split form's neighbour lists and
-    sph::DevBuf<uint32_t> ncount;          // their lengths,
-    sph::DevBuf<uint32_t> mask_hi;         // second mask words
+    sph::DevBuf<uint32_t> spare;           // spares, in one allocation (each costs a new handle 30 us):
+    uint16_t* nlist = nullptr;             // the split form's neighbour lists and
+    uint32_t* ncount = nullptr;            // their lengths,
+    uint32_t* mask_hi = nullptr;           // second mask words
     sph::DevBuf<uint32_t> tmp;             // cell-count sort: members of the tiles too full for LDS
     sph::StepBufs work;
     sph::DevBuf<uint32_t> hist, status, tickets, err, queue;

@@ -177,8 +177,8 @@ int sph_rollout_backward(sph_handle* h, const float* dL_dx_final, float* dL_dB, 
             if (split_form(h)) {
                 a.tiles = split_tiles;
                 a.ntiles = n_split;
-                a.nlist = h->nlist.p;
-                a.ncount = h->ncount.p;
+                a.nlist = h->nlist;
+                a.ncount = h->ncount;
                 a.tile_first = R.tile_first.p;
                 // This step's acceleration has been used: its room holds the
                 // particles' parameter terms.
