@@ -124,19 +124,28 @@ extern "C" int sph_autotune(sph_handle* h) {
         *ax.field = best_v;
         if (rc != SPH_OK) break;
     }
+    // Staged or gathered: the form of the handle's size unless the other is
+    // 5 % faster.  The trials are a few steps from the state as it is, often a
+    // fresh one, whose forms can lie within the trials' noise of each other
+    // while compression and the reverse pass, which takes the force pass's
+    // form, favour the size's: 16 scenes of 32,768 particles reverse 200 steps
+    // in 36.0 ms staged and in 41.9 where a trial preferred the gathered force.
+    const int of_size = n >= kStagedFrom ? 1 : 0;
+    auto beats = [&](double t, double best_ms, int staged) { return t < (staged == of_size ? 1.0 : 0.95) * best_ms; };
     // Launch form of density and force (persistent or one block per tile;
     // force rows staged in LDS or gathered), judged on their summed time.
     if (rc == SPH_OK) {
         double best_ms = 1e30;
-        int best_v = 0;
-        for (int c = 0; c < 4; ++c) {
+        int best_v = of_size << 1;
+        for (int i = 0; i < 4; ++i) {
+            const int c = i ^ (of_size << 1);  // the form of the size first
             best.persistent = c & 1;
             best.force_staged = c >> 1;
             h->tune = best;
             rc = trial(ms);
             if (rc != SPH_OK) break;
             const double t = ms[SPH_PASS_DENSITY] + ms[SPH_PASS_FORCE];
-            if (t < best_ms) { best_ms = t; best_v = c; }
+            if (beats(t, best_ms, c >> 1)) { best_ms = t; best_v = c; }
         }
         best.persistent = best_v & 1;
         best.force_staged = best_v >> 1;
@@ -144,13 +153,14 @@ extern "C" int sph_autotune(sph_handle* h) {
     // Density rows staged in LDS or read from global memory.
     if (rc == SPH_OK) {
         double best_ms = 1e30;
-        int best_v = 0;
-        for (int c = 0; c < 2; ++c) {
+        int best_v = of_size;
+        for (int i = 0; i < 2; ++i) {
+            const int c = i ^ of_size;
             best.density_staged = c;
             h->tune = best;
             rc = trial(ms);
             if (rc != SPH_OK) break;
-            if (ms[SPH_PASS_DENSITY] < best_ms) { best_ms = ms[SPH_PASS_DENSITY]; best_v = c; }
+            if (beats(ms[SPH_PASS_DENSITY], best_ms, c)) { best_ms = ms[SPH_PASS_DENSITY]; best_v = c; }
         }
         best.density_staged = best_v;
     }
