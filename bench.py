@@ -2,7 +2,7 @@
 
 Default workload: the 1,048,576-particle double dam break (two jittered
 128x64x64 blocks, box [0,2]x[0,1]x[0,2], r 0.005, h 0.02, dt 1e-4), FP32.
-A step = counting sort of the cell keys (keys and per-cell counts come from
+A step = counting sort of the cell keys (keys and cell chains come from
 the previous step's force pass, so no hash pass runs per step), reorder + cell
 table, density + EOS, pressure/viscosity force + integrate + clamp.
 

@@ -106,7 +106,7 @@ struct Tuning {
     int persistent = 0;   // density and force: 0 one block per tile, 1 persistent blocks over tile queues
     int force_staged = 0; // force: 1 each row's candidates staged in LDS, 0 gathered from global memory
     int density_staged = 0;  // density: the same choice
-    int by_size = 1;      // 1 force and density are staged by the handle's size (staged_form), 0 as the two fields
+    int by_size = 1;      // 1 force and density are staged by the handle's size (kStagedFrom), 0 as the two fields
                           // above say (sph_set_tuning, sph_autotune)
     int split = 1;        // density and force: 1 the split form where it applies (split_form), 0 the forms above
                           // (sph_set_tuning)

@@ -1,5 +1,5 @@
 // Per-particle passes of one SPH step on gfx950:
-//   hash     cell key and per-cell count of every state position (first step
+//   hash     cell key and chain links of every state position (first step
 //            only; afterwards the integrate pass produces the next keys)
 //   density  rho, EOS, neighbour bit masks (candidate tests happen here once)
 //   force    pressure + viscosity from the masks, integrate, clamp, next key
