@@ -529,7 +529,10 @@ static int download(sph_handle* h, const void* src, size_t words, Use&& use) {
     // the flag behind it, where the next piece's words then go.
     const size_t marks = std::min(pieces, h->copy_events.size());
     auto mark_end = [&](size_t m) { return std::min(words, (m + 1) * pieces / marks * kPiece); };
-    hipError_t e = hipSuccess;
+    // The flag alone first: nothing is handed over where it is raised.
+    hipError_t e = launch_copy_out(h->stream, nullptr, 0, h->err.p, reinterpret_cast<uint32_t*>(h->host_pinned) + words);
+    int device = 0;
+    if (e == hipSuccess) e = hipGetDevice(&device);
     size_t at = 0;
     for (size_t m = 0; m < marks && e == hipSuccess; ++m) {
         const size_t end = m + 1 == marks ? words : mark_end(m);
@@ -544,11 +547,15 @@ static int download(sph_handle* h, const void* src, size_t words, Use&& use) {
     }
     std::atomic<int> bad{0};
     auto work = [&](size_t first) {
+        (void)hipSetDevice(device);  // a new thread starts on the first one
         for (size_t m = first; m < marks; m += kThreads) {
             if (hipEventSynchronize(h->copy_events[m]) != hipSuccess) {
                 bad.store(1);
                 return;
             }
+            uint32_t raised;
+            std::memcpy(&raised, h->host_pinned + words, sizeof(raised));
+            if (raised) return;
             const size_t beg = m ? mark_end(m - 1) : 0, end = m + 1 == marks ? words : mark_end(m);
             use(beg, end - beg);
         }

@@ -3,6 +3,7 @@ last 16 bytes, the last size that goes in one piece and the first that goes
 in several, and many pieces with a ragged last one.  What was uploaded comes
 back bit for bit, also while another handle's download runs on another
 thread."""
+import ctypes
 import threading
 
 import numpy as np
@@ -51,3 +52,19 @@ def test_downloads_on_two_threads():
     assert not bad
     for e, _, _ in held:
         e.close()
+
+
+@pytest.mark.parametrize("n", [READ, READ + 1, 300_000])
+def test_nothing_is_handed_over_where_the_error_flag_is_raised(n):
+    """1,200 particles in one cell, more than the cell-count sort ranks: the
+    read reports it and leaves the caller's array alone, on each path."""
+    from simplefluid_amd import engine as E
+    e, x, _ = upload(n, n)
+    x[:1200] = np.nan
+    e.set_particles(x)
+    e.make_ready()
+    e.advance_steps(1)
+    out = np.full((n, 3), 7.0, np.float32)
+    rc = e._L.sph_get_particles(e._h, out.ctypes.data_as(ctypes.c_void_p))
+    assert rc == E.SPH_E_DEVICE and (out == 7.0).all()
+    e.close()
