@@ -5,7 +5,8 @@
 // with HIP events on the handle's own state.  The state is saved first and
 // restored before every trial, so all candidates run the same steps.
 // Results are cached per process, keyed by device arch, particle-count
-// bucket (power of two) and scene count.  A handle small enough for the split
+// bucket (power of two), scene count, x subdivision and sort mode (which is
+// the handle's own: its buffers are allocated for it).  A handle small enough for the split
 // form runs that, which has no shape to choose.
 #include <algorithm>
 #include <cmath>
@@ -26,7 +27,7 @@ std::string cache_key(const sph_handle* h) {
     int bucket = 0;
     while ((1u << bucket) < h->n && bucket < 31) ++bucket;
     return h->arch + ":" + std::to_string(bucket) + ":" + std::to_string(h->sc_h.size()) + ":" +
-           std::to_string(h->xsub);
+           std::to_string(h->xsub) + ":" + std::to_string(h->tune.sort_mode);
 }
 
 struct Saved {
@@ -50,7 +51,9 @@ extern "C" int sph_autotune(sph_handle* h) {
         std::lock_guard<std::mutex> lk(g_mu);
         auto it = g_cache.find(key);
         if (it != g_cache.end()) {
+            const int mode = h->tune.sort_mode;
             h->tune = it->second;
+            h->tune.sort_mode = mode;
             invalidate_graph(h);
             return SPH_OK;
         }

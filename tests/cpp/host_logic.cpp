@@ -1,0 +1,208 @@
+// The engine's host code without a GPU: this program defines the HIP runtime
+// calls the library makes (its own definitions win over the runtime's), with
+// host memory for device memory and kernels that do nothing but are noted by
+// name.  Each check, named on the command line, drives the C ABI into a state
+// that is hard to reach on a GPU and looks at what the host code asked for.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "sph_engine.h"
+
+namespace fake {
+
+// Host stub -> kernel name.  The library registers its kernels before this
+// program's own objects are built.
+std::map<const void*, std::string>& kernels() {
+    static std::map<const void*, std::string> m;
+    return m;
+}
+std::vector<std::string> launched;
+std::set<void*> held;      // device allocations
+uint64_t frees = 0;        // device allocations given back so far
+bool capturing = false;
+std::map<void*, uint64_t> graphs;  // executable graph -> frees when it was captured
+uint64_t captured_at = 0;
+bool stale = false;        // a graph ran after a buffer it may name was given back
+uint64_t device_left = ~0ull;  // bytes hipMalloc still hands out
+std::map<void*, uint64_t> sizes;
+
+int count(const char* what) {
+    int n = 0;
+    for (const std::string& s : launched) n += s.find(what) != std::string::npos;
+    return n;
+}
+
+}  // namespace fake
+
+#define API extern "C" __attribute__((visibility("default")))
+
+API void** __hipRegisterFatBinary(const void*) { static void* m; return &m; }
+API void __hipUnregisterFatBinary(void**) {}
+API void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*,
+                               int*) {
+    fake::kernels()[host] = name;
+}
+API void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+API hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+API hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* st) {
+    *g = dim3(1);
+    *b = dim3(1);
+    *s = 0;
+    *st = nullptr;
+    return hipSuccess;
+}
+API hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t) {
+    fake::launched.push_back(fake::kernels()[f]);
+    return hipSuccess;
+}
+API hipError_t hipMalloc(void** p, size_t n) {
+    *p = nullptr;
+    if (n > fake::device_left) return hipErrorOutOfMemory;
+    fake::device_left -= n;
+    *p = std::calloc(1, n);
+    fake::held.insert(*p);
+    fake::sizes[*p] = n;
+    return hipSuccess;
+}
+API hipError_t hipFree(void* p) {
+    if (!p) return hipSuccess;
+    if (!fake::held.erase(p)) {
+        std::printf("hipFree of memory that is not held\n");
+        std::exit(3);
+    }
+    fake::device_left += fake::sizes[p];
+    ++fake::frees;
+    std::free(p);
+    return hipSuccess;
+}
+API hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = std::calloc(1, n); return hipSuccess; }
+API hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+API hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
+API hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+API hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { std::memset(d, v, n); return hipSuccess; }
+API hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+API hipError_t hipSetDevice(int) { return hipSuccess; }
+API hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
+    std::memset(p, 0, sizeof(*p));
+    p->multiProcessorCount = 256;
+    std::strcpy(p->gcnArchName, "gfx950");
+    return hipSuccess;
+}
+API const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
+API hipError_t hipGetLastError() { return hipSuccess; }
+API hipError_t hipGetSymbolAddress(void** p, const void* s) { *p = const_cast<void*>(s); return hipSuccess; }
+API hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) { *n = 4; return hipSuccess; }
+API hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+    *s = reinterpret_cast<hipStream_t>(std::malloc(1));
+    return hipSuccess;
+}
+API hipError_t hipStreamDestroy(hipStream_t s) { std::free(s); return hipSuccess; }
+API hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+API hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+API hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    *e = reinterpret_cast<hipEvent_t>(std::malloc(1));
+    return hipSuccess;
+}
+API hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+API hipError_t hipEventDestroy(hipEvent_t e) { std::free(e); return hipSuccess; }
+API hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+API hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+API hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0.005f; return hipSuccess; }
+API hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
+    fake::capturing = true;
+    fake::captured_at = fake::frees;
+    return hipSuccess;
+}
+API hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
+    fake::capturing = false;
+    *g = reinterpret_cast<hipGraph_t>(std::malloc(1));
+    return hipSuccess;
+}
+API hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+    *x = reinterpret_cast<hipGraphExec_t>(std::malloc(1));
+    fake::graphs[*x] = fake::captured_at;
+    return hipSuccess;
+}
+API hipError_t hipGraphExecDestroy(hipGraphExec_t x) {
+    fake::graphs.erase(x);
+    std::free(x);
+    return hipSuccess;
+}
+API hipError_t hipGraphDestroy(hipGraph_t g) { std::free(g); return hipSuccess; }
+API hipError_t hipGraphLaunch(hipGraphExec_t x, hipStream_t) {
+    fake::launched.push_back("graph");
+    fake::stale |= fake::graphs.at(x) != fake::frees;
+    return hipSuccess;
+}
+
+// ------------------------------------------------------------------ checks
+
+namespace {
+
+#define CHECK(c)                                                      \
+    do {                                                              \
+        if (!(c)) {                                                   \
+            std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);       \
+            return 1;                                                 \
+        }                                                             \
+    } while (0)
+
+sph_handle* make(uint32_t n, float h = 0.02f) {
+    sph_params p;
+    sph_params_default(&p);
+    p.kernel_radius = h;
+    p.particle_radius = h / 4;
+    sph_handle* e = nullptr;
+    if (sph_create(&p, &e) != SPH_OK) std::exit(4);
+    std::vector<float> x(3 * (size_t)n, 0.1f);
+    if (sph_set_particles(e, x.data(), nullptr, n) != SPH_OK || sph_make_ready(e) != SPH_OK) std::exit(5);
+    return e;
+}
+
+// A process's autotuned shapes are shared by handles of the same size bucket;
+// how a handle sorts is its own.
+int autotune_keeps_the_sort() {
+    for (int first : {SPH_SORT_RADIX, SPH_SORT_CELL_COUNT}) {
+        const uint32_t n = first == SPH_SORT_RADIX ? 50000u : 100000u;  // a bucket each
+        sph_handle* e[2] = {make(n), make(n)};
+        const int mode[2] = {first, first == SPH_SORT_RADIX ? SPH_SORT_CELL_COUNT : SPH_SORT_RADIX};
+        for (int i = 0; i < 2; ++i) {
+            CHECK(sph_set_sort_mode(e[i], mode[i]) == SPH_OK);
+            CHECK(sph_autotune(e[i]) == SPH_OK);
+            CHECK(sph_get_sort_mode(e[i]) == mode[i]);
+            fake::launched.clear();
+            CHECK(sph_set_use_graph(e[i], 0) == SPH_OK);
+            CHECK(sph_advance_steps(e[i], 1) == SPH_OK);
+            CHECK((fake::count("radix_pass") > 0) == (mode[i] == SPH_SORT_RADIX));
+        }
+        for (sph_handle* h : e) sph_destroy(h);
+    }
+    return 0;
+}
+
+struct Check {
+    const char* name;
+    int (*run)();
+};
+const Check kChecks[] = {
+    {"autotune_keeps_the_sort", autotune_keeps_the_sort},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    for (const Check& c : kChecks)
+        if (argc == 2 && std::strcmp(argv[1], c.name) == 0) return c.run();
+    std::printf("no such check\n");
+    return 2;
+}
