@@ -336,10 +336,11 @@ static void prof_record(sph_handle* h, int slot) {
 // New state: the chains start empty, then every particle is hashed.
 static int enqueue_hash(sph_handle* h) {
     hipStream_t st = h->stream;
-    hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells));
-    if (e == hipSuccess && h->cfl) e = launch_fill_u32(st, h->vmax2.p, 0u, kSpeedSlots);
     uint32_t nt = 0;
     const uint2* tl = tiles_for(h, 256, nt);
+    if (!tl) return fail(h, SPH_E_OOM, "tile table");
+    hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells));
+    if (e == hipSuccess && h->cfl) e = launch_fill_u32(st, h->vmax2.p, 0u, kSpeedSlots);
     if (e == hipSuccess)
         e = launch_hash(st, 256, nt, h->pos.p, h->vel.p, h->key0.p, h->next.p, h->head.p, h->ncells,
                         h->cfl ? h->vmax2.p : nullptr, h->sc_d.p, tl, nt);
@@ -1435,6 +1436,7 @@ int sph_debug_neighbors(sph_handle* h, uint32_t* offsets, uint32_t* list, uint64
     DevBuf<uint32_t> cnt, off, lst;
     if (cnt.ensure(n + 1) != hipSuccess || off.ensure(n + 1) != hipSuccess) return fail(h, SPH_E_OOM, "neighbour buffers");
     StepArgs a = step_args(h, h->work, 256);
+    if (!a.tiles) return fail(h, SPH_E_OOM, "tile table");
     hipError_t e = launch_neighbors(h->stream, 256, a.ntiles, a, nullptr, cnt.p, 0);
     std::vector<uint32_t> c(n);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);

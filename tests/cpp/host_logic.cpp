@@ -190,12 +190,50 @@ int autotune_keeps_the_sort() {
     return 0;
 }
 
+// A step whose tables do not fit fails, and with room for them the next one
+// hashes the state as if that one had not been asked for.
+int hash_without_its_table_fails() {
+    const uint32_t n = 5000;
+    const uint64_t spares = n * (9ull * 4 + 128 * 2 + 4);
+    sph_handle* full = make(n);
+    uint64_t used = 0;
+    CHECK(sph_device_memory_used(full, &used) == SPH_OK);
+    sph_destroy(full);
+    for (int frame = 0; frame < 2; ++frame) {
+        sph_params p;
+        sph_params_default(&p);
+        p.kernel_radius = 0.02f;
+        p.particle_radius = 0.005f;
+        p.cfl_number = frame ? 0.3f : 0.0f;
+        sph_handle* e = nullptr;
+        CHECK(sph_create(&p, &e) == SPH_OK);
+        CHECK(sph_set_device_memory_limit(e, used - spares) == SPH_OK);
+        std::vector<float> x(3 * n, 0.1f);
+        CHECK(sph_set_particles(e, x.data(), nullptr, n) == SPH_OK && sph_make_ready(e) == SPH_OK);
+        const int cfg[5] = {64, 64, 256, 8, 0};
+        CHECK(sph_set_tuning(e, cfg) == SPH_OK);
+        // Room for the table of 64-particle tiles, not for the hash's of 256.
+        CHECK(sph_set_device_memory_limit(e, used - spares + (n + 63) / 64 * 8) == SPH_OK);
+        fake::launched.clear();
+        const int rc = frame ? sph_run_frame(e, nullptr, nullptr) : sph_advance_steps(e, 1);
+        CHECK(rc == SPH_E_OOM);
+        CHECK(fake::count("force") == 0 && fake::count("graph") == 0);
+        CHECK(sph_set_device_memory_limit(e, 0) == SPH_OK);
+        fake::launched.clear();
+        CHECK(sph_advance_steps(e, 1) == SPH_OK);
+        CHECK(fake::count("hash_kernel") == 1 && fake::count("force") == 1);
+        sph_destroy(e);
+    }
+    return 0;
+}
+
 struct Check {
     const char* name;
     int (*run)();
 };
 const Check kChecks[] = {
     {"autotune_keeps_the_sort", autotune_keeps_the_sort},
+    {"hash_without_its_table_fails", hash_without_its_table_fails},
 };
 
 }  // namespace
