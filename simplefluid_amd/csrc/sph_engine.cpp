@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <thread>
+#include <utility>
 
 using namespace sph;
 
@@ -302,6 +303,7 @@ static int ensure_buffers(sph_handle* h) {
     if (rc != SPH_OK) return rc;
     // These only speed the step up: a handle with no room for them does
     // without, and they are given back when another buffer needs the room.
+    const auto before = std::make_pair(h->nlist, h->mask_hi);
     h->mem.spares = nullptr;
     h->mask_hi = h->ncount = nullptr;
     h->nlist = nullptr;
@@ -320,6 +322,8 @@ static int ensure_buffers(sph_handle* h) {
         h->mem.refused = 0;
         (void)hipGetLastError();
     }
+    // Others than before (there was no room, or there is now): the graphs name those.
+    if (before != std::make_pair(h->nlist, h->mask_hi)) invalidate_graph(h);
     return SPH_OK;
 }
 

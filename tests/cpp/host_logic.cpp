@@ -228,6 +228,39 @@ int hash_without_its_table_fails() {
     return 0;
 }
 
+// Making a handle ready again when there is more room gives it the neighbour
+// lists it did without: no graph that names the buffers before runs on.
+int new_spares_drop_the_graphs() {
+    const uint32_t n = 5000;
+    const uint64_t lists = n * (128ull * 2 + 4);
+    sph_handle* full = make(n);
+    uint64_t used = 0;
+    CHECK(sph_device_memory_used(full, &used) == SPH_OK);
+    sph_destroy(full);
+    sph_params p;
+    sph_params_default(&p);
+    p.kernel_radius = 0.02f;
+    p.particle_radius = 0.005f;
+    sph_handle* e = nullptr;
+    CHECK(sph_create(&p, &e) == SPH_OK);
+    CHECK(sph_set_device_memory_limit(e, used - lists) == SPH_OK);
+    std::vector<float> x(3 * n, 0.1f);
+    CHECK(sph_set_particles(e, x.data(), nullptr, n) == SPH_OK && sph_make_ready(e) == SPH_OK);
+    CHECK(sph_set_device_memory_limit(e, used) == SPH_OK);  // the tile tables
+    fake::launched.clear();
+    CHECK(sph_advance_steps(e, 2) == SPH_OK);  // the second one's is a graph
+    CHECK(fake::count("split") == 0 && fake::count("graph") == 1);
+    CHECK(sph_set_device_memory_limit(e, 0) == SPH_OK);
+    CHECK(sph_make_ready(e) == SPH_OK);
+    fake::launched.clear();
+    fake::stale = false;
+    CHECK(sph_advance_steps(e, 1) == SPH_OK);
+    CHECK(fake::count("graph") == 1 && !fake::stale);
+    CHECK(fake::count("force_split") == 1);  // captured anew, with the lists
+    sph_destroy(e);
+    return 0;
+}
+
 struct Check {
     const char* name;
     int (*run)();
@@ -235,6 +268,7 @@ struct Check {
 const Check kChecks[] = {
     {"autotune_keeps_the_sort", autotune_keeps_the_sort},
     {"hash_without_its_table_fails", hash_without_its_table_fails},
+    {"new_spares_drop_the_graphs", new_spares_drop_the_graphs},
 };
 
 }  // namespace
