@@ -397,12 +397,27 @@ __device__ __forceinline__ uint32_t cell_key(const SceneConst& sc, float x, floa
 // tiles of 512, 9.2 with 256; DoubleDambreak at resolution 24, 55k cells:
 // frame 8.06 ms, 7.76 with 256).  Above 2^20 cells more tiles cost
 // more in the sums each block adds up than their balance gives.
+// Cells that hold more than the usual few particles each (a support radius of
+// more than four particle radii; `members`: of a cell of fluid at rest) come
+// in tiles of fewer, down to four, so that a full tile holds about 2,048
+// particles, as long as there are no more tiles than a 64th of the particles:
+// with 54 and 250 particles a cell (216,000 particles, support 12 and 20
+// radii) tiles of 256 cells left 16 to 76 blocks to move them, sort 230 and
+// 2,935 us; with fewer cells, and runs ranked instead of members, 17.6 and 28.
 constexpr uint32_t kTileShiftMax = 10;
-__host__ __device__ constexpr uint32_t tile_shift(uint32_t ncells) {
+constexpr uint32_t kTileShiftMin = 2;
+constexpr uint32_t tile_shift_for(uint32_t ncells) {
     return ncells <= (1u << 19) ? 8u : ncells <= (1u << 20) ? 9u : kTileShiftMax;
 }
-__host__ __device__ constexpr uint32_t scan_tiles(uint32_t ncells) {
-    return (ncells + (1u << tile_shift(ncells)) - 1u) >> tile_shift(ncells);
+constexpr uint32_t tile_shift_for(uint32_t ncells, uint32_t n, float members) {
+    uint32_t shift = tile_shift_for(ncells);
+    if (members > 8.0f)
+        while (shift > kTileShiftMin && members * (float)(1u << shift) > 2048.0f && ncells >> (shift - 1u) <= n / 64u)
+            --shift;
+    return shift;
+}
+__host__ __device__ constexpr uint32_t scan_tiles(uint32_t ncells, uint32_t shift) {
+    return (ncells + (1u << shift) - 1u) >> shift;
 }
 
 // Runs.  A cell's members are kept as a chain of runs: consecutive particles

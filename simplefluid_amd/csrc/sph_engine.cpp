@@ -237,6 +237,7 @@ StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     a.tiles = tiles_for(h, block, a.ntiles);
     a.n = h->n;
     a.ncells = h->ncells;
+    a.tile_shift = h->tile_shift;
     return a;
 }
 
@@ -252,13 +253,17 @@ int alloc_step_bufs(sph_handle* h, StepBufs& w) {
     chk(w.perm.ensure(n));
     // A table that is new or held another grid's cells: every tile is
     // rewritten at the next sort.
-    const uint32_t T = scan_tiles(h->ncells);
-    const bool stale = w.cstart.count < (size_t)h->ncells + 1 || w.tile_pre.count < T || w.tile_cells != h->ncells;
+    const uint32_t T = scan_tiles(h->ncells, h->tile_shift);
+    const bool stale = w.cstart.count < (size_t)h->ncells + 1 || w.tile_pre.count < T || w.tile_cells != h->ncells ||
+                       w.tile_shift != h->tile_shift;
     w.tile_cells = 0;
     chk(w.cstart.ensure((size_t)h->ncells + 1));
     chk(w.tile_pre.ensure(T));
     if (e == hipSuccess && stale) chk(launch_fill_u32(h->stream, w.tile_pre.p, 0xffffffffu, T));
-    if (e == hipSuccess) w.tile_cells = h->ncells;
+    if (e == hipSuccess) {
+        w.tile_cells = h->ncells;
+        w.tile_shift = h->tile_shift;
+    }
     if (h->tune.sort_mode == kSortRadix)
         for (int i = 0; i < 2; ++i) { chk(w.kbuf[i].ensure(n)); chk(w.vbuf[i].ensure(n)); }
     else
@@ -278,7 +283,7 @@ static int ensure_buffers(sph_handle* h) {
     chk(h->id.ensure(n));
     chk(h->key0.ensure(n));
     chk(h->next.ensure(n));
-    const size_t head_words = (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells);
+    const size_t head_words = (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells, h->tile_shift);
     const bool fresh_head = h->head.count < head_words || !h->head.p;
     chk(h->head.ensure(head_words));
     chk(h->hist.ensure(kMaxPasses * 256));
@@ -343,11 +348,11 @@ static int enqueue_hash(sph_handle* h) {
     uint32_t nt = 0;
     const uint2* tl = tiles_for(h, 256, nt);
     if (!tl) return fail(h, SPH_E_OOM, "tile table");
-    hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells));
+    hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells, h->tile_shift));
     if (e == hipSuccess && h->cfl) e = launch_fill_u32(st, h->vmax2.p, 0u, kSpeedSlots);
     if (e == hipSuccess)
         e = launch_hash(st, 256, nt, h->pos.p, h->vel.p, h->key0.p, h->next.p, h->head.p, h->ncells,
-                        h->cfl ? h->vmax2.p : nullptr, h->sc_d.p, tl, nt);
+                        h->tile_shift, h->cfl ? h->vmax2.p : nullptr, h->sc_d.p, tl, nt);
     if (e != hipSuccess) return hip_fail(h, e, "hash launch");
     h->keys_valid = true;
     return SPH_OK;
@@ -375,6 +380,7 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     SortPlan sp;
     sp.n = h->n;
     sp.ncells = h->ncells;
+    sp.tile_shift = h->tile_shift;
     sp.mode = h->tune.sort_mode;
     sp.passes = h->passes;
     sp.items = h->tune.sort_items;
@@ -645,6 +651,9 @@ static int configure(sph_handle* h, const std::vector<sph_params>& ps, const std
     h->n = (uint32_t)p_off;
     h->ncells = (uint32_t)cell_off;
     h->passes = sort_key_passes(h->ncells);
+    float members = 0.0f;  // of the fullest scene's cells at rest
+    for (const sph_params& p : ps) members = std::max(members, cell_members(p, xsub));
+    h->tile_shift = tile_shift_for(h->ncells, h->n, members);
     h->split_tiles = 0;
     for (uint32_t v : ns) h->split_tiles += (v + kSplitTile - 1) / kSplitTile;
     h->xsub = xsub;

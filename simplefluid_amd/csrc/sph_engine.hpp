@@ -91,7 +91,8 @@ struct StepBufs {
     DevBuf<uint32_t> skey, perm;   // sorted keys, sorted index -> state index
     DevBuf<uint32_t> cstart;       // C + 1 lower-bound cell-start table
     DevBuf<uint32_t> tile_pre;     // per tile of cstart: prefix held by an empty tile, or ~0u
-    uint32_t tile_cells = 0;       // cells of the grid tile_pre describes cstart for
+    uint32_t tile_cells = 0;       // cells of the grid tile_pre describes cstart for, and of its tiles (shift)
+    uint32_t tile_shift = 0;
     DevBuf<uint32_t> kbuf[2], vbuf[2];  // radix ping-pong (radix mode only)
     DevBuf<float> rho;
     DevBuf<uint32_t> mask;
@@ -149,6 +150,7 @@ struct sph_handle {
     bool batched = false;
     uint32_t n = 0;
     uint32_t ncells = 0;
+    uint32_t tile_shift = 0;               // cells per tile of the sort, as a shift
     int passes = 1;
     uint32_t split_tiles = 0;              // tiles of the split form, scene by scene
     int xsub = 1;                          // x cells per y/z cell size
@@ -170,7 +172,7 @@ struct sph_handle {
     uint16_t* nlist = nullptr;             // the split form's neighbour lists and
     uint32_t* ncount = nullptr;            // their lengths,
     uint32_t* mask_hi = nullptr;           // second mask words
-    sph::DevBuf<uint32_t> tmp;             // cell-count sort: members of the tiles too full for LDS
+    sph::DevBuf<uint32_t> tmp;             // cell-count sort: a tile's runs or members on their way to their order
     sph::StepBufs work;
     sph::DevBuf<uint32_t> hist, status, tickets, err, queue;
     bool cfl = false;                      // adaptive step (single scene)
@@ -231,6 +233,11 @@ int hip_fail(sph_handle* h, hipError_t e, const char* what);
 int derive_scene(const sph_params& p, SceneConst& sc, std::string& err, int xsub);
 // The same checks and constants without building a message (allocates nothing).
 int derive_scene_noalloc(const sph_params& p, SceneConst& sc, int xsub);
+// Particles of a cell of fluid at rest: the lattice's, one per (2 r)^3.
+inline float cell_members(const sph_params& p, int xsub) {
+    const float s = p.kernel_radius / (2.0f * p.particle_radius);
+    return s * s * s / (float)xsub;
+}
 // Records the failure message of a call that has no handle (sph_last_error(NULL)).
 void set_thread_error(const char* msg);
 int alloc_step_bufs(sph_handle* h, StepBufs& w);

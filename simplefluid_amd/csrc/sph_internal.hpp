@@ -16,6 +16,7 @@ constexpr int kSortRadix = 1;       // multi-pass 8-bit LSD radix sort
 struct SortPlan {
     uint32_t n = 0;
     uint32_t ncells = 0;
+    uint32_t tile_shift = 0;          // cells per tile, as a shift
     int mode = kSortCellCount;
     int passes = 1;                   // radix: 8-bit digits
     int items = 8;                    // radix: keys per thread of a digit-pass tile
@@ -26,7 +27,7 @@ struct SortPlan {
     uint32_t* cstart = nullptr;       // C + 1, written by the sort
     uint32_t* tile_pre = nullptr;     // per tile: the prefix this cstart holds in all its cells
                                       // when the tile was empty at its last write, else 0xffffffff
-    uint32_t* tmp = nullptr;          // cell-count: members of the tiles too full for LDS (n)
+    uint32_t* tmp = nullptr;          // cell-count: runs or members of a tile on their way to their order (n)
     uint32_t* kbuf[2] = {nullptr, nullptr};  // radix ping-pong
     uint32_t* vbuf[2] = {nullptr, nullptr};
     uint32_t* skey = nullptr;         // radix: sorted keys
@@ -48,7 +49,7 @@ struct SortPlan {
 };
 
 uint32_t sort_tiles(uint32_t n, int items);
-// head holds C chain heads, then T = scan_tiles(C) per-tile sums, then their
+// head holds C chain heads, then T = scan_tiles(C, tile_shift) per-tile sums, then their
 // exclusive scan (T words).
 int sort_key_passes(uint32_t ncells);
 // Cell-start table and the sort; cell-count mode gathers the state too ...
@@ -81,7 +82,11 @@ struct StepArgs {
     const SceneConst* scenes;
     const uint2* tiles;
     uint32_t ntiles;
-    uint32_t n;
+    // One word for both: with a register more to hold, the staged force pass
+    // fetched its buffer descriptors back from vector lanes in its walk over
+    // global memory (216,000 particles, rows of 200 candidates: 257 -> 278 us).
+    uint32_t n : 28;         // below 2^28
+    uint32_t tile_shift : 4; // cells per tile of the sort, as a shift
     uint32_t ncells;
     uint32_t* queue;         // persistent launch: 8 tile counters (zeroed by the sort), else null
     uint32_t* vmax2;         // CFL: kSpeedSlots words of max |v|^2 (float bits) of the state the step starts
@@ -96,12 +101,12 @@ struct StepArgs {
 constexpr int kQueueWords = 16;
 
 hipError_t launch_hash(hipStream_t st, int block, uint32_t grid, const float4* pos, const float4* vel,
-                       uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t ncells, uint32_t* vmax2,
-                       const SceneConst* scenes, const uint2* tiles, uint32_t ntiles);
+                       uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t ncells, uint32_t tile_shift,
+                       uint32_t* vmax2, const SceneConst* scenes, const uint2* tiles, uint32_t ntiles);
 // Upload and hash of one scene in one pass (vel_in null: zero velocity).
 hipError_t launch_upload_hash(hipStream_t st, const float* xyz, const float* vel_in, float4* pos, float4* vel,
                               uint32_t* id, uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t n,
-                              uint32_t ncells, const SceneConst& sc);
+                              uint32_t ncells, uint32_t tile_shift, const SceneConst& sc);
 // Device frame loop state, 4 words: halt (steps are skipped), pending (the
 // frame reached 1/30 s in the current step), steps taken, frame time (float
 // bits).  reset zeroes them; the density pass adds its step and sets pending,

@@ -30,7 +30,8 @@ constexpr uint32_t kMaxCells = 1u << 20;
 constexpr uint32_t kMaxTiles = kMaxParticles / kSplitTile;
 static_assert(kMaxParticles <= kSplitMax, "the step runs in the split form");
 constexpr uint32_t kScanTilesMax = 2048;
-static_assert(scan_tiles(kMaxCells) <= kScanTilesMax && scan_tiles(1u << 19) <= kScanTilesMax,
+static_assert(scan_tiles(kMaxCells, tile_shift_for(kMaxCells)) <= kScanTilesMax &&
+                  scan_tiles(1u << 19, tile_shift_for(1u << 19)) <= kScanTilesMax && kMaxParticles / 64 < kScanTilesMax,
               "the most tiles of each tile size");
 
 // Byte offsets of the arrays inside the scratch, each 256-byte aligned.
@@ -46,7 +47,8 @@ struct Layout {
     static constexpr size_t key0 = align256(id_s + 4 * N);
     static constexpr size_t next = align256(key0 + 4 * N);
     static constexpr size_t tmp = align256(next + 4 * N);
-    static constexpr size_t nlist = align256(tmp + 4 * N);
+    static constexpr size_t perm = align256(tmp + 4 * N);
+    static constexpr size_t nlist = align256(perm + 4 * N);
     static constexpr size_t ncount = align256(nlist + 2 * (size_t)kListMax * N);
     static constexpr size_t rho = align256(ncount + 4 * N);
     static constexpr size_t mask = align256(rho + 4 * N);
@@ -70,13 +72,13 @@ void* g_scratch[kMaxDevices] = {};
 
 // Scene constants, the tile table (scene 0, first particle t * kSplitTile),
 // empty chains, tile sums and tile prefixes, and the error word cleared.
-__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint8_t* __restrict__ base) {
+__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint32_t tile_shift, uint8_t* __restrict__ base) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
     if (i == 0) {
         *reinterpret_cast<SceneConst*>(base + Layout::scene) = sc;
         *reinterpret_cast<uint32_t*>(base + Layout::err) = 0u;
     }
-    const uint32_t T = scan_tiles(ncells);
+    const uint32_t T = scan_tiles(ncells, tile_shift);
     uint32_t* head = reinterpret_cast<uint32_t*>(base + Layout::head);
     // Whole 16-byte words; the scratch behind the last tile sum is unused.
     for (uint32_t w = i; w < (ncells + 2u * T + 3u) / 4u; w += stride)
@@ -124,16 +126,20 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     // The grid a handle of n <= 65536 particles picks: the largest x
     // subdivision whose cell count stays within 2^20.
     SceneConst sc;
-    int rc = SPH_E_INVALID;
+    int rc = SPH_E_INVALID, sub = 1;
     for (int xsub : {4, 2, 1}) {
         rc = derive_scene_noalloc(*p, sc, xsub);
         if (rc != SPH_OK) return fail_noalloc(rc, "sph_step_noalloc: invalid parameters (as sph_create checks them)");
-        if ((uint64_t)sc.G[0] * sc.G[1] * sc.G[2] <= kMaxCells) break;
+        if ((uint64_t)sc.G[0] * sc.G[1] * sc.G[2] <= kMaxCells) {
+            sub = xsub;
+            break;
+        }
         rc = SPH_E_CAPACITY;
     }
     if (rc != SPH_OK)
         return fail_noalloc(SPH_E_INVALID, "sph_step_noalloc: the grid exceeds 2^20 cells (the scratch's cell limit)");
     const uint32_t C = (uint32_t)((uint64_t)sc.G[0] * sc.G[1] * sc.G[2]);
+    const uint32_t shift = tile_shift_for(C, n, cell_members(*p, sub));
     sc.cell_offset = 0;
     sc.p_begin = 0;
     sc.p_end = n;
@@ -152,12 +158,13 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
 
     // Five launches: setup, upload and hash, sort, density, force (which
     // writes the caller's arrays itself).
-    hipLaunchKernelGGL(noalloc_setup_kernel, dim3(256), dim3(256), 0, st, sc, C, base);
+    hipLaunchKernelGGL(noalloc_setup_kernel, dim3(256), dim3(256), 0, st, sc, C, shift, base);
     e = hipGetLastError();
-    if (e == hipSuccess) e = launch_upload_hash(st, xyz_in, vel_in, pos, vel, id, key0, next, head, n, C, sc);
+    if (e == hipSuccess) e = launch_upload_hash(st, xyz_in, vel_in, pos, vel, id, key0, next, head, n, C, shift, sc);
     SortPlan sp;
     sp.n = n;
     sp.ncells = C;
+    sp.tile_shift = shift;
     sp.mode = kSortCellCount;
     sp.key0 = key0;
     sp.head = head;
@@ -165,6 +172,7 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     sp.cstart = reinterpret_cast<uint32_t*>(at(Layout::cstart));
     sp.tile_pre = reinterpret_cast<uint32_t*>(at(Layout::tile_pre));
     sp.tmp = reinterpret_cast<uint32_t*>(at(Layout::tmp));
+    sp.perm = reinterpret_cast<uint32_t*>(at(Layout::perm));
     sp.err = reinterpret_cast<uint32_t*>(at(Layout::err));
     sp.pos_in = pos;
     sp.vel_in = vel;

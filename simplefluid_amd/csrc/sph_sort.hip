@@ -7,9 +7,10 @@
 // each particle into its cell's chain of runs and counted particles per tile
 // of cells, so a block of cell_sort_kernel owns a tile: it takes its
 // prefix from the tile sums, counts its cells by following their chains,
-// scans the counts (cstart), lists the members cell by cell in LDS, each
-// cell's by ascending input index, and
-// gathers its state straight into its sorted place (pos, vel, id, perm).  No block waits for another.
+// scans the counts (cstart), lists the members cell by cell, each cell's by
+// ascending input index (from the chain's links in registers; a longer
+// chain's runs are ranked among each other first), and gathers their state
+// into its sorted place (pos, vel, id, perm).  No block waits for another.
 // Radix sort: one histogram kernel for all 8-bit digits, then one kernel per
 // digit that ranks a tile of keys in LDS (wave64 ballot-matching of the
 // digit bits, so equal digits rank in lane order without LDS atomics) and
@@ -19,6 +20,8 @@
 // Look-back waits are bounded: a wait that exceeds its bound raises the
 // device error flag instead of hanging, and every data-dependent store is
 // range-checked.
+#include <algorithm>
+
 #include "sph_internal.hpp"
 
 namespace sph {
@@ -147,25 +150,31 @@ __global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __r
     if (i < T) head[C + T + i] = run;
 }
 
-// Members a cell may hold for the stable in-cell rank (a member's rank scans
-// its cell).  Rest-density fluid holds a few per cell.
+// Members a cell may hold for the stable in-cell rank.  Rest-density fluid
+// holds a few per cell.
 constexpr uint32_t kMaxRankCell = 1024;
 // Members of a tile listed in LDS, at most eight per cell; a fuller tile lists
 // them in global memory.
 constexpr uint32_t kTileMembers = 4096;
 // Links of one cell followed in its chain; a longer chain (a pile of
 // particles in one cell, or an upload in random order of a very full one)
-// makes the block find the tile's members by scanning all keys instead.
-constexpr int kMaxLinks = 256;
+// makes the block find the tile's members by scanning all keys instead.  A
+// link costs a read's latency twice, the scan the keys' bytes at one CU's
+// rate, kScanQuads 16-byte loads in flight per lane: about the same at one
+// link per 2,048 keys.
+constexpr uint32_t kMinLinks = 32, kMaxLinks = 1024;
+constexpr uint32_t kScanQuads = 6;
 
 struct CellSortArgs {
     uint32_t n, C;
+    uint32_t shift;      // cells per tile, as a shift
+    uint32_t max_links;
     uint32_t* head;
     const uint32_t* next;
     const uint32_t* key0;
     uint32_t* cstart;
     uint32_t* tile_pre;
-    uint32_t* tmp;       // members of the tiles too full for LDS, at their sorted place
+    uint32_t* tmp;       // a tile's runs or members on their way to their order, from its sorted place on
     const float4* pos_in;
     const float4* vel_in;
     const uint32_t* id_in;
@@ -180,8 +189,8 @@ struct CellSortArgs {
     int gather;          // 0: the cell-start table only (radix mode)
 };
 
-// Block b sorts the particles of tile b, of BLOCK V cells.  Thread t owns
-// V consecutive cells; their chains are followed together, so a wave waits
+// Block b sorts the particles of tile b, of up to BLOCK V cells.  Thread t
+// owns V consecutive cells; their chains are followed together, so a wave waits
 // once per link for the longest chain among its cells, and the first
 // kHeldLinks links stay in registers for the listing.  The kernel is bound
 // by the latency of its dependent steps at small sizes (tile sums and heads,
@@ -205,6 +214,8 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     }
     constexpr uint32_t kCells = (uint32_t)(BLOCK * V);
     constexpr uint32_t kMembers = kCells * 8u < kTileMembers ? kCells * 8u : kTileMembers;
+    // A tile whose runs are ranked keeps each cell's first run in that room.
+    constexpr uint32_t kRanked = kMembers - (kCells + 1u);
     static_assert(kCells <= 1u << kTileShiftMax, "a tile");
     constexpr int kWaves = BLOCK / 64;
     static_assert(V == 1 || V == 4, "one head, or four in one 16-byte load, per thread");
@@ -219,10 +230,14 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     // Tile counters of this step's persistent density and force launches.
     if (b == 0 && tid < kQueueWords && a.queue) a.queue[tid] = 0u;
     const uint32_t T = gridDim.x;
-    const uint32_t base = b * kCells;
+    const uint32_t cells = 1u << a.shift;
+    const uint32_t base = b << a.shift;
     const uint32_t i0 = base + (uint32_t)(V * tid);
     uint32_t r[kHeldLinks + 1][V];
-    const bool whole = i0 + (uint32_t)V <= C;
+    // Cells of this thread: V == 4 has four of a whole tile, one or none where
+    // V == 1; past the grid none.
+    const uint32_t Ce = V == 1 && base + cells < C ? base + cells : C;
+    const bool whole = i0 + (uint32_t)V <= Ce;
     if (V == 4 && whole) {
         const uint4 hv = *reinterpret_cast<const uint4*>(a.head + i0);
         r[0][0] = hv.x;
@@ -231,7 +246,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
         r[0][V > 3 ? 3 : 0] = V > 3 ? hv.w : hv.x;
     } else {
 #pragma unroll
-        for (int v = 0; v < V; ++v) r[0][v] = i0 + (uint32_t)v < C ? a.head[i0 + v] : 0u;
+        for (int v = 0; v < V; ++v) r[0][v] = i0 + (uint32_t)v < Ce ? a.head[i0 + v] : 0u;
     }
     // What the table holds for this tile, read by every thread before any
     // thread of the block rewrites it.
@@ -264,7 +279,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
         if (V == 4 && whole) {
             *reinterpret_cast<uint4*>(a.cstart + i0) = make_uint4(pre, pre, pre, pre);
         } else {
-            for (uint32_t e = i0; e < C && e < i0 + (uint32_t)V; ++e) a.cstart[e] = pre;
+            for (uint32_t e = i0; e < Ce && e < i0 + (uint32_t)V; ++e) a.cstart[e] = pre;
         }
         if (b == T - 1u && tid == 0) a.cstart[C] = pre;
         return;
@@ -281,9 +296,12 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
         for (int v = 0; v < V; ++v) o |= q[v];
         return o != 0u;
     };
-    uint32_t cnt[V];
+    uint32_t cnt[V], more[V];  // per cell: members, links past the held ones
 #pragma unroll
-    for (int v = 0; v < V; ++v) cnt[v] = run_len(r[0][v]);
+    for (int v = 0; v < V; ++v) {
+        cnt[v] = run_len(r[0][v]);
+        more[v] = 0u;
+    }
 #pragma unroll
     for (int l = 0; l < kHeldLinks; ++l) {
 #pragma unroll
@@ -300,22 +318,23 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
         if (V == 4 && whole) {
             *reinterpret_cast<uint4*>(a.head + i0) = make_uint4(0u, 0u, 0u, 0u);
         } else {
-            for (uint32_t e = i0; e < C && e < i0 + (uint32_t)V; ++e) a.head[e] = 0u;
+            for (uint32_t e = i0; e < Ce && e < i0 + (uint32_t)V; ++e) a.head[e] = 0u;
         }
     }
     {
         uint32_t q[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) q[v] = r[kHeldLinks][v];
-        int links = kHeldLinks;
+        uint32_t links = (uint32_t)kHeldLinks;
         if (any(q)) s_unsorted = 1u;  // longer than the registers hold (a last run may follow none: no matter)
         while (any(q)) {
-            if (++links > kMaxLinks) {
+            if (++links > a.max_links) {
                 s_big = 1u;
                 break;
             }
 #pragma unroll
             for (int v = 0; v < V; ++v) {
+                more[v] += q[v] ? 1u : 0u;
                 q[v] = link(q[v]);
                 cnt[v] += run_len(q[v]);
             }
@@ -324,12 +343,32 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     __syncthreads();
     const bool big = s_big != 0u;
     if (big) {
-        // Count by scanning all keys (s_off as the counters).
-        for (uint32_t i = (uint32_t)tid; i < kCells; i += BLOCK) s_off[i] = 0u;
+        // Find the tile's members by scanning all keys: their counts per cell
+        // (s_off) and, in any order, themselves (tmp; s_off's last word counts
+        // them).
+        for (uint32_t i = (uint32_t)tid; i <= kCells; i += BLOCK) s_off[i] = 0u;
         __syncthreads();
-        for (uint32_t k = (uint32_t)tid; k < a.n; k += BLOCK) {
-            const uint32_t c = a.key0[k] - base;
-            if (c < kCells) atomicAdd(&s_off[c], 1u);
+        const __amdgpu_buffer_rsrc_t rkey = buffer_of(a.key0, a.n);
+        const uint32_t room = a.gather && pre < a.n ? min(members, a.n - pre) : 0u;
+        for (uint32_t q0 = (uint32_t)tid; 4u * q0 < a.n; q0 += kScanQuads * (uint32_t)BLOCK) {
+            u32x4 key[kScanQuads];
+#pragma unroll
+            for (uint32_t u = 0; u < kScanQuads; ++u)
+                key[u] = __builtin_amdgcn_raw_buffer_load_b128(rkey, (int)(q0 << 4), (int)(u * (uint32_t)BLOCK * 16u), 0);
+#pragma unroll
+            for (uint32_t u = 0; u < kScanQuads; ++u) {
+                const uint32_t c[4] = {key[u].x - base, key[u].y - base, key[u].z - base, key[u].w - base};
+                if (min(min(c[0], c[1]), min(c[2], c[3])) >= cells) continue;
+#pragma unroll
+                for (uint32_t e = 0; e < 4u; ++e) {
+                    const uint32_t k = 4u * (q0 + u * (uint32_t)BLOCK) + e;
+                    if (c[e] < cells && k < a.n) {
+                        atomicAdd(&s_off[c[e]], 1u);
+                        const uint32_t at = atomicAdd(&s_off[kCells], 1u);
+                        if (at < room) a.tmp[pre + at] = k;
+                    }
+                }
+            }
         }
         __syncthreads();
 #pragma unroll
@@ -349,26 +388,26 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     } else {
 #pragma unroll
         for (int v = 0; v < V; ++v)
-            if (i0 + (uint32_t)v < C) a.cstart[i0 + v] = pre + off[v];
+            if (i0 + (uint32_t)v < Ce) a.cstart[i0 + v] = pre + off[v];
     }
     if (b == T - 1u && tid == 0) a.cstart[C] = pre + total;
     if (!a.gather) return;
-    if (pre > a.n || total > a.n - pre) {  // inconsistent sums: never write out of bounds
+    if (pre > a.n || total > a.n - pre || total > members) {  // inconsistent sums: never write out of bounds
         if (tid == 0) atomicOr(a.err, 2u);
         return;
     }
 #pragma unroll
     for (int v = 0; v < V; ++v) s_off[V * tid + v] = off[v];
     if (tid == 0) s_off[kCells] = total;
-    // The members, cell by cell.  A cell whose runs are all in registers
-    // lists them by their first particles, so its members come sorted; with a
-    // longer chain in the tile, all come as their runs do and are ranked
-    // below.
+    // The members, cell by cell, each cell's by ascending index.
     const bool unsorted = big || s_unsorted != 0u;
-    const bool in_lds = total <= kMembers && !big;
+    const bool in_lds = !big && total <= (unsorted ? kRanked : kMembers);
+    uint32_t* const s_list = unsorted ? s_mem + (kCells + 1u) : s_mem;
+    uint32_t* const list = a.perm + pre;  // too many for LDS: where they end up
     uint32_t* const tmp = a.tmp + pre;
     if (!unsorted) {
-        auto list = [&](auto&& put) __attribute__((always_inline)) {
+        // Every cell's runs are in registers: their first particles order them.
+        auto put_all = [&](auto&& put) __attribute__((always_inline)) {
 #pragma unroll
             for (int l = 0; l < kHeldLinks; ++l) {
                 if (__ballot(any(r[l])) != 0u) {
@@ -386,44 +425,124 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
             }
         };
         if (in_lds)
-            list([&](uint32_t i, uint32_t k) { s_mem[i] = k; });
+            put_all([&](uint32_t i, uint32_t k) { s_mem[i] = k; });
         else
-            list([&](uint32_t i, uint32_t k) { tmp[i] = k; });
+            put_all([&](uint32_t i, uint32_t k) { list[i] = k; });
     } else if (!big) {
-        auto list = [&](const uint32_t* q) __attribute__((always_inline)) {
+        // Longer chains: all runs of the tile go to tmp, cell by cell, and each
+        // finds its place among its cell's (a rank by members costs that many
+        // times more: cells of 54, 216,000 particles, 230 us).
+        uint32_t* const s_first = s_mem;  // each cell's first run in tmp
+        uint32_t runs[V], mine = 0u;
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                const uint32_t k = run_first(q[v]), len = run_len(q[v]);
-                for (uint32_t t = 0; t < len; ++t) {
-                    if (in_lds)
-                        s_mem[off[v] + t] = k + t;
-                    else
-                        tmp[off[v] + t] = k + t;
-                }
-                off[v] += len;
-            }
-        };
+        for (int v = 0; v < V; ++v) {
+            runs[v] = more[v];
 #pragma unroll
-        for (int l = 0; l <= kHeldLinks; ++l)
-            if (any(r[l])) list(r[l]);
+            for (int l = 0; l < kHeldLinks; ++l) runs[v] += r[l][v] ? 1u : 0u;
+            mine += runs[v];
+        }
+        uint32_t nruns, at[V];
+        __syncthreads();  // s_w is read by the scan before
+        at[0] = block_scan<BLOCK>(mine, s_w, nruns);
+#pragma unroll
+        for (int v = 1; v < V; ++v) at[v] = at[v - 1] + runs[v - 1];
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            s_first[V * tid + v] = at[v];
+#pragma unroll
+            for (int l = 0; l < kHeldLinks; ++l)
+                if (r[l][v]) tmp[at[v]++] = r[l][v];
+        }
         uint32_t q[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) q[v] = r[kHeldLinks][v];
         while (any(q)) {
 #pragma unroll
-            for (int v = 0; v < V; ++v) q[v] = link(q[v]);
-            list(q);
+            for (int v = 0; v < V; ++v) {
+                if (q[v]) tmp[at[v]++] = q[v];
+                q[v] = link(q[v]);
+            }
+        }
+        if (tid == 0) s_first[kCells] = nruns;
+        __threadfence_block();
+        __syncthreads();
+        for (uint32_t i = (uint32_t)tid; i < nruns; i += BLOCK) {
+            const uint32_t k = run_first(tmp[i]), len = run_len(tmp[i]);
+            const uint32_t c = k < a.n ? a.key0[k] - base : cells;
+            if (c >= cells) {
+                atomicOr(a.err, 4u);
+                continue;
+            }
+            uint32_t d = s_off[c];
+#pragma unroll 4
+            for (uint32_t t = s_first[c]; t < s_first[c + 1u]; ++t) {
+                const uint32_t q = tmp[t];
+                d += run_first(q) < k ? run_len(q) : 0u;
+            }
+            if (s_off[c + 1u] - s_off[c] > kMaxRankCell) atomicOr(a.err, 8u);
+            for (uint32_t t = 0; t < len && d + t < total; ++t) {
+                if (in_lds)
+                    s_list[d + t] = k + t;
+                else
+                    list[d + t] = k + t;
+            }
         }
     } else {
+        // From tmp to their cells, then each to its rank, in tmp again.
+        // f(j, k, c): member j of src, k, lies in cell c; eight loads of each
+        // kind in flight.
+        auto each = [&](const uint32_t* src, auto&& f) __attribute__((always_inline)) {
+            constexpr int kEach = 8;
+            for (uint32_t j0 = (uint32_t)tid; j0 < total; j0 += (uint32_t)(kEach * BLOCK)) {
+                uint32_t k[kEach], c[kEach];
+#pragma unroll
+                for (int u = 0; u < kEach; ++u) k[u] = src[min(j0 + (uint32_t)(u * BLOCK), total - 1u)];
+#pragma unroll
+                for (int u = 0; u < kEach; ++u) c[u] = a.key0[min(k[u], a.n - 1u)] - base;
+#pragma unroll
+                for (int u = 0; u < kEach; ++u) {
+                    const uint32_t j = j0 + (uint32_t)(u * BLOCK);
+                    if (j >= total) break;
+                    if (k[u] < a.n && c[u] < cells)
+                        f(j, k[u], c[u]);
+                    else
+                        atomicOr(a.err, 4u);
+                }
+            }
+        };
+        __threadfence_block();
         __syncthreads();
-        for (uint32_t k = (uint32_t)tid; k < a.n; k += BLOCK) {
-            const uint32_t c = a.key0[k] - base;
-            if (c < kCells) tmp[atomicAdd(&s_off[c], 1u)] = k;
-        }
+        each(tmp, [&](uint32_t, uint32_t k, uint32_t c) {
+            const uint32_t at = atomicAdd(&s_off[c], 1u);
+            if (at < total) list[at] = k;
+        });
         __syncthreads();
         // The counters ended at the next cell's start.
 #pragma unroll
         for (int v = 0; v < V; ++v) s_off[V * tid + v] = off[v];
+        __threadfence_block();
+        __syncthreads();
+        bool over = false;
+        each(list, [&](uint32_t j, uint32_t k, uint32_t c) {
+            const uint32_t lo = s_off[c], hi = s_off[c + 1u];
+            uint32_t d = j;
+            if (hi - lo <= kMaxRankCell) {
+                d = lo;
+#pragma unroll 8
+                for (uint32_t t = lo; t < hi; ++t) d += list[t] < k ? 1u : 0u;
+            } else {
+                // A cell this full only arises from collapsed or non-finite
+                // positions (clamped into one cell).  Ranking it costs its
+                // size per member, so it keeps the order its members were
+                // listed in (a valid permutation, not the stable one) and
+                // raises the error flag instead.  The block moves it alone:
+                // 20,000 such particles among 1.9M make the sort 540 us, 200,000
+                // among 1M 1,120 (one key at a time per lane: 4,700 and 4,600).
+                over = true;
+            }
+            tmp[d] = k;
+        });
+        if (over) atomicOr(a.err, 8u);
     }
     __threadfence_block();
     __syncthreads();
@@ -441,7 +560,7 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
         for (int v = 0; v < V; ++v) {
             const uint32_t j = j0 + (uint32_t)(v * BLOCK);
             k[v] = 0xffffffffu;
-            if (j < total) k[v] = in_lds ? s_mem[j] : tmp[j];
+            if (j < total) k[v] = in_lds ? s_list[j] : big ? tmp[j] : list[j];
         }
 #pragma unroll
         for (int v = 0; v < V; ++v) {
@@ -458,37 +577,8 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
                 atomicOr(a.err, 4u);
                 continue;
             }
-            uint32_t d = j;
-            if (unsorted) {
-                const uint32_t c = a.key0[k[v]] - base;
-                if (c >= kCells) {
-                    atomicOr(a.err, 4u);
-                    continue;
-                }
-                const uint32_t lo = s_off[c], hi = s_off[c + 1u];
-                if (hi - lo <= kMaxRankCell) {
-                    d = lo;
-                    if (in_lds) {
-#pragma unroll 4
-                        for (uint32_t t = lo; t < hi; ++t) d += s_mem[t] < k[v] ? 1u : 0u;
-                    } else {
-                        for (uint32_t t = lo; t < hi; ++t) d += tmp[t] < k[v] ? 1u : 0u;
-                    }
-                } else {
-                    // A cell this full only arises from collapsed or
-                    // non-finite positions (clamped into one cell).  Ranking
-                    // it costs its size per member, so it keeps the order its
-                    // members were listed in (a valid permutation, not the
-                    // stable one) and raises the error flag instead.
-                    atomicOr(a.err, 8u);
-                }
-            }
-            const uint32_t dst = pre + d;
-            if (dst >= a.n) {
-                atomicOr(a.err, 4u);
-                continue;
-            }
-            if (a.perm) a.perm[dst] = k[v];
+            const uint32_t dst = pre + j;
+            if (in_lds || big) a.perm[dst] = k[v];
             a.pos_out[dst] = pk[v];
             if (a.soa) {  // the planes, for the gathered density pass
                 a.soa[dst] = pk[v].x;
@@ -695,13 +785,15 @@ int sort_key_passes(uint32_t ncells) {
 #define SPH_CELL_SORT(block, v) HIP_KERNEL_NAME(cell_sort_kernel<block, v>)
 
 static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
-    const uint32_t tiles = scan_tiles(sp.ncells);
+    const uint32_t tiles = scan_tiles(sp.ncells, sp.tile_shift);
     if (tiles > kInlineTiles)
         hipLaunchKernelGGL(tile_scan_kernel, dim3((tiles + kTileScanBlock - 1) / kTileScanBlock), dim3(kTileScanBlock),
                            0, st, sp.head, sp.ncells, tiles, sp.frame);
     CellSortArgs a;
     a.n = sp.n;
     a.C = sp.ncells;
+    a.shift = sp.tile_shift;
+    a.max_links = std::min(std::max(sp.n >> 11, kMinLinks), kMaxLinks);
     a.head = sp.head;
     a.next = sp.next;
     a.key0 = sp.key0;
@@ -720,10 +812,9 @@ static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
     a.err = sp.err;
     a.frame = sp.frame;
     a.gather = gather;
-    const uint32_t shift = tile_shift(sp.ncells);
-    if (shift == 8u)
+    if (sp.tile_shift <= 8u)
         hipLaunchKernelGGL(SPH_CELL_SORT(256, 1), dim3(tiles), dim3(256), 0, st, a);
-    else if (shift == 9u)
+    else if (sp.tile_shift == 9u)
         hipLaunchKernelGGL(SPH_CELL_SORT(512, 1), dim3(tiles), dim3(512), 0, st, a);
     else
         hipLaunchKernelGGL(SPH_CELL_SORT(256, 4), dim3(tiles), dim3(256), 0, st, a);

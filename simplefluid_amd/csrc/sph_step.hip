@@ -597,7 +597,7 @@ __device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
         }
     }
     if (!a.head) return;
-    const uint32_t words = scan_tiles(a.ncells);
+    const uint32_t words = scan_tiles(a.ncells, a.tile_shift);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
         a.head[a.ncells + i] = 0u;
 }
@@ -607,7 +607,7 @@ __device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
 __device__ __forceinline__ void finish_particle(const StepArgs& a, uint32_t k, const Moved& to, bool active) {
     const uint32_t key = to.key;
     if (!a.head) return;  // a single step: there is no next one
-    add_tile_sums(a.head + a.ncells, tile_shift(a.ncells), key, active);
+    add_tile_sums(a.head + a.ncells, a.tile_shift, key, active);
     if (a.vmax2) wave_max_v2(a.vmax2, to.v2);
     if (active) a.key0[k] = key;
     push_run(a.head, a.next, key, k, active);  // last: it waits for its exchange's answer
@@ -1129,8 +1129,8 @@ struct BlockTileSums {
     uint32_t* tsum;
     uint32_t shift, tiles;
     uint32_t* local;  // kHashTiles words of LDS; null: straight to memory
-    __device__ __forceinline__ BlockTileSums(uint32_t* head, uint32_t ncells, uint32_t* lds)
-        : tsum(head + ncells), shift(tile_shift(ncells)), tiles(scan_tiles(ncells)) {
+    __device__ __forceinline__ BlockTileSums(uint32_t* head, uint32_t ncells, uint32_t shift_, uint32_t* lds)
+        : tsum(head + ncells), shift(shift_), tiles(scan_tiles(ncells, shift_)) {
         local = tiles <= kHashTiles ? lds : nullptr;
         if (local) {
             for (uint32_t i = threadIdx.x; i < tiles; i += blockDim.x) local[i] = 0u;
@@ -1153,10 +1153,10 @@ struct BlockTileSums {
 
 __global__ void hash_kernel(const float4* __restrict__ pos, const float4* __restrict__ vel,
                             uint32_t* __restrict__ key0, uint32_t* __restrict__ next, uint32_t* __restrict__ head,
-                            uint32_t ncells, uint32_t* __restrict__ vmax2, const SceneConst* __restrict__ scenes,
-                            const uint2* __restrict__ tiles, uint32_t ntiles) {
+                            uint32_t ncells, uint32_t tile_shift, uint32_t* __restrict__ vmax2,
+                            const SceneConst* __restrict__ scenes, const uint2* __restrict__ tiles, uint32_t ntiles) {
     __shared__ uint32_t s_sum[kHashTiles];
-    BlockTileSums sums(head, ncells, s_sum);
+    BlockTileSums sums(head, ncells, tile_shift, s_sum);
     uint32_t t0, t1;
     tile_span(ntiles, t0, t1);
     for (uint32_t t = t0; t < t1; ++t) {
@@ -1187,9 +1187,10 @@ __global__ __launch_bounds__(256) void upload_hash_kernel(const float* __restric
                                                           float4* __restrict__ pos, float4* __restrict__ vel,
                                                           uint32_t* __restrict__ id, uint32_t* __restrict__ key0,
                                                           uint32_t* __restrict__ next, uint32_t* __restrict__ head,
-                                                          uint32_t n, uint32_t ncells, SceneConst sc) {
+                                                          uint32_t n, uint32_t ncells, uint32_t tile_shift,
+                                                          SceneConst sc) {
     __shared__ uint32_t s_sum[kHashTiles];
-    BlockTileSums sums(head, ncells, s_sum);
+    BlockTileSums sums(head, ncells, tile_shift, s_sum);
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = k < n;
     uint32_t key = 0;
@@ -1399,20 +1400,20 @@ int force_blocks_per_cu(int block, int staged) {
 }
 
 hipError_t launch_hash(hipStream_t st, int block, uint32_t grid, const float4* pos, const float4* vel,
-                       uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t ncells, uint32_t* vmax2,
-                       const SceneConst* scenes, const uint2* tiles, uint32_t ntiles) {
+                       uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t ncells, uint32_t tile_shift,
+                       uint32_t* vmax2, const SceneConst* scenes, const uint2* tiles, uint32_t ntiles) {
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL(hash_kernel, dim3(grid), dim3(block), 0, st, pos, vel, key0, next, head, ncells, vmax2,
-                       scenes, tiles, ntiles);
+    hipLaunchKernelGGL(hash_kernel, dim3(grid), dim3(block), 0, st, pos, vel, key0, next, head, ncells,
+                       tile_shift, vmax2, scenes, tiles, ntiles);
     return hipGetLastError();
 }
 
 hipError_t launch_upload_hash(hipStream_t st, const float* xyz, const float* vel_in, float4* pos, float4* vel,
                               uint32_t* id, uint32_t* key0, uint32_t* next, uint32_t* head, uint32_t n,
-                              uint32_t ncells, const SceneConst& sc) {
+                              uint32_t ncells, uint32_t tile_shift, const SceneConst& sc) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(upload_hash_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, st, xyz, vel_in, pos, vel, id, key0,
-                       next, head, n, ncells, sc);
+                       next, head, n, ncells, tile_shift, sc);
     return hipGetLastError();
 }
 
