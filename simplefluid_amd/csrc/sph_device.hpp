@@ -6,10 +6,11 @@
 //                                (written by the density pass for the force pass)
 //   id[2]           uint32 x N   original particle id, state / sorted order
 //   key0            uint32 x N   cell key of the state positions (written by integrate)
-//   head            uint32 x C+2T per cell, the newest run of particles that entered it
+//   head            uint32 x C+3T+1 per cell, the newest run of particles that entered it
 //                                (0: none; built by the integrate pass, cleared by the
-//                                sort), then particles per tile of cells, then the
-//                                exclusive scan of the tile sums
+//                                sort), then particles per tile of cells, then (with many
+//                                tiles) the list of those that need work: its length, the
+//                                exclusive scan of the tile sums, the list
 //   next            uint32 x N   per run (at its first particle), the cell's run before it
 //   radix ping-pong 2 x (uint32 key + uint32 value) x N (radix mode)
 //   cstart          uint32 x C+1 lower-bound cell-start table: cstart[c] = #particles with key < c

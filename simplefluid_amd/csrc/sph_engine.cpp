@@ -283,7 +283,7 @@ static int ensure_buffers(sph_handle* h) {
     chk(h->id.ensure(n));
     chk(h->key0.ensure(n));
     chk(h->next.ensure(n));
-    const size_t head_words = (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells, h->tile_shift);
+    const size_t head_words = sort_head_words(h->ncells, h->tile_shift);
     const bool fresh_head = h->head.count < head_words || !h->head.p;
     chk(h->head.ensure(head_words));
     chk(h->hist.ensure(kMaxPasses * 256));
@@ -348,7 +348,7 @@ static int enqueue_hash(sph_handle* h) {
     uint32_t nt = 0;
     const uint2* tl = tiles_for(h, 256, nt);
     if (!tl) return fail(h, SPH_E_OOM, "tile table");
-    hipError_t e = launch_fill_u32(st, h->head.p, 0u, (size_t)h->ncells + 2 * (size_t)scan_tiles(h->ncells, h->tile_shift));
+    hipError_t e = launch_fill_u32(st, h->head.p, 0u, sort_head_words(h->ncells, h->tile_shift));
     if (e == hipSuccess && h->cfl) e = launch_fill_u32(st, h->vmax2.p, 0u, kSpeedSlots);
     if (e == hipSuccess)
         e = launch_hash(st, 256, nt, h->pos.p, h->vel.p, h->key0.p, h->next.p, h->head.p, h->ncells,

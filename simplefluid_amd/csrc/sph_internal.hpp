@@ -22,7 +22,7 @@ struct SortPlan {
     int items = 8;                    // radix: keys per thread of a digit-pass tile
     int reorder_block = 256;
     const uint32_t* key0 = nullptr;   // unsorted keys (state order)
-    uint32_t* head = nullptr;         // C chain heads (cleared by the sort), T tile sums, T words for their scan
+    uint32_t* head = nullptr;         // C chain heads (cleared by the sort), T tile sums and the sort's room
     const uint32_t* next = nullptr;   // per run, the cell's run before it
     uint32_t* cstart = nullptr;       // C + 1, written by the sort
     uint32_t* tile_pre = nullptr;     // per tile: the prefix this cstart holds in all its cells
@@ -49,8 +49,13 @@ struct SortPlan {
 };
 
 uint32_t sort_tiles(uint32_t n, int items);
-// head holds C chain heads, then T = scan_tiles(C, tile_shift) per-tile sums, then their
-// exclusive scan (T words).
+// head holds C chain heads, then T = scan_tiles(C, tile_shift) per-tile sums, the
+// length of the list of tiles that need work, the sums' exclusive scan and
+// that list (T words each; both only where there are more tiles than a block
+// sums itself).
+inline size_t sort_head_words(uint32_t ncells, uint32_t shift) {
+    return (size_t)ncells + 3 * (size_t)scan_tiles(ncells, shift) + 1;
+}
 int sort_key_passes(uint32_t ncells);
 // Cell-start table and the sort; cell-count mode gathers the state too ...
 hipError_t launch_sort_keys(hipStream_t st, const SortPlan& sp);

@@ -119,7 +119,9 @@ __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s_w, uint32
 }
 
 // Exclusive scan of the T per-tile sums (head[C .. C+T)) into
-// head[C+T .. C+2T).  Block i scans sums [1024 i, 1024 (i + 1)) and adds up
+// head[C+T+1 .. C+2T+1); with tile_pre, a list of the tiles that need work (not
+// empty, or their cells hold another prefix) behind it, its length in
+// head[C+T].  Block i scans sums [1024 i, 1024 (i + 1)) and adds up
 // all the ones before itself: the reads are coalesced, independent and in
 // cache, where one block over all of them waited on itself round by round
 // (22k tiles: 14 us).
@@ -130,16 +132,19 @@ constexpr int kTileScanBlock = 1024;
 constexpr uint32_t kInlineTiles = 6144;
 
 __global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __restrict__ head, uint32_t C,
-                                                                   uint32_t T, const uint32_t* __restrict__ frame) {
+                                                                   uint32_t T, const uint32_t* __restrict__ frame,
+                                                                   const uint32_t* __restrict__ tile_pre) {
     if (frame && (frame[0] | frame[1])) return;
     __shared__ uint32_t s_w[kTileScanBlock / 64];
     __shared__ uint32_t s_pre[kTileScanBlock / 64];
+    __shared__ uint32_t s_at;
     const uint32_t* tsum = head + C;
     const uint32_t i0 = blockIdx.x * (uint32_t)kTileScanBlock, i = i0 + threadIdx.x;
     uint32_t before = 0;
 #pragma unroll 8
     for (uint32_t e = threadIdx.x; e < i0; e += (uint32_t)kTileScanBlock) before += tsum[e];
     const uint32_t own = i < T ? tsum[i] : 0u;
+    const uint32_t held = tile_pre && i < T ? tile_pre[i] : 0u;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
     if ((threadIdx.x & 63u) == 0u) s_pre[threadIdx.x >> 6] = before;
@@ -147,7 +152,15 @@ __global__ __launch_bounds__(kTileScanBlock) void tile_scan_kernel(uint32_t* __r
     uint32_t run = block_scan<kTileScanBlock>(own, s_w, total);
 #pragma unroll
     for (int w = 0; w < kTileScanBlock / 64; ++w) run += s_pre[w];
-    if (i < T) head[C + T + i] = run;
+    if (i < T) head[C + T + 1u + i] = run;
+    if (!tile_pre) return;
+    const bool need = i < T && (own != 0u || held != run);
+    uint32_t listed;
+    __syncthreads();  // s_w is read by the scan before
+    const uint32_t at = block_scan<kTileScanBlock>(need ? 1u : 0u, s_w, listed);
+    if (threadIdx.x == 0 && listed) s_at = atomicAdd(head + C + T, listed);
+    __syncthreads();
+    if (need) head[C + 2u * T + 1u + s_at + at] = i;
 }
 
 // Members a cell may hold for the stable in-cell rank.  Rest-density fluid
@@ -205,71 +218,68 @@ constexpr int kHeldLinks = 5;
 // (54 tiles) 7.0 against 11.5 us, 65k dam break (489 tiles) 7.8 against 11.3
 // us, 1M (2013 tiles) 29.2 against 23.1 us.
 template <int BLOCK, int V>
-__global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
-    // A frame that is complete (pending, or halted already) skips the step;
-    // the first kernel of the step turns pending into halt for the others.
-    if (a.frame && (a.frame[0] | a.frame[1])) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) a.frame[0] = 1u;
-        return;
-    }
-    constexpr uint32_t kCells = (uint32_t)(BLOCK * V);
-    constexpr uint32_t kMembers = kCells * 8u < kTileMembers ? kCells * 8u : kTileMembers;
+struct TileSort {
+    static constexpr uint32_t kCells = (uint32_t)(BLOCK * V);
+    static constexpr uint32_t kMembers = kCells * 8u < kTileMembers ? kCells * 8u : kTileMembers;
     // A tile whose runs are ranked keeps each cell's first run in that room.
-    constexpr uint32_t kRanked = kMembers - (kCells + 1u);
+    static constexpr uint32_t kRanked = kMembers - (kCells + 1u);
     static_assert(kCells <= 1u << kTileShiftMax, "a tile");
-    constexpr int kWaves = BLOCK / 64;
     static_assert(V == 1 || V == 4, "one head, or four in one 16-byte load, per thread");
-    __shared__ uint32_t s_w[kWaves];
-    __shared__ uint32_t s_pre[kWaves];
-    __shared__ uint32_t s_big;
-    __shared__ uint32_t s_off[kCells + 1];
-    __shared__ uint32_t s_mem[kMembers];
-    __shared__ uint32_t s_unsorted;
-    const uint32_t b = blockIdx.x, C = a.C;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // Tile counters of this step's persistent density and force launches.
-    if (b == 0 && tid < kQueueWords && a.queue) a.queue[tid] = 0u;
-    const uint32_t T = gridDim.x;
+    uint32_t w[BLOCK / 64];
+    uint32_t pre[BLOCK / 64];
+    uint32_t big, unsorted;
+    uint32_t off[kCells + 1];
+    uint32_t mem[kMembers];
+};
+
+// The cells of tile b that a thread owns: V == 4 has four of a whole tile, one
+// or none where V == 1; past the grid none.  [i0, end), whole: V of them.
+template <int V>
+struct OwnCells {
+    uint32_t i0, end;
+    bool whole;
+    __device__ __forceinline__ OwnCells(const CellSortArgs& a, uint32_t b) {
+        const uint32_t base = b << a.shift, cells = 1u << a.shift;
+        i0 = base + (uint32_t)V * threadIdx.x;
+        end = V == 1 && base + cells < a.C ? base + cells : a.C;
+        whole = i0 + (uint32_t)V <= end;
+    }
+    __device__ __forceinline__ void heads(const CellSortArgs& a, uint32_t (&r)[V]) const {
+        if (V == 4 && whole) {
+            const uint4 hv = *reinterpret_cast<const uint4*>(a.head + i0);
+            r[0] = hv.x;
+            r[V > 1 ? 1 : 0] = V > 1 ? hv.y : hv.x;
+            r[V > 2 ? 2 : 0] = V > 2 ? hv.z : hv.x;
+            r[V > 3 ? 3 : 0] = V > 3 ? hv.w : hv.x;
+        } else {
+#pragma unroll
+            for (int v = 0; v < V; ++v) r[v] = i0 + (uint32_t)v < end ? a.head[i0 + v] : 0u;
+        }
+    }
+};
+
+// Sorts tile b of T: pre particles before it, `members` in it, heads its own
+// cells' chains, held what tile_pre says of it (read by every thread before any
+// thread of the block rewrites it).  sh.big and sh.unsorted are 0.
+template <int BLOCK, int V>
+__device__ __forceinline__ void sort_tile(const CellSortArgs& a, TileSort<BLOCK, V>& sh, uint32_t T, uint32_t b,
+                                          uint32_t pre, uint32_t members, uint32_t held, const OwnCells<V>& own_cells,
+                                          const uint32_t (&heads)[V]) {
+    constexpr uint32_t kCells = TileSort<BLOCK, V>::kCells, kMembers = TileSort<BLOCK, V>::kMembers,
+                       kRanked = TileSort<BLOCK, V>::kRanked;
+    uint32_t(&s_w)[BLOCK / 64] = sh.w;
+    uint32_t &s_big = sh.big, &s_unsorted = sh.unsorted;
+    uint32_t(&s_off)[kCells + 1] = sh.off;
+    uint32_t(&s_mem)[kMembers] = sh.mem;
+    const uint32_t C = a.C;
+    const int tid = threadIdx.x;
     const uint32_t cells = 1u << a.shift;
     const uint32_t base = b << a.shift;
-    const uint32_t i0 = base + (uint32_t)(V * tid);
+    const uint32_t i0 = own_cells.i0, Ce = own_cells.end;
+    const bool whole = own_cells.whole;
     uint32_t r[kHeldLinks + 1][V];
-    // Cells of this thread: V == 4 has four of a whole tile, one or none where
-    // V == 1; past the grid none.
-    const uint32_t Ce = V == 1 && base + cells < C ? base + cells : C;
-    const bool whole = i0 + (uint32_t)V <= Ce;
-    if (V == 4 && whole) {
-        const uint4 hv = *reinterpret_cast<const uint4*>(a.head + i0);
-        r[0][0] = hv.x;
-        r[0][V > 1 ? 1 : 0] = V > 1 ? hv.y : hv.x;
-        r[0][V > 2 ? 2 : 0] = V > 2 ? hv.z : hv.x;
-        r[0][V > 3 ? 3 : 0] = V > 3 ? hv.w : hv.x;
-    } else {
 #pragma unroll
-        for (int v = 0; v < V; ++v) r[0][v] = i0 + (uint32_t)v < Ce ? a.head[i0 + v] : 0u;
-    }
-    // What the table holds for this tile, read by every thread before any
-    // thread of the block rewrites it.
-    const uint32_t held = a.tile_pre[b];
-    const uint32_t members = a.head[C + b];
-    uint32_t pre;
-    if (T <= kInlineTiles) {
-        uint32_t x = 0;
-#pragma unroll 8
-        for (uint32_t i = (uint32_t)tid; i < b; i += BLOCK) x += a.head[C + i];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-        if (lane == 0) s_pre[wave] = x;
-        if (tid == 0) s_big = s_unsorted = 0u;
-        __syncthreads();
-        pre = 0u;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) pre += s_pre[w];
-    } else {
-        pre = a.head[C + T + b];
-        if (tid == 0) s_big = s_unsorted = 0u;
-        __syncthreads();
-    }
+    for (int v = 0; v < V; ++v) r[0][v] = heads[v];
     if (members == 0u) {
         // An empty tile's cells all hold its prefix; skip the rewrite when
         // this table already holds that prefix there (most empty tiles of
@@ -591,6 +601,83 @@ __global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
     }
 }
 
+template <int BLOCK, int V>
+__global__ __launch_bounds__(BLOCK) void cell_sort_kernel(CellSortArgs a) {
+    // A frame that is complete (pending, or halted already) skips the step;
+    // the first kernel of the step turns pending into halt for the others.
+    if (a.frame && (a.frame[0] | a.frame[1])) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.frame[0] = 1u;
+        return;
+    }
+    constexpr int kWaves = BLOCK / 64;
+    __shared__ TileSort<BLOCK, V> sh;
+    const uint32_t b = blockIdx.x, C = a.C;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // Tile counters of this step's persistent density and force launches.
+    if (b == 0 && tid < kQueueWords && a.queue) a.queue[tid] = 0u;
+    const uint32_t T = gridDim.x;
+    const OwnCells<V> own(a, b);
+    uint32_t heads[V];
+    own.heads(a, heads);
+    const uint32_t held = a.tile_pre[b];
+    const uint32_t members = a.head[C + b];
+    uint32_t pre;
+    if (T <= kInlineTiles) {
+        uint32_t x = 0;
+#pragma unroll 8
+        for (uint32_t i = (uint32_t)tid; i < b; i += BLOCK) x += a.head[C + i];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+        if (lane == 0) sh.pre[wave] = x;
+        if (tid == 0) sh.big = sh.unsorted = 0u;
+        __syncthreads();
+        pre = 0u;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) pre += sh.pre[w];
+    } else {
+        pre = a.head[C + T + 1u + b];
+        if (tid == 0) sh.big = sh.unsorted = 0u;
+        __syncthreads();
+    }
+    sort_tile<BLOCK, V>(a, sh, T, b, pre, members, held, own, heads);
+}
+
+// A sparse grid's tiles are mostly empty, and a block of its own for each of
+// them, whose reads of the prefix and of the table wait on each other, takes
+// most of the sort.  Where tile_scan_kernel runs anyway it lists the tiles
+// that need work, and as many blocks as are resident at once take those in
+// turn.  Sort pass, block per tile against list: 1,100 scenes of 125 particles
+// (134,000 tiles) 115 -> 33 us, 260 of 512 (32,000) 35 -> 20, 60 of 180 (7,300)
+// 16.1 -> 15.0.  With fewer tiles the scan's launch costs what the list saves
+// (30 scenes of 4,600, 3,700 tiles: 15.6 against 18.1); with more particles a
+// tile few are empty.
+constexpr uint32_t kSparseMembers = 64;    // particles per tile below which
+constexpr uint32_t kSparseBlocks = 1536;   // six a CU, as registers allow
+
+template <int BLOCK, int V>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) void cell_sort_sparse_kernel(
+    CellSortArgs a, uint32_t T) {
+    if (a.frame && (a.frame[0] | a.frame[1])) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.frame[0] = 1u;
+        return;
+    }
+    __shared__ TileSort<BLOCK, V> sh;
+    const uint32_t C = a.C;
+    if (blockIdx.x == 0 && threadIdx.x < (uint32_t)kQueueWords && a.queue) a.queue[threadIdx.x] = 0u;
+    const uint32_t listed = a.head[C + T];
+    for (uint32_t i = blockIdx.x; i < listed; i += gridDim.x) {
+        const uint32_t t = a.head[C + 2u * T + 1u + i];
+        const OwnCells<V> own(a, t);
+        uint32_t heads[V];
+        own.heads(a, heads);
+        const uint32_t pre = a.head[C + T + 1u + t], members = a.head[C + t], held = a.tile_pre[t];
+        __syncthreads();  // the tile before is done with the room they share
+        if (threadIdx.x == 0) sh.big = sh.unsorted = 0u;
+        __syncthreads();
+        sort_tile<BLOCK, V>(a, sh, T, t, pre, members, held, own, heads);
+    }
+}
+
 // --------------------------------------------------------------------- radix
 
 // Digit histograms of all passes; zeroes the look-back status words and the
@@ -786,9 +873,10 @@ int sort_key_passes(uint32_t ncells) {
 
 static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
     const uint32_t tiles = scan_tiles(sp.ncells, sp.tile_shift);
+    const bool sparse = tiles > kInlineTiles && sp.n / tiles < kSparseMembers && sp.tile_shift == kTileShiftMax;
     if (tiles > kInlineTiles)
         hipLaunchKernelGGL(tile_scan_kernel, dim3((tiles + kTileScanBlock - 1) / kTileScanBlock), dim3(kTileScanBlock),
-                           0, st, sp.head, sp.ncells, tiles, sp.frame);
+                           0, st, sp.head, sp.ncells, tiles, sp.frame, sparse ? sp.tile_pre : nullptr);
     CellSortArgs a;
     a.n = sp.n;
     a.C = sp.ncells;
@@ -816,6 +904,9 @@ static void launch_cell_sort(hipStream_t st, const SortPlan& sp, int gather) {
         hipLaunchKernelGGL(SPH_CELL_SORT(256, 1), dim3(tiles), dim3(256), 0, st, a);
     else if (sp.tile_shift == 9u)
         hipLaunchKernelGGL(SPH_CELL_SORT(512, 1), dim3(tiles), dim3(512), 0, st, a);
+    else if (sparse)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(cell_sort_sparse_kernel<256, 4>), dim3(kSparseBlocks), dim3(256), 0, st, a,
+                           tiles);
     else
         hipLaunchKernelGGL(SPH_CELL_SORT(256, 4), dim3(tiles), dim3(256), 0, st, a);
 }

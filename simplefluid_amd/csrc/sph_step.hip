@@ -597,7 +597,7 @@ __device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
         }
     }
     if (!a.head) return;
-    const uint32_t words = scan_tiles(a.ncells, a.tile_shift);
+    const uint32_t words = scan_tiles(a.ncells, a.tile_shift) + 1u;  // and the sparse sort's count
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
         a.head[a.ncells + i] = 0u;
 }
