@@ -133,7 +133,7 @@ extern "C" int sph_autotune(sph_handle* h) {
     // while compression and the reverse pass, which takes the force pass's
     // form, favour the size's: 16 scenes of 32,768 particles reverse 200 steps
     // in 36.0 ms staged and in 41.9 where a trial preferred the gathered force.
-    const int of_size = n >= kStagedFrom ? 1 : 0;
+    const int of_size = staged_by_size(h);
     auto beats = [&](double t, double best_ms, int staged) { return t < (staged == of_size ? 1.0 : 0.95) * best_ms; };
     // Launch form of density and force (persistent or one block per tile;
     // force rows staged in LDS or gathered), judged on their summed time.

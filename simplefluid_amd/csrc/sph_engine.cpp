@@ -205,7 +205,7 @@ uint32_t grid_for(sph_handle* h, int block, uint32_t ntiles, uint32_t** queue, i
 }
 
 bool split_form(const sph_handle* h) {
-    return h->tune.split && h->split_tiles <= kSplitTiles && h->nlist;
+    return h->tune.split && h->split_tiles <= kSplitTiles && !h->wide_rows && h->nlist;
 }
 
 StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
@@ -313,7 +313,7 @@ static int ensure_buffers(sph_handle* h) {
     h->mask_hi = h->ncount = nullptr;
     h->nlist = nullptr;
     static_assert(kListMax % 2 == 0, "lists of whole words");
-    const size_t list_words = h->split_tiles <= kSplitTiles ? (kListMax / 2 + 1) * n : 0;
+    const size_t list_words = h->split_tiles <= kSplitTiles && !h->wide_rows ? (kListMax / 2 + 1) * n : 0;
     for (const size_t words : {list_words, (size_t)0}) {  // without the lists where only the masks fit
         if (h->spare.ensure(words + (size_t)kRows * n) == hipSuccess) {
             if (words) {
@@ -656,6 +656,8 @@ static int configure(sph_handle* h, const std::vector<sph_params>& ps, const std
     h->tile_shift = tile_shift_for(h->ncells, h->n, members);
     h->split_tiles = 0;
     for (uint32_t v : ns) h->split_tiles += (v + kSplitTile - 1) / kSplitTile;
+    h->wide_rows = false;
+    for (const sph_params& p : ps) h->wide_rows |= cell_members(p, 1) > kWideRows;
     h->xsub = xsub;
     h->cfl = ps.size() == 1 && ps[0].cfl_number > 0.f;
     h->tiles.clear();

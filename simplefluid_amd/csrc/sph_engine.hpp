@@ -153,6 +153,7 @@ struct sph_handle {
     uint32_t tile_shift = 0;               // cells per tile of the sort, as a shift
     int passes = 1;
     uint32_t split_tiles = 0;              // tiles of the split form, scene by scene
+    bool wide_rows = false;                // a support of more than kWideRows
     int xsub = 1;                          // x cells per y/z cell size
     int xsub_override = 0;                 // 0 = automatic
     bool ready = false;
@@ -247,9 +248,18 @@ uint2* tiles_for(sph_handle* h, int block, uint32_t& ntiles);
 // the launch is persistent, else null.
 // blocks_per_cu: the kernel's resident blocks per CU (0: 2048 lanes' worth).
 uint32_t grid_for(sph_handle* h, int block, uint32_t ntiles, uint32_t** queue, int blocks_per_cu = 0);
-// Density and force run in the split form: few enough tiles, its lists
-// allocated, and no other form asked for (sph_set_tuning).
+// Density and force run in the split form: few enough tiles, rows not too
+// wide, its lists allocated, and no other form asked for (sph_set_tuning).
 bool split_form(const sph_handle* h);
+// Particles of fluid at rest in a cube of the support radius's side up to
+// which a row's candidates fit a wave's copy (64 + twice as many are 124 of
+// 120) and a particle's neighbours its list (4 pi / 3 times as many are 126 of
+// 128).  Measured per step, gathered against the form of the handle's size, at
+// a support of 6, 7, 8 and 12 particle radii (27, 43, 64 and 216 in the cube):
+// 31,713 particles 78 / 64, 185 / 195, 244 / 267, 1,022 / 1,020 us; 216,000
+// 146 / 144, 296 / 349, 396 / 528, 1,497 / 1,802; 1M 499 / 470, 1,063 / 1,170,
+// 1,525 / 1,910 (at 8).
+constexpr float kWideRows = 30.0f;
 // Particles from which a handle no one has tuned stages density and force.
 // Below, a wave's copies and bounds cost more than its gathers, whose records
 // are in cache.  Measured per step, gathered against staged, fresh and after
@@ -258,11 +268,12 @@ bool split_form(const sph_handle* h);
 // 64.5 / 74.6 against 62.2 / 69.7, 40 scenes of 25k 236.7 / 302.0 against
 // 186.7 / 238.0, 1M 216.8 / 322.8 against 167.0 / 233.2.
 constexpr uint32_t kStagedFrom = 1u << 17;
+inline int staged_by_size(const sph_handle* h) { return h->n >= kStagedFrom && !h->wide_rows; }
 inline int force_staged(const sph_handle* h) {
-    return h->tune.by_size ? h->n >= kStagedFrom : h->tune.force_staged;
+    return h->tune.by_size ? staged_by_size(h) : h->tune.force_staged;
 }
 inline int density_staged(const sph_handle* h) {
-    return h->tune.by_size ? h->n >= kStagedFrom : h->tune.density_staged;
+    return h->tune.by_size ? staged_by_size(h) : h->tune.density_staged;
 }
 StepArgs step_args(sph_handle* h, StepBufs& w, int block);
 // Enqueue one step reading/writing the state buffers with intermediates in w.

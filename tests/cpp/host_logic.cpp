@@ -157,11 +157,12 @@ namespace {
         }                                                             \
     } while (0)
 
-sph_handle* make(uint32_t n, float h = 0.02f) {
+// ratio: the support in particle radii.
+sph_handle* make(uint32_t n, float ratio = 4.0f) {
     sph_params p;
     sph_params_default(&p);
-    p.kernel_radius = h;
-    p.particle_radius = h / 4;
+    p.particle_radius = 0.005f;
+    p.kernel_radius = ratio * 0.005f;
     sph_handle* e = nullptr;
     if (sph_create(&p, &e) != SPH_OK) std::exit(4);
     std::vector<float> x(3 * (size_t)n, 0.1f);
@@ -261,6 +262,24 @@ int new_spares_drop_the_graphs() {
     return 0;
 }
 
+// The forms that hold a row's candidates or a particle's neighbours in room of
+// a fixed size are left to supports whose rows and neighbours fit them.
+int wide_rows_are_gathered() {
+    for (uint32_t n : {5000u, 200000u})
+        for (float ratio : {4.0f, 6.0f, 7.0f, 12.0f}) {
+            sph_handle* e = make(n, ratio);
+            CHECK(sph_set_use_graph(e, 0) == SPH_OK);
+            fake::launched.clear();
+            CHECK(sph_advance_steps(e, 1) == SPH_OK);
+            const bool wide = ratio > 6.5f;
+            CHECK(fake::count("density_kernel") == wide && fake::count("force_kernel") == wide);
+            CHECK(fake::count("split") == (!wide && n == 5000u ? 2 : 0));
+            CHECK(fake::count("staged") == (!wide && n == 200000u ? 2 : 0));
+            sph_destroy(e);
+        }
+    return 0;
+}
+
 struct Check {
     const char* name;
     int (*run)();
@@ -269,6 +288,7 @@ const Check kChecks[] = {
     {"autotune_keeps_the_sort", autotune_keeps_the_sort},
     {"hash_without_its_table_fails", hash_without_its_table_fails},
     {"new_spares_drop_the_graphs", new_spares_drop_the_graphs},
+    {"wide_rows_are_gathered", wide_rows_are_gathered},
 };
 
 }  // namespace
