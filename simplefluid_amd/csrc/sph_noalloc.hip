@@ -6,9 +6,9 @@
 // capture or a serving loop that runs one fluid step per request.
 //
 // The step is the one sph_advance_steps runs as the first step after
-// sph_set_particles (hash, cell-count sort, gather, density, force), with the
-// same kernels in their split form and the same grid rule, so its results
-// equal that entry point's bit for bit.
+// sph_set_particles (hash, cell-count sort, density, force), with the same
+// kernels, form and grid rule, so its results equal that entry point's bit for
+// bit.
 //
 // Limits: at most kMaxParticles particles and kMaxCells grid cells (the
 // largest x subdivision of 4, 2, 1 whose grid fits is used, as a handle of
@@ -28,7 +28,7 @@ namespace {
 constexpr uint32_t kMaxParticles = 65536;
 constexpr uint32_t kMaxCells = 1u << 20;
 constexpr uint32_t kMaxTiles = kMaxParticles / kSplitTile;
-static_assert(kMaxParticles <= kSplitMax, "the step runs in the split form");
+constexpr uint32_t kBlock = 256;  // tiles of the gathered form
 constexpr uint32_t kScanTilesMax = 2048;
 static_assert(scan_tiles(kMaxCells, tile_shift_for(kMaxCells)) <= kScanTilesMax &&
                   scan_tiles(1u << 19, tile_shift_for(1u << 19)) <= kScanTilesMax && kMaxParticles / 64 < kScanTilesMax,
@@ -49,6 +49,10 @@ struct Layout {
     static constexpr size_t tmp = align256(next + 4 * N);
     static constexpr size_t perm = align256(tmp + 4 * N);
     static constexpr size_t nlist = align256(perm + 4 * N);
+    // The gathered form's planes and second mask words, in the lists' room.
+    static constexpr size_t soa = nlist;
+    static constexpr size_t mask_hi = align256(soa + 12 * N);
+    static_assert(mask_hi + 4 * (size_t)kRows * N <= nlist + 2 * (size_t)kListMax * N, "they fit there");
     static constexpr size_t ncount = align256(nlist + 2 * (size_t)kListMax * N);
     static constexpr size_t rho = align256(ncount + 4 * N);
     static constexpr size_t mask = align256(rho + 4 * N);
@@ -70,9 +74,10 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 void* g_scratch[kMaxDevices] = {};
 
-// Scene constants, the tile table (scene 0, first particle t * kSplitTile),
-// empty chains, tile sums and tile prefixes, and the error word cleared.
-__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint32_t tile_shift, uint8_t* __restrict__ base) {
+// Scene constants, the tile table (scene 0, first particle t * block), empty
+// chains, tile sums and tile prefixes, and the error word cleared.
+__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint32_t tile_shift, uint32_t block,
+                                     uint8_t* __restrict__ base) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
     if (i == 0) {
         *reinterpret_cast<SceneConst*>(base + Layout::scene) = sc;
@@ -86,7 +91,7 @@ __global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint32_t ti
     uint32_t* tile_pre = reinterpret_cast<uint32_t*>(base + Layout::tile_pre);
     for (uint32_t t = i; t < T; t += stride) tile_pre[t] = 0xffffffffu;
     uint2* tiles = reinterpret_cast<uint2*>(base + Layout::tiles);
-    for (uint32_t t = i; t * kSplitTile < sc.p_end; t += stride) tiles[t] = make_uint2(0u, t * kSplitTile);
+    for (uint32_t t = i; t * block < sc.p_end; t += stride) tiles[t] = make_uint2(0u, t * block);
 }
 
 // The scratch address on the current device, looked up once per device.
@@ -156,9 +161,12 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     uint32_t* next = reinterpret_cast<uint32_t*>(at(Layout::next));
     const SceneConst* scd = reinterpret_cast<const SceneConst*>(at(Layout::scene));
 
+    // The form a handle of so many particles and such rows takes.
+    const bool split = (n + kSplitTile - 1) / kSplitTile <= kSplitTiles && !(cell_members(*p, 1) > kWideRows);
+    const uint32_t block = split ? (uint32_t)kSplitTile : kBlock;
     // Five launches: setup, upload and hash, sort, density, force (which
     // writes the caller's arrays itself).
-    hipLaunchKernelGGL(noalloc_setup_kernel, dim3(256), dim3(256), 0, st, sc, C, shift, base);
+    hipLaunchKernelGGL(noalloc_setup_kernel, dim3(256), dim3(256), 0, st, sc, C, shift, block, base);
     e = hipGetLastError();
     if (e == hipSuccess) e = launch_upload_hash(st, xyz_in, vel_in, pos, vel, id, key0, next, head, n, C, shift, sc);
     SortPlan sp;
@@ -180,6 +188,7 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     sp.pos_out = reinterpret_cast<float4*>(at(Layout::pos_s));
     sp.vel_out = reinterpret_cast<float4*>(at(Layout::vel_s));
     sp.id_out = reinterpret_cast<uint32_t*>(at(Layout::id_s));
+    if (!split) sp.soa_out = reinterpret_cast<float*>(at(Layout::soa));
     if (e == hipSuccess) e = launch_sort_keys(st, sp);
     StepArgs a;
     std::memset(&a, 0, sizeof(a));
@@ -191,15 +200,20 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     a.cstart = sp.cstart;
     a.rho = reinterpret_cast<float*>(at(Layout::rho));
     a.mask = reinterpret_cast<uint32_t*>(at(Layout::mask));
-    a.nlist = reinterpret_cast<uint16_t*>(at(Layout::nlist));
-    a.ncount = reinterpret_cast<uint32_t*>(at(Layout::ncount));
+    if (split) {
+        a.nlist = reinterpret_cast<uint16_t*>(at(Layout::nlist));
+        a.ncount = reinterpret_cast<uint32_t*>(at(Layout::ncount));
+    } else {
+        a.soa = sp.soa_out;
+        a.mask_hi = reinterpret_cast<uint32_t*>(at(Layout::mask_hi));
+    }
     a.scenes = scd;
     a.tiles = reinterpret_cast<const uint2*>(at(Layout::tiles));
-    a.ntiles = (n + kSplitTile - 1) / kSplitTile;
+    a.ntiles = (n + block - 1) / block;
     a.n = n;
     a.ncells = C;
-    if (e == hipSuccess) e = launch_density_split(st, a);
-    if (e == hipSuccess) e = launch_force_split(st, a);
+    if (e == hipSuccess) e = split ? launch_density_split(st, a) : launch_density(st, (int)block, a.ntiles, a);
+    if (e == hipSuccess) e = split ? launch_force_split(st, a) : launch_force(st, (int)block, a.ntiles, a);
     if (e != hipSuccess) return fail_noalloc(SPH_E_HIP, "sph_step_noalloc: kernel launch failed");
     return SPH_OK;
 }
