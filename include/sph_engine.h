@@ -229,16 +229,19 @@ int  sph_profile_read(sph_handle* h, double* ms_per_pass, uint32_t* steps);
  * fastest (state is saved and restored).  Results are cached per process
  * keyed by (device arch, particle-count bucket, scene count).               */
 int  sph_autotune(sph_handle* h);
-/* Current choice (5 ints): block sizes of density, force and reorder, the
- * sort items per thread, and the launch form: bit 0 set when density and
- * force run as persistent blocks taking tiles from per-XCD queues (clear:
- * one block per tile), bit 1 set when the force pass stages each row's
- * candidates in LDS (clear: it gathers them from global memory), bit 2 the
- * same for the density pass.  A handle of at most 40,960 particles (640 tiles
- * of 64, scene by scene) runs density and force in a form of its own that
- * none of these shape, until sph_set_tuning asks for the forms above; one of
- * 131,072 particles or more stages both until it is tuned or set.  Every
- * choice gives the same results bit for bit.                                */
+/* What the handle runs now (5 ints): block sizes of density, force and
+ * reorder, the sort items per thread, and the launch form: bit 0 set when
+ * density and force run as persistent blocks taking tiles from per-XCD queues
+ * (clear: one block per tile), bit 1 set when the force pass stages each
+ * row's candidates in LDS (clear: it gathers them from global memory), bit 2
+ * the same for the density pass, bit 3 set when both run in the small
+ * handles' form, which the others do not shape.  Until it is tuned or set, a
+ * handle picks its form by its size: the small handles' up to 40,960
+ * particles (640 tiles of 64, scene by scene), staged from 131,072 on,
+ * gathered between and where a support is more than six particle radii.
+ * sph_set_tuning asks for a form whatever the size, the small handles' (bit
+ * 3) wherever it applies; setting what sph_get_tuning returned changes
+ * nothing.  Every choice gives the same results bit for bit.                */
 int  sph_get_tuning(const sph_handle* h, int* cfg5);
 int  sph_set_tuning(sph_handle* h, const int* cfg5);
 /* Sort used to order particles by cell (no reference counterpart; both give

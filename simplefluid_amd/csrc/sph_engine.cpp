@@ -1256,7 +1256,8 @@ int sph_get_tuning(const sph_handle* h, int* cfg) {
     cfg[1] = h->tune.force_block;
     cfg[2] = h->tune.reorder_block;
     cfg[3] = h->tune.sort_items;
-    cfg[4] = h->tune.persistent | (h->tune.force_staged << 1) | (h->tune.density_staged << 2);
+    // What runs, whether asked for or picked by the handle's size.
+    cfg[4] = h->tune.persistent | (force_staged(h) << 1) | (density_staged(h) << 2) | (split_form(h) ? 8 : 0);
     return SPH_OK;
 }
 
@@ -1269,9 +1270,10 @@ int sph_set_tuning(sph_handle* h, const int* cfg) {
         return fail(h, SPH_E_INVALID, "block sizes must be 64, 128, 256 or 512");
     if (cfg[3] != 4 && cfg[3] != 8 && cfg[3] != 12 && cfg[3] != 16)
         return fail(h, SPH_E_INVALID, "sort items must be 4, 8, 12 or 16");
-    if (cfg[4] < 0 || cfg[4] > 7)
+    if (cfg[4] < 0 || cfg[4] > 15)
         return fail(h, SPH_E_INVALID,
-                    "launch form must be 0 to 7 (bit 0 persistent, bit 1 staged force, bit 2 staged density)");
+                    "launch form must be 0 to 15 (bit 0 persistent, bit 1 staged force, bit 2 staged density, bit 3 "
+                    "split where it applies)");
     h->tune.density_block = cfg[0];
     h->tune.force_block = cfg[1];
     h->tune.reorder_block = cfg[2];
@@ -1280,7 +1282,7 @@ int sph_set_tuning(sph_handle* h, const int* cfg) {
     h->tune.force_staged = (cfg[4] >> 1) & 1;
     h->tune.density_staged = (cfg[4] >> 2) & 1;
     h->tune.by_size = 0;
-    h->tune.split = 0;
+    h->tune.split = (cfg[4] >> 3) & 1;
     invalidate_graph(h);
     return SPH_OK;
 }

@@ -110,7 +110,7 @@ struct Tuning {
     int by_size = 1;      // 1 force and density are staged by the handle's size (kStagedFrom), 0 as the two fields
                           // above say (sph_set_tuning, sph_autotune)
     int split = 1;        // density and force: 1 the split form where it applies (split_form), 0 the forms above
-                          // (sph_set_tuning)
+                          // (sph_set_tuning without its bit)
     int sort_mode = kSortCellCount;
 };
 

@@ -280,6 +280,47 @@ int wide_rows_are_gathered() {
     return 0;
 }
 
+// sph_get_tuning says what runs, and setting that changes nothing: small, in
+// between, large, tuned and set handles.
+int tuning_round_trip() {
+    struct {
+        uint32_t n;
+        float ratio;
+        int form;  // launch form an untuned handle reports
+    } const kinds[] = {{5000u, 4.0f, 8}, {40960u, 4.0f, 8}, {40961u, 4.0f, 0}, {131071u, 4.0f, 0},
+                       {131072u, 4.0f, 6}, {5000u, 8.0f, 0}, {200000u, 8.0f, 0}};
+    for (const auto& kind : kinds)
+        for (int how = 0; how < 3; ++how) {  // untuned, autotuned, set to other forms
+            sph_handle* e = make(kind.n, kind.ratio);
+            CHECK(sph_set_use_graph(e, 0) == SPH_OK);
+            if (how == 1) CHECK(sph_autotune(e) == SPH_OK);
+            const int other[5] = {128, 64, 256, 8, 4};
+            if (how == 2) CHECK(sph_set_tuning(e, other) == SPH_OK);
+            int cfg[5], again[5];
+            CHECK(sph_get_tuning(e, cfg) == SPH_OK);
+            if (how == 0) CHECK(cfg[4] == kind.form);
+            if (how == 2) CHECK(std::memcmp(cfg, other, sizeof(cfg)) == 0);
+            CHECK(sph_advance_steps(e, 1) == SPH_OK);
+            fake::launched.clear();
+            CHECK(sph_advance_steps(e, 1) == SPH_OK);
+            const std::vector<std::string> before = fake::launched;
+            CHECK(fake::count("split") == ((cfg[4] & 8) ? 2 : 0));
+            if (!(cfg[4] & 8)) {
+                CHECK(fake::count("force_staged") == ((cfg[4] >> 1) & 1));
+                CHECK(fake::count("density_staged") == ((cfg[4] >> 2) & 1));
+            }
+            CHECK(sph_set_tuning(e, cfg) == SPH_OK);
+            CHECK(sph_get_tuning(e, again) == SPH_OK && std::memcmp(cfg, again, sizeof(cfg)) == 0);
+            fake::launched.clear();
+            CHECK(sph_advance_steps(e, 1) == SPH_OK);
+            CHECK(fake::launched == before);
+            const int bad[5] = {256, 256, 256, 8, 16};
+            CHECK(sph_set_tuning(e, bad) == SPH_E_INVALID);
+            sph_destroy(e);
+        }
+    return 0;
+}
+
 struct Check {
     const char* name;
     int (*run)();
@@ -289,6 +330,7 @@ const Check kChecks[] = {
     {"hash_without_its_table_fails", hash_without_its_table_fails},
     {"new_spares_drop_the_graphs", new_spares_drop_the_graphs},
     {"wide_rows_are_gathered", wide_rows_are_gathered},
+    {"tuning_round_trip", tuning_round_trip},
 };
 
 }  // namespace
