@@ -6,8 +6,9 @@
 // restored before every trial, so all candidates run the same steps.
 // Results are cached per process, keyed by device arch, particle-count
 // bucket (power of two), scene count, x subdivision and sort mode (which is
-// the handle's own: its buffers are allocated for it).  A handle small enough for the split
-// form runs that, which has no shape to choose.
+// the handle's own: its buffers are allocated for it).  A handle small enough
+// for the split form runs density and force in that, which has no shape to
+// choose; its sort has one in radix mode.
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -23,11 +24,11 @@ namespace {
 std::mutex g_mu;
 std::map<std::string, Tuning> g_cache;
 
-std::string cache_key(const sph_handle* h) {
+std::string cache_key(const sph_handle* h, bool split) {
     int bucket = 0;
     while ((1u << bucket) < h->n && bucket < 31) ++bucket;
     return h->arch + ":" + std::to_string(bucket) + ":" + std::to_string(h->sc_h.size()) + ":" +
-           std::to_string(h->xsub) + ":" + std::to_string(h->tune.sort_mode);
+           std::to_string(h->xsub) + ":" + std::to_string(h->tune.sort_mode) + (split ? ":split" : h->wide_rows ? ":wide" : "");
 }
 
 struct Saved {
@@ -42,14 +43,14 @@ extern "C" int sph_autotune(sph_handle* h) {
     if (!h) return SPH_E_INVALID;
     if (!h->ready) return fail(h, SPH_E_NOT_READY, "call sph_make_ready first");
     h->tune.split = 1;
-    if (split_form(h)) {  // has no shape to choose
+    const bool radix = h->tune.sort_mode == kSortRadix;
+    if (split_form(h) && !radix) {  // no shape to choose
         invalidate_graph(h);
         return SPH_OK;
     }
-    const std::string key = cache_key(h);
     {
         std::lock_guard<std::mutex> lk(g_mu);
-        auto it = g_cache.find(key);
+        auto it = g_cache.find(cache_key(h, split_form(h)));
         if (it != g_cache.end()) {
             const int mode = h->tune.sort_mode;
             h->tune = it->second;
@@ -67,6 +68,8 @@ extern "C" int sph_autotune(sph_handle* h) {
     if (e == hipSuccess) e = hipMemcpyAsync(sv.vel.p, h->vel.p, n * sizeof(float4), hipMemcpyDeviceToDevice, h->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(sv.id.p, h->id.p, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "autotune save");
+    const bool split = split_form(h);  // still, with the state saved
+    const std::string key = cache_key(h, split);
 
     const bool prof_was = h->prof;
     auto restore = [&]() -> hipError_t {
@@ -101,7 +104,7 @@ extern "C" int sph_autotune(sph_handle* h) {
     const int items[] = {4, 8, 12, 16};
     const Tuning before = h->tune;
     Tuning best = h->tune;
-    best.by_size = 0;
+    if (!split) best.by_size = 0;
     double ms[SPH_NUM_PASSES];
     int rc = SPH_OK;
     // Density and force blocks, then reorder block, then sort items.
@@ -112,9 +115,10 @@ extern "C" int sph_autotune(sph_handle* h) {
                    {&best.sort_items, items, 4, SPH_PASS_SORT}};
     for (const Axis& ax : axes) {
         if (rc != SPH_OK) break;
-        // The gather's block and the keys per thread only shape the radix sort.
-        if ((ax.field == &best.sort_items || ax.field == &best.reorder_block) && best.sort_mode != kSortRadix)
-            continue;
+        // The gather's block and the keys per thread only shape the radix sort,
+        // the others only the forms that are not split.
+        const bool of_sort = ax.field == &best.sort_items || ax.field == &best.reorder_block;
+        if (of_sort ? !radix : split) continue;
         double best_ms = 1e30;
         int best_v = *ax.field;
         for (int c = 0; c < ax.ncand; ++c) {
@@ -137,7 +141,7 @@ extern "C" int sph_autotune(sph_handle* h) {
     auto beats = [&](double t, double best_ms, int staged) { return t < (staged == of_size ? 1.0 : 0.95) * best_ms; };
     // Launch form of density and force (persistent or one block per tile;
     // force rows staged in LDS or gathered), judged on their summed time.
-    if (rc == SPH_OK) {
+    if (rc == SPH_OK && !split) {
         double best_ms = 1e30;
         int best_v = of_size << 1;
         for (int i = 0; i < 4; ++i) {
@@ -154,7 +158,7 @@ extern "C" int sph_autotune(sph_handle* h) {
         best.force_staged = best_v >> 1;
     }
     // Density rows staged in LDS or read from global memory.
-    if (rc == SPH_OK) {
+    if (rc == SPH_OK && !split) {
         double best_ms = 1e30;
         int best_v = of_size;
         for (int i = 0; i < 2; ++i) {

@@ -321,6 +321,27 @@ int tuning_round_trip() {
     return 0;
 }
 
+// Small handles have no density and force shapes to choose, but the radix
+// sort's are timed for them as for others, for each a set of its own.
+int autotune_times_the_radix_sort() {
+    for (uint32_t n : {5000u, 33000u, 60000u}) {  // two of one size bucket
+        sph_handle* e = make(n);
+        CHECK(sph_set_sort_mode(e, SPH_SORT_RADIX) == SPH_OK);
+        fake::launched.clear();
+        CHECK(sph_autotune(e) == SPH_OK);
+        for (const char* kernel : {"radix_pass_kernelILi4E", "radix_pass_kernelILi16E"}) CHECK(fake::count(kernel) > 0);
+        CHECK((fake::count("split") > 0) == (n < 40960u));
+        CHECK((fake::count("staged") > 0) == (n > 40960u));
+        sph_destroy(e);
+        e = make(n);  // cell counts: nothing to time where the form has no shape
+        fake::launched.clear();
+        CHECK(sph_autotune(e) == SPH_OK);
+        CHECK((fake::launched.size() > 0) == (n > 40960u));
+        sph_destroy(e);
+    }
+    return 0;
+}
+
 struct Check {
     const char* name;
     int (*run)();
@@ -331,6 +352,7 @@ const Check kChecks[] = {
     {"new_spares_drop_the_graphs", new_spares_drop_the_graphs},
     {"wide_rows_are_gathered", wide_rows_are_gathered},
     {"tuning_round_trip", tuning_round_trip},
+    {"autotune_times_the_radix_sort", autotune_times_the_radix_sort},
 };
 
 }  // namespace
