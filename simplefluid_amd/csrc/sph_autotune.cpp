@@ -100,76 +100,74 @@ extern "C" int sph_autotune(sph_handle* h) {
         return check_device_error(h);
     };
 
+    // The form of the handle's size: its blocks are timed first, and it stays
+    // unless the other is 5 % faster.
+    const int of_size = staged_by_size(h);
     const int blocks[] = {64, 128, 256, 512};
     const int items[] = {4, 8, 12, 16};
     const Tuning before = h->tune;
     Tuning best = h->tune;
-    if (!split) best.by_size = 0;
+    if (!split) {
+        best.by_size = 0;
+        best.force_staged = best.density_staged = of_size;
+    }
     double ms[SPH_NUM_PASSES];
     int rc = SPH_OK;
-    // Density and force blocks, then reorder block, then sort items.
-    struct Axis { int* field; const int* cand; int ncand; int pass; };
-    Axis axes[] = {{&best.density_block, blocks, 4, SPH_PASS_DENSITY},
-                   {&best.force_block, blocks, 4, SPH_PASS_FORCE},
-                   {&best.reorder_block, blocks, 4, SPH_PASS_REORDER},
-                   {&best.sort_items, items, 4, SPH_PASS_SORT}};
-    for (const Axis& ax : axes) {
-        if (rc != SPH_OK) break;
-        // The gather's block and the keys per thread only shape the radix sort,
-        // the others only the forms that are not split.
-        const bool of_sort = ax.field == &best.sort_items || ax.field == &best.reorder_block;
-        if (of_sort ? !radix : split) continue;
+    // Takes the candidate with the least time in a pass (or two) as the field's value.
+    auto choose = [&](int& field, const int* cand, int ncand, int pass) {
         double best_ms = 1e30;
-        int best_v = *ax.field;
-        for (int c = 0; c < ax.ncand; ++c) {
-            *ax.field = ax.cand[c];
+        int best_v = field;
+        for (int c = 0; c < ncand && rc == SPH_OK; ++c) {
+            field = cand[c];
             h->tune = best;
             rc = trial(ms);
-            if (rc != SPH_OK) break;
-            if (ms[ax.pass] < best_ms) { best_ms = ms[ax.pass]; best_v = ax.cand[c]; }
+            if (rc == SPH_OK && ms[pass] < best_ms) { best_ms = ms[pass]; best_v = cand[c]; }
         }
-        *ax.field = best_v;
-        if (rc != SPH_OK) break;
+        field = best_v;
+    };
+    if (!split) {
+        choose(best.density_block, blocks, 4, SPH_PASS_DENSITY);
+        choose(best.force_block, blocks, 4, SPH_PASS_FORCE);
     }
-    // Staged or gathered: the form of the handle's size unless the other is
-    // 5 % faster.  The trials are a few steps from the state as it is, often a
-    // fresh one, whose forms can lie within the trials' noise of each other
-    // while compression and the reverse pass, which takes the force pass's
-    // form, favour the size's: 16 scenes of 32,768 particles reverse 200 steps
-    // in 36.0 ms staged and in 41.9 where a trial preferred the gathered force.
-    const int of_size = staged_by_size(h);
-    auto beats = [&](double t, double best_ms, int staged) { return t < (staged == of_size ? 1.0 : 0.95) * best_ms; };
-    // Launch form of density and force (persistent or one block per tile;
-    // force rows staged in LDS or gathered), judged on their summed time.
-    if (rc == SPH_OK && !split) {
-        double best_ms = 1e30;
-        int best_v = of_size << 1;
-        for (int i = 0; i < 4; ++i) {
-            const int c = i ^ (of_size << 1);  // the form of the size first
+    // The gather's block and the keys per thread only shape the radix sort.
+    if (radix) {
+        choose(best.reorder_block, blocks, 4, SPH_PASS_REORDER);
+        choose(best.sort_items, items, 4, SPH_PASS_SORT);
+    }
+    // Staged or gathered: the trials are a few steps from the state as it is,
+    // often a fresh one, whose forms can lie within the trials' noise of each
+    // other while compression and the reverse pass, which takes the force
+    // pass's form, favour the size's: 16 scenes of 32,768 particles reverse 200
+    // steps in 36.0 ms staged and in 41.9 where a trial preferred the gathered
+    // force.  t[form]: each form's least time.
+    auto form = [&](const double (&t)[2]) { return t[!of_size] < 0.95 * t[of_size] ? !of_size : of_size; };
+    if (!split) {
+        // Launch form of density and force (persistent or one block per tile;
+        // force rows staged in LDS or gathered), judged on their summed time.
+        double t[2] = {1e30, 1e30};
+        int persistent[2] = {0, 0};
+        for (int c = 0; c < 4 && rc == SPH_OK; ++c) {
             best.persistent = c & 1;
             best.force_staged = c >> 1;
             h->tune = best;
             rc = trial(ms);
-            if (rc != SPH_OK) break;
-            const double t = ms[SPH_PASS_DENSITY] + ms[SPH_PASS_FORCE];
-            if (beats(t, best_ms, c >> 1)) { best_ms = t; best_v = c; }
+            const double sum = ms[SPH_PASS_DENSITY] + ms[SPH_PASS_FORCE];
+            if (rc == SPH_OK && sum < t[c >> 1]) { t[c >> 1] = sum; persistent[c >> 1] = c & 1; }
         }
-        best.persistent = best_v & 1;
-        best.force_staged = best_v >> 1;
-    }
-    // Density rows staged in LDS or read from global memory.
-    if (rc == SPH_OK && !split) {
-        double best_ms = 1e30;
-        int best_v = of_size;
-        for (int i = 0; i < 2; ++i) {
-            const int c = i ^ of_size;
+        best.force_staged = form(t);
+        best.persistent = persistent[best.force_staged];
+        // Density rows staged in LDS or read from global memory.
+        double d[2] = {1e30, 1e30};
+        for (int c = 0; c < 2 && rc == SPH_OK; ++c) {
             best.density_staged = c;
             h->tune = best;
             rc = trial(ms);
-            if (rc != SPH_OK) break;
-            if (beats(ms[SPH_PASS_DENSITY], best_ms, c)) { best_ms = ms[SPH_PASS_DENSITY]; best_v = c; }
+            if (rc == SPH_OK) d[c] = ms[SPH_PASS_DENSITY];
         }
-        best.density_staged = best_v;
+        best.density_staged = form(d);
+        // A form other than the blocks were timed in gets its own.
+        if (best.density_staged != of_size) choose(best.density_block, blocks, 4, SPH_PASS_DENSITY);
+        if (best.force_staged != of_size) choose(best.force_block, blocks, 4, SPH_PASS_FORCE);
     }
     h->tune = rc == SPH_OK ? best : before;
     h->prof = prof_was;
