@@ -42,6 +42,7 @@ extern "C" int sph_autotune(sph_handle* h) {
     BudgetScope budget_scope(h ? &h->mem : nullptr);
     if (!h) return SPH_E_INVALID;
     if (!h->ready) return fail(h, SPH_E_NOT_READY, "call sph_make_ready first");
+    const Tuning before = h->tune;  // stays where tuning fails
     h->tune.split = 1;
     const bool radix = h->tune.sort_mode == kSortRadix;
     if (split_form(h) && !radix) {  // no shape to choose
@@ -67,7 +68,10 @@ extern "C" int sph_autotune(sph_handle* h) {
     if (e == hipSuccess) e = hipMemcpyAsync(sv.pos.p, h->pos.p, n * sizeof(float4), hipMemcpyDeviceToDevice, h->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(sv.vel.p, h->vel.p, n * sizeof(float4), hipMemcpyDeviceToDevice, h->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(sv.id.p, h->id.p, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, h->stream);
-    if (e != hipSuccess) return hip_fail(h, e, "autotune save");
+    if (e != hipSuccess) {
+        h->tune = before;
+        return hip_fail(h, e, "autotune save");
+    }
     const bool split = split_form(h);  // still, with the state saved
     const std::string key = cache_key(h, split);
 
@@ -105,7 +109,6 @@ extern "C" int sph_autotune(sph_handle* h) {
     const int of_size = staged_by_size(h);
     const int blocks[] = {64, 128, 256, 512};
     const int items[] = {4, 8, 12, 16};
-    const Tuning before = h->tune;
     Tuning best = h->tune;
     if (!split) {
         best.by_size = 0;

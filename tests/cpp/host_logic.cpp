@@ -396,6 +396,31 @@ int autotune_compares_forms() {
     return 0;
 }
 
+// A tuning that fails leaves the shapes as they were.
+int failed_autotune_changes_nothing() {
+    const uint32_t n = 30000;
+    sph_handle* e = make(n);
+    uint64_t used = 0;
+    CHECK(sph_device_memory_used(e, &used) == SPH_OK);
+    sph_params p;
+    CHECK(sph_get_params(e, &p) == SPH_OK);
+    sph_destroy(e);
+    // No room for the spares, nor for the state to be saved.
+    CHECK(sph_create(&p, &e) == SPH_OK);
+    CHECK(sph_set_device_memory_limit(e, used - n * (9ull * 4 + 128 * 2 + 4) + 1000) == SPH_OK);
+    std::vector<float> x(3 * n, 0.1f);
+    CHECK(sph_set_particles(e, x.data(), nullptr, n) == SPH_OK && sph_make_ready(e) == SPH_OK);
+    const int other[5] = {128, 64, 256, 8, 4};
+    CHECK(sph_set_tuning(e, other) == SPH_OK);
+    CHECK(sph_autotune(e) == SPH_E_OOM);
+    CHECK(sph_set_device_memory_limit(e, 0) == SPH_OK);
+    CHECK(sph_make_ready(e) == SPH_OK);  // with its spares again
+    int cfg[5];
+    CHECK(sph_get_tuning(e, cfg) == SPH_OK && std::memcmp(cfg, other, sizeof(cfg)) == 0);
+    sph_destroy(e);
+    return 0;
+}
+
 struct Check {
     const char* name;
     int (*run)();
@@ -408,6 +433,7 @@ const Check kChecks[] = {
     {"tuning_round_trip", tuning_round_trip},
     {"autotune_times_the_radix_sort", autotune_times_the_radix_sort},
     {"autotune_compares_forms", autotune_compares_forms},
+    {"failed_autotune_changes_nothing", failed_autotune_changes_nothing},
 };
 
 }  // namespace
