@@ -215,8 +215,11 @@ int  sph_device_memory_used(const sph_handle* h, uint64_t* bytes);
 
 /* ---- measurement ---- */
 #define SPH_PASS_HASH      0   /* standalone cell hash (first step only)        */
-#define SPH_PASS_SORT      1   /* cell-start scan + sort of keys                */
-#define SPH_PASS_REORDER   2   /* gather of the state into sorted order         */
+#define SPH_PASS_SORT      1   /* cell-start scan + sort of keys; by cell counts
+                                  the gather of the state into sorted order too */
+#define SPH_PASS_REORDER   2   /* that gather after the radix sort; by cell counts
+                                  nothing runs here and the time is the events'
+                                  own, about 5 us                               */
 #define SPH_PASS_DENSITY   3   /* density, EOS, neighbour masks                 */
 #define SPH_PASS_FORCE     4   /* pressure + viscosity + integrate + clamp      */
 #define SPH_NUM_PASSES     5
