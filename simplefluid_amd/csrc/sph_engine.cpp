@@ -13,6 +13,7 @@
 using namespace sph;
 
 sph_handle::~sph_handle() {
+    sph::forget_spares(mem);
     if (copy_stream) (void)hipStreamSynchronize(copy_stream);
     if (snap_host) (void)hipHostFree(snap_host);
     if (snap_ready) (void)hipEventDestroy(snap_ready);
@@ -169,6 +170,37 @@ void give_back_spares(MemBudget& b) {
     h->nlist = nullptr;
 }
 
+// Budgets of the handles that may hold spares.  Whoever has this lock waits for
+// no handle's call: a handle in one is passed over.
+static std::mutex g_spares_mu;
+static std::vector<MemBudget*> g_spares;
+
+void remember_spares(MemBudget& b) {
+    (void)hipGetDevice(&b.device);
+    std::lock_guard<std::mutex> lk(g_spares_mu);
+    if (std::find(g_spares.begin(), g_spares.end(), &b) == g_spares.end()) g_spares.push_back(&b);
+}
+
+void forget_spares(MemBudget& b) {
+    std::lock_guard<std::mutex> lk(g_spares_mu);
+    g_spares.erase(std::remove(g_spares.begin(), g_spares.end(), &b), g_spares.end());
+}
+
+bool give_back_others(const MemBudget* b) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return false;
+    bool any = false;
+    std::lock_guard<std::mutex> lk(g_spares_mu);
+    for (MemBudget* o : g_spares) {
+        if (o == b || o->device != device) continue;
+        std::unique_lock<std::mutex> call(o->in_call, std::try_to_lock);
+        if (!call.owns_lock() || !o->spares) continue;
+        give_back_spares(*o);
+        any = true;
+    }
+    return any;
+}
+
 uint2* tiles_for(sph_handle* h, int block, uint32_t& ntiles) {
     auto it = h->tiles.find(block);
     if (it != h->tiles.end() && it->second.p) {
@@ -315,12 +347,13 @@ static int ensure_buffers(sph_handle* h) {
     static_assert(kListMax % 2 == 0, "lists of whole words");
     const size_t list_words = h->split_tiles <= kSplitTiles && !h->wide_rows ? (kListMax / 2 + 1) * n : 0;
     for (const size_t words : {list_words, (size_t)0}) {  // without the lists where only the masks fit
-        if (h->spare.ensure(words + (size_t)kRows * n) == hipSuccess) {
+        if (h->spare.ensure(words + (size_t)kRows * n, kSpare) == hipSuccess) {
             if (words) {
                 h->nlist = reinterpret_cast<uint16_t*>(h->spare.p);
                 h->ncount = h->spare.p + (kListMax / 2) * n;
             }
             h->mask_hi = h->spare.p ? h->spare.p + words : nullptr;
+            if (h->spare.p) remember_spares(h->mem);
             h->mem.spares = h->spare.p ? h : nullptr;
             break;
         }
@@ -735,7 +768,6 @@ int sph_create(const sph_params* p, sph_handle** out) {
 }
 
 void sph_destroy(sph_handle* h) {
-    BudgetScope budget_scope(h ? &h->mem : nullptr);
     if (!h) return;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     delete h;
@@ -1155,9 +1187,11 @@ int sph_batch_create(const sph_scene_desc* scenes, uint32_t nscenes, sph_handle*
     std::vector<uint32_t> ns(nscenes);
     for (uint32_t s = 0; s < nscenes; ++s) { ps[s] = scenes[s].params; ns[s] = scenes[s].num_particles; }
     h->batched = true;
-    BudgetScope budget_scope(&h->mem);
-    rc = configure(h, ps, ns);
-    if (rc == SPH_OK) rc = ensure_buffers(h);
+    {
+        BudgetScope budget_scope(&h->mem);
+        rc = configure(h, ps, ns);
+        if (rc == SPH_OK) rc = ensure_buffers(h);
+    }
     if (rc != SPH_OK) {
         const std::string msg = h->last_error;
         delete h;
@@ -1205,6 +1239,7 @@ int sph_set_scene_params(sph_handle* h, uint32_t scene, const sph_params* p) {
 // ---- device memory ----
 
 int sph_set_device_memory_limit(sph_handle* h, uint64_t bytes) {
+    BudgetScope budget_scope(h ? &h->mem : nullptr);
     if (!h) return SPH_E_INVALID;
     h->mem.limit = bytes;
     return SPH_OK;
@@ -1212,6 +1247,7 @@ int sph_set_device_memory_limit(sph_handle* h, uint64_t bytes) {
 
 int sph_device_memory_used(const sph_handle* h, uint64_t* bytes) {
     if (!h || !bytes) return SPH_E_INVALID;
+    BudgetScope budget_scope(const_cast<MemBudget*>(&h->mem));  // another handle's call may take the spares
     *bytes = h->mem.used;
     return SPH_OK;
 }
@@ -1252,6 +1288,7 @@ int sph_profile_read(sph_handle* h, double* ms, uint32_t* steps) {
 
 int sph_get_tuning(const sph_handle* h, int* cfg) {
     if (!h || !cfg) return SPH_E_INVALID;
+    BudgetScope budget_scope(const_cast<MemBudget*>(&h->mem));
     cfg[0] = h->tune.density_block;
     cfg[1] = h->tune.force_block;
     cfg[2] = h->tune.reorder_block;

@@ -3,6 +3,7 @@
 
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -17,12 +18,21 @@ struct MemBudget {
     uint64_t used = 0;
     uint64_t refused = 0;   // size of the last allocation the cap refused
     sph_handle* spares = nullptr;  // the handle, while it holds buffers it can do without
+    int device = 0;                // where they are
+    std::mutex in_call;            // held by the thread that is in a call on the handle
     bool over(uint64_t bytes) const { return limit && used + bytes > limit; }
 };
 
 // Frees the buffers that only speed the step up (and the graphs that name
 // them): an allocation that does not fit beside them takes their place.
 void give_back_spares(MemBudget& b);
+// The same for every other handle of this device that no thread is in a call
+// on; true if any had some.
+bool give_back_others(const MemBudget* b);
+// Lists a handle's budget among those that may hold spares, until it is
+// forgotten (before the handle goes).
+void remember_spares(MemBudget& b);
+void forget_spares(MemBudget& b);
 
 // The budget that buffers allocated on this thread are charged to: each C-ABI
 // entry point sets it to its handle's for the duration of the call (a handle
@@ -32,11 +42,18 @@ extern thread_local MemBudget* t_budget;
 
 struct BudgetScope {
     MemBudget* prev;
-    explicit BudgetScope(MemBudget* b) : prev(t_budget) { t_budget = b; }
+    std::unique_lock<std::mutex> call;  // not for a call within one on the same handle
+    explicit BudgetScope(MemBudget* b) : prev(t_budget) {
+        if (b && b != prev) call = std::unique_lock<std::mutex>(b->in_call);
+        t_budget = b;
+    }
     ~BudgetScope() { t_budget = prev; }
     BudgetScope(const BudgetScope&) = delete;
     BudgetScope& operator=(const BudgetScope&) = delete;
 };
+
+// Spare buffers do not take other handles' spares' place.
+enum BufNeed { kNeeded, kSpare };
 
 // Device buffer owned by the handle.
 template <class T>
@@ -57,7 +74,7 @@ struct DevBuf {
         count = 0;
         owner = nullptr;
     }
-    hipError_t ensure(size_t n) {
+    hipError_t ensure(size_t n, BufNeed need = kNeeded) {
         if (n <= count && p) return hipSuccess;
         release();
         if (n == 0) return hipSuccess;
@@ -72,6 +89,10 @@ struct DevBuf {
         if (e != hipSuccess && b && b->spares) {
             (void)hipGetLastError();
             give_back_spares(*b);
+            e = hipMalloc((void**)&p, bytes);
+        }
+        if (e != hipSuccess && need == kNeeded && give_back_others(b)) {
+            (void)hipGetLastError();
             e = hipMalloc((void**)&p, bytes);
         }
         if (e != hipSuccess) { p = nullptr; return e; }

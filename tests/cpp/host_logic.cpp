@@ -421,6 +421,36 @@ int failed_autotune_changes_nothing() {
     return 0;
 }
 
+// What a handle can do without makes room for another handle's buffers.
+int spares_make_room_for_others() {
+    sph_handle* a = make(30000);
+    CHECK(sph_advance_steps(a, 2) == SPH_OK);
+    fake::launched.clear();
+    CHECK(sph_advance_steps(a, 1) == SPH_OK && fake::count("graph") == 1);
+    uint64_t used = 0, after = 0;
+    CHECK(sph_device_memory_used(a, &used) == SPH_OK);
+    sph_handle* b = make(20000);
+    uint64_t need = 0;
+    CHECK(sph_device_memory_used(b, &need) == SPH_OK);
+    sph_destroy(b);
+    const uint64_t spares_a = 30000ull * (9 * 4 + 128 * 2 + 4), spares_b = 20000ull * (9 * 4 + 128 * 2 + 4);
+    // Room for all but a kilobyte of b's own buffers.
+    fake::device_left = need - spares_b - 1024;
+    b = make(20000);
+    CHECK(sph_device_memory_used(a, &after) == SPH_OK && after == used - spares_a);
+    fake::device_left = ~0ull >> 1;
+    fake::stale = false;
+    for (sph_handle* h : {a, b}) CHECK(sph_advance_steps(h, 2) == SPH_OK);
+    CHECK(!fake::stale);
+    // Spares alone take nothing from other handles.
+    CHECK(sph_make_ready(a) == SPH_OK && sph_device_memory_used(a, &after) == SPH_OK && after >= used);
+    fake::device_left = 0;
+    CHECK(sph_make_ready(b) == SPH_OK && sph_device_memory_used(a, &used) == SPH_OK && used == after);
+    sph_destroy(a);
+    sph_destroy(b);
+    return 0;
+}
+
 struct Check {
     const char* name;
     int (*run)();
@@ -434,6 +464,7 @@ const Check kChecks[] = {
     {"autotune_times_the_radix_sort", autotune_times_the_radix_sort},
     {"autotune_compares_forms", autotune_compares_forms},
     {"failed_autotune_changes_nothing", failed_autotune_changes_nothing},
+    {"spares_make_room_for_others", spares_make_room_for_others},
 };
 
 }  // namespace

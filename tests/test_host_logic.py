@@ -29,7 +29,8 @@ def exe(tmp_path_factory):
 @pytest.mark.parametrize("check", ["autotune_keeps_the_sort", "hash_without_its_table_fails",
                                    "new_spares_drop_the_graphs", "wide_rows_are_gathered",
                                    "tuning_round_trip", "autotune_times_the_radix_sort",
-                                   "autotune_compares_forms", "failed_autotune_changes_nothing"])
+                                   "autotune_compares_forms", "failed_autotune_changes_nothing",
+                                   "spares_make_room_for_others"])
 def test_host_logic(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
