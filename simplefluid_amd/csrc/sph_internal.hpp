@@ -96,7 +96,8 @@ struct StepArgs {
     uint32_t* queue;         // persistent launch: 8 tile counters (zeroed by the sort), else null
     uint32_t* vmax2;         // CFL: kSpeedSlots words of max |v|^2 (float bits) of the state the step starts
                              // from (density), of the new state (force), else null
-    SceneConst* cfl_scene;   // CFL: the scene whose dt the density pass sets from vmax2 (one scene), else null
+    SceneConst* cfl_scene;   // CFL: receives the scene (one) with the dt that the density pass finds from vmax2,
+                             // for the force pass to read, else null
     float* dt_out;           // CFL: receives that dt
     uint32_t* frame;         // device frame loop's state, else null
 };

@@ -11,6 +11,7 @@
 // two forms with the same results: candidates read from global memory, or
 // each row's candidates first copied by the wave into LDS ("staged").
 #include <atomic>
+#include <cstddef>
 
 #include "sph_internal.hpp"
 
@@ -576,17 +577,22 @@ __device__ __forceinline__ Moved force_one_staged(const StepArgs& a, const Scene
 // force pass: the sort has read the tile sums, which are cleared for the
 // integrate pass, and the CFL step is set (launches of their own cost 4-6 us
 // of a 40 us step each: 26k particles).  dt = min(dt_max, (cfl h) / (c0 +
-// |v|max)), in this op order; no density reads dt.  With a frame state, the
+// |v|max)), in this op order; it goes into the copy of the scene that the force
+// pass reads, since this pass's own blocks read the table.  With a frame state, the
 // step is added to the frame time (float, as the host frame loop adds it) and
 // a frame of at least 1/30 s marks pending.
 __device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
     if (a.cfl_scene && blockIdx.x == 0 && threadIdx.x < kSpeedSlots) {  // the first wave
         const uint32_t v2 = wave_umax(a.vmax2[threadIdx.x]);
         a.vmax2[threadIdx.x] = 0u;
+        const SceneConst sc = scene_at(a.scenes, 0u);
+        const float dt = fminf(sc.dt_max, (sc.cfl * sc.h) / (sc.c0 + sqrtf(__uint_as_float(v2))));
+        constexpr uint32_t kWords = sizeof(SceneConst) / 4u, kDt = offsetof(SceneConst, dt) / 4u;
+        static_assert(kWords <= kSpeedSlots, "a lane a word");
+        if (threadIdx.x < kWords)
+            reinterpret_cast<uint32_t*>(a.cfl_scene)[threadIdx.x] =
+                threadIdx.x == kDt ? __float_as_uint(dt) : reinterpret_cast<const uint32_t*>(a.scenes)[threadIdx.x];
         if (threadIdx.x == 0) {
-            SceneConst& sc = *a.cfl_scene;
-            const float dt = fminf(sc.dt_max, (sc.cfl * sc.h) / (sc.c0 + sqrtf(__uint_as_float(v2))));
-            sc.dt = dt;
             *a.dt_out = dt;
             if (a.frame) {
                 const float ft = __uint_as_float(a.frame[3]) + dt;
