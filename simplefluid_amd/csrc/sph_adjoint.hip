@@ -112,7 +112,7 @@ __device__ __forceinline__ void adj_integrate_one(const AdjArgs& a, const SceneC
     }
     a.xbar_o[k] = make_float4(xo[0], xo[1], xo[2], 0.0f);
     a.vbar_o[k] = make_float4(vo[0], vo[1], vo[2], 0.0f);
-    a.abar[k] = make_float4(ab[0], ab[1], ab[2], pw);
+    a.abar[k] = make_float4(sc.scale_a * ab[0], sc.scale_a * ab[1], sc.scale_a * ab[2], sc.scale_a * pw);
 }
 
 // The last step of a segment (the others' is done by the density pass of the
@@ -133,8 +133,10 @@ __global__ void adj_integrate_kernel(AdjArgs a) {
 }
 
 // Per-particle sums of the adjoint force pass, without their constant factors
-// (adj_force_finish applies those): g without cP, h without -cV q_i, Pb
-// without cP, qb without cV.
+// (adj_finish_* apply those): g without cP, h without -cV q_i, Pb without cP,
+// qb without cV; these four by scale_a, as abar is in memory.  Without the
+// scale, seeds whose gradients were far inside the float range lost bits of
+// their pairs' terms at its end (h = 0.0056, seeds of 1e-23: 1e-5).
 struct AdjForceAcc {
     float gx, gy, gz, hx, hy, hz, Pb, qb, Ax, Ay, Az;
 };
@@ -195,24 +197,25 @@ __device__ __forceinline__ float visc_ratio(const SceneConst& sc, const float4& 
 
 // The sums' ends: the position adjoint ...
 __device__ __forceinline__ float4 adj_finish_x(const SceneConst& sc, float4 xs, float gx, float gy, float gz) {
-    xs.x = fmaf(sc.cP, gx, xs.x); xs.y = fmaf(sc.cP, gy, xs.y); xs.z = fmaf(sc.cP, gz, xs.z);
+    const float c = sc.cP * sc.unscale_a;
+    xs.x = fmaf(c, gx, xs.x); xs.y = fmaf(c, gy, xs.y); xs.z = fmaf(c, gz, xs.z);
     return xs;
 }
 // ... the velocity adjoint, ...
 __device__ __forceinline__ float4 adj_finish_v(const SceneConst& sc, float4 vs, float qi, float hx, float hy, float hz) {
-    const float cvq = sc.cV * qi;
+    const float cvq = sc.cV * qi * sc.unscale_a;
     vs.x = fmaf(-cvq, hx, vs.x); vs.y = fmaf(-cvq, hy, vs.y); vs.z = fmaf(-cvq, hz, vs.z);
     return vs;
 }
 // ... the dL/dmu term, ...
 __device__ __forceinline__ float adj_finish_mu(const SceneConst& sc, float qi, const float4& abi, float Ax, float Ay,
                                                float Az) {
-    return sc.cP * qi * (abi.x * Ax + abi.y * Ay + abi.z * Az);
+    return sc.cP * qi * (abi.x * Ax + abi.y * Ay + abi.z * Az) * sc.unscale_a;
 }
-// ... and the EOS reverse: the density adjoint and the dL/dB term.
+// ... and the EOS reverse: the density adjoint (by scale_r) and the dL/dB term.
 __device__ __forceinline__ float adj_finish_rho(const SceneConst& sc, float rho, float qi, const float4& abi, float Pbs,
                                                 float qbs, float& rhobar) {
-    const float Pb = fmaf(sc.cP, Pbs, abi.w), qb = sc.cV * qbs;
+    const float Pb = fmaf(sc.cP * sc.unscale_a, Pbs, abi.w * sc.unscale_a), qb = sc.cV * sc.unscale_a * qbs;
     // EOS derivatives (clamped Tait, exponent 7).
     const float x = rho * sc.inv_rho0;
     const float x2 = x * x, x4 = x2 * x2, x6 = x4 * x2, x7 = x6 * x;
@@ -221,7 +224,7 @@ __device__ __forceinline__ float adj_finish_rho(const SceneConst& sc, float rho,
     const float p = praw * sgn;
     const float dp_drho = sgn * sc.B * 7.0f * x6 * sc.inv_rho0;
     const float dp_dB = sgn * (x7 - 1.0f);
-    rhobar = Pb * (dp_drho * qi * qi - 2.0f * p * qi * qi * qi) - qb * qi * qi;
+    rhobar = sc.scale_r * (Pb * (dp_drho * qi * qi - 2.0f * p * qi * qi * qi) - qb * qi * qi);
     return Pb * qi * qi * dp_dB;
 }
 
@@ -433,7 +436,7 @@ __device__ __forceinline__ float adj_density_factor(const SceneConst& sc, float 
     return (tt * tt) * (rbi + rbj);
 }
 // One neighbour's term of the adjoint density pass, without its factor -6 cD
-// (adj_density_finish applies it).
+// (adj_scatter applies it), by scale_r as the density adjoint is.
 __device__ __forceinline__ void adj_density_pair(const SceneConst& sc, const float4& pi, float rbi, const float4& pj,
                                                  float rbj, float& gx, float& gy, float& gz) {
     const float rx = pi.x - pj.x, ry = pi.y - pj.y, rz = pi.z - pj.z;
@@ -470,12 +473,12 @@ __device__ __forceinline__ void adj_density_walls(const SceneConst& sc, const fl
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const float ul = (pk[d] - sc.bmin[d]) * sc.inv_h, uh = (sc.wmax[d] - pk[d]) * sc.inv_h;
-        gw[d] = (rbi * sc.rho0) * (sc.inv_h * (wall_rho_du(ul) - wall_rho_du(uh)));
+        gw[d] = (rbi * sc.unscale_r * sc.rho0) * (sc.inv_h * (wall_rho_du(ul) - wall_rho_du(uh)));
     }
 }
 __device__ __forceinline__ void adj_scatter(const AdjArgs& a, const SceneConst& sc, AdjMove& m, float gx, float gy,
                                             float gz, const float gw[3], const float wj[3], const float wd[3]) {
-    const float cg = -6.0f * sc.cD;
+    const float cg = -6.0f * sc.cD * sc.unscale_r;
     m.xs.x += fmaf(cg, gx, gw[0]);
     m.xs.y += fmaf(cg, gy, gw[1]);
     m.xs.z += fmaf(cg, gz, gw[2]);

@@ -60,7 +60,10 @@ struct SceneConst {
     float inv_h;       // 1 / h
     float cW;          // 2 * 45 rho0 / h: the walls' pressure term
     float wmax[3];     // box_max (box_min is bmin)
-    uint32_t pad[4];
+    float scale_a;     // powers of two that the reverse pass keeps the acceleration's and the density's
+    float unscale_a;   // adjoint by, and their inverses: the pairs' terms leave the constant factors of their
+    float scale_r;     // sums out (up to 10^16), and so lie as far inside the float range as with them
+    float unscale_r;
 };
 static_assert(sizeof(SceneConst) == 192, "SceneConst layout");
 

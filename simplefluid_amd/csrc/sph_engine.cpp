@@ -111,6 +111,16 @@ int derive_scene_core(const sph_params& p, SceneConst& sc, const char** err, int
     sc.rho0 = p.rest_density;
     sc.inv_h = (float)(1.0 / (double)p.kernel_radius);
     sc.cW = (float)(90.0 * (double)p.rest_density / (double)p.kernel_radius);
+    // Largest powers of two up to the sizes of the pairs' factors, cP h^2 and 6 cD h^4.
+    auto scales = [](double size, float& up, float& down) {
+        int e = 0;
+        if (std::isfinite(size) && size > 0.0) (void)std::frexp(size, &e);
+        e = std::min(std::max(e - 1, -100), 100);
+        up = std::ldexp(1.0f, e);
+        down = std::ldexp(1.0f, -e);
+    };
+    scales((double)sc.cP * sc.h2, sc.scale_a, sc.unscale_a);
+    scales(6.0 * (double)sc.cD * sc.h2 * sc.h2, sc.scale_r, sc.unscale_r);
     uint64_t cells = 1;
     for (int k = 0; k < 3; ++k) {
         sc.g[k] = p.gravity[k];
