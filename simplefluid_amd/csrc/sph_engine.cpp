@@ -22,7 +22,8 @@ sph_handle::~sph_handle() {
     if (host_pinned) (void)hipHostFree(host_pinned);
     sph::invalidate_graph(this);
     for (auto e : prof_events) (void)hipEventDestroy(e);
-    for (auto e : copy_events) (void)hipEventDestroy(e);
+    for (auto e : copy_events)
+        if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -188,7 +189,11 @@ static std::vector<MemBudget*> g_spares;
 void remember_spares(MemBudget& b) {
     (void)hipGetDevice(&b.device);
     std::lock_guard<std::mutex> lk(g_spares_mu);
-    if (std::find(g_spares.begin(), g_spares.end(), &b) == g_spares.end()) g_spares.push_back(&b);
+    if (std::find(g_spares.begin(), g_spares.end(), &b) != g_spares.end()) return;
+    try {
+        g_spares.push_back(&b);
+    } catch (...) {  // not listed: this handle keeps its spares
+    }
 }
 
 void forget_spares(MemBudget& b) {
@@ -576,15 +581,17 @@ static int download(sph_handle* h, const void* src, size_t words, Use&& use) {
     constexpr size_t kPiece = (size_t)1 << 18;  // words: 1 MB
     constexpr int kThreads = 4;
     const size_t pieces = (words + kPiece - 1) / kPiece;
-    while (h->copy_events.size() < (size_t)kThreads * 2) {
-        hipEvent_t ev;
+    for (hipEvent_t& ev : h->copy_events) {
+        if (ev) continue;
         const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-        if (e != hipSuccess) return hip_fail(h, e, "download event");
-        h->copy_events.push_back(ev);
+        if (e != hipSuccess) {
+            ev = nullptr;
+            return hip_fail(h, e, "download event");
+        }
     }
     // Events mark up to eight points of the copy; each piece's launch writes
     // the flag behind it, where the next piece's words then go.
-    const size_t marks = std::min(pieces, h->copy_events.size());
+    const size_t marks = std::min(pieces, (size_t)sph_handle::kCopyEvents);
     auto mark_end = [&](size_t m) { return std::min(words, (m + 1) * pieces / marks * kPiece); };
     // The flag alone first: nothing is handed over where it is raised.
     hipError_t e = launch_copy_out(h->stream, nullptr, 0, h->err.p, reinterpret_cast<uint32_t*>(h->host_pinned) + words);

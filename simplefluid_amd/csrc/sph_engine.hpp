@@ -207,7 +207,8 @@ struct sph_handle {
     sph::DevBuf<float> staging;
     float* host_pinned = nullptr;          // page-locked host memory for downloads, one word longer than
     size_t host_pinned_n = 0;              // host_pinned_n
-    std::vector<hipEvent_t> copy_events;   // points of a large download
+    static constexpr int kCopyEvents = 8;
+    hipEvent_t copy_events[kCopyEvents] = {};  // points of a large download
     // Asynchronous frame snapshot: positions un-permuted on the step stream
     // into snap_d, copied to snap_host on copy_stream while steps continue.
     hipStream_t copy_stream = nullptr;
