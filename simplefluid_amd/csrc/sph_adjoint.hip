@@ -25,9 +25,10 @@
 //   adj_force      starts Pbar_i from it (the term involves particle i alone)
 //   adj_density:   xbar_i,d += rhobar_i rho0 (wall_rho'(u_lo) - wall_rho'(u_hi)) / h
 // Each kernel reads neighbour values written by the previous kernel only.
-// adj_force and adj_density come in two forms with identical results: the
-// neighbours' records gathered from global memory, or each row's candidates
-// staged in LDS by the wave first (the forward passes' staged form).
+// adj_force and adj_density come in three forms with identical results: the
+// neighbours' records gathered from global memory, each row's candidates
+// staged in LDS by the wave first, or split over several waves (as the forward
+// passes).
 #include "sph_internal.hpp"
 
 namespace sph {
@@ -394,7 +395,7 @@ __device__ __forceinline__ void add_tile_terms(const AdjArgs& a, uint32_t t, dou
     __syncthreads();
 }
 
-// Eight waves per SIMD (64 VGPRs, a 36-byte spill): the backward pass was
+// Eight waves per SIMD (64 VGPRs, three spilled): the backward pass was
 // 3 % faster than without the bound (47.0 against 48.3 ms, 16 x 32k
 // particles x 200 steps, with the walls' reverse still in this kernel).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void adj_force_kernel(AdjArgs a) {
@@ -499,7 +500,7 @@ __device__ __forceinline__ void adj_density_finish(const AdjArgs& a, const Scene
 }
 
 // adj_density_kernel with the rows staged in LDS (1.9 KB per wave).
-// Eight waves per SIMD: the bound fits it in 64 VGPRs.
+// Eight waves per SIMD: the bound fits it in 64 VGPRs (25 SGPRs in lanes).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void adj_density_staged_kernel(AdjArgs a) {
     uint32_t t0, t1;
     tile_span(a.ntiles, t0, t1);

@@ -378,14 +378,6 @@ __device__ __forceinline__ float4 load4(__amdgpu_buffer_rsrc_t r, uint32_t byte_
     return f;
 }
 
-__device__ __forceinline__ float2 load2(__amdgpu_buffer_rsrc_t r, uint32_t byte_off) {
-    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)byte_off, 0, 0);
-    float2 f;
-    f.x = __uint_as_float(v.x);
-    f.y = __uint_as_float(v.y);
-    return f;
-}
-
 __device__ __forceinline__ uint32_t cell_key(const SceneConst& sc, float x, float y, float z) {
     const int cx = cell_coord(x, sc.bmin[0], sc.inv_csx, sc.G[0]);
     const int cy = cell_coord(y, sc.bmin[1], sc.inv_cs, sc.G[1]);

@@ -611,7 +611,7 @@ static int download(sph_handle* h, const void* src, size_t words, Use&& use) {
     }
     std::atomic<int> bad{0};
     auto work = [&](size_t first) {
-        (void)hipSetDevice(device);  // a new thread starts on the first one
+        (void)hipSetDevice(device);  // the caller's: a new thread starts on the first one
         for (size_t m = first; m < marks; m += kThreads) {
             if (hipEventSynchronize(h->copy_events[m]) != hipSuccess) {
                 bad.store(1);
@@ -946,8 +946,8 @@ int sph_advance_steps(sph_handle* h, uint32_t k) {
     if (!h) return SPH_E_INVALID;
     if (!h->ready) return fail(h, SPH_E_NOT_READY, "call sph_make_ready first");
     for (uint32_t i = 0; i < k;) {
-        // The graphs hold steady-state steps: keys from the last integrate,
-        // a cell table to clear sparsely.  Earlier steps run eagerly.
+        // The graphs hold steady-state steps, which take their keys from the
+        // last one's integration.  Earlier steps run eagerly.
         const bool steady = h->keys_valid && !h->keep_acc;
         if (h->use_graph && steady && !h->prof) {
             const bool multi = k - i >= kGraphSteps;

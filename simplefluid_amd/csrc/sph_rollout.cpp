@@ -3,7 +3,7 @@
 // runs the hand-written adjoint kernels over it (sph_adjoint.hip).
 //
 // Memory: (steps/every + 1) state checkpoints of 36 B per particle, plus
-// `every` taped steps of ~116 B per particle and 8 B per cell.
+// `every` taped steps of 112 B per particle and 4 B per cell.
 #include <algorithm>
 #include <cstring>
 

@@ -7,9 +7,10 @@
 // Neighbour order is canonical: rows (dz, dy) = (-1..1, -1..1), dz outer; a
 // row is the contiguous sorted range of the x cells inside the support
 // sphere's chord at that row; ascending index.  Density sums and force sums
-// run in that order, one particle per lane.  Density and force each come in
-// two forms with the same results: candidates read from global memory, or
-// each row's candidates first copied by the wave into LDS ("staged").
+// run in that order.  Density and force each come in three forms with the same
+// results: candidates read from global memory ("gathered"), each row's
+// candidates first copied by the wave into LDS ("staged"), both one particle
+// per lane, or several waves to 64 particles ("split").
 #include <atomic>
 #include <cstddef>
 
@@ -637,7 +638,7 @@ __global__ __launch_bounds__(BLOCK) void density_kernel(StepArgs a) {
 }
 
 // density_kernel with the rows staged in LDS (1.5 KB per wave).  Eight
-// waves per SIMD: the bound fits it in 59 VGPRs without spills (65 without).
+// waves per SIMD: the bound fits it in 56 VGPRs (33 SGPRs in lanes of others).
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8, 8))) void density_staged_kernel(StepArgs a) {
     if (a.frame && a.frame[0]) return;
