@@ -278,7 +278,7 @@ StepArgs step_args(sph_handle* h, StepBufs& w, int block) {
     a.scenes = h->sc_d.p;
     if (h->cfl) {
         a.vmax2 = h->vmax2.p;
-        a.cfl_scene = h->sc_cfl.p;
+        a.cfl_scene = h->sc_d.p + h->sc_h.size();
         a.dt_out = h->dt_dev.p;
     }
     a.tiles = tiles_for(h, block, a.ntiles);
@@ -340,10 +340,9 @@ static int ensure_buffers(sph_handle* h) {
     chk(h->queue.ensure(kQueueWords));
     chk(h->vmax2.ensure(kSpeedSlots));
     chk(h->dt_dev.ensure(1));
-    chk(h->sc_cfl.ensure(1));
     chk(h->frame.ensure(kFrameWords));
     chk(h->staging.ensure(3 * n + 1));
-    chk(h->sc_d.ensure(h->sc_h.size()));
+    chk(h->sc_d.ensure(h->sc_h.size() + 1));
     if (e != hipSuccess) return hip_fail(h, e, "device allocation");
     chk(launch_fill_u32(h->stream, h->hist.p, 0u, kMaxPasses * 256));
     chk(launch_fill_u32(h->stream, h->err.p, 0u, 1));
@@ -479,13 +478,13 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     if (split) {
         StepArgs a = step_args(h, w, kSplitTile);
         a.frame = frame;
-        if (h->cfl) a.scenes = h->sc_cfl.p;
+        if (h->cfl) a.scenes = a.cfl_scene;
         e = launch_force_split(st, a);
         if (e != hipSuccess) return hip_fail(h, e, "force launch");
     } else {
         StepArgs a = step_args(h, w, h->tune.force_block);
         a.frame = frame;
-        if (h->cfl) a.scenes = h->sc_cfl.p;
+        if (h->cfl) a.scenes = a.cfl_scene;
         const uint32_t grid = grid_for(h, h->tune.force_block, a.ntiles, &a.queue,
                                        force_blocks_per_cu(h->tune.force_block, force_staged(h)));
         e = launch_force(st, h->tune.force_block, grid, a, force_staged(h));

@@ -200,8 +200,8 @@ struct sph_handle {
     bool cfl = false;                      // adaptive step (single scene)
     sph::DevBuf<uint32_t> vmax2;           // max |v|^2 bits for the next step (kSpeedSlots words)
     sph::DevBuf<float> dt_dev;             // step length of the last step (scene 0)
-    sph::DevBuf<sph::SceneConst> sc_d;
-    sph::DevBuf<sph::SceneConst> sc_cfl;   // scene 0 with the step's length, written by the density pass
+    sph::DevBuf<sph::SceneConst> sc_d;     // behind the scenes, CFL: scene 0 with the step's length, written by
+                                           // the density pass
     std::map<int, sph::DevBuf<uint2>> tiles;
     std::map<int, uint32_t> ntiles;
     sph::DevBuf<float> staging;

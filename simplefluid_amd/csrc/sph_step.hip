@@ -584,15 +584,15 @@ __device__ __forceinline__ Moved force_one_staged(const StepArgs& a, const Scene
 // a frame of at least 1/30 s marks pending.
 __device__ __forceinline__ void step_bookkeeping(const StepArgs& a) {
     if (a.cfl_scene && blockIdx.x == 0 && threadIdx.x < kSpeedSlots) {  // the first wave
+        constexpr uint32_t kWords = sizeof(SceneConst) / 4u, kDt = offsetof(SceneConst, dt) / 4u;
+        static_assert(kWords <= kSpeedSlots, "a lane a word");
+        const uint32_t word = reinterpret_cast<const uint32_t*>(a.scenes)[min(threadIdx.x, kWords - 1u)];
         const uint32_t v2 = wave_umax(a.vmax2[threadIdx.x]);
         a.vmax2[threadIdx.x] = 0u;
         const SceneConst sc = scene_at(a.scenes, 0u);
         const float dt = fminf(sc.dt_max, (sc.cfl * sc.h) / (sc.c0 + sqrtf(__uint_as_float(v2))));
-        constexpr uint32_t kWords = sizeof(SceneConst) / 4u, kDt = offsetof(SceneConst, dt) / 4u;
-        static_assert(kWords <= kSpeedSlots, "a lane a word");
         if (threadIdx.x < kWords)
-            reinterpret_cast<uint32_t*>(a.cfl_scene)[threadIdx.x] =
-                threadIdx.x == kDt ? __float_as_uint(dt) : reinterpret_cast<const uint32_t*>(a.scenes)[threadIdx.x];
+            reinterpret_cast<uint32_t*>(a.cfl_scene)[threadIdx.x] = threadIdx.x == kDt ? __float_as_uint(dt) : word;
         if (threadIdx.x == 0) {
             *a.dt_out = dt;
             if (a.frame) {
