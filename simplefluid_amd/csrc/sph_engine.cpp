@@ -415,7 +415,7 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
     const uint8_t hashed = h->keys_valid ? 0 : 1;
     // Tile tables first: their allocation may give the spares back, and the
     // step's form and both its passes have to see the same ones.
-    for (int b : {h->tune.density_block, h->tune.force_block, kSplitTile}) {
+    for (int b : {density_block(h), force_block(h), kSplitTile}) {
         uint32_t nt = 0;
         if (!tiles_for(h, b, nt)) return fail(h, SPH_E_OOM, "tile table");
     }
@@ -468,10 +468,10 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
         e = launch_density_split(st, a);
         if (e != hipSuccess) return hip_fail(h, e, "density launch");
     } else {
-        StepArgs a = step_args(h, w, h->tune.density_block);
+        StepArgs a = step_args(h, w, density_block(h));
         a.frame = frame;
-        const uint32_t grid = grid_for(h, h->tune.density_block, a.ntiles, &a.queue);
-        e = launch_density(st, h->tune.density_block, grid, a, density_staged(h));
+        const uint32_t grid = grid_for(h, density_block(h), a.ntiles, &a.queue);
+        e = launch_density(st, density_block(h), grid, a, density_staged(h));
         if (e != hipSuccess) return hip_fail(h, e, "density launch");
     }
     if (record_prof) prof_record(h, 4);
@@ -482,12 +482,12 @@ int enqueue_step(sph_handle* h, StepBufs& w, bool record_prof, uint32_t* frame) 
         e = launch_force_split(st, a);
         if (e != hipSuccess) return hip_fail(h, e, "force launch");
     } else {
-        StepArgs a = step_args(h, w, h->tune.force_block);
+        StepArgs a = step_args(h, w, force_block(h));
         a.frame = frame;
         if (h->cfl) a.scenes = a.cfl_scene;
-        const uint32_t grid = grid_for(h, h->tune.force_block, a.ntiles, &a.queue,
-                                       force_blocks_per_cu(h->tune.force_block, force_staged(h)));
-        e = launch_force(st, h->tune.force_block, grid, a, force_staged(h));
+        const uint32_t grid = grid_for(h, force_block(h), a.ntiles, &a.queue,
+                                       force_blocks_per_cu(force_block(h), force_staged(h)));
+        e = launch_force(st, force_block(h), grid, a, force_staged(h));
         if (e != hipSuccess) return hip_fail(h, e, "force launch");
     }
     if (record_prof) {
@@ -898,12 +898,12 @@ static int capture_graph(sph_handle* h, GraphKind kind = kGraphOne) {
     // Tile tables are built on first use with a synchronous copy, which a
     // capturing stream does not allow: build the ones the step uses first
     // (a block size set after steps have run has none yet).
-    const int blocks[] = {h->tune.density_block, h->tune.force_block, kSplitTile};
+    const int blocks[] = {density_block(h), force_block(h), kSplitTile};
     for (int b : blocks) {
         uint32_t nt = 0;
         if (!tiles_for(h, b, nt)) return fail(h, SPH_E_OOM, "tile table");
     }
-    (void)force_blocks_per_cu(h->tune.force_block, force_staged(h));  // runtime query, outside capture
+    (void)force_blocks_per_cu(force_block(h), force_staged(h));  // runtime query, outside capture
     hipError_t e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(h, e, "begin capture");
     int rc = SPH_OK;
@@ -1308,8 +1308,8 @@ int sph_profile_read(sph_handle* h, double* ms, uint32_t* steps) {
 int sph_get_tuning(const sph_handle* h, int* cfg) {
     if (!h || !cfg) return SPH_E_INVALID;
     BudgetScope budget_scope(const_cast<MemBudget*>(&h->mem));
-    cfg[0] = h->tune.density_block;
-    cfg[1] = h->tune.force_block;
+    cfg[0] = density_block(h);
+    cfg[1] = force_block(h);
     cfg[2] = h->tune.reorder_block;
     cfg[3] = h->tune.sort_items;
     // What runs, whether asked for or picked by the handle's size.

@@ -277,11 +277,11 @@ bool split_form(const sph_handle* h);
 // Particles of fluid at rest in a cube of the support radius's side up to
 // which a row's candidates fit a wave's copy (64 + twice as many are 124 of
 // 120) and a particle's neighbours its list (4 pi / 3 times as many are 126 of
-// 128).  Measured per step, gathered against the form of the handle's size, at
-// a support of 6, 7, 8 and 12 particle radii (27, 43, 64 and 216 in the cube):
-// 31,713 particles 78 / 64, 185 / 195, 244 / 267, 1,022 / 1,020 us; 216,000
-// 146 / 144, 296 / 349, 396 / 528, 1,497 / 1,802; 1M 499 / 470, 1,063 / 1,170,
-// 1,525 / 1,910 (at 8).
+// 128).  Measured per step, gathered (in blocks of 256) against the form of
+// the handle's size, at a support of 6, 7, 8 and 12 particle radii (27, 43, 64
+// and 216 in the cube): 31,713 particles 78 / 64, 185 / 195, 244 / 267, 1,022 /
+// 1,020 us; 216,000 146 / 144, 296 / 349, 396 / 528, 1,497 / 1,802; 1M 499 /
+// 470, 1,063 / 1,170, 1,525 / 1,910 (at 8).
 constexpr float kWideRows = 30.0f;
 // Particles from which a handle no one has tuned stages density and force.
 // Below, a wave's copies and bounds cost more than its gathers, whose records
@@ -292,6 +292,13 @@ constexpr float kWideRows = 30.0f;
 // 186.7 / 238.0, 1M 216.8 / 322.8 against 167.0 / 233.2.
 constexpr uint32_t kStagedFrom = 1u << 17;
 inline int staged_by_size(const sph_handle* h) { return h->n >= kStagedFrom && !h->wide_rows; }
+// Blocks of the two passes.  Wide rows come in blocks of a wave, which spread
+// over more CUs (support of 8 radii, blocks of 256 and of 64: 7,220 particles
+// 251 / 224 us a step, 216,000 396 / 360; the split form 237 and 528).
+inline int density_block(const sph_handle* h) {
+    return h->tune.by_size && h->wide_rows ? 64 : h->tune.density_block;
+}
+inline int force_block(const sph_handle* h) { return h->tune.by_size && h->wide_rows ? 64 : h->tune.force_block; }
 inline int force_staged(const sph_handle* h) {
     return h->tune.by_size ? staged_by_size(h) : h->tune.force_staged;
 }

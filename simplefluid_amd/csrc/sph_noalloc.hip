@@ -28,7 +28,6 @@ namespace {
 constexpr uint32_t kMaxParticles = 65536;
 constexpr uint32_t kMaxCells = 1u << 20;
 constexpr uint32_t kMaxTiles = kMaxParticles / kSplitTile;
-constexpr uint32_t kBlock = 256;  // tiles of the gathered form
 constexpr uint32_t kScanTilesMax = 2048;
 static_assert(scan_tiles(kMaxCells, tile_shift_for(kMaxCells)) <= kScanTilesMax &&
                   scan_tiles(1u << 19, tile_shift_for(1u << 19)) <= kScanTilesMax && kMaxParticles / 64 < kScanTilesMax,
@@ -74,10 +73,10 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 void* g_scratch[kMaxDevices] = {};
 
-// Scene constants, the tile table (scene 0, first particle t * block), empty
+// Scene constants, the tile table (scene 0, first particle t * kSplitTile, in
+// every form: a wave's tiles spread over more CUs than larger ones), empty
 // chains, tile sums and tile prefixes, and the error word cleared.
-__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint32_t tile_shift, uint32_t block,
-                                     uint8_t* __restrict__ base) {
+__global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint32_t tile_shift, uint8_t* __restrict__ base) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
     if (i == 0) {
         *reinterpret_cast<SceneConst*>(base + Layout::scene) = sc;
@@ -91,7 +90,7 @@ __global__ void noalloc_setup_kernel(SceneConst sc, uint32_t ncells, uint32_t ti
     uint32_t* tile_pre = reinterpret_cast<uint32_t*>(base + Layout::tile_pre);
     for (uint32_t t = i; t < T; t += stride) tile_pre[t] = 0xffffffffu;
     uint2* tiles = reinterpret_cast<uint2*>(base + Layout::tiles);
-    for (uint32_t t = i; t * block < sc.p_end; t += stride) tiles[t] = make_uint2(0u, t * block);
+    for (uint32_t t = i; t * kSplitTile < sc.p_end; t += stride) tiles[t] = make_uint2(0u, t * kSplitTile);
 }
 
 // The scratch address on the current device, looked up once per device.
@@ -163,10 +162,9 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
 
     // The form a handle of so many particles and such rows takes.
     const bool split = (n + kSplitTile - 1) / kSplitTile <= kSplitTiles && !(cell_members(*p, 1) > kWideRows);
-    const uint32_t block = split ? (uint32_t)kSplitTile : kBlock;
     // Five launches: setup, upload and hash, sort, density, force (which
     // writes the caller's arrays itself).
-    hipLaunchKernelGGL(noalloc_setup_kernel, dim3(256), dim3(256), 0, st, sc, C, shift, block, base);
+    hipLaunchKernelGGL(noalloc_setup_kernel, dim3(256), dim3(256), 0, st, sc, C, shift, base);
     e = hipGetLastError();
     if (e == hipSuccess) e = launch_upload_hash(st, xyz_in, vel_in, pos, vel, id, key0, next, head, n, C, shift, sc);
     SortPlan sp;
@@ -209,11 +207,11 @@ extern "C" int sph_step_noalloc(const sph_params* p, const float* xyz_in, const 
     }
     a.scenes = scd;
     a.tiles = reinterpret_cast<const uint2*>(at(Layout::tiles));
-    a.ntiles = (n + block - 1) / block;
+    a.ntiles = (n + kSplitTile - 1) / kSplitTile;
     a.n = n;
     a.ncells = C;
-    if (e == hipSuccess) e = split ? launch_density_split(st, a) : launch_density(st, (int)block, a.ntiles, a);
-    if (e == hipSuccess) e = split ? launch_force_split(st, a) : launch_force(st, (int)block, a.ntiles, a);
+    if (e == hipSuccess) e = split ? launch_density_split(st, a) : launch_density(st, kSplitTile, a.ntiles, a);
+    if (e == hipSuccess) e = split ? launch_force_split(st, a) : launch_force(st, kSplitTile, a.ntiles, a);
     if (e != hipSuccess) return fail_noalloc(SPH_E_HIP, "sph_step_noalloc: kernel launch failed");
     return SPH_OK;
 }
