@@ -187,7 +187,13 @@ int sph_rollout_backward(sph_handle* h, const float* dL_dx_final, float* dL_dB, 
                 chk(launch_adj_density_split(st, a));
             } else {
                 chk(launch_adj_force(st, 256, grid, a, force_staged(h)));
-                chk(launch_adj_density(st, 256, grid, a, force_staged(h)));
+                if (h->wide_rows && !force_staged(h)) {  // blocks of a wave, as the forward passes
+                    a.tiles = split_tiles;
+                    a.ntiles = n_split;
+                    chk(launch_adj_density(st, kSplitTile, n_split, a, 0));
+                } else {
+                    chk(launch_adj_density(st, 256, grid, a, force_staged(h)));
+                }
             }
             swap();
             if (e != hipSuccess) return hip_fail(h, e, "adjoint launch");
