@@ -187,8 +187,8 @@ static std::mutex g_spares_mu;
 static std::vector<MemBudget*> g_spares;
 
 void remember_spares(MemBudget& b) {
-    (void)hipGetDevice(&b.device);
     std::lock_guard<std::mutex> lk(g_spares_mu);
+    (void)hipGetDevice(&b.device);
     if (std::find(g_spares.begin(), g_spares.end(), &b) != g_spares.end()) return;
     try {
         g_spares.push_back(&b);
